@@ -22,14 +22,14 @@ The default run also measures, each in a block of its own under "configs":
       precision, learned parameters, beside the fallback ncrit 64 / theta 0.4.
   c1_cartesian  c1 in the Cartesian Taylor basis (ExaFMM's
       LaplaceCartesianCPU.cxx; FP64 expansions, the M2L through the FP64
-      tile kernel between exact basis changes).
+      set kernel between exact basis changes).
       --cart-m2l 1: the direct Cartesian M2L kernel instead.
 --only-headline skips them; --batch K / --dist / --n measure one workload
 (--basis cartesian: in the Cartesian basis).
 
 roofline: the P2P kernel (20 flops per evaluated body pair against the FP32
 vector peak; the FP64 kernel against the FP64 vector peak), timed by HIP
-events on the stream it runs on; the M2L tile kernel is reported beside it.
+events on the stream it runs on; the M2L set kernel is reported beside it.
 """
 import argparse
 import json
@@ -77,11 +77,11 @@ def parse():
     ap.add_argument("--config-steps", type=int, default=5,
                     help="timed steps of each c1 / c3 / c4 block")
     ap.add_argument("--no-autotune", action="store_true",
-                    help="keep the default tile-kernel knobs instead of autotuning them")
+                    help="keep the default set-kernel knobs instead of autotuning them")
     ap.add_argument("--unit-factor", type=float, default=None,
-                    help="M2L work-unit size in mean items per tile (0: one unit per tile)")
+                    help="M2L work-unit size in mean items per target set (0: automatic)")
     ap.add_argument("--xcd-run", type=int, default=None,
-                    help="M2L work units dealt to one XCD in a row")
+                    help="groups of 8 M2L work units dealt to one XCD in a row")
     ap.add_argument("--p2p-schedule", type=int, default=None, choices=[0, 1, 2, 3, 4],
                     help="0: P2P from the numeric phase's start, 1: beside the M2L tiles, "
                          "2: from phase A, beside the M2L batch building, 3: as 2, drained "
@@ -94,7 +94,7 @@ def parse():
     ap.add_argument("--basis", default="spherical", choices=["spherical", "cartesian"],
                     help="expansion basis of a single-workload run")
     ap.add_argument("--cart-m2l", type=int, default=0, choices=[0, 1],
-                    help="route of the Cartesian M2L: 0 the FP64 tile kernel between basis "
+                    help="route of the Cartesian M2L: 0 the FP64 set kernel between basis "
                          "changes, 1 the direct Cartesian kernel")
     ap.add_argument("--calibrate-copy", action="store_true",
                     help="only copy a 256 MiB device buffer three times (the reference kernel "
@@ -279,7 +279,7 @@ def errors(ctx, targets, direct):
 def kernels(st, phases, precision, workload, basis="spherical", cart_direct=False,
             resident=False):
     """Achieved rates of the P2P kernel (20 flops per evaluated body pair)
-    and the M2L tile kernel (9,680 flops per grouped pair; the Cartesian
+    and the M2L set kernel (9,680 flops per grouped pair; the Cartesian
     basis's direct kernel k_cart_m2l: CART_M2L_FLOPS_PER_PAIR per pair, FP64
     vector) over their HIP-event times on the streams they run on."""
     import tfmm
@@ -293,7 +293,7 @@ def kernels(st, phases, precision, workload, basis="spherical", cart_direct=Fals
     grouped = st["n_m2l_exec"] - st["n_m2l_fallback"]
     tiles_ms = phases["ms_m2l_tiles"]
     m2l_tf = M2L_FLOPS_PER_PAIR * grouped / (tiles_ms * 1e-3) / 1e12 if tiles_ms > 0 else 0.0
-    tile_name = "k_m2l_tiles<%s>" % ("float" if mixed else "double")
+    tile_name = "k_m2l_sets<%s>" % ("float" if mixed else "double")
     tile_peak = PEAK_FP32_TFLOPS if mixed else PEAK_FP64_TFLOPS
     p2p_traffic = measured_traffic(workload, p2p_name)
     tile_traffic = measured_traffic(workload, tile_name)
@@ -392,7 +392,7 @@ def autotune(ctx, prm, fixed, enabled):
     return {"m2l_unit_factor": unit, "m2l_xcd_run": run, "p2p_schedule": sched,
             "p2p_waves": int(ctx.get_tuning(tfmm.TUNE_P2P_WAVES)),
             "ms_per_evaluation": tms, "seconds": time.perf_counter() - t0,
-            "note": "16 tile-kernel settings, then up to 8 P2P schedule/resident-wave "
+            "note": "16 set-kernel settings, then up to 8 P2P schedule/resident-wave "
                     "settings, x 5 evaluations each, outside the timed steps"}
 
 

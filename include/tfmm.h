@@ -103,10 +103,11 @@ typedef struct {
    * context stream; kernel entries are summed over their launches */
   double ms_tree, ms_upward, ms_traverse, ms_downward, ms_total;
   double ms_p2p, ms_m2l, ms_dtt;
-  /* M2L batching: offset groups, MFMA work items (<= 16 pairs of one group
-   * and one 128-cell target tile each) and pairs outside the groups */
+  /* M2L batching: offset groups (offsets up to mirroring), MFMA work items
+   * (one group, at most one pair for each of 16 consecutive target cells) and
+   * pairs outside the groups */
   uint64_t n_m2l_groups, n_m2l_items, n_m2l_fallback;
-  /* the batched M2L tile kernel alone (its one launch, inside ms_m2l) */
+  /* the batched M2L set kernel alone (its one launch, inside ms_m2l) */
   double ms_m2l_tiles;
   /* problems in the forest (1 unless the bodies were set as a batch);
    * region_min/max above are those of problem 0 */
@@ -180,8 +181,8 @@ int tfmm_set_periodic(tfmm_ctx *ctx, int images, double cycle);
  * d (d+1) (d+2) / 6 + (y + z) (y + z + 1) / 2 + z).  Both bases truncate
  * the same series at total degree 9, so their fields agree to rounding.
  * TFMM_TUNE_CART_M2L picks the route of the Cartesian M2L (by default the
- * FP64 tile kernel between exact basis changes; the stats' group, item and
- * fallback counts are then the tile kernel's, and 0 for the direct kernel).
+ * FP64 set kernel between exact basis changes; the stats' group, item and
+ * fallback counts are then the set kernel's, and 0 for the direct kernel).
  * The P2P follows the precision parameter; the Cartesian expansions and
  * their M2L are FP64 in either precision.  Mutual interaction, batches and
  * periodic images work in either basis; TFMM_TUNE_GRAPH 2 evaluates the
@@ -246,25 +247,27 @@ int tfmm_get_lists(tfmm_ctx *ctx, int32_t *m2l_off, int32_t *m2l_src, int32_t *p
 
 /* Tuning knobs of the kernels (no counterpart in the reference; results do
  * not depend on them beyond the summation order).
- * TFMM_TUNE_M2L_UNIT: the batched M2L kernel runs each 128-cell target tile
- * as work units of at most factor x (mean items per tile) items, so that a
- * few heavy tiles do not hold the launch back; 0 = one unit per tile. */
+ * TFMM_TUNE_M2L_UNIT: the batched M2L kernel runs each set of 16 target cells
+ * as work units of at most factor x (mean items per set) items, so that a
+ * few heavy sets do not hold the launch back; 0 = a size from the number of
+ * items. */
 #define TFMM_TUNE_M2L_UNIT 1
-/* TFMM_TUNE_M2L_XCD_RUN: consecutive work units dealt to one of the 8 XCDs
- * (each has its own L2; neighbouring tiles share source expansions). */
+/* TFMM_TUNE_M2L_XCD_RUN: groups of 8 consecutive work units dealt to one of
+ * the 8 XCDs (each has its own L2; neighbouring sets share source
+ * expansions). */
 #define TFMM_TUNE_M2L_XCD_RUN 2
 /* TFMM_TUNE_P2P_SCHEDULE: where the P2P kernel (second stream) starts.  In
  * tfmm_evaluate, 0 starts it with the numeric phase, beside the upward pass
- * and the M2L kernels; 1 starts it with the M2L tile kernel; 2 as soon as
+ * and the M2L kernels; 1 starts it with the M2L set kernel; 2 as soon as
  * its list is sorted, beside the M2L batch building (also inside the
  * one-launch graph of TFMM_TUNE_GRAPH 2; with TFMM_TUNE_GRAPH 1 as 0); 3 as 2 with the resident FP32 P2P (TFMM_TUNE_P2P_WAVES > 0,
- * mixed precision) holding its few waves until the tile kernel is done, when
+ * mixed precision) holding its few waves until the set kernel is done, when
  * a full-occupancy launch of the same kernel on the context stream takes the
  * target cells still left on its counter (each cell is computed by one
  * wave either way: the fields do not change); 4 runs it on the context
  * stream with nothing beside it (from phase A, serially: for timing the
  * kernel alone).  In the separate
- * tfmm_traverse, 1 starts it with the tile kernel, any other value as soon
+ * tfmm_traverse, 1 starts it with the set kernel, any other value as soon
  * as its list is sorted. */
 #define TFMM_TUNE_P2P_SCHEDULE 3
 /* TFMM_TUNE_GRAPH: 1 records tfmm_evaluate's numeric phase (P2M, M2M, P2P,
@@ -300,7 +303,7 @@ int tfmm_get_lists(tfmm_ctx *ctx, int32_t *m2l_off, int32_t *m2l_src, int32_t *p
  * failure path. */
 #define TFMM_TUNE_DEVICE_LIMIT 6
 /* TFMM_TUNE_CART_M2L: the M2L of the Cartesian basis (tfmm_set_basis).
- * 0 (default): through the spherical tile kernel, exactly -- the Cartesian
+ * 0 (default): through the spherical set kernel, exactly -- the Cartesian
  * multipoles turned into spherical ones per degree (T1), the FP64 tile
  * kernel (and its per-pair FP64 fallback, and the far field of periodic
  * images), the spherical locals turned back (T2); both bases truncate the
@@ -314,7 +317,7 @@ int tfmm_set_tuning(tfmm_ctx *ctx, int knob, double value);
 int tfmm_get_tuning(tfmm_ctx *ctx, int knob, double *value);
 /* Autotuner: evaluates the current bodies with params, reps times per
  * candidate (after 2 uncounted evaluations of the candidate, which let the
- * device settle to the setting), in two stages -- the tile-kernel knobs (unit factor {0, 1.5,
+ * device settle to the setting), in two stages -- the set-kernel knobs (unit factor {0, 1.5,
  * 2, 3} x XCD run {8, 16, 32, 64}) at the current P2P setting, then the
  * P2P's schedule {0, 1, 2} x resident waves {0, 3, 4} (waves for mixed
  * precision only, schedule 2 not with TFMM_TUNE_GRAPH 1) at the best tile

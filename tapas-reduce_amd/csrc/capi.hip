@@ -12,6 +12,8 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <tuple>
+#include <utility>
 #include <vector>
 
 #include "../../include/tfmm.h"
@@ -118,14 +120,14 @@ struct tfmm_ctx {
   uint32_t dtt_steps = 0;
 
   // batched M2L (offset groups)
-  DevBuf g_used, g_gid, g_y64, g_y32, g_af, g_dl, g_lt, g_cnt;
+  DevBuf g_used, g_gid, g_y64, g_y32, g_af, g_dl, g_cnt;
   DevBuf gkeys, gvals, gkeys_alt, gvals_alt, fkeys, fvals, fkeys_alt, fvals_alt;
-  // it_flag: position in segment per grouped pair; it_iflag/it_iexcl: item starts per block
-  DevBuf it_flag, it_iflag, it_iexcl, items, cols, tile_off, mq, codes;
+  // it_cnt/it_start: items per block of grouped pairs; items: every item's key
+  DevBuf it_cnt, it_start, items, cols, set_off, mq, codes;
   DevBuf fb_off, fb_src, fb_part, relpos, leaf_of, tops, slot_of;
   DevBuf u_cnt, u_off, units, u_part;
-  double m2l_unit_factor = 0.0;  // tile work-unit size in mean items per tile (0: off)
-  int m2l_xcd_run = 32;          // consecutive work units dealt to one XCD
+  double m2l_unit_factor = 0.0;  // M2L work-unit size in mean items per set (0: automatic)
+  int m2l_xcd_run = 32;          // groups of 8 consecutive work units dealt to one XCD
   int p2p_schedule = 0;          // where the P2P starts (TFMM_TUNE_P2P_SCHEDULE)
   int use_graph = 0;             // tfmm_evaluate's numeric phase as one hipGraph
   int p2p_waves = 0;             // resident P2P waves per SIMD (0: one workgroup per cell)
@@ -152,13 +154,14 @@ struct tfmm_ctx {
   DevBuf cart_tab;
   bool cart_ready = false;
   // Cartesian expansions (CART_TERMS doubles per cell); M and L then hold
-  // the spherical images the tile kernel works on (TFMM_TUNE_CART_M2L 0)
+  // the spherical images the set kernel works on (TFMM_TUNE_CART_M2L 0)
   DevBuf Mc, Lc;
   int cart_direct = 0;  // TFMM_TUNE_CART_M2L: 1 = the direct Cartesian M2L kernel
   int32_t unit_chunk = 0;
   uint32_t units_bound = 0;
   bool codes_ready = false;
   uint32_t n_groups = 0, n_grouped = 0, n_fallback = 0, n_items = 0;
+  int group_bits = 0;  // of a key's group field
   bool grouped_keys_in_alt = false;
 
   // picker
@@ -254,10 +257,9 @@ std::vector<DevBuf *> all_buffers(tfmm_ctx *c) {
           &c->p2p_pairs, &c->cnt, &c->lkeys, &c->lkeys_alt, &c->lidx, &c->lidx_alt,
           &c->m2l_off, &c->m2l_src, &c->p2p_off, &c->p2p_src, &c->acc,
           &c->trg, &c->out, &c->g_used, &c->g_gid, &c->g_y64, &c->g_y32, &c->g_af, &c->g_dl,
-          &c->g_lt, &c->g_cnt, &c->gkeys, &c->gvals, &c->gkeys_alt, &c->gvals_alt,
-          &c->fkeys, &c->fvals, &c->fkeys_alt, &c->fvals_alt, &c->it_flag,
-          &c->it_iflag, &c->it_iexcl, &c->items,
-          &c->tile_off, &c->cols, &c->mq, &c->codes, &c->fb_off, &c->fb_src, &c->fb_part,
+          &c->g_cnt, &c->gkeys, &c->gvals, &c->gkeys_alt, &c->gvals_alt,
+          &c->fkeys, &c->fvals, &c->fkeys_alt, &c->fvals_alt, &c->it_cnt,
+          &c->it_start, &c->items, &c->set_off, &c->cols, &c->mq, &c->codes, &c->fb_off, &c->fb_src, &c->fb_part,
           &c->relpos, &c->leaf_of, &c->tops, &c->slot_of,
           &c->feat_acc, &c->feat_x, &c->feat_out, &c->d_prob_off, &c->bprob,
           &c->pkey, &c->pkey_alt, &c->ppos, &c->ppos_alt, &c->brec, &c->lev,
@@ -291,7 +293,7 @@ double period(const tfmm_ctx *c) { return c->images > 0 ? c->cycle : 0.0; }
 bool cartesian(const tfmm_ctx *c) { return c->basis == TFMM_BASIS_CARTESIAN; }
 // the Cartesian basis with its own M2L kernel (no spherical images)
 bool cart_direct(const tfmm_ctx *c) { return cartesian(c) && c->cart_direct; }
-// the tile kernel in FP32 (mixed precision, spherical basis); the Cartesian
+// the set kernel in FP32 (mixed precision, spherical basis); the Cartesian
 // basis keeps its expansions and their M2L in FP64
 bool m2l_fp32(const tfmm_ctx *c) { return c->prm.precision == TFMM_MIXED && !cartesian(c); }
 
@@ -522,7 +524,7 @@ hipError_t rec(tfmm_ctx *c, int ev, hipStream_t st);
 int sort_list(tfmm_ctx *c, DevBuf &pairs, uint32_t npairs, DevBuf &off, DevBuf &src);
 
 // The Cartesian basis's upward pass: P2M, then M2M level by level (Mc);
-// for the tile kernel's route also the spherical images of the multipoles (M).
+// for the set kernel's route also the spherical images of the multipoles (M).
 int cart_upward(tfmm_ctx *c) {
   hipStream_t s = c->stream;
   const Cells k = cells_of(c);
@@ -563,7 +565,7 @@ int cart_lists(tfmm_ctx *c) {
   return cart_tables(c);
 }
 
-// The tile kernel's route: its spherical locals (L) into the Cartesian ones.
+// The set kernel's route: its spherical locals (L) into the Cartesian ones.
 hipError_t cart_from_tiles(tfmm_ctx *c) {
   if (!cartesian(c) || c->cart_direct) return hipSuccess;
   return launch_sph_to_cart((int32_t)c->ncells, dp<double>(c->L), dp<double>(c->Lc),
@@ -656,7 +658,7 @@ int do_dtt(tfmm_ctx *c) {
   // seen after an overflow are lower bounds: capacities at least double.
   // M2L group-table flags (one per slot), then the count of M2L pairs
   // outside the table, filled by the steps beside the lists
-  const int32_t nslots = m2l_group_slots(max_depth);
+  const int32_t nslots = m2l_group_slots();
   TRY(dev_reserve(c->g_used, (size_t)(nslots + 1) * 4));
   for (int attempt = 0; attempt < 12; attempt++) {
     TRY(dev_reserve(c->m2l_pairs, (size_t)c->m2l_cap * 8));
@@ -721,14 +723,45 @@ int do_dtt(tfmm_ctx *c) {
   return fail(c, TFMM_EHIP, "traversal lists did not converge");
 }
 
-// Group the executed M2L pairs by (target level, source level, offset), build
+// An item takes one source per target and mirrored offset, which is all the
+// traversal makes.  Lists that the caller gives (given) may hold more: all but
+// one of them then go to the per-pair kernel.
+int repeats_to_fallback(tfmm_ctx *c) {
+  hipStream_t s = c->stream;
+  const uint32_t n = c->n_m2l_exec;
+  const int32_t nslots = m2l_group_slots();
+  std::vector<int2> pairs(n);
+  std::vector<int32_t> slot(n);
+  std::vector<uint32_t> order;
+  TRY(hipMemcpyAsync(pairs.data(), c->m2l_pairs.ptr, (size_t)n * 8, hipMemcpyDeviceToHost, s));
+  TRY(hipMemcpyAsync(slot.data(), c->slot_of.ptr, (size_t)n * 4, hipMemcpyDeviceToHost, s));
+  TRY(hipStreamSynchronize(s));
+  for (uint32_t i = 0; i < n; i++)
+    if (slot[i] >= 0) order.push_back(i);
+  auto place = [&](uint32_t i) { return std::make_pair(pairs[i].x, slot[i]); };
+  std::sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) {
+    return std::make_tuple(place(a), a) < std::make_tuple(place(b), b);
+  });
+  uint32_t outside = n - (uint32_t)order.size();
+  std::vector<uint32_t> repeated;
+  for (size_t e = 1; e < order.size(); e++)
+    if (place(order[e]) == place(order[e - 1])) repeated.push_back(order[e]);
+  for (uint32_t i : repeated) slot[i] = -1;
+  outside += (uint32_t)repeated.size();
+  TRY(hipMemcpyAsync(c->slot_of.ptr, slot.data(), (size_t)n * 4, hipMemcpyHostToDevice, s));
+  TRY(hipMemcpyAsync(dp<uint32_t>(c->g_used) + nslots, &outside, 4, hipMemcpyHostToDevice, s));
+  TRY(hipStreamSynchronize(s));
+  return TFMM_OK;
+}
+
+// Group the executed M2L pairs by (level difference, offset up to mirrors), build
 // the MFMA work items and the per-target list of the pairs outside the groups.
-int build_m2l_batches(tfmm_ctx *c) {
+int build_m2l_batches(tfmm_ctx *c, bool given = false) {
   hipStream_t s = c->stream;
   const Cells k = cells_of(c);
   const uint32_t n = c->n_m2l_exec;
   const int max_depth = (int)c->lvl.size() - 2;
-  const int32_t nslots = m2l_group_slots(max_depth);
+  const int32_t nslots = m2l_group_slots();
   // g_used (nslots flags, then the count of pairs outside the table) and
   // slot_of (every pair's slot) come from the traversal
   TRY(dev_reserve(c->g_gid, (size_t)nslots * 4));
@@ -746,10 +779,9 @@ int build_m2l_batches(tfmm_ctx *c) {
   TRY(dev_reserve(c->g_y64, ngr * 112 * 8));
   TRY(dev_reserve(c->g_y32, ngr * 112 * 4));
   TRY(dev_reserve(c->g_dl, ngr));
-  TRY(dev_reserve(c->g_lt, ngr));
-  TRY(launch_m2l_group_harmonics(dp<uint32_t>(c->g_used), dp<uint32_t>(c->g_gid), nslots,
+  TRY(launch_m2l_group_harmonics(dp<uint32_t>(c->g_used), dp<uint32_t>(c->g_gid),
                                  dp<double>(c->g_y64), dp<float>(c->g_y32), dp<int8_t>(c->g_dl),
-                                 dp<int8_t>(c->g_lt), s));
+                                 s));
   // split grouped / fallback pairs
   const size_t nn = (size_t)std::max<uint32_t>(n, 1);
   TRY(dev_reserve(c->gkeys, nn * 4));
@@ -766,8 +798,7 @@ int build_m2l_batches(tfmm_ctx *c) {
   const int sbits = bits_for(c->ncells);
   {
     const int64_t nt = (c->ncells + m2l_tile_size() - 1) / m2l_tile_size();
-    if (bits_for(nt) + gbits > 32 || gbits > m2l_group_bits() ||
-        c->ncells >= ((int64_t)1 << m2l_src_bits()))
+    if (bits_for(nt) + gbits > 32 || c->ncells >= ((int64_t)1 << m2l_src_bits()))
       return fail(c, TFMM_EHIP, "tree too large for the batched M2L keys");
   }
   uint32_t ngp = n, nfb = 0;
@@ -798,25 +829,29 @@ int build_m2l_batches(tfmm_ctx *c) {
                          &alt));
   c->grouped_keys_in_alt = alt;
   const uint32_t *gk = dp<uint32_t>(alt ? c->gkeys_alt : c->gkeys);
-  // work items: runs of <= 16 pairs of one group within one tile
-  const size_t ng1 = (size_t)std::max<uint32_t>(ngp, 1);
-  TRY(dev_reserve(c->it_flag, ng1 * 4));
-  const size_t nblk = (ng1 + 1023) / 1024;
-  TRY(dev_reserve(c->it_iflag, nblk * 4));
-  TRY(dev_reserve(c->it_iexcl, nblk * 4));
-  uint32_t nitems = 0;
-  TRY(launch_m2l_count_items(gk, ngp, dp<uint32_t>(c->it_flag), dp<uint32_t>(c->it_iflag),
-                             dp<uint32_t>(c->it_iexcl), c->scan_tmp.ptr, c->h_u32, &nitems, s));
-  const size_t ni1 = std::max<uint32_t>(nitems, 1);
-  TRY(dev_reserve(c->items, ni1 * 16));
-  TRY(dev_reserve(c->cols, ni1 * 16 * 8));
   const uint32_t *gvs = dp<uint32_t>(alt ? c->gvals_alt : c->gvals);
-  TRY(launch_m2l_write_items(gk, gvs, ngp, gbits, dp<uint32_t>(c->it_flag),
-                             dp<uint32_t>(c->it_iexcl), dp<int8_t>(c->g_dl), dp<int4>(c->items),
-                             dp<uint2>(c->cols), s));
+  // work items: one group and at most one pair per target of one set
+  const size_t nblk = m2l_item_blocks(ngp);
+  TRY(dev_reserve(c->it_cnt, nblk * 4));
+  TRY(dev_reserve(c->it_start, nblk * 4));
+  uint32_t nitems = 0;
+  TRY(launch_m2l_count_items(gk, gvs, ngp, dp<uint32_t>(c->it_cnt), dp<uint32_t>(c->it_start),
+                             c->scan_tmp.ptr, c->h_u32, &nitems, s,
+                             given ? dp<uint32_t>(c->g_cnt) + 2 : nullptr));
+  if (given && c->h_u32[2]) {
+    const int rc = repeats_to_fallback(c);
+    return rc ? rc : build_m2l_batches(c);
+  }
+  const size_t ni1 = std::max<uint32_t>(nitems, 1);
+  TRY(dev_reserve(c->items, ni1 * 4));
+  TRY(dev_reserve(c->cols, ni1 * 16 * 4));
+  TRY(launch_m2l_write_items(gk, gvs, ngp, dp<uint32_t>(c->it_start), (int32_t)c->ncells,
+                             dp<uint32_t>(c->items), dp<uint32_t>(c->cols), s));
   c->n_items = nitems;
-  TRY(dev_reserve(c->tile_off, (size_t)(ntiles + 1) * 4));
-  TRY(launch_m2l_tile_offsets(dp<int4>(c->items), nitems, ntiles, dp<int32_t>(c->tile_off), s));
+  c->group_bits = gbits;
+  TRY(dev_reserve(c->set_off, (size_t)(ntiles + 1) * 4));
+  TRY(launch_m2l_set_offsets(dp<uint32_t>(c->items), nitems, gbits, ntiles, dp<int32_t>(c->set_off),
+                             s));
   c->unit_chunk = m2l_unit_chunk(nitems, ntiles, c->m2l_unit_factor);
   c->units_bound = m2l_units_bound(nitems, ntiles, c->unit_chunk);
   TRY(dev_reserve(c->u_cnt, (size_t)ntiles * 4));
@@ -824,7 +859,7 @@ int build_m2l_batches(tfmm_ctx *c) {
   TRY(dev_reserve(c->units, (size_t)c->units_bound * 8));
   TRY(dev_reserve(c->u_part, m2l_unit_part_bytes(c->units_bound, ntiles)));
   TRY(dev_reserve(c->scan_tmp, scan_tmp_bytes(std::max<int64_t>(ntiles, std::max<int64_t>(nslots, n)))));
-  TRY(launch_m2l_units(dp<int32_t>(c->tile_off), ntiles, c->unit_chunk, dp<uint32_t>(c->u_cnt),
+  TRY(launch_m2l_units(dp<int32_t>(c->set_off), ntiles, c->unit_chunk, dp<uint32_t>(c->u_cnt),
                        dp<uint32_t>(c->u_off), dp<int2>(c->units), c->scan_tmp.ptr, s));
   // fallback pairs: per-target list sorted by (target, source)
   bool falt = false;
@@ -843,7 +878,7 @@ int build_m2l_batches(tfmm_ctx *c) {
     TRY(e);
     c->codes_ready = true;
   }
-  // every group's A operands in the tile kernel's order
+  // every group's A operands in the set kernel's order
   const bool mixed = m2l_fp32(c);
   TRY(dev_reserve(c->g_af, m2l_afrag_bytes(ng, mixed)));
   TRY(launch_m2l_group_afrag(mixed ? (const void *)c->g_y32.ptr : (const void *)c->g_y64.ptr,
@@ -858,7 +893,7 @@ int p2p_resident(tfmm_ctx *c) { return c->p2p_waves > 0 ? c->p2p_waves * 4 * c->
 // The M2L and P2P pairs of the traversal (c->m2l_pairs with their group
 // slots, c->p2p_pairs, the counters) into sorted lists, M2L batches and the
 // M2L and P2P kernels.
-int run_lists(tfmm_ctx *c) {
+int run_lists(tfmm_ctx *c, bool given = false) {
   hipStream_t s = c->stream;
   const Cells k = cells_of(c);
   const bool mixed = c->prm.precision == TFMM_MIXED;
@@ -871,8 +906,8 @@ int run_lists(tfmm_ctx *c) {
   // P2P on the side stream: it needs only the P2P list and the bodies.
   // Schedule 0 starts it as soon as its list is sorted, so it covers the host
   // round trips of the M2L batch building (which then gets few CU slots);
-  // schedule 1 starts it together with the tile kernel, so the P2P (FP32
-  // VALU) and the tiles (MFMA, LDS) share the CUs.  Joined before the
+  // schedule 1 starts it together with the set kernel, so the P2P (FP32
+  // VALU) and the M2L (MFMA) share the CUs.  Joined before the
   // downward pass.
   TRY(dev_reserve(c->acc, (size_t)c->n * 32));
   auto launch_p2p = [&]() -> int {
@@ -909,19 +944,17 @@ int run_lists(tfmm_ctx *c) {
                        hipMemcpyDeviceToHost, s));
     return TFMM_OK;
   }
-  rc = build_m2l_batches(c);
+  rc = build_m2l_batches(c, given);
   if (rc) {
     if (p2p_early) (void)hipStreamWaitEvent(s, c->ev[EV_P2P1], 0);
     return rc;
   }
   // M~ in the MFMA operand layout
   const bool tf32 = m2l_fp32(c);
-  TRY(dev_reserve(c->mq, (size_t)c->ncells * 112 * (tf32 ? 4 : 8)));
+  TRY(dev_reserve(c->mq, m2l_mq_bytes(c->ncells, tf32)));
   TRY(launch_m2l_scale_m(k, (int32_t)c->ncells, dp<double>(c->M), c->mq.ptr, tf32, s));
   TRY(hipEventRecord(c->ev[EV_DTT1], s));
 
-  const size_t lbytes = sph_bytes(c->ncells);
-  TRY(hipMemsetAsync(c->L.ptr, 0, lbytes, s));
   TRY(hipEventRecord(c->ev[EV_M2L0], s));
   if (!p2p_early) {
     rc = launch_p2p();
@@ -929,12 +962,11 @@ int run_lists(tfmm_ctx *c) {
   }
   const int32_t tile = m2l_tile_size();
   const int32_t ntiles = (int32_t)((c->ncells + tile - 1) / tile);
-  TRY(launch_m2l_tiles(dp<int32_t>(c->tile_off), dp<int2>(c->units), dp<uint32_t>(c->u_cnt),
-                       dp<uint32_t>(c->u_off), ntiles, c->unit_chunk, c->m2l_xcd_run,
-                       c->units_bound,
-                       dp<uint2>(c->cols),
-                       c->g_af.ptr, c->mq.ptr, k, (int32_t)c->ncells,
-                       dp<double>(c->L), dp<double>(c->u_part), tf32, s));
+  TRY(launch_m2l_sets(dp<int32_t>(c->set_off), dp<int2>(c->units), dp<uint32_t>(c->u_cnt),
+                      dp<uint32_t>(c->u_off), ntiles, c->unit_chunk, c->m2l_xcd_run,
+                      c->units_bound, dp<uint32_t>(c->items), c->group_bits,
+                      dp<uint32_t>(c->cols), c->g_af.ptr, c->mq.ptr, k, (int32_t)c->ncells,
+                      dp<double>(c->L), dp<double>(c->u_part), tf32, s));
   TRY(hipEventRecord(c->ev[EV_M2LT], s));
   if (c->n_fallback) {
     Csr fl{dp<int32_t>(c->fb_off), dp<int32_t>(c->fb_src)};
@@ -1013,7 +1045,7 @@ int traverse_given(tfmm_ctx *c, const int32_t *m2l, int64_t nm, const int32_t *p
   }
   TRY(hipEventRecord(c->ev[EV_DTT0], s));
   const int max_depth = (int)c->lvl.size() - 2;
-  const int32_t nslots = m2l_group_slots(max_depth);
+  const int32_t nslots = m2l_group_slots();
   const size_t nme = std::max<size_t>(me.size(), 1), npe = std::max<size_t>(pe.size(), 1);
   TRY(dev_reserve(c->cnt, 16 * 4));
   TRY(dev_reserve(c->g_used, (size_t)(nslots + 1) * 4));
@@ -1041,7 +1073,7 @@ int traverse_given(tfmm_ctx *c, const int32_t *m2l, int64_t nm, const int32_t *p
   c->n_m2l_all = m2l_calls;
   c->n_p2p = (uint32_t)pe.size();
   c->n_p2p_calls_leaf = p2p_calls;
-  return run_lists(c);
+  return run_lists(c, true);
 }
 
 int do_downward(tfmm_ctx *c) {
@@ -1104,7 +1136,7 @@ void probe_external_events(tfmm_ctx *c) {
 // stream by events).
 // Schedule 3: the resident FP32 P2P starts early with its few waves, and a
 // full-occupancy launch of the same kernel on the context stream takes the
-// target cells still left on its counter once the tile kernel is done.
+// target cells still left on its counter once the set kernel is done.
 bool p2p_drains(const tfmm_ctx *c) {
   return c->p2p_schedule == 3 && c->p2p_waves > 0 && c->prm.precision == TFMM_MIXED;
 }
@@ -1193,7 +1225,7 @@ int fused_prepare(tfmm_ctx *c) {
     TRY(launch_translation_ops(dp<double>(c->tops), s));
     c->tops_ready = true;
   }
-  TRY(dev_reserve(c->mq, (size_t)c->ncells * 112 * (m2l_fp32(c) ? 4 : 8)));
+  TRY(dev_reserve(c->mq, m2l_mq_bytes(c->ncells, m2l_fp32(c))));
   TRY(dev_reserve(c->trg, (size_t)c->n * 32));
   TRY(dev_reserve(c->out, (size_t)c->n * 32));
   TRY(dev_reserve(c->leaf_of, (size_t)c->n * 4));
@@ -1207,7 +1239,7 @@ int fused_numeric(tfmm_ctx *c) {
   hipStream_t s = c->stream;
   const Cells k = cells_of(c);
   // P2P on the second stream, joined before the downward pass; forked at the
-  // start of the phase (schedule 0), at the tile kernel (1), or already in
+  // start of the phase (schedule 0), at the set kernel (1), or already in
   // phase A (2)
   int rc;
   if (!c->p2p_forked && c->p2p_schedule != 1 && (rc = fork_p2p(c))) return rc;
@@ -1240,16 +1272,15 @@ int fused_numeric(tfmm_ctx *c) {
   // M2L
   const bool mixed = m2l_fp32(c);
   TRY(launch_m2l_scale_m(k, (int32_t)c->ncells, dp<double>(c->M), c->mq.ptr, mixed, s));
-  TRY(launch_fill_zero(c->L.ptr, ebytes, s));
   TRY(rec(c, EV_M2L0, s));
   if (!c->p2p_forked && c->p2p_schedule == 1 && (rc = fork_p2p(c))) return rc;
   const int32_t tile = m2l_tile_size();
   const int32_t ntiles = (int32_t)((c->ncells + tile - 1) / tile);
-  TRY(launch_m2l_tiles(dp<int32_t>(c->tile_off), dp<int2>(c->units), dp<uint32_t>(c->u_cnt),
-                       dp<uint32_t>(c->u_off), ntiles, c->unit_chunk, c->m2l_xcd_run,
-                       c->units_bound, dp<uint2>(c->cols),
-                       c->g_af.ptr, c->mq.ptr, k, (int32_t)c->ncells,
-                       dp<double>(c->L), dp<double>(c->u_part), mixed, s));
+  TRY(launch_m2l_sets(dp<int32_t>(c->set_off), dp<int2>(c->units), dp<uint32_t>(c->u_cnt),
+                      dp<uint32_t>(c->u_off), ntiles, c->unit_chunk, c->m2l_xcd_run,
+                      c->units_bound, dp<uint32_t>(c->items), c->group_bits,
+                      dp<uint32_t>(c->cols), c->g_af.ptr, c->mq.ptr, k, (int32_t)c->ncells,
+                      dp<double>(c->L), dp<double>(c->u_part), mixed, s));
   TRY(rec(c, EV_M2LT, s));
   if (c->n_fallback) {
     Csr fl{dp<int32_t>(c->fb_off), dp<int32_t>(c->fb_src)};
@@ -1390,7 +1421,7 @@ void plan_make(tfmm_ctx *c) {
   pl.nsteps = 2 * pl.max_depth + 2;
   pl.cwords = 16 + pl.nsteps + 1;
   if (pl.cwords > PLAN_MAX_CWORDS) return;
-  pl.nslots = m2l_group_slots(pl.max_depth);
+  pl.nslots = m2l_group_slots();
   int64_t fmax = 0;
   pl.step_grid.resize(pl.nsteps);
   for (int st = 0; st < pl.nsteps; st++) {
@@ -1406,14 +1437,11 @@ void plan_make(tfmm_ctx *c) {
   pl.caps.fallback = cap32(more(c->n_fallback, 4096));
   pl.groups = cap32(more(c->n_groups, 256));
   pl.ntiles = (int32_t)((pl.cells + m2l_tile_size() - 1) / m2l_tile_size());
-  const double f = c->m2l_unit_factor;
-  pl.caps.units =
-      cap32(f > 0 ? pl.ntiles + (int64_t)std::ceil(pl.ntiles / f) + 1 : (int64_t)pl.ntiles);
+  pl.caps.units = m2l_units_cap(pl.caps.items, pl.ntiles, c->m2l_unit_factor);
   pl.gbits = bits_for(pl.groups);
   pl.sbits = bits_for(pl.cells);
   pl.tbits = bits_for(pl.ntiles);
-  if (pl.tbits + pl.gbits > 32 || pl.gbits > m2l_group_bits() ||
-      pl.cells >= ((int64_t)1 << m2l_src_bits()) || FB_SRC_BITS + pl.sbits > 64 ||
+  if (pl.tbits + pl.gbits > 32 || pl.cells >= ((int64_t)1 << m2l_src_bits()) || FB_SRC_BITS + pl.sbits > 64 ||
       (int64_t)pl.caps.fallback > (1 << 22))
     return;
   pl.valid = true;
@@ -1481,7 +1509,7 @@ int plan_reserve(tfmm_ctx *c) {
   TRY(dev_reserve(c->acc, (size_t)n * 32));
   // M2L batches
   const size_t ng = pl.groups;
-  const size_t item_blocks = (nm + 1023) / 1024;
+  const size_t item_blocks = m2l_item_blocks((uint32_t)nm);
   TRY(dev_reserve(c->g_gid, (size_t)pl.nslots * 4));
   TRY(dev_reserve(c->scan_tmp,
                   scan_tmp_bytes(std::max<int64_t>({(int64_t)pl.nslots, (int64_t)pl.ntiles,
@@ -1489,7 +1517,6 @@ int plan_reserve(tfmm_ctx *c) {
   TRY(dev_reserve(c->g_y64, ng * 112 * 8));
   TRY(dev_reserve(c->g_y32, ng * 112 * 4));
   TRY(dev_reserve(c->g_dl, ng));
-  TRY(dev_reserve(c->g_lt, ng));
   TRY(dev_reserve(c->g_af, m2l_afrag_bytes((uint32_t)ng, mixed)));
   TRY(dev_reserve(c->gkeys, nm * 4));
   TRY(dev_reserve(c->gvals, nm * 4));
@@ -1500,12 +1527,11 @@ int plan_reserve(tfmm_ctx *c) {
   TRY(dev_reserve(c->fkeys_alt, nm * 8));
   TRY(dev_reserve(c->fvals_alt, nm * 4));
   TRY(dev_reserve(c->g_cnt, 16));
-  TRY(dev_reserve(c->it_flag, nm * 4));
-  TRY(dev_reserve(c->it_iflag, item_blocks * 4));
-  TRY(dev_reserve(c->it_iexcl, item_blocks * 4));
-  TRY(dev_reserve(c->items, (size_t)pl.caps.items * 16));
-  TRY(dev_reserve(c->cols, (size_t)pl.caps.items * 16 * 8));
-  TRY(dev_reserve(c->tile_off, (size_t)(pl.ntiles + 1) * 4));
+  TRY(dev_reserve(c->it_cnt, item_blocks * 4));
+  TRY(dev_reserve(c->it_start, item_blocks * 4));
+  TRY(dev_reserve(c->items, (size_t)pl.caps.items * 4));
+  TRY(dev_reserve(c->cols, (size_t)pl.caps.items * 16 * 4));
+  TRY(dev_reserve(c->set_off, (size_t)(pl.ntiles + 1) * 4));
   TRY(dev_reserve(c->u_cnt, (size_t)pl.ntiles * 4));
   TRY(dev_reserve(c->u_off, (size_t)pl.ntiles * 4));
   TRY(dev_reserve(c->units, (size_t)pl.caps.units * 8));
@@ -1529,7 +1555,7 @@ int plan_reserve(tfmm_ctx *c) {
     TRY(launch_translation_ops(dp<double>(c->tops), s));
     c->tops_ready = true;
   }
-  TRY(dev_reserve(c->mq, cells * 112 * (mixed ? 4 : 8)));
+  TRY(dev_reserve(c->mq, m2l_mq_bytes(pl.cells, mixed)));
   TRY(dev_reserve(c->trg, (size_t)n * 32));
   TRY(dev_reserve(c->out, (size_t)n * 32));
   TRY(dev_reserve(c->leaf_of, (size_t)n * 4));
@@ -1649,9 +1675,8 @@ int whole_record(tfmm_ctx *c) {
     uint32_t *gcnt = dp<uint32_t>(c->g_cnt);
     TRY(scan_exclusive_u32(used, dp<uint32_t>(c->g_gid), pl.nslots, c->scan_tmp.ptr, s));
     TRY(launch_groups_count(dp<uint32_t>(c->g_gid), used, pl.nslots, pl.groups, sz, s));
-    TRY(launch_m2l_group_harmonics(used, dp<uint32_t>(c->g_gid), pl.nslots,
-                                   dp<double>(c->g_y64), dp<float>(c->g_y32),
-                                   dp<int8_t>(c->g_dl), dp<int8_t>(c->g_lt), s, pl.groups));
+    TRY(launch_m2l_group_harmonics(used, dp<uint32_t>(c->g_gid), dp<double>(c->g_y64),
+                                   dp<float>(c->g_y32), dp<int8_t>(c->g_dl), s, pl.groups));
     TRY(launch_fill_zero(gcnt, 16, s));
     TRY(launch_m2l_classify(dp<int2>(c->m2l_pairs), dp<int32_t>(c->slot_of), nm,
                             dp<uint32_t>(c->g_gid), pl.gbits, FB_SRC_BITS, dp<uint32_t>(c->gkeys),
@@ -1665,17 +1690,15 @@ int whole_record(tfmm_ctx *c) {
     pl.gkeys_alt = galt;
     const uint32_t *gk = dp<uint32_t>(galt ? c->gkeys_alt : c->gkeys);
     const uint32_t *gv = dp<uint32_t>(galt ? c->gvals_alt : c->gvals);
-    TRY(launch_m2l_count_items_dev(gk, nm, gcnt, dp<uint32_t>(c->it_flag),
-                                   dp<uint32_t>(c->it_iflag), dp<uint32_t>(c->it_iexcl),
-                                   c->scan_tmp.ptr, sz + SZ_NITEMS, s));
-    TRY(launch_m2l_write_items(gk, gv, nm, pl.gbits, dp<uint32_t>(c->it_flag),
-                               dp<uint32_t>(c->it_iexcl), dp<int8_t>(c->g_dl), dp<int4>(c->items),
-                               dp<uint2>(c->cols), s, gcnt, pl.caps.items));
-    TRY(launch_m2l_tile_offsets(dp<int4>(c->items), pl.caps.items, pl.ntiles,
-                                dp<int32_t>(c->tile_off), s, sz + SZ_NITEMS));
+    TRY(launch_m2l_count_items_dev(gk, gv, nm, gcnt, dp<uint32_t>(c->it_cnt),
+                                   dp<uint32_t>(c->it_start), c->scan_tmp.ptr, sz + SZ_NITEMS, s));
+    TRY(launch_m2l_write_items(gk, gv, nm, dp<uint32_t>(c->it_start), cells, dp<uint32_t>(c->items),
+                               dp<uint32_t>(c->cols), s, gcnt, pl.caps.items));
+    TRY(launch_m2l_set_offsets(dp<uint32_t>(c->items), pl.caps.items, pl.gbits, pl.ntiles,
+                               dp<int32_t>(c->set_off), s, sz + SZ_NITEMS));
     int32_t *chunk = reinterpret_cast<int32_t *>(sz + SZ_CHUNK);
     TRY(launch_m2l_unit_chunk(sz + SZ_NITEMS, sz + SZ_NTILES, c->m2l_unit_factor, chunk, s));
-    TRY(launch_m2l_units(dp<int32_t>(c->tile_off), pl.ntiles, 0, dp<uint32_t>(c->u_cnt),
+    TRY(launch_m2l_units(dp<int32_t>(c->set_off), pl.ntiles, 0, dp<uint32_t>(c->u_cnt),
                          dp<uint32_t>(c->u_off), dp<int2>(c->units), c->scan_tmp.ptr, s,
                          pl.caps.units, chunk));
     // the pairs outside the groups (appended compactly): at most the
@@ -1703,14 +1726,13 @@ int whole_record(tfmm_ctx *c) {
                    d + 1));
   TRY(rec(c, EV_UP, s));
   TRY(launch_m2l_scale_m(k, cells, dp<double>(c->M), c->mq.ptr, mixed, s));
-  TRY(launch_fill_zero(c->L.ptr, ebytes, s));
   TRY(rec(c, EV_M2L0, s));
   if (c->p2p_schedule == 1 && (rc = fork_p2p(c, cells))) return rc;
-  TRY(launch_m2l_tiles(dp<int32_t>(c->tile_off), dp<int2>(c->units), dp<uint32_t>(c->u_cnt),
-                       dp<uint32_t>(c->u_off), pl.ntiles, 0, c->m2l_xcd_run, pl.caps.units,
-                       dp<uint2>(c->cols), c->g_af.ptr, c->mq.ptr, k, cells, dp<double>(c->L),
-                       dp<double>(c->u_part), mixed, s,
-                       reinterpret_cast<const int32_t *>(sz + SZ_CHUNK)));
+  TRY(launch_m2l_sets(dp<int32_t>(c->set_off), dp<int2>(c->units), dp<uint32_t>(c->u_cnt),
+                      dp<uint32_t>(c->u_off), pl.ntiles, 0, c->m2l_xcd_run, pl.caps.units,
+                      dp<uint32_t>(c->items), pl.gbits, dp<uint32_t>(c->cols), c->g_af.ptr,
+                      c->mq.ptr, k, cells, dp<double>(c->L), dp<double>(c->u_part), mixed, s,
+                      reinterpret_cast<const int32_t *>(sz + SZ_CHUNK)));
   TRY(rec(c, EV_M2LT, s));
   if (pl.caps.fallback > 0) {
     Csr fl{dp<int32_t>(c->fb_off), dp<int32_t>(c->fb_src)};
@@ -2011,12 +2033,12 @@ int tfmm_set_tuning(tfmm_ctx *c, int knob, double value) {
   }
 }
 
-// Candidates of the tile-kernel knobs, tried jointly; the evaluation's time
+// Candidates of the set-kernel knobs, tried jointly; the evaluation's time
 // (HIP events around it) decides, median over the repetitions.  The P2P
 // schedule stays as set: running the P2P beside the tiles measured within
 // noise of running it beside the batch building, and it would fold the
-// P2P's time into the tile kernel's.
-// Candidates of the kernel knobs, timed in two stages: the tile kernel's
+// P2P's time into the set kernel's.
+// Candidates of the kernel knobs, timed in two stages: the set kernel's
 // (unit factor x XCD run) at the current P2P setting, then where the P2P
 // starts and how many resident waves it holds, at the best tile setting
 // (running the P2P from phase A with a few resident waves lets the upward

@@ -11,9 +11,11 @@
 //
 // Cells of one level sit on a lattice, so dX of a pair is an integer
 // multiple of half the finer cell's width: pairs are grouped by
-// (target level, source level, offset).  Every pair of a group shares T, so a
-// group's pairs become the columns of a matrix product T * [M_s1 ... M_s16].
-// The harmonics of each group are formed once, in FP64.
+// (level difference, offset), offsets that mirror each other in one group
+// (their operators differ by signs, which the kernel applies to the operands
+// as it takes a group's mirror).  Every pair of a group shares T, so a group's pairs
+// become the columns of a matrix product T * [M_s1 ... M_s16].  The harmonics
+// of each group are formed once, in FP64.
 //
 // Scaling: with sigma the width of each cell, the kernel works on
 //   M~_n = M_n / sigma_s^n,  L~_j = L_j sigma_t^(j+1),  Y~_p = Y_p sigma_t^(p+1)
@@ -22,27 +24,31 @@
 // power-of-two factors are exact.  Y~ depends only on the offset in units of
 // the cells' widths, so one group serves every tree of a batch.
 //
-// Work decomposition: targets are tiled by 128 consecutive cells (breadth
-// first, so one tile is one Morton range of one level); the pairs of a tile
-// are sorted by group, and each run of up to 16 pairs of one group is a work
-// item = 18 blocks x 4 MFMA 16x16x4 steps.  One workgroup (4 waves) owns a
-// tile and accumulates its local expansions in LDS; each wave owns fixed row
-// blocks of T, so the waves never write the same LDS word, walk the tile's
-// items independently, and the accumulation order is fixed (deterministic).
-// The item loop is software pipelined (the next items' operands are in
-// flight while an item is multiplied), and tiles are dealt to the XCDs in
-// runs of consecutive tiles so that one XCD's L2 holds the sources its tiles
-// share.  Pairs whose offset falls outside the group table (level
-// difference above 3, or an offset beyond the table's range) go to the
-// per-pair kernel of m2l.hip.
+// Work decomposition: targets are taken in sets of 16 consecutive cells (breadth
+// first, so one set is two families of siblings), and the 16 cells are the 16
+// columns of every product of the set: a column never changes its target, so
+// the 110 x 16 local expansions of a set stay in one wave's MFMA accumulators
+// over all its work, and nothing is read, added and written back per item.  The
+// pairs of a set are sorted by group; a work item is one group and, for each
+// target, one of the target's pairs in that group (in different mirrors, since
+// a target meets each offset once), or none.  That the mirrors of an offset
+// share a group is what fills the columns: siblings see the same offsets
+// mirrored, and a target at the edge of a region lacks some mirrors of many
+// offsets rather than whole offsets.  An item is 61 MFMA 16x16x4 steps.  A
+// set's items are cut into work units, one wave each, so that few or uneven
+// sets still fill the chip; the first unit writes the set's local expansions,
+// the others leave FP64 slabs that a second kernel adds in unit order.  Pairs
+// whose offset falls outside the group table (level difference above 3, or an
+// offset beyond the table's range) go to the per-pair kernel of m2l.hip.
 //
 // Per-group factors: the level factor 2^(n dl), n the source degree and
 // dl = l_t - l_s, is split as 2^(p dl) 2^(-j dl) with p = j + n, the first
 // folded into the group's harmonics (index p) and the second into the rows
 // (degree j) of the group's A operands, which are formed once per group
-// before the tile kernel; both are exact powers of two.
+// before the set kernel; both are exact powers of two.
 #include <algorithm>
 #include <cmath>
+#include <utility>
 #include <vector>
 
 #include "m2l_codes.h"
@@ -64,56 +70,25 @@ using m2lc::NBLK;
 using m2lc::NR;
 constexpr int NCODE = NBLK * 4 * 64;
 constexpr int SRC_BITS = 25;  // source cell bits of a grouped pair's value
-constexpr int TILE = 128;
-constexpr int TILE_WAVES = 4;
-constexpr int WAVE_SYNC = 64;  // items between block barriers in the tile loop
+constexpr int TILE = 16;      // cells of a target set
+constexpr int SET_BITS = 4;
 
 // ---------------------------------------------------------------------------
 // group table
 // ---------------------------------------------------------------------------
-// group table (m2l_groups.h)
-using m2lg::CROSS_MAX;
-using m2lg::CROSS_N;
-using m2lg::DL_MAX;
-using m2lg::SAME_HALF;
-using m2lg::SAME_N;
-using m2lg::SLOTS_CROSS;
-using m2lg::SLOTS_PER_LEVEL;
-using m2lg::SLOTS_SAME;
-// column word of the tile kernel: target slot (7 bits) | 128 | (l_t - l_s +
-// DL_MAX) << COL_DL | group << COL_G
-constexpr int COL_DL = 8;
-constexpr int COL_G = 11;
+using m2lg::MIRROR_BITS;
+// A grouped pair's value and an item's column word: source cell (SRC_BITS) |
+// in a value the target's place in its set << SRC_BITS | mirror bits << MIR_AT.
+constexpr int MIR_AT = SRC_BITS + SET_BITS;
+static_assert(MIR_AT + MIRROR_BITS == 32, "a value is one word");
 
-__device__ inline void slot_decode(int32_t slot, int &lt, int &ls, int o[3]) {
-  lt = slot / SLOTS_PER_LEVEL;
-  int idx = slot - lt * SLOTS_PER_LEVEL;
-  if (idx < SLOTS_SAME) {
-    ls = lt;
-    o[2] = (idx % SAME_N - SAME_HALF) * 2;
-    idx /= SAME_N;
-    o[1] = (idx % SAME_N - SAME_HALF) * 2;
-    o[0] = (idx / SAME_N - SAME_HALF) * 2;
-  } else {
-    idx -= SLOTS_SAME;
-    const int blk = idx / SLOTS_CROSS;
-    ls = lt + ((blk & 1) ? -(blk / 2 + 1) : (blk / 2 + 1));
-    idx %= SLOTS_CROSS;
-    o[2] = (idx % CROSS_N) * 2 - CROSS_MAX;
-    idx /= CROSS_N;
-    o[1] = (idx % CROSS_N) * 2 - CROSS_MAX;
-    o[0] = (idx / CROSS_N) * 2 - CROSS_MAX;
-  }
-}
-
-
-// Split the executed M2L pairs into grouped ones (sort key: tile << gbits |
-// group, value: source cell | slot in tile << SRC_BITS) and the rest (key:
-// target | source).  Within one (tile, group) segment every target occurs at
-// most once, so the order inside a segment does not affect any sum and the
-// key needs no slot bits.
+// Split the executed M2L pairs into grouped ones (sort key: set << gbits |
+// group) and the rest (key: target | source).  Among the pairs of one key,
+// target and mirror name the pair (a target has one level, so they fix the
+// source): k_items places each by them alone, whatever order the traversal's
+// atomics left.
 // Grouped keys stay at the pair's index; a pair outside the groups leaves
-// the key NO_GROUP there, which sorts after every grouped key (the tile
+// the key NO_GROUP there, which sorts after every grouped key (the set
 // field of a key is at most 2^tbits - 2), so a sort of all n keys puts the
 // grouped pairs first.  The pairs outside the groups are appended compactly
 // (counters[1], one atomic per block that has any); k_grouped_count then
@@ -121,6 +96,11 @@ __device__ inline void slot_decode(int32_t slot, int &lt, int &ls, int o[3]) {
 // With dn the pair count is *dn (n its capacity), and group indices are
 // clamped below gcap (a capacity the caller checks after the launch).
 constexpr uint32_t NO_GROUP = 0xffffffffu;
+
+__device__ inline uint32_t pair_value(int2 p, uint32_t slot) {
+  return ((uint32_t)p.y & CELL_MASK) | ((uint32_t)p.x % TILE) << SRC_BITS |
+         (slot & ((1u << MIRROR_BITS) - 1u)) << MIR_AT;
+}
 
 __global__ __launch_bounds__(1024) void k_classify(const int2 *pairs, const int32_t *slot_of,
                                                   uint32_t n, const uint32_t *gid_of_slot, int gbits,
@@ -142,9 +122,9 @@ __global__ __launch_bounds__(1024) void k_classify(const int2 *pairs, const int3
   const bool grouped = valid && slot >= 0;
   const bool fallback = valid && slot < 0;
   if (valid) {
-    const uint64_t tile = (uint32_t)p.x / TILE, in_tile = (uint32_t)p.x % TILE;
-    gkeys[i] = grouped ? (uint32_t)(tile << gbits) | min(gid_of_slot[slot], gcap - 1u) : NO_GROUP;
-    gvals[i] = grouped ? ((uint32_t)p.y & CELL_MASK) | (uint32_t)(in_tile << SRC_BITS) : 0u;
+    gkeys[i] = grouped ? ((uint32_t)p.x / TILE) << gbits | min(gid_of_slot[slot >> MIRROR_BITS], gcap - 1u)
+                       : NO_GROUP;
+    gvals[i] = grouped ? pair_value(p, (uint32_t)slot) : 0u;
   }
   if (!__syncthreads_or(fallback)) return;  // the usual block: nothing outside the groups
   const uint32_t af = block_append<16>(&counters[1], fallback, 1, scratch);
@@ -169,39 +149,35 @@ __global__ void k_classify_all(const int2 *pairs, const int32_t *slot_of, uint32
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int2 p = pairs[i];
-  const uint64_t tile = (uint32_t)p.x / TILE, in_tile = (uint32_t)p.x % TILE;
-  gkeys[i] = (uint32_t)(tile << gbits) | gid_of_slot[slot_of[i]];
-  gvals[i] = ((uint32_t)p.y & CELL_MASK) | (uint32_t)(in_tile << SRC_BITS);
+  const uint32_t slot = (uint32_t)slot_of[i];
+  gkeys[i] = ((uint32_t)p.x / TILE) << gbits | gid_of_slot[slot >> MIRROR_BITS];
+  gvals[i] = pair_value(p, slot);
 }
 
 // Harmonics of every used group, FP64, scaled: Y~_p^q = Y_p^q sigma_t^(p+1)
 // 2^(p dl), dl = l_t - l_s, i.e. the harmonics of the offset measured in
 // target widths.  Stored as NR reals (re/im interleaved, index 2 tri(p, q)),
 // in FP64 and FP32.
-__global__ void k_group_harmonics(const uint32_t *used, const uint32_t *gid_of_slot,
-                                  int32_t nslots, double *Y64, float *Y32, int8_t *gdl,
-                                  int8_t *glt, uint32_t gcap) {
+__global__ void k_group_harmonics(const uint32_t *used, const uint32_t *gid_of_slot, double *Y64,
+                                  float *Y32, int8_t *gdl, uint32_t gcap) {
   critical_path_priority();
   const int32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
-  if (slot >= nslots || !used[slot]) return;
+  if (slot >= m2lg::SLOTS || !used[slot]) return;
   const uint32_t g = gid_of_slot[slot];
   if (g >= gcap) return;  // more groups than the buffers hold (checked by the caller)
-  int lt, ls, o[3];
-  slot_decode(slot, lt, ls, o);
-  const int lf = lt > ls ? lt : ls;
-  const double half = ldexp(0.5, lt - lf);  // half the finer width, target width = 1
+  int sl, o[3];  // source level less target level
+  m2lg::slot_decode(slot, sl, o);
+  const double half = ldexp(0.5, -max(sl, 0));  // half the finer width, target width = 1
   const double dx = o[0] * half, dy = o[1] * half, dz = o[2] * half;
   double rho, alpha, beta;
   cart2sph(dx, dy, dz, rho, alpha, beta);
-  const double sig = 1.0;
   const double x = cos(alpha), y = sin(alpha);
   const cd ei = mk(cos(beta), sin(beta));
   double *yo = Y64 + (int64_t)g * NR;
   float *yf = Y32 + (int64_t)g * NR;
   for (int m = 0; m < P; m++) {
     local_column(m, rho, x, y, ei, [&](int n, int mm, cd v) {
-      double sc = ldexp(sig, n * (lt - ls));  // sigma^(n+1) 2^(n dl)
-      for (int i = 0; i < n; i++) sc *= sig;
+      const double sc = ldexp(1.0, -n * sl);  // 2^(n dl)
       const int t = tri(n, mm);
       yo[2 * t] = v.re * sc;
       yo[2 * t + 1] = v.im * sc;
@@ -211,22 +187,26 @@ __global__ void k_group_harmonics(const uint32_t *used, const uint32_t *gid_of_s
   }
   yo[110] = yo[111] = 0;
   yf[110] = yf[111] = 0;
-  gdl[g] = (int8_t)(lt - ls);
-  glt[g] = (int8_t)lt;
+  gdl[g] = (int8_t)-sl;
 }
 
-// M~ of every cell, in the quad-interleaved layout the MFMA B operand reads:
-// Mq[cell][q][t] = M~[cell][4 t + q], row r = 2 tri(n, m) + (0 re | 1 im).
+// M~ of every cell, in the order the MFMA B operands are read: row r = 4 t + q
+// (r = 2 tri(n, m) + (0 re | 1 im)) at 16 (t / 4) + 4 q + t % 4, so that the
+// four lanes (q) that read a column vector (four k-steps) of one source read
+// 64 contiguous bytes in FP32 (128 in FP64).  With each lane's 28 values
+// contiguous instead, every lane of a load would touch a cache line of its own,
+// 64 lines an instruction instead of 16.
+// Cell ncells is the source of empty columns: zeros.
 template <class T>
 __global__ void k_scale_m(Cells c, int32_t ncells, const double *M, T *Mq) {
   critical_path_priority();
   const int32_t ci = blockIdx.x;
-  if (ci >= ncells) return;
+  if (ci > ncells) return;
   const int r = threadIdx.x;  // 0..111
   if (r >= NR) return;
   const int q = r & 3, t = r >> 2;
   double v = 0;
-  if (r < 110) {
+  if (r < 110 && ci < ncells) {
     const int tt = r >> 1;
     int n = 0;
     while (tri(n + 1, 0) <= tt) n++;
@@ -236,145 +216,157 @@ __global__ void k_scale_m(Cells c, int32_t ncells, const double *M, T *Mq) {
     for (int i = 0; i < n; i++) sc *= isig;
     v = M[2 * ((int64_t)ci * NTERM + tt) + (r & 1)] * sc;
   }
-  Mq[(int64_t)ci * NR + q * 28 + t] = (T)v;
+  Mq[(int64_t)ci * NR + 16 * (t >> 2) + 4 * q + (t & 3)] = (T)v;
 }
 
 // ---------------------------------------------------------------------------
 // work items
 // ---------------------------------------------------------------------------
-// Position of every grouped pair in its (tile, group) segment, from the
-// sorted keys alone.  A target occurs at most once per segment, so a segment
-// holds at most TILE = 128 pairs: the block reads the 128 keys before its
-// own and 64 after, marks the segment starts (ballot per row of 64 keys),
-// and every pair finds its segment's start among the marks of its row and
-// the two rows before, and the next start among those of its row and the
-// row after.  Items are runs of 16 pairs of one segment: a pair starts one
-// when its position in the segment is a multiple of 16; ipos = position in
-// the segment | (pairs of the item) << 8 for an item start, and bcount[b]
-// the item starts among block b's pairs.
-constexpr int IP_WAVES = 16;
-constexpr int IP_ROWS = IP_WAVES + 3;  // 2 rows before the block's, 1 after
+// The items of the sorted pairs.  The pairs of one key (a segment: one set and
+// group) have at most 16 targets x 8 mirrors, each combination once, so a
+// segment is a 128-bit presence mask, and everything follows from it: the
+// segment needs as many items as its fullest target has pairs, and a pair goes
+// to the item given by its rank among its target's mirrors.  A block handles
+// the segments that start among its 1024 keys and reads 128 keys more for the
+// end of the last one.  The first pass (WRITE false) counts the block's items;
+// the second, with the exclusive prefix of the blocks' counts in bstart,
+// writes every item's key and 16 column words (empty: empty).  With dn the
+// pair count is *dn (n its capacity); items at or past items_cap are not
+// written (a capacity the caller checks).  Lists that the caller of the library
+// gives may repeat a target's place in a group (a pair twice, or sources of two
+// problems); the counting pass then sets *repeats.  (A segment longer than the
+// block can see has a repeat among the 129 keys that it does see.)
+constexpr int IT_THREADS = 1024;
+constexpr int IT_ROWS = IT_THREADS / 64 + 2;  // 2 rows after the block's own
+constexpr int SEG_WORDS = TILE * 8 / 32;      // words of a segment's mask
 
-__global__ __launch_bounds__(64 * IP_WAVES) void k_item_pos(const uint32_t *keys, uint32_t n,
-                                                            uint32_t *ipos, uint32_t *bcount,
-                                                            const uint32_t *dn) {
+template <bool WRITE>
+__global__ __launch_bounds__(IT_THREADS) void k_items(const uint32_t *keys, const uint32_t *vals,
+                                                      uint32_t n, uint32_t *bcount,
+                                                      const uint32_t *bstart, uint32_t empty,
+                                                      uint32_t *ikey, uint32_t *cols,
+                                                      const uint32_t *dn, uint32_t items_cap,
+                                                      uint32_t *repeats) {
   critical_path_priority();
-  __shared__ uint32_t sk[IP_ROWS * 64];
-  __shared__ uint64_t mark[IP_ROWS];
-  __shared__ uint32_t wcount[IP_WAVES];
+  __shared__ uint32_t sk[IT_ROWS * 64];        // keys of the window
+  __shared__ uint32_t rowstart[IT_ROWS + 1];   // segments that start before a row
+  __shared__ uint64_t mark[IT_ROWS];           // segment starts of a row
+  __shared__ uint32_t mask[IT_THREADS * SEG_WORDS];
+  __shared__ uint32_t first[IT_THREADS];       // a segment's first item, in the block
+  __shared__ uint32_t segkey[IT_THREADS];
+  __shared__ uint32_t wsum[IT_THREADS / 64];
   if (dn) n = min(n, *dn);
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int64_t w0 = (int64_t)blockIdx.x * (64 * IP_WAVES) - 128;  // key of window slot 0
-  for (int t = threadIdx.x; t < IP_ROWS * 64; t += 64 * IP_WAVES) {
-    const int64_t j = w0 + t;
-    // outside [0, n): a value no key takes (the tile field of a key is at
-    // most 2^tbits - 2), so the last segment ends at n
-    sk[t] = (j >= 0 && j < (int64_t)n) ? keys[j] : 0xffffffffu;
-  }
+  const int64_t w0 = (int64_t)blockIdx.x * IT_THREADS;
+  const uint32_t before = w0 > 0 && w0 - 1 < (int64_t)n ? keys[w0 - 1] : NO_GROUP;
+  for (int t = threadIdx.x; t < IT_ROWS * 64; t += IT_THREADS)
+    sk[t] = w0 + t < (int64_t)n ? keys[w0 + t] : NO_GROUP;
+  for (int t = threadIdx.x; t < IT_THREADS * SEG_WORDS; t += IT_THREADS) mask[t] = 0;
   __syncthreads();
-  for (int r = wid; r < IP_ROWS; r += IP_WAVES) {
+  for (int r = wid; r < IT_ROWS; r += IT_THREADS / 64) {
     const int t = 64 * r + lane;
-    const uint64_t m = __ballot(t == 0 || sk[t] != sk[t - 1]);
+    const uint64_t m = __ballot(sk[t] != NO_GROUP && sk[t] != (t ? sk[t - 1] : before));
     if (lane == 0) mark[r] = m;
   }
   __syncthreads();
-  const int R = wid + 2;
-  const int64_t i = w0 + 64 * R + lane;
-  bool first = false;
-  if (i < (int64_t)n) {
-    const uint64_t upto = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);  // bits <= lane
-    int start;  // window slot of the segment's first pair
-    if (mark[R] & upto) start = 64 * R + 63 - __clzll(mark[R] & upto);
-    else if (mark[R - 1]) start = 64 * (R - 1) + 63 - __clzll(mark[R - 1]);
-    else start = 64 * (R - 2) + 63 - __clzll(mark[R - 2]);  // mark[R - 2] has slot 0 at least
-    const int d = min(64 * R + lane - start, TILE - 1);
-    int next;  // window slot of the next segment's first pair
-    if (mark[R] & ~upto) next = 64 * R + __ffsll((unsigned long long)(mark[R] & ~upto)) - 1;
-    else if (mark[R + 1]) next = 64 * (R + 1) + __ffsll((unsigned long long)mark[R + 1]) - 1;
-    else next = 64 * (R + 2);
-    const int cnt = min(16, next - (64 * R + lane));
-    first = (d & 15) == 0;
-    ipos[i] = (uint32_t)d | (first ? (uint32_t)cnt << 8 : 0u);
-  }
-  const uint64_t fm = __ballot(first);
-  if (lane == 0) wcount[wid] = (uint32_t)__popcll(fm);
-  __syncthreads();
   if (threadIdx.x == 0) {
-    uint32_t t = 0;
-    for (int w = 0; w < IP_WAVES; w++) t += wcount[w];
-    bcount[blockIdx.x] = t;
+    uint32_t run = 0;
+    for (int r = 0; r < IT_ROWS; r++) {
+      rowstart[r] = run;
+      run += (uint32_t)__popcll(mark[r]);
+    }
+    rowstart[IT_ROWS] = run;
   }
-}
-
-// Item descriptors (first pair, pairs, group, tile) and the item's 16 column
-// descriptors: cols[16 item + j] = (source cell, target slot in tile
-// | 128 if column j holds a pair | (level difference + DL_MAX) << COL_DL
-// | group << COL_G).
-// Every column carries the group, so that every lane of the tile kernel can
-// fetch the group's data.
-// Blocks as in k_item_pos; bstart: exclusive prefix of its block counts.
-// With dn the pair count is *dn (n its capacity); items at or past
-// items_cap are not written (a capacity the caller checks).
-__global__ __launch_bounds__(64 * IP_WAVES) void k_items(const uint32_t *keys,
-                                                         const uint32_t *vals,
-                                                         const uint32_t *ipos,
-                                                         const uint32_t *bstart, uint32_t n,
-                                                         int gbits, const int8_t *gdl,
-                                                         int4 *items, uint2 *cols,
-                                                         const uint32_t *dn, uint32_t items_cap) {
-  critical_path_priority();
-  __shared__ uint32_t wcount[IP_WAVES];
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (dn) n = min(n, *dn);
-  const bool valid = i < n;
-  const uint32_t ip = valid ? ipos[i] : 1u;
-  const bool first = valid && (ip & 15u) == 0;
-  // item of pair i = item starts at or before i, less one
-  const uint64_t fm = __ballot(first);
-  if (lane == 0) wcount[wid] = (uint32_t)__popcll(fm);
   __syncthreads();
-  if (!valid) return;
-  uint32_t before = bstart[blockIdx.x];
-  for (int w = 0; w < wid; w++) before += wcount[w];
-  const uint64_t upto = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
-  const uint32_t item = before + (uint32_t)__popcll(fm & upto) - 1;
-  const uint32_t jj = ip & 15u;
-  const uint32_t k = keys[i], v = vals[i];
-  const uint32_t g = k & ((1u << gbits) - 1u);
-  const uint32_t gw = (uint32_t)(gdl[g] + DL_MAX) << COL_DL | (g << COL_G);
-  if (item >= items_cap) return;
-  cols[(int64_t)item * 16 + jj] =
-      make_uint2(v & ((1u << SRC_BITS) - 1u), (v >> SRC_BITS) | 128u | gw);
-  if (first) {  // first pair of the item: descriptor and padding columns
-    const uint32_t cnt = ip >> 8;  // pairs of the segment from i on, at most 16
-    int4 it;
-    it.x = (int)i;                             // first pair
-    it.y = (int)cnt;                           // pairs in the item
-    it.z = (int)g;                             // group
-    it.w = (int)(k >> gbits);                  // tile
-    items[item] = it;
-    for (uint32_t j2 = cnt; j2 < 16; j2++) cols[(int64_t)item * 16 + j2] = make_uint2(0u, gw);
+  const uint32_t nseg = rowstart[IT_THREADS / 64];  // segments that start in the block's own keys
+  const uint64_t upto = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);  // bits <= lane
+  // segment of window key t, or -1: it starts before the block or after its keys
+  auto segment = [&](int t) -> int {
+    if (sk[t] == NO_GROUP) return -1;
+    const int s = (int)(rowstart[t >> 6] + (uint32_t)__popcll(mark[t >> 6] & upto)) - 1;
+    return s < (int)nseg ? s : -1;
+  };
+  for (int t = threadIdx.x; t < IT_ROWS * 64; t += IT_THREADS) {
+    const int s = segment(t);
+    if (s < 0) continue;
+    const uint32_t v = vals[w0 + t];
+    const uint32_t sl = (v >> SRC_BITS) & (TILE - 1), mi = v >> MIR_AT;
+    const uint32_t bit = 1u << (8 * (sl & 3) + mi);
+    if ((atomicOr(&mask[s * SEG_WORDS + (sl >> 2)], bit) & bit) && !WRITE && repeats) *repeats = 1;
+    segkey[s] = sk[t];
+  }
+  __syncthreads();
+  // items of segment threadIdx.x, and their exclusive prefix in the block
+  uint32_t cnt = 0;
+  if (threadIdx.x < nseg) {
+    for (int w = 0; w < SEG_WORDS; w++) {
+      const uint32_t m = mask[threadIdx.x * SEG_WORDS + w];
+      for (int b = 0; b < 4; b++) cnt = max(cnt, (uint32_t)__popc((m >> (8 * b)) & 0xffu));
+    }
+  }
+  uint32_t inc = cnt;
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t u = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += u;
+  }
+  if (lane == 63) wsum[wid] = inc;
+  __syncthreads();
+  uint32_t pre = 0, tot = 0;
+  for (int w = 0; w < IT_THREADS / 64; w++) {
+    pre += w < wid ? wsum[w] : 0u;
+    tot += wsum[w];
+  }
+  if (!WRITE) {
+    if (threadIdx.x == 0) bcount[blockIdx.x] = tot;
+    return;
+  }
+  const uint32_t base = bstart[blockIdx.x];
+  first[threadIdx.x] = pre + inc - cnt;
+  if (threadIdx.x < nseg)
+    for (uint32_t k = 0; k < cnt; k++) {
+      const uint32_t it = base + first[threadIdx.x] + k;
+      if (it < items_cap) ikey[it] = segkey[threadIdx.x];
+    }
+  __syncthreads();
+  // the pairs' columns
+  for (int t = threadIdx.x; t < IT_ROWS * 64; t += IT_THREADS) {
+    const int s = segment(t);
+    if (s < 0) continue;
+    const uint32_t v = vals[w0 + t];
+    const uint32_t sl = (v >> SRC_BITS) & (TILE - 1), mi = v >> MIR_AT;
+    const uint32_t m = (mask[s * SEG_WORDS + (sl >> 2)] >> (8 * (sl & 3))) & 0xffu;
+    const uint32_t it = base + first[s] + (uint32_t)__popc(m & ((1u << mi) - 1u));
+    if (it < items_cap)
+      cols[(int64_t)it * TILE + sl] = (v & ((1u << SRC_BITS) - 1u)) | mi << MIR_AT;
+  }
+  // the empty columns
+  for (uint32_t e = threadIdx.x; e < nseg * TILE; e += IT_THREADS) {
+    const uint32_t s = e / TILE, sl = e % TILE;
+    const uint32_t end = s + 1 < nseg ? first[s + 1] : tot;
+    const uint32_t m = (mask[s * SEG_WORDS + (sl >> 2)] >> (8 * (sl & 3))) & 0xffu;
+    for (uint32_t it = first[s] + (uint32_t)__popc(m); it < end; it++)
+      if (base + it < items_cap) cols[(int64_t)(base + it) * TILE + sl] = empty;
   }
 }
 
-__global__ void k_tile_offsets(const int4 *items, uint32_t nitems, int32_t ntiles,
-                               int32_t *off, const uint32_t *dnitems) {
+// first item of every set
+__global__ void k_set_offsets(const uint32_t *ikey, uint32_t nitems, int gbits, int32_t nsets,
+                              int32_t *off, const uint32_t *dnitems) {
   critical_path_priority();
   const int32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t > ntiles) return;
+  if (t > nsets) return;
   if (dnitems) nitems = min(nitems, *dnitems);
   uint32_t lo = 0, hi = nitems;
   while (lo < hi) {
     const uint32_t mid = lo + ((hi - lo) >> 1);
-    if (items[mid].w < t) lo = mid + 1;
+    if ((ikey[mid] >> gbits) < (uint32_t)t) lo = mid + 1;
     else hi = mid;
   }
   off[t] = (int32_t)lo;
 }
 
 // ---------------------------------------------------------------------------
-// the tile kernel
+// the set kernel
 // ---------------------------------------------------------------------------
 template <class T>
 struct Mfma;
@@ -387,7 +379,7 @@ struct Mfma<float> {
   static __device__ inline V step(float a, float b, V c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
-  static __device__ inline int row(int q, int i) { return 4 * q + i; }
+  static __host__ __device__ constexpr int row(int q, int i) { return 4 * q + i; }
 };
 template <>
 struct Mfma<double> {
@@ -395,32 +387,65 @@ struct Mfma<double> {
   static __device__ inline V step(double a, double b, V c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
-  static __device__ inline int row(int q, int i) { return q + 4 * i; }
+  static __host__ __device__ constexpr int row(int q, int i) { return q + 4 * i; }
 };
 
-// Work split of one item over the 4 waves of a tile: each wave owns fixed
-// (row block, column block) pairs of T, so the waves write disjoint rows of
-// the tile's expansions and need no atomics and no barriers between items.
-// Row block 0 has 7 column blocks and is split between waves 0 and 1 (wave 1
-// accumulates its part in a separate array, added at the end).
-//   wave 0: (0,0) (0,1) (0,2) (0,3) (6,0)
-//   wave 1: (0,4) (0,5) (0,6) (4,0) (5,0)
-//   wave 2: (1,0) (1,1) (1,2) (1,3)
-//   wave 3: (2,0) (2,1) (3,0) (3,1)
-// Blocks of one row block accumulate into one MFMA accumulator (WAVE_F).
-constexpr int WAVE_NBLK[TILE_WAVES] = {5, 5, 4, 4};
-constexpr int WAVE_BLK[TILE_WAVES][5] = {
-    {0, 1, 2, 3, 17}, {4, 5, 6, 15, 16}, {7, 8, 9, 10, -1}, {11, 12, 13, 14, -1}};
-constexpr int WAVE_NRB[TILE_WAVES] = {2, 3, 1, 2};
-constexpr int WAVE_RBS[TILE_WAVES][3] = {{0, 6, -1}, {0, 4, 5}, {1, -1, -1}, {2, 3, -1}};
-constexpr int WAVE_F[TILE_WAVES][5] = {
-    {0, 0, 0, 0, 1}, {0, 0, 0, 1, 2}, {0, 0, 0, 0, -1}, {0, 0, 1, 1, -1}};
+// The steps of one item.  T has 7 row blocks of 16 rows and 28 k-steps of 4
+// columns; the step (row block, k-step) is non-zero only while the smallest
+// degrees of its rows and columns add up to at most P - 1, which leaves 61 of
+// the 196 (18 whole 16 x 16 blocks would be 72): the first RB_STEPS[rb] k-steps
+// of row block rb.  They are taken row block by row block, the last three
+// (6 steps) in turn: an MFMA's results take a while to arrive, and a row block
+// is added to the sums some steps after its last one.
+constexpr int NRB = 7;
+constexpr int RB_STEPS[NRB] = {28, 14, 8, 5, 3, 2, 1};
+constexpr int NST = 61;
+constexpr int NAV = (NST + 3) / 4;  // A operand vectors of an item (four steps each)
+constexpr int NBV = NR / 16;        // B operand vectors (four k-steps each)
 
-__host__ __device__ constexpr bool wave_needs_cb(int w, int cb) {
-  for (int e = 0; e < WAVE_NBLK[w]; e++)
-    if (BLK_CB[WAVE_BLK[w][e]] == cb) return true;
-  return false;
+__host__ __device__ constexpr int coef_degree(int r) {
+  int n = 0;
+  while ((n + 1) * (n + 2) / 2 <= r / 2) n++;
+  return n;
 }
+constexpr bool steps_cover() {
+  int n = 0;
+  for (int rb = 0; rb < NRB; rb++)
+    for (int t = 0; t < 28; t++) {
+      const bool need = coef_degree(16 * rb) + coef_degree(4 * t) <= P - 1;
+      if (need != (t < RB_STEPS[rb])) return false;
+      n += need;
+    }
+  return n == NST;
+}
+static_assert(steps_cover(), "every non-zero k-step of the operator once");
+// row block, k-step and MFMA block (m2l_codes.h; block * 4 + k-step in it) of
+// every step, -1 for the padding of the last vector
+struct StepTab {
+  int16_t rb[NAV * 4], t[NAV * 4], code[NAV * 4];
+};
+constexpr StepTab make_steps() {
+  StepTab s{};
+  int n = 0;
+  for (int rb = 0; rb < 4; rb++)
+    for (int t = 0; t < RB_STEPS[rb]; t++, n++) {
+      s.rb[n] = (int16_t)rb;
+      s.t[n] = (int16_t)t;
+    }
+  for (int t = 0; t < 3; t++)
+    for (int rb = 4; rb < NRB; rb++)
+      if (t < RB_STEPS[rb]) {
+        s.rb[n] = (int16_t)rb;
+        s.t[n++] = (int16_t)t;
+      }
+  for (int i = 0; i < n; i++)
+    for (int b = 0; b < NBLK; b++)
+      if (BLK_RB[b] == s.rb[i] && BLK_CB[b] == s.t[i] / 4) s.code[i] = (int16_t)(4 * b + s.t[i] % 4);
+  for (; n < NAV * 4; n++) s.rb[n] = s.t[n] = s.code[n] = -1;
+  return s;
+}
+constexpr StepTab STEP = make_steps();
+__constant__ StepTab c_steps = make_steps();
 
 __device__ inline int row_degree(int r) {
   if (r >= 110) return 0;
@@ -430,31 +455,10 @@ __device__ inline int row_degree(int r) {
   return n;
 }
 
-// B fragments (4 k-steps) of the column blocks wave W multiplies, for the
-// source whose M~ starts at mq (already offset by the lane's k-row quad)
-template <class T, int W>
-__device__ inline void load_b(T (&b)[7][4], const T *mq) {
-#pragma unroll
-  for (int cb = 0; cb < 7; cb++) {
-    if (wave_needs_cb(W, cb)) {
-#pragma unroll
-      for (int kk = 0; kk < 4; kk++) b[cb][kk] = mq[4 * cb + kk];
-    }
-  }
-}
-
-// A operands of every group, in the order the tile kernel's lanes read them:
-// Af[g][AF_SLOT(w, e)][lane][kk] is the entry of block WAVE_BLK[w][e] at
-// k-step kk that lane supplies (a 16-byte vector per lane and block in FP32,
-// 32 in FP64), so a wave reads its operands of a new group with one
-// contiguous, conflict-free load per block.  Slots number the (wave, block)
-// pairs wave by wave: slot = sum of WAVE_NBLK[0 .. w-1] + e.
-constexpr int AF_PER_GROUP = NBLK * 64 * 4;  // elements per group
-__host__ __device__ constexpr int af_slot(int w, int e) {
-  int s = e;
-  for (int i = 0; i < w; i++) s += WAVE_NBLK[i];
-  return s;
-}
+// A operands of every group, in the order the set kernel's lanes read them:
+// Af[g][s / 4][lane][s % 4] is what lane supplies at step s (four steps are a
+// 16-byte vector per lane in FP32, 32 in FP64).
+constexpr int AF_PER_GROUP = NAV * 4 * 64;  // elements per group
 
 template <class T>
 struct Vec4;
@@ -467,146 +471,152 @@ struct Vec4<double> {
   typedef d4 V;
 };
 
-// A operands of wave W for the group whose fragments start at af
-template <class T, int W>
-__device__ inline void load_a(T (&a)[WAVE_NBLK[W] * 4], const T *af, int lane) {
-  typedef typename Vec4<T>::V V;
+// Signs of a mirrored offset (m2l_groups.h): T(R o) = S T(o) S.  The operator
+// stays that of the unmirrored offset; a column's source and its products are
+// multiplied by S.  Bit t of b[d][q]: mirroring axis d changes the sign of row
+// 4 t + q (a lane's B operands).
+// p[FP64][d][q]: the same for bit 4 rb + i, result i of row block rb.
+struct MirrorTab {
+  uint32_t b[3][4], p[2][3][4];
+};
+constexpr MirrorTab make_mirror() {
+  MirrorTab t{};
+  for (int d = 0; d < 3; d++) {
+    for (int r = 0; r < NR; r++) t.b[d][r & 3] |= (uint32_t)m2lg::mirror_sign(d, r) << (r >> 2);
+    for (int q = 0; q < 4; q++)
+      for (int rb = 0; rb < NRB; rb++)
+        for (int i = 0; i < 4; i++) {
+          const int bit = 4 * rb + i;
+          t.p[0][d][q] |= (uint32_t)m2lg::mirror_sign(d, 16 * rb + Mfma<float>::row(q, i)) << bit;
+          t.p[1][d][q] |= (uint32_t)m2lg::mirror_sign(d, 16 * rb + Mfma<double>::row(q, i)) << bit;
+        }
+  }
+  return t;
+}
+__constant__ MirrorTab c_mirror = make_mirror();
+
+// a lane's sign masks for the three axes: its B operands and its products
+struct LaneSigns {
+  uint32_t b[3], p[3];
+  __device__ static uint32_t of(const uint32_t (&m)[3], uint32_t mirror) {
+    return ((mirror & 1u) ? m[0] : 0u) ^ ((mirror & 2u) ? m[1] : 0u) ^ ((mirror & 4u) ? m[2] : 0u);
+  }
+};
+template <class T>
+__device__ inline LaneSigns lane_signs(int q) {
+  LaneSigns s;
 #pragma unroll
-  for (int e = 0; e < WAVE_NBLK[W]; e++) {
-    const V v = *reinterpret_cast<const V *>(af + (af_slot(W, e) * 64 + lane) * 4);
+  for (int d = 0; d < 3; d++) {
+    s.b[d] = c_mirror.b[d][q];
+    s.p[d] = c_mirror.p[sizeof(T) == 8][d][q];
+  }
+  return s;
+}
+
+// x with its sign changed where bit `at` of mask is set
+__device__ inline float flip(float x, uint32_t mask, int at) {
+  return __uint_as_float(__float_as_uint(x) ^ ((mask << (31 - at)) & 0x80000000u));
+}
+__device__ inline double flip(double x, uint32_t mask, int at) {
+  return __hiloint2double(__double2hiint(x) ^ (int)((mask << (31 - at)) & 0x80000000u),
+                          __double2loint(x));
+}
+
+// sums of row block rb += products, with their signs
+template <class T>
+__device__ inline void add_products(typename Mfma<T>::V (&sum)[NRB], int rb,
+                                    const typename Mfma<T>::V &v, uint32_t signs) {
 #pragma unroll
-    for (int kk = 0; kk < 4; kk++) a[e * 4 + kk] = v[kk];
+  for (int i = 0; i < 4; i++) {
+    sum[rb][i] += flip(v[i], signs, 4 * rb + i);
+    asm volatile("" : "+v"(sum[rb][i]));  // added here, not when the sum is next needed
   }
 }
 
-// Pipeline state of one wave at item it: everything was loaded during item
-// it - 1, so nothing the item consumes is still in flight when it starts;
-// acc holds the products of item it - 1, stored during item it.
-template <class T, int W>
-struct WaveState {
-  uint2 c_cur;  // columns of it (sources of its B operands were c_b of it - 1)
-  uint2 c_b;    // columns of it + 1 (sources and group of the next operands)
-  uint2 c_st;   // columns of it - 1 (target slots and level difference of acc)
-  T b[7][4];    // B operands of it
-  typename Mfma<T>::V acc[WAVE_NRB[W]];  // products of it - 1
+// One wave's registers: the operands of the current group, the sums, and the
+// products of the last three row blocks of the item before (with their signs),
+// which are added during this one.
+template <class T>
+struct SetRegs {
+  typename Vec4<T>::V a[NAV];
+  typename Mfma<T>::V sum[NRB], late[3];
+  uint32_t late_signs;
 };
 
-// add the products of one item (columns c) into the tile's expansions
-template <class T, int W>
-__device__ inline void store_item(const typename Mfma<T>::V (&acc)[WAVE_NRB[W]], uint2 c,
-                                  T (*Lt)[NR + 1], T (*Lt0b)[17], int q) {
-  if (!(c.y & 128u)) return;
-  const uint32_t ts = c.y & 127u;
+// One item: 61 MFMAs, and between them the loads of the next item's B operands
+// (from next into bn) and, when its group differs (change), of its A operands
+// (from af, each vector over itself once its last step is issued): they have
+// most of an item to arrive.  A wave issues in order and waits at an MFMA until
+// the matrix unit is free, so what is written between two MFMAs costs no time
+// as long as it is short, and what is loaded after the last one is waited for.
+// The loads over a vector in use stand in branches of their own because the
+// compiler would otherwise lift them above the vector's last use and move the
+// values back at the end, waiting for them.
+// Every row block's products are summed from zero over the item and then added
+// to the target's sums: long chains into the sums themselves would lose more to
+// rounding in FP32 (relative 1.2e-6 between two groupings of one problem's
+// pairs, against 6e-7).  bs, ss: signs of b and of the products.
+template <class T, int S>
+__device__ inline void set_step(SetRegs<T> &r, typename Vec4<T>::V (&b)[NBV],
+                                typename Vec4<T>::V (&bn)[NBV], typename Mfma<T>::V (&p)[NRB],
+                                uint32_t bs, uint32_t ss, const T *next, bool change,
+                                const T *af) {
+  typedef typename Vec4<T>::V V;
+  constexpr int rb = STEP.rb[S], t = STEP.t[S];
+  if constexpr (S < 28 && S % 4 == 0) {
+    bn[S / 4] = *reinterpret_cast<const V *>(next + 4 * S);
 #pragma unroll
-  for (int f = 0; f < WAVE_NRB[W]; f++) {
+    for (int k = 0; k < 4; k++) b[S / 4][k] = flip(b[S / 4][k], bs, S + k);
+  }
+  if constexpr (t == 0) p[rb] = (typename Mfma<T>::V){0, 0, 0, 0};
+  p[rb] = Mfma<T>::step(r.a[S / 4][S % 4], b[t / 4][t % 4], p[rb]);
+  if constexpr (S == 11) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int r = Mfma<T>::row(q, i);
-      const T v = acc[f][i];
-      if (W == 1 && WAVE_RBS[W][f] == 0) {
-        Lt0b[ts][r] += v;
-      } else {
-        const int row = WAVE_RBS[W][f] * 16 + r;
-        if (row < 110) Lt[ts][row] += v;
-      }
-    }
+    for (int i = 0; i < 3; i++) add_products<T>(r.sum, 4 + i, r.late[i], r.late_signs);
+  }
+  // row block rb is added four steps into the next one
+  constexpr int end[4] = {28, 28 + 14, 28 + 14 + 8, 28 + 14 + 8 + 5};
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+    if (S == end[k] + 3) add_products<T>(r.sum, k, p[k], ss);
+  if constexpr (S % 4 == 3 || S == NST - 1) {
+    if (change) r.a[S / 4] = *reinterpret_cast<const V *>(af + (S / 4) * 256);
   }
 }
 
-// One item of wave W with the state of it in cur; fills nxt for it + 1.
-// Order: the item's MFMAs are issued first; the loads of the next item's
-// operands and the store of the previous item's products are independent of
-// them and overlap their execution.  Loads issued here are consumed by the
-// next call.  The state is double buffered by unrolling the caller's loop by
-// two (a register rotation would wait for the loads just issued).
-template <class T, int W>
-__device__ inline void wave_item(WaveState<T, W> &cur, WaveState<T, W> &nxt,
-                                 T (&a)[WAVE_NBLK[W] * 4], int32_t it, int32_t ib, int32_t last,
-                                 const uint2 *cols, const T *Af, const T *Mq, T (*Lt)[NR + 1],
-                                 T (*Lt0b)[17], int lane) {
-  constexpr int NB = WAVE_NBLK[W], NF = WAVE_NRB[W];
-  const int q = lane >> 4, j = lane & 15;
-  // the matrix work of it
+template <class T, int... S>
+__device__ inline void set_steps(std::integer_sequence<int, S...>, SetRegs<T> &r,
+                                 typename Vec4<T>::V (&b)[NBV], typename Vec4<T>::V (&bn)[NBV],
+                                 uint32_t bs, uint32_t ss, const T *next, bool change,
+                                 const T *af) {
+  typename Mfma<T>::V p[NRB];
+  (set_step<T, S>(r, b, bn, p, bs, ss, next, change, af), ...);
 #pragma unroll
-  for (int f = 0; f < NF; f++) nxt.acc[f] = (typename Mfma<T>::V){0, 0, 0, 0};
-#pragma unroll
-  for (int kk = 0; kk < 4; kk++) {
-#pragma unroll
-    for (int e = 0; e < NB; e++)
-      nxt.acc[WAVE_F[W][e]] = Mfma<T>::step(a[e * 4 + kk], cur.b[BLK_CB[WAVE_BLK[W][e]]][kk],
-                                            nxt.acc[WAVE_F[W][e]]);
-  }
-  nxt.c_st = cur.c_cur;
-  // loads for the next items (indices clamped: loads stay in range)
-  nxt.c_cur = cur.c_b;
-  nxt.c_b = cols[(int64_t)min(it + 2, last) * 16 + j];
-  load_b<T, W>(nxt.b, Mq + (int64_t)cur.c_b.x * NR + q * 28);
-  // A operands of it + 1, loaded over those of it (the MFMAs above have
-  // read them) when the group changes: consecutive items of one group share
-  // them, and every column of an item carries its group, so the branch is
-  // uniform
-  const uint32_t gn = cur.c_b.y >> COL_G;
-  if (gn != (cur.c_cur.y >> COL_G)) load_a<T, W>(a, Af + (int64_t)gn * AF_PER_GROUP, lane);
-  // the products of it - 1
-  store_item<T, W>(cur.acc, cur.c_st, Lt, Lt0b, q);
-  // keep the 4 waves within a few items of each other: they read the same
-  // source multipoles, which then come from L2 once instead of 4 times
-  if (((it - ib) & (WAVE_SYNC - 1)) == WAVE_SYNC - 1) __syncthreads();
-}
-
-// The item loop of wave W over the tile's items [ib, ie).
-template <class T, int W>
-__device__ inline void run_wave(const uint2 *cols, int32_t ib, int32_t ie, const T *Af,
-                                const T *Mq, T (*Lt)[NR + 1], T (*Lt0b)[17], int lane) {
-  constexpr int NF = WAVE_NRB[W];
-  if (ib >= ie) return;
-  const int q = lane >> 4, j = lane & 15;
-  const int32_t last = ie - 1;
-
-  WaveState<T, W> s0, s1;
-  s0.c_cur = cols[(int64_t)ib * 16 + j];
-  s0.c_b = cols[(int64_t)min(ib + 1, last) * 16 + j];
-  s0.c_st = make_uint2(0u, 0u);  // no previous item
-#pragma unroll
-  for (int f = 0; f < NF; f++) s0.acc[f] = (typename Mfma<T>::V){0, 0, 0, 0};
-  load_b<T, W>(s0.b, Mq + (int64_t)s0.c_cur.x * NR + q * 28);
-  T a[WAVE_NBLK[W] * 4];  // A operands of the current item
-  load_a<T, W>(a, Af + (int64_t)(s0.c_cur.y >> COL_G) * AF_PER_GROUP, lane);
-  for (int32_t it = ib; it < ie; it += 2) {
-    wave_item<T, W>(s0, s1, a, it, ib, last, cols, Af, Mq, Lt, Lt0b, lane);
-    if (it + 1 < ie) wave_item<T, W>(s1, s0, a, it + 1, ib, last, cols, Af, Mq, Lt, Lt0b, lane);
-  }
-  // the products of the last item
-  if ((ie - ib) & 1) store_item<T, W>(s1.acc, s1.c_st, Lt, Lt0b, q);
-  else store_item<T, W>(s0.acc, s0.c_st, Lt, Lt0b, q);
+  for (int i = 0; i < 3; i++) r.late[i] = p[4 + i];
+  r.late_signs = ss;
 }
 
 // Workgroups are dispatched to the 8 XCDs round robin (workgroup b to XCD
-// b % 8) and every XCD has its own L2.  Consecutive tiles are neighbouring
-// target ranges of one level and share most of their source cells, so each
-// run of 256 tiles is dealt out as 8 blocks of 32 consecutive tiles, one per
-// XCD: the tiles an XCD runs at the same time read the same sources from
-// its L2.  The last partial run keeps the identity order (a bijection).
+// b % 8) and every XCD has its own L2.  Consecutive sets are neighbouring
+// target ranges of one level and share most of their source cells, so units
+// are dealt out in runs of RUN_UNITS x run consecutive units, one run per XCD
+// in turn: the units an XCD runs at the same time read the same sources from
+// its L2.  The last partial round keeps the identity order (a bijection).
 // The run length is a tuning knob (32 by default).
+constexpr int RUN_UNITS = 8;
 constexpr int NXCD = 8;
-__device__ inline int tile_of_block(int b, int ntiles, int run) {
+__device__ inline int unit_of_block(int b, int nunits, int run) {
+  run *= RUN_UNITS;
   const int S = NXCD * run;
-  if (run <= 1 || b >= (ntiles / S) * S) return b;
+  if (b >= (nunits / S) * S) return b;
   const int local = b % S;
   return (b - local) + (local % NXCD) * run + local / NXCD;
 }
 
-// Work units: a tile's items are cut into runs of about `chunk` items, one
-// workgroup each, so that a tile with many sparse groups (a coarse leaf next
-// to a much finer region) does not hold the whole launch back.  Unit k of a
-// tile starts at the first segment (group) boundary at or after item
-// k chunk: a segment never straddles two units, and since a target occurs
-// at most once per segment, which of a target's terms a unit sums does not
-// depend on the order of the items inside a segment (which the traversal's
-// atomics leave open).  The first unit adds its products to L directly, the
-// others leave theirs in part[] (one 128 x 110 slab per extra unit, FP64),
-// which k_unit_combine adds in unit order after the launch, so the sums do
-// not depend on timing.
+// Work units: unit k of a set is its items [k chunk, (k + 1) chunk).  The first
+// unit writes the set's L, the others leave theirs in part[] (one 16 x 110 slab
+// per extra unit, FP64), which k_unit_combine adds in unit order after the
+// launch, so the sums do not depend on timing.
 __global__ void k_unit_counts(const int32_t *tile_off, int32_t ntiles, int32_t chunk,
                               uint32_t *ucnt, const int32_t *dchunk) {
   critical_path_priority();
@@ -641,15 +651,24 @@ __global__ void k_unit_combine(const uint32_t *ucnt, const uint32_t *uoff, int32
   while (n > 1 && extra_slab(uoff, t, n - 1) >= nslab) n--;
   if (n <= 1) return;
   const int32_t first = t * TILE;
-  for (int e = threadIdx.x; e < TILE * 110; e += blockDim.x) {
-    const int sl = e / 110, row = e - sl * 110;
-    const int32_t ci = first + sl;
-    if (ci >= ncells) continue;
-    double *dst = &L[2 * ((int64_t)ci * NTERM + (row >> 1)) + (row & 1)];
-    double v = *dst;
-    for (int k = 1; k < n; k++) v += part[extra_slab(uoff, t, k) * (TILE * 110) + e];
-    *dst = v;
+  const int e = blockIdx.y * blockDim.x + threadIdx.x;
+  if (e >= TILE * 110) return;
+  const int sl = e / 110, row = e - sl * 110;
+  const int32_t ci = first + sl;
+  if (ci >= ncells) return;
+  double *dst = &L[2 * ((int64_t)ci * NTERM + (row >> 1)) + (row & 1)];
+  const double *p = part + extra_slab(uoff, t, 1) * (TILE * 110) + e;
+  double v = *dst;
+  int k = 1;
+  for (; k + 8 <= n; k += 8) {  // eight loads in flight, added in order
+    double x[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) x[i] = p[(int64_t)(k - 1 + i) * (TILE * 110)];
+#pragma unroll
+    for (int i = 0; i < 8; i++) v += x[i];
   }
+  for (; k < n; k++) v += p[(int64_t)(k - 1) * (TILE * 110)];
+  *dst = v;
 }
 
 // A fragments of every group from its harmonics: the entry that lane
@@ -668,94 +687,137 @@ template <class T>
 __global__ void k_group_afrag(const T *Yg, uint32_t ng, const uint32_t *codes, const int8_t *gdl,
                               T *Af, const uint32_t *dng) {
   critical_path_priority();
+  constexpr int VPG = AF_PER_GROUP / 4;  // vectors per group
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (dng) ng = min(ng, *dng);
-  if (t >= (int64_t)ng * (NBLK * 64)) return;
-  const int64_t g = t / (NBLK * 64);
-  const int r = (int)(t - g * (NBLK * 64));
+  if (t >= (int64_t)ng * VPG) return;
+  const int64_t g = t / VPG;
+  const int r = (int)(t - g * VPG);
   const int slot = r >> 6, lane = r & 63;
-  int w = 0, e = slot;
-  while (w < TILE_WAVES - 1 && e >= WAVE_NBLK[w]) {
-    e -= WAVE_NBLK[w];
-    w++;
-  }
-  const int b = WAVE_BLK[w][e];
   const T *y = Yg + g * NR;
-  // row factor 2^(-j dl) of the entry's row (degree j)
-  const int rexp = -row_degree(BLK_RB[b] * 16 + (lane & 15)) * (int)gdl[g];
   typename Vec4<T>::V out;
 #pragma unroll
   for (int kk = 0; kk < 4; kk++) {
-    const uint32_t cw = codes[(b * 4 + kk) * 64 + lane];
+    const int at = c_steps.code[slot * 4 + kk];
+    if (at < 0) {
+      out[kk] = 0;
+      continue;
+    }
+    // row factor 2^(-j dl) of the entry's row (degree j)
+    const int rexp = -row_degree(BLK_RB[at >> 2] * 16 + (lane & 15)) * (int)gdl[g];
+    const uint32_t cw = codes[at * 64 + lane];
     out[kk] = ldexp(table_elem(y, cw & 0xffffu) + table_elem(y, cw >> 16), rexp);
   }
-  *reinterpret_cast<typename Vec4<T>::V *>(Af + g * AF_PER_GROUP + (slot * 64 + lane) * 4) = out;
+  *reinterpret_cast<typename Vec4<T>::V *>(Af + t * 4) = out;
 }
 
+// degree of result i of row block rb: a constant per lane quarter q
 template <class T>
-__global__ __launch_bounds__(64 * TILE_WAVES) void k_m2l_tiles(
-    const int32_t *tile_off, const int2 *units, const uint32_t *ucnt, const uint32_t *uoff,
-    int32_t ntiles, int32_t chunk, int xcd_run, const uint2 *cols, const T *Af, const T *Mq,
-    Cells c, int32_t ncells, double *L, double *part, const int32_t *dchunk, int64_t nslab) {
+__device__ inline int result_degree(int rb, int i, int q) {
+  uint32_t d = 0;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const int row = 16 * rb + Mfma<T>::row(k, i);
+    d |= (uint32_t)(row < 110 ? coef_degree(row) : 0) << (8 * k);
+  }
+  return (int)((d >> (8 * q)) & 0xffu);
+}
+
+// One work unit per wave.
+template <class T>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 2 : 1)))
+void k_m2l_sets(
+    const int32_t *set_off, const int2 *units, const uint32_t *ucnt, const uint32_t *uoff,
+    int32_t nsets, int32_t chunk, int xcd_run, const uint32_t *ikey, int gbits,
+    const uint32_t *cols, const T *Af, const T *Mq, Cells c, int32_t ncells, double *L,
+    double *part, const int32_t *dchunk, int64_t nslab) {
   critical_path_priority();
-  __shared__ T Lt[TILE][NR + 1];
-  __shared__ T Lt0b[TILE][17];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int u = tile_of_block(blockIdx.x, gridDim.x, xcd_run);
-  if ((uint32_t)u >= uoff[ntiles - 1] + ucnt[ntiles - 1]) return;  // grid is an upper bound
-  const int2 tu = units[u];
-  const int tile = tu.x, k = tu.y;
-  if (k > 0 && extra_slab(uoff, tile, k) >= nslab) return;  // no slab (capacity exceeded)
+  typedef typename Vec4<T>::V V;
+  const int lane = threadIdx.x & 63;
+  const int q = lane >> 4, j = lane & 15;
+  const int u = unit_of_block(blockIdx.x, gridDim.x, xcd_run);
+  if ((uint32_t)u >= uoff[nsets - 1] + ucnt[nsets - 1]) return;  // grid is an upper bound
+  const int2 su = units[u];
+  const int set = su.x, k = su.y;
+  if (k > 0 && extra_slab(uoff, set, k) >= nslab) return;  // no slab (capacity exceeded)
   if (dchunk) chunk = *dchunk;
-  for (int i = threadIdx.x; i < TILE * (NR + 1); i += 64 * TILE_WAVES) (&Lt[0][0])[i] = 0;
-  for (int i = threadIdx.x; i < TILE * 17; i += 64 * TILE_WAVES) (&Lt0b[0][0])[i] = 0;
-  __syncthreads();
-  const int32_t tb = tile_off[tile], te = tile_off[tile + 1];
-  // first segment start at or after item j of the tile (a segment holds at
-  // most TILE / 16 items, so the walk is short)
-  auto seg_start = [&](int64_t j) -> int32_t {
-    if (j <= tb) return tb;
-    if (j >= te) return te;
-    int32_t i = (int32_t)j;
-    while (i < te && (cols[(int64_t)i * 16].y >> COL_G) == (cols[(int64_t)(i - 1) * 16].y >> COL_G)) i++;
-    return i;
-  };
-  const int32_t ib = seg_start((int64_t)tb + (int64_t)k * chunk);
-  const int32_t ie = seg_start((int64_t)tb + (int64_t)(k + 1) * chunk);
-  // every wave walks all items of the tile, in order, for its own blocks
-  switch (wave) {
-    case 0: run_wave<T, 0>(cols, ib, ie, Af, Mq, Lt, Lt0b, lane); break;
-    case 1: run_wave<T, 1>(cols, ib, ie, Af, Mq, Lt, Lt0b, lane); break;
-    case 2: run_wave<T, 2>(cols, ib, ie, Af, Mq, Lt, Lt0b, lane); break;
-    default: run_wave<T, 3>(cols, ib, ie, Af, Mq, Lt, Lt0b, lane); break;
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < TILE * 16; e += 64 * TILE_WAVES) {
-    const int sl = e >> 4, r = e & 15;
-    Lt[sl][r] += Lt0b[sl][r];
-  }
-  __syncthreads();
-  // L_j = L~_j / sigma_t^(j+1): added to the target's FP64 local expansion
-  // by the tile's first unit, kept in the unit's slab by the others
-  const int32_t first = tile * TILE;
-  double *slab = k ? part + extra_slab(uoff, tile, k) * (TILE * 110) : nullptr;
-  for (int e = threadIdx.x; e < TILE * 110; e += 64 * TILE_WAVES) {
-    const int sl = e / 110, row = e - sl * 110;
-    const int32_t ci = first + sl;
-    if (ci >= ncells) continue;
-    const int jk = row >> 1;
-    int jj = 0;
-    while (tri(jj + 1, 0) <= jk) jj++;
-    const double v = (double)Lt[sl][row];
-    double out = 0;
-    if (v != 0) {  // (nothing arrived; a zero-width tree must not form 0 * inf)
-      const double isig = 1.0 / c.width[ci];
-      double sc = isig;
-      for (int i = 0; i < jj; i++) sc *= isig;
-      out = v * sc;
+  const int32_t sb = set_off[set], se = set_off[set + 1];
+  const int32_t ib = (int32_t)min((int64_t)sb + (int64_t)k * chunk, (int64_t)se);
+  const int32_t ie = (int32_t)min((int64_t)ib + chunk, (int64_t)se);
+  SetRegs<T> r;
+#pragma unroll
+  for (int rb = 0; rb < NRB; rb++) r.sum[rb] = (typename Mfma<T>::V){0, 0, 0, 0};
+  if (ib < ie) {
+    const int32_t last = ie - 1;
+    const uint32_t gmask = (1u << gbits) - 1u;
+    auto word = [&](int32_t it) { return cols[(int64_t)min(it, last) * TILE + j]; };
+    auto key = [&](int32_t it) { return ikey[min(it, last)]; };
+    auto group = [&](uint32_t k) {
+      return (uint32_t)__builtin_amdgcn_readfirstlane((int)(k & gmask));
+    };
+    auto source = [&](uint32_t w) {
+      return Mq + (int64_t)(w & ((1u << SRC_BITS) - 1u)) * NR + 4 * q;
+    };
+    auto operands = [&](uint32_t g) { return Af + (int64_t)g * AF_PER_GROUP + lane * 4; };
+    const LaneSigns signs = lane_signs<T>(q);
+    V b0[NBV], b1[NBV];
+    // keys and column words are loaded two items ahead of their use
+    uint32_t w0 = word(ib), w1 = word(ib + 1), k1 = key(ib + 1), k0 = key(ib + 2);
+    uint32_t g = group(key(ib));
+    {
+      const T *m = source(w0), *af = operands(g);
+#pragma unroll
+      for (int v = 0; v < NBV; v++) b0[v] = *reinterpret_cast<const V *>(m + 16 * v);
+#pragma unroll
+      for (int v = 0; v < NAV; v++) r.a[v] = *reinterpret_cast<const V *>(af + v * 256);
     }
-    if (slab) slab[e] = out;
-    else if (v != 0) L[2 * ((int64_t)ci * NTERM + jk) + (row & 1)] += out;
+#pragma unroll
+    for (int i = 0; i < 3; i++) r.late[i] = (typename Mfma<T>::V){0, 0, 0, 0};
+    r.late_signs = 0;
+    // wa, wb: column words of this item and the next; kb: the next item's key
+    auto item = [&](V (&b)[NBV], V (&bn)[NBV], uint32_t &wa, uint32_t wb, uint32_t &kb,
+                    int32_t it) {
+      const uint32_t gn = group(kb), m = wa >> MIR_AT;
+      kb = key(it + 3);
+      wa = word(it + 2);
+      set_steps<T>(std::make_integer_sequence<int, NST>{}, r, b, bn, LaneSigns::of(signs.b, m),
+                   LaneSigns::of(signs.p, m), source(wb), gn != g, operands(gn));
+      g = gn;
+    };
+    for (int32_t it = ib;; it += 2) {
+      item(b0, b1, w0, w1, k1, it);
+      if (it + 1 >= ie) break;
+      item(b1, b0, w1, w0, k0, it + 1);
+      if (it + 2 >= ie) break;
+    }
+#pragma unroll
+    for (int i = 0; i < 3; i++) add_products<T>(r.sum, 4 + i, r.late[i], r.late_signs);
+  }
+  // L_j = L~_j / sigma_t^(j+1)
+  const int32_t ci = set * TILE + j;
+  if (ci >= ncells) return;
+  const double w = c.width[ci];
+  double *dst = k ? part + extra_slab(uoff, set, k) * (TILE * 110) + j * 110
+                  : L + 2 * (int64_t)ci * NTERM;
+  const double p1 = 1.0 / w, p2 = p1 * p1, p4 = p2 * p2, p8 = p4 * p4;
+#pragma unroll
+  for (int rb = 0; rb < NRB; rb++) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int row = 16 * rb + Mfma<T>::row(q, i);
+      const double v = (double)r.sum[rb][i];
+      const int n = result_degree<T>(rb, i, q);
+      double out = 0;
+      if (v != 0) {  // (nothing arrived; a zero-width tree must not form 0 * inf)
+        double sc = p1;
+        if (n & 1) sc *= p1;
+        if (n & 2) sc *= p2;
+        if (n & 4) sc *= p4;
+        if (n & 8) sc *= p8;
+        out = v * sc;
+      }
+      if (row < 110) dst[row] = out;
+    }
   }
 }
 
@@ -778,8 +840,7 @@ hipError_t m2l_upload_codes(uint32_t *dev_codes, hipStream_t s) {
 
 size_t m2l_codes_bytes() { return (size_t)2 * NCODE * 4; }
 
-int32_t m2l_group_slots(int max_depth) { return (max_depth + 1) * SLOTS_PER_LEVEL; }
-int m2l_group_bits() { return 32 - COL_G; }
+int32_t m2l_group_slots() { return m2lg::SLOTS; }
 
 hipError_t launch_m2l_classify_all(const int2 *pairs, const int32_t *slot_of, uint32_t n,
                                    const uint32_t *gid_of_slot, int gbits, uint32_t *gkeys,
@@ -804,34 +865,45 @@ hipError_t launch_m2l_classify(const int2 *pairs, const int32_t *slot_of, uint32
 }
 
 hipError_t launch_m2l_group_harmonics(const uint32_t *used, const uint32_t *gid_of_slot,
-                                      int32_t nslots, double *Y64, float *Y32, int8_t *gdl,
-                                      int8_t *glt, hipStream_t s, uint32_t gcap) {
-  if (nslots <= 0) return hipSuccess;
-  k_group_harmonics<<<(nslots + 127) / 128, 128, 0, s>>>(used, gid_of_slot, nslots, Y64, Y32,
-                                                         gdl, glt, gcap);
+                                      double *Y64, float *Y32, int8_t *gdl, hipStream_t s,
+                                      uint32_t gcap) {
+  k_group_harmonics<<<(m2lg::SLOTS + 63) / 64, 64, 0, s>>>(used, gid_of_slot, Y64, Y32, gdl, gcap);
   return hipGetLastError();
 }
 
 hipError_t launch_m2l_scale_m(Cells c, int32_t ncells, const double *M, void *Mq, bool fp32,
                               hipStream_t s) {
   if (ncells <= 0) return hipSuccess;
-  if (fp32) k_scale_m<float><<<ncells, NR, 0, s>>>(c, ncells, M, (float *)Mq);
-  else k_scale_m<double><<<ncells, NR, 0, s>>>(c, ncells, M, (double *)Mq);
+  if (fp32) k_scale_m<float><<<ncells + 1, NR, 0, s>>>(c, ncells, M, (float *)Mq);
+  else k_scale_m<double><<<ncells + 1, NR, 0, s>>>(c, ncells, M, (double *)Mq);
   return hipGetLastError();
 }
 
-hipError_t launch_m2l_count_items(const uint32_t *keys, uint32_t n, uint32_t *ipos,
+size_t m2l_mq_bytes(int64_t ncells, bool fp32) {
+  return (size_t)(ncells + 1) * NR * (fp32 ? 4 : 8);
+}
+
+uint32_t m2l_item_blocks(uint32_t n) {
+  return std::max<uint32_t>(1, (n + IT_THREADS - 1) / IT_THREADS);
+}
+
+hipError_t launch_m2l_count_items(const uint32_t *keys, const uint32_t *vals, uint32_t n,
                                   uint32_t *bcount, uint32_t *bstart, void *scan_tmp,
-                                  uint32_t *h_pinned, uint32_t *nitems_out, hipStream_t s) {
+                                  uint32_t *h_pinned, uint32_t *nitems_out, hipStream_t s,
+                                  uint32_t *repeats) {
   *nitems_out = 0;
+  h_pinned[2] = 0;
   if (n == 0) return hipSuccess;
-  const unsigned per = 64 * IP_WAVES, nb = (n + per - 1) / per;
-  k_item_pos<<<nb, per, 0, s>>>(keys, n, ipos, bcount, nullptr);
+  const unsigned nb = m2l_item_blocks(n);
+  k_items<false><<<nb, IT_THREADS, 0, s>>>(keys, vals, n, bcount, nullptr, 0, nullptr, nullptr,
+                                           nullptr, 0, repeats);
   hipError_t e = scan_exclusive_u32(bcount, bstart, nb, scan_tmp, s);
   if (e != hipSuccess) return e;
   e = hipMemcpyAsync(h_pinned, bstart + (nb - 1), 4, hipMemcpyDeviceToHost, s);
   if (e != hipSuccess) return e;
   e = hipMemcpyAsync(h_pinned + 1, bcount + (nb - 1), 4, hipMemcpyDeviceToHost, s);
+  if (e != hipSuccess) return e;
+  if (repeats) e = hipMemcpyAsync(h_pinned + 2, repeats, 4, hipMemcpyDeviceToHost, s);
   if (e != hipSuccess) return e;
   e = hipStreamSynchronize(s);
   if (e != hipSuccess) return e;
@@ -839,17 +911,18 @@ hipError_t launch_m2l_count_items(const uint32_t *keys, uint32_t n, uint32_t *ip
   return hipGetLastError();
 }
 
-// the item count on the device: the block counts of k_item_pos summed
+// the item count on the device: the block counts summed
 __global__ void k_items_total(const uint32_t *bcount, const uint32_t *bstart, uint32_t nb,
                               uint32_t *nitems) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *nitems = bstart[nb - 1] + bcount[nb - 1];
 }
 
-hipError_t launch_m2l_count_items_dev(const uint32_t *keys, uint32_t n, const uint32_t *dn,
-                                      uint32_t *ipos, uint32_t *bcount, uint32_t *bstart,
+hipError_t launch_m2l_count_items_dev(const uint32_t *keys, const uint32_t *vals, uint32_t n,
+                                      const uint32_t *dn, uint32_t *bcount, uint32_t *bstart,
                                       void *scan_tmp, uint32_t *nitems, hipStream_t s) {
-  const unsigned per = 64 * IP_WAVES, nb = (std::max<uint32_t>(n, 1) + per - 1) / per;
-  k_item_pos<<<nb, per, 0, s>>>(keys, n, ipos, bcount, dn);
+  const unsigned nb = m2l_item_blocks(n);
+  k_items<false><<<nb, IT_THREADS, 0, s>>>(keys, vals, n, bcount, nullptr, 0, nullptr, nullptr, dn,
+                                           0, nullptr);
   hipError_t e = scan_exclusive_u32(bcount, bstart, nb, scan_tmp, s);
   if (e != hipSuccess) return e;
   k_items_total<<<1, 64, 0, s>>>(bcount, bstart, nb, nitems);
@@ -857,32 +930,42 @@ hipError_t launch_m2l_count_items_dev(const uint32_t *keys, uint32_t n, const ui
 }
 
 hipError_t launch_m2l_write_items(const uint32_t *keys, const uint32_t *vals, uint32_t n,
-                                  int gbits, const uint32_t *ipos, const uint32_t *bstart,
-                                  const int8_t *gdl, int4 *items, uint2 *cols, hipStream_t s,
-                                  const uint32_t *dn, uint32_t items_cap) {
+                                  const uint32_t *bstart, int32_t ncells, uint32_t *ikey,
+                                  uint32_t *cols, hipStream_t s, const uint32_t *dn,
+                                  uint32_t items_cap) {
   if (n == 0) return hipSuccess;
-  const unsigned per = 64 * IP_WAVES;
-  k_items<<<(n + per - 1) / per, per, 0, s>>>(keys, vals, ipos, bstart, n, gbits, gdl, items,
-                                             cols, dn, items_cap);
+  k_items<true><<<m2l_item_blocks(n), IT_THREADS, 0, s>>>(keys, vals, n, nullptr, bstart,
+                                                          (uint32_t)ncells, ikey, cols, dn,
+                                                          items_cap, nullptr);
   return hipGetLastError();
 }
 
-hipError_t launch_m2l_tile_offsets(const int4 *items, uint32_t nitems, int32_t ntiles,
-                                   int32_t *off, hipStream_t s, const uint32_t *dnitems) {
-  k_tile_offsets<<<(ntiles + 1 + 255) / 256, 256, 0, s>>>(items, nitems, ntiles, off, dnitems);
+hipError_t launch_m2l_set_offsets(const uint32_t *ikey, uint32_t nitems, int gbits, int32_t nsets,
+                                  int32_t *off, hipStream_t s, const uint32_t *dnitems) {
+  k_set_offsets<<<(nsets + 1 + 255) / 256, 256, 0, s>>>(ikey, nitems, gbits, nsets, off, dnitems);
   return hipGetLastError();
 }
 
-// m2l_unit_chunk on the device, from the item and tile counts there
-__global__ void k_unit_chunk(const uint32_t *nitems, const uint32_t *ntiles, double factor,
+// Items of a work unit.  With a factor, factor x the mean items per set.
+// Without, enough units for several turns of the chip's 2,048 wave slots
+// (UNITS), but a unit of at least UNIT_MIN items (its start and end, about
+// UNIT_MIN items' time, must not outweigh it) and at most UNIT_MAX (the last
+// units to start leave the rest of the chip idle).
+constexpr int UNITS = 8192, UNIT_MIN = 8, UNIT_MAX = 128;
+__host__ __device__ inline int32_t unit_chunk(uint32_t nitems, int32_t nsets, double factor) {
+  if (factor <= 0) {
+    const uint32_t want = (nitems + UNITS - 1) / UNITS;
+    return (int32_t)(want < UNIT_MIN ? UNIT_MIN : want > UNIT_MAX ? UNIT_MAX : want);
+  }
+  const double mean = nsets > 0 ? (double)nitems / (double)nsets : 1.0;
+  return (int32_t)fmin((double)(INT32_MAX / 2), fmax((double)UNIT_MIN, ceil(mean * factor)));
+}
+
+// m2l_unit_chunk on the device, from the item and set counts there
+__global__ void k_unit_chunk(const uint32_t *nitems, const uint32_t *nsets, double factor,
                              int32_t *chunk) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  if (factor <= 0) {
-    *chunk = INT32_MAX / 2;
-    return;
-  }
-  const double mean = *ntiles > 0 ? (double)*nitems / (double)*ntiles : 1.0;
-  *chunk = (int32_t)fmin((double)(INT32_MAX / 2), fmax(64.0, ceil(mean * factor)));
+  *chunk = unit_chunk(*nitems, (int32_t)*nsets, factor);
 }
 
 hipError_t launch_m2l_unit_chunk(const uint32_t *nitems, const uint32_t *ntiles, double factor,
@@ -891,14 +974,20 @@ hipError_t launch_m2l_unit_chunk(const uint32_t *nitems, const uint32_t *ntiles,
   return hipGetLastError();
 }
 
-int32_t m2l_unit_chunk(uint32_t nitems, int32_t ntiles, double factor) {
-  if (factor <= 0) return INT32_MAX / 2;  // one unit per tile
-  const double mean = ntiles > 0 ? (double)nitems / ntiles : 1.0;
-  return (int32_t)std::min<double>(INT32_MAX / 2, std::max(64.0, std::ceil(mean * factor)));
+int32_t m2l_unit_chunk(uint32_t nitems, int32_t nsets, double factor) {
+  return unit_chunk(nitems, nsets, factor);
 }
 
 uint32_t m2l_units_bound(uint32_t nitems, int32_t ntiles, int32_t chunk) {
   return (uint32_t)ntiles + nitems / (uint32_t)chunk;
+}
+
+// the same for a chunk chosen on the device from at most nitems items and
+// nsets sets
+uint32_t m2l_units_cap(uint32_t nitems, int32_t nsets, double factor) {
+  const double extra = factor > 0 ? std::ceil(nsets / factor) + 1
+                                  : std::max<double>(UNITS, nitems / (double)UNIT_MAX) + 1;
+  return (uint32_t)std::min<double>(UINT32_MAX / 4, nsets + extra);
 }
 
 size_t m2l_unit_part_bytes(uint32_t units_bound, int32_t ntiles) {
@@ -925,7 +1014,7 @@ hipError_t launch_m2l_group_afrag(const void *Yg, uint32_t ngroups, const uint32
                                   const int8_t *gdl, void *Af, bool fp32, hipStream_t s,
                                   const uint32_t *dng) {
   if (ngroups == 0) return hipSuccess;
-  const int64_t n = (int64_t)ngroups * NBLK * 64;
+  const int64_t n = (int64_t)ngroups * (AF_PER_GROUP / 4);
   const unsigned nb = (unsigned)((n + 255) / 256);
   if (fp32)
     k_group_afrag<float><<<nb, 256, 0, s>>>((const float *)Yg, ngroups, codes, gdl, (float *)Af,
@@ -936,25 +1025,29 @@ hipError_t launch_m2l_group_afrag(const void *Yg, uint32_t ngroups, const uint32
   return hipGetLastError();
 }
 
-hipError_t launch_m2l_tiles(const int32_t *tile_off, const int2 *units, const uint32_t *ucnt,
-                            const uint32_t *uoff, int32_t ntiles, int32_t chunk, int xcd_run,
-                            uint32_t units_bound, const uint2 *cols, const void *Af,
-                            const void *Mq, Cells c, int32_t ncells, double *L, double *part,
-                            bool fp32, hipStream_t s, const int32_t *dchunk) {
-  if (ntiles <= 0) return hipSuccess;
+hipError_t launch_m2l_sets(const int32_t *set_off, const int2 *units, const uint32_t *ucnt,
+                           const uint32_t *uoff, int32_t nsets, int32_t chunk, int xcd_run,
+                           uint32_t units_bound, const uint32_t *ikey, int gbits,
+                           const uint32_t *cols, const void *Af, const void *Mq, Cells c,
+                           int32_t ncells, double *L, double *part, bool fp32, hipStream_t s,
+                           const int32_t *dchunk) {
+  if (nsets <= 0) return hipSuccess;
   // slabs of the part buffer (m2l_unit_part_bytes)
-  const int64_t nslab = units_bound > (uint32_t)ntiles ? (int64_t)units_bound - ntiles : 0;
+  const int64_t nslab = units_bound > (uint32_t)nsets ? (int64_t)units_bound - nsets : 0;
   if (fp32)
-    k_m2l_tiles<float><<<units_bound, 64 * TILE_WAVES, 0, s>>>(
-        tile_off, units, ucnt, uoff, ntiles, chunk, xcd_run, cols, (const float *)Af,
-        (const float *)Mq, c, ncells, L, part, dchunk, nslab);
+    k_m2l_sets<float><<<units_bound, 64, 0, s>>>(set_off, units, ucnt, uoff, nsets, chunk, xcd_run,
+                                                 ikey, gbits, cols, (const float *)Af,
+                                                 (const float *)Mq, c, ncells, L, part, dchunk,
+                                                 nslab);
   else
-    k_m2l_tiles<double><<<units_bound, 64 * TILE_WAVES, 0, s>>>(
-        tile_off, units, ucnt, uoff, ntiles, chunk, xcd_run, cols, (const double *)Af,
-        (const double *)Mq, c, ncells, L, part, dchunk, nslab);
+    k_m2l_sets<double><<<units_bound, 64, 0, s>>>(set_off, units, ucnt, uoff, nsets, chunk,
+                                                  xcd_run, ikey, gbits, cols, (const double *)Af,
+                                                  (const double *)Mq, c, ncells, L, part, dchunk,
+                                                  nslab);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  k_unit_combine<<<ntiles, 256, 0, s>>>(ucnt, uoff, ntiles, part, ncells, L, nslab);
+  k_unit_combine<<<dim3(nsets, (TILE * 110 + 255) / 256), 256, 0, s>>>(ucnt, uoff, nsets, part,
+                                                                      ncells, L, nslab);
   return hipGetLastError();
 }
 

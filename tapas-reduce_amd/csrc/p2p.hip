@@ -417,11 +417,14 @@ void k_p2p_fp32(Cells c, Csr list, Bodies b, const float4 *rel, double *acc, dou
 // (zeroed before the launch) until none are left: the P2P then holds a
 // bounded share of the CUs, and kernels on the other stream still find
 // slots.  Each target is computed by one wave exactly as above, so the order
-// in which the waves take them does not change any result.
-__global__ __launch_bounds__(64) void k_p2p_fp32_resident(Cells c, int32_t ncells, Csr list,
-                                                         Bodies b, const float4 *rel,
-                                                         double *acc, uint32_t *next,
-                                                         double cycle) {
+// in which the waves take them does not change any result.  80 registers (3
+// spilled, outside the pair loop) and not the 94 of a free choice: the M2L set
+// kernel takes 232 of a SIMD's 512, which three waves of 94 would not leave, and
+// the M2L then ran mostly after the P2P (two clusters of 4M bodies 21.9 ms an
+// evaluation against 20.4, one cluster 12.2 against 11.5).
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8)))
+void k_p2p_fp32_resident(Cells c, int32_t ncells, Csr list, Bodies b, const float4 *rel,
+                         double *acc, uint32_t *next, double cycle) {
   __shared__ float4 ring[ring_entries(RING32)];
   __shared__ uint32_t take;
   while (true) {

@@ -224,8 +224,7 @@ hipError_t launch_direct_fp64(const double *x, const double *y, const double *z,
 
 namespace tfmm {
 // m2l_batched.hip
-int m2l_group_bits();  // bits of a group index in the tile kernel's column word
-int32_t m2l_group_slots(int max_depth);
+int32_t m2l_group_slots();
 int m2l_tile_size();
 int m2l_src_bits();
 hipError_t m2l_upload_codes(uint32_t *dev_codes, hipStream_t s);
@@ -246,35 +245,40 @@ hipError_t launch_m2l_classify(const int2 *pairs, const int32_t *slot_of, uint32
                                uint32_t *fvals, uint32_t *counters, hipStream_t s,
                                const uint32_t *dn = nullptr, uint32_t gcap = UINT32_MAX);
 hipError_t launch_m2l_group_harmonics(const uint32_t *used, const uint32_t *gid_of_slot,
-                                      int32_t nslots, double *Y64, float *Y32, int8_t *gdl,
-                                      int8_t *glt, hipStream_t s, uint32_t gcap = UINT32_MAX);
+                                      double *Y64, float *Y32, int8_t *gdl, hipStream_t s,
+                                      uint32_t gcap = UINT32_MAX);
 hipError_t launch_m2l_scale_m(Cells c, int32_t ncells, const double *M, void *Mq, bool fp32,
                               hipStream_t s);
-// items of the (tile, group)-sorted grouped pairs: every pair's position in
-// its segment and the item starts (runs of 16) per block of 1024 pairs,
-// their count read back; bcount/bstart: one word per block
-hipError_t launch_m2l_count_items(const uint32_t *keys, uint32_t n, uint32_t *ipos,
+// bytes of the scaled multipoles (one cell more: the source of empty columns)
+size_t m2l_mq_bytes(int64_t ncells, bool fp32);
+// items of the (set, group)-sorted grouped pairs, counted per block of pairs
+// (m2l_item_blocks words in bcount and bstart) and read back
+uint32_t m2l_item_blocks(uint32_t n);
+hipError_t launch_m2l_count_items(const uint32_t *keys, const uint32_t *vals, uint32_t n,
                                   uint32_t *bcount, uint32_t *bstart, void *scan_tmp,
-                                  uint32_t *h_pinned, uint32_t *nitems_out, hipStream_t s);
+                                  uint32_t *h_pinned, uint32_t *nitems_out, hipStream_t s,
+                                  uint32_t *repeats = nullptr);
 // the same with the pair count *dn on the device (n its capacity) and the
 // item count left on the device in *nitems
-hipError_t launch_m2l_count_items_dev(const uint32_t *keys, uint32_t n, const uint32_t *dn,
-                                      uint32_t *ipos, uint32_t *bcount, uint32_t *bstart,
+hipError_t launch_m2l_count_items_dev(const uint32_t *keys, const uint32_t *vals, uint32_t n,
+                                      const uint32_t *dn, uint32_t *bcount, uint32_t *bstart,
                                       void *scan_tmp, uint32_t *nitems, hipStream_t s);
-// items at or past items_cap are not written
+// every item's key and 16 column words (ncells: as the launch of the set
+// kernel); items at or past items_cap are not written
 hipError_t launch_m2l_write_items(const uint32_t *keys, const uint32_t *vals, uint32_t n,
-                                  int gbits, const uint32_t *ipos, const uint32_t *bstart,
-                                  const int8_t *gdl, int4 *items, uint2 *cols, hipStream_t s,
-                                  const uint32_t *dn = nullptr, uint32_t items_cap = UINT32_MAX);
-hipError_t launch_m2l_tile_offsets(const int4 *items, uint32_t nitems, int32_t ntiles,
-                                   int32_t *off, hipStream_t s,
-                                   const uint32_t *dnitems = nullptr);
+                                  const uint32_t *bstart, int32_t ncells, uint32_t *ikey,
+                                  uint32_t *cols, hipStream_t s, const uint32_t *dn = nullptr,
+                                  uint32_t items_cap = UINT32_MAX);
+hipError_t launch_m2l_set_offsets(const uint32_t *ikey, uint32_t nitems, int gbits, int32_t nsets,
+                                  int32_t *off, hipStream_t s,
+                                  const uint32_t *dnitems = nullptr);
 // m2l_unit_chunk of the device's item and tile counts, into *chunk
 hipError_t launch_m2l_unit_chunk(const uint32_t *nitems, const uint32_t *ntiles, double factor,
                                  int32_t *chunk, hipStream_t s);
-// work units of the tile kernel: runs of at most `chunk` items of one tile
+// work units of the set kernel: runs of at most `chunk` items of one set
 int32_t m2l_unit_chunk(uint32_t nitems, int32_t ntiles, double factor);
 uint32_t m2l_units_bound(uint32_t nitems, int32_t ntiles, int32_t chunk);
+uint32_t m2l_units_cap(uint32_t nitems, int32_t nsets, double factor);
 size_t m2l_unit_part_bytes(uint32_t units_bound, int32_t ntiles);
 // units at or past units_cap are not written; with dchunk the chunk is read
 // on the device
@@ -282,18 +286,19 @@ hipError_t launch_m2l_units(const int32_t *tile_off, int32_t ntiles, int32_t chu
                             uint32_t *ucnt, uint32_t *uoff, int2 *units, void *scan_tmp,
                             hipStream_t s, uint32_t units_cap = UINT32_MAX,
                             const int32_t *dchunk = nullptr);
-// A fragments of every group (the tile kernel's operand order, row factors
+// A fragments of every group (the set kernel's operand order, row factors
 // 2^(-j dl) included) from the group harmonics (FP32 or FP64), the operand
 // codes of both types and the groups' level differences
 size_t m2l_afrag_bytes(uint32_t ngroups, bool fp32);
 hipError_t launch_m2l_group_afrag(const void *Yg, uint32_t ngroups, const uint32_t *codes,
                                   const int8_t *gdl, void *Af, bool fp32, hipStream_t s,
                                   const uint32_t *dng = nullptr);
-hipError_t launch_m2l_tiles(const int32_t *tile_off, const int2 *units, const uint32_t *ucnt,
-                            const uint32_t *uoff, int32_t ntiles, int32_t chunk, int xcd_run,
-                            uint32_t units_bound, const uint2 *cols, const void *Af,
-                            const void *Mq, Cells c, int32_t ncells, double *L, double *part,
-                            bool fp32, hipStream_t s, const int32_t *dchunk = nullptr);
+hipError_t launch_m2l_sets(const int32_t *set_off, const int2 *units, const uint32_t *ucnt,
+                           const uint32_t *uoff, int32_t nsets, int32_t chunk, int xcd_run,
+                           uint32_t units_bound, const uint32_t *ikey, int gbits,
+                           const uint32_t *cols, const void *Af, const void *Mq, Cells c,
+                           int32_t ncells, double *L, double *part, bool fp32, hipStream_t s,
+                           const int32_t *dchunk = nullptr);
 
 // p2p.hip (mixed precision)
 hipError_t launch_leaf_relpos(Cells c, int32_t ncells, Bodies b, float4 *rel, hipStream_t s);

@@ -221,7 +221,7 @@ __global__ __launch_bounds__(DTT_THREADS) void k_dtt_step(const int2 *in, const 
         if (sl + e < m2l_cap) {
           m2l[sl + e] = e ? make_int2(j, i) : make_int2(i, j);
           m2l_slot[sl + e] = ge;
-          if (ge >= 0) used[ge] = 1u;
+          if (ge >= 0) used[ge >> m2lg::MIRROR_BITS] = 1u;
           else outside++;
         }
       }
@@ -266,7 +266,7 @@ __global__ void k_pair_slots(const int2 *pairs, uint32_t n, const double4 *geo,
   const double ci[3] = {gi.x, gi.y, gi.z}, cj[3] = {gj.x, gj.y, gj.z};
   const int32_t g = m2lg::pair_slot(depth[pr.x], depth[pr.y], width[pr.x], width[pr.y], ci, cj);
   slot[t] = g;
-  if (g >= 0) used[g] = 1u;
+  if (g >= 0) used[g >> m2lg::MIRROR_BITS] = 1u;
   else atomicAdd(n_outside, 1u);
 }
 
