@@ -1134,15 +1134,19 @@ void probe_external_events(tfmm_ctx *c) {
 
 // The P2P on the second stream (forked from and later joined to the context
 // stream by events).
-// Schedule 3: the resident FP32 P2P starts early with its few waves, and a
-// full-occupancy launch of the same kernel on the context stream takes the
-// target cells still left on its counter once the set kernel is done.
+// The resident FP32 P2P holds few waves so that the kernels of the critical path
+// find room beside it.  When those are done, nothing is left to make room for: a
+// full-occupancy launch of the same kernel on the context stream then takes the
+// target cells still left on its counter, after the L2L, or with schedule 3
+// already once the set kernel is done.  (Two clusters of 4M bodies, mixed, 3
+// resident waves: 19.9 ms with the drain, 20.3 without, where the 3 waves
+// ended alone.)
 bool p2p_drains(const tfmm_ctx *c) {
-  return c->p2p_schedule == 3 && c->p2p_waves > 0 && c->prm.precision == TFMM_MIXED;
+  return c->p2p_schedule != 4 && c->p2p_waves > 0 && c->prm.precision == TFMM_MIXED;
 }
 
-int drain_p2p(tfmm_ctx *c, int64_t ncells) {
-  if (!p2p_drains(c)) return TFMM_OK;
+int drain_p2p(tfmm_ctx *c, int64_t ncells, bool l2l_done) {
+  if (!p2p_drains(c) || l2l_done == (c->p2p_schedule == 3)) return TFMM_OK;
   const Cells k = cells_of(c);
   Csr pl{dp<int32_t>(c->p2p_off), dp<int32_t>(c->p2p_src)};
   TRY(launch_p2p_fp32_drain(k, (int32_t)ncells, pl, sorted_bodies(c), dp<float4>(c->relpos),
@@ -1249,7 +1253,7 @@ int fused_numeric(tfmm_ctx *c) {
     if (!c->p2p_forked && c->p2p_schedule == 1 && (rc = fork_p2p(c))) return rc;
     if ((rc = cart_m2l(c))) return rc;
     TRY(rec(c, EV_M2L1, s));
-    if ((rc = drain_p2p(c, c->ncells))) return rc;
+    if ((rc = drain_p2p(c, c->ncells, c->p2p_schedule != 3))) return rc;
     TRY(hipStreamWaitEvent(s, c->ev[EV_P2PJOIN], 0));
     TRY(rec(c, EV_TRAV, s));
     if ((rc = cart_downward(c))) return rc;
@@ -1290,18 +1294,20 @@ int fused_numeric(tfmm_ctx *c) {
   TRY(launch_periodic_far(dp<double>(c->M), dp<double>(c->L), c->cycle, c->images, s));
   TRY(cart_from_tiles(c));
   TRY(rec(c, EV_M2L1, s));
-  if ((rc = drain_p2p(c, c->ncells))) return rc;
+  // downward: the L2L needs no P2P, so the join stands before the L2P
+  if ((rc = drain_p2p(c, c->ncells, false))) return rc;
+  if (!cartesian(c))
+    for (int d = 0; d + 1 < nl; d++)
+      TRY(launch_l2l(k, c->lvl[d + 1], (c->lvl[d + 2] - c->lvl[d + 1]) / 8, dp<double>(c->tops),
+                     dp<double>(c->L), s));
+  if ((rc = drain_p2p(c, c->ncells, true))) return rc;
   TRY(hipStreamWaitEvent(s, c->ev[EV_P2PJOIN], 0));
   TRY(rec(c, EV_TRAV, s));
-  // downward
   if (cartesian(c)) {
     if ((rc = cart_downward(c))) return rc;
     TRY(rec(c, EV_DOWN, s));
     return TFMM_OK;
   }
-  for (int d = 0; d + 1 < nl; d++)
-    TRY(launch_l2l(k, c->lvl[d + 1], (c->lvl[d + 2] - c->lvl[d + 1]) / 8, dp<double>(c->tops),
-                   dp<double>(c->L), s));
   TRY(launch_l2p(k, (int32_t)c->ncells, sorted_bodies(c), dp<double>(c->L), dp<double>(c->acc),
                  dp<int32_t>(c->perm), dp<int32_t>(c->leaf_of), dp<double>(c->trg),
                  dp<double>(c->out), s));
@@ -1740,12 +1746,13 @@ int whole_record(tfmm_ctx *c) {
                         dp<double>(c->L), c->fb_part.ptr, s, dp<uint32_t>(c->g_cnt) + 1));
   }
   TRY(rec(c, EV_M2L1, s));
-  if ((rc = drain_p2p(c, cells))) return rc;
-  TRY(hipStreamWaitEvent(s, c->ev[EV_P2PJOIN], 0));
-  TRY(rec(c, EV_TRAV, s));
+  if ((rc = drain_p2p(c, cells, false))) return rc;
   for (int d = 0; d + 1 < pl.L; d++)
     TRY(launch_l2l(k, 0, pl.grid[d + 1] / 8 + 1, dp<double>(c->tops), dp<double>(c->L), s, lev,
                    d + 1));
+  if ((rc = drain_p2p(c, cells, true))) return rc;
+  TRY(hipStreamWaitEvent(s, c->ev[EV_P2PJOIN], 0));
+  TRY(rec(c, EV_TRAV, s));
   TRY(launch_l2p(k, cells, sorted_bodies(c), dp<double>(c->L), dp<double>(c->acc),
                  dp<int32_t>(c->perm), dp<int32_t>(c->leaf_of), dp<double>(c->trg),
                  dp<double>(c->out), s));
