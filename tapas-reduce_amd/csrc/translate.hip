@@ -21,6 +21,8 @@
 // v_mfma_f64_16x16x4 in FP64.  (dX of the reference comes from the cell
 // centres, which equal sigma_p u_o up to rounding.)
 #include <algorithm>
+#include <cmath>
+#include <cstdlib>
 
 #include "tfmm_device.h"
 #include "tfmm_kernels.h"
@@ -492,29 +494,6 @@ size_t translation_ops_doubles() {
 
 namespace {
 
-// M2L output coefficient (j, k) from source coefficients Ms and the singular
-// harmonics Ys of dX (LaplaceSphericalCPU_tapas.h:227-250, mutual = 0)
-__device__ inline cd m2l_entry(int j, int k, const cd *Ms, const cd *Ys) {
-  const double Cnm = sgn(j);
-  cd acc = mk(0, 0);
-  for (int n = 0; n < P - j; n++) {
-    for (int m = -n; m < 0; m++)
-      acc = cadd(acc, cmul(cscale(cconj(Ms[tri(n, -m)]), Cnm), yfull(Ys, j + n, m - k)));
-    for (int m = 0; m <= n; m++) {
-      const double Cnm2 = Cnm * sgn((k - m) * (k < m) + m);
-      acc = cadd(acc, cmul(cscale(Ms[tri(n, m)], Cnm2), yfull(Ys, j + n, m - k)));
-    }
-  }
-  return acc;
-}
-
-// image (ix, iy, iz) in {-1, 0, 1}^3 of index a in the reference's loop order
-__device__ inline void image_of(int a, int &ix, int &iy, int &iz) {
-  ix = a / 9 - 1;
-  iy = a / 3 % 3 - 1;
-  iz = a % 3 - 1;
-}
-
 // The far field of the periodic images beyond the first shell
 // (EX/include/traversal.h:126-185, images > 1): at sublevel l the copies of
 // the periodic cell form cells of side cycle_l = cycle 3^l whose multipole
@@ -525,72 +504,114 @@ __device__ inline void image_of(int a, int &ix, int &iy, int &iz) {
 // into the cell three times larger.  (The copy at the centre is part of that
 // cell: the reference's loop resets the parent before its M2M, which would
 // leave it out; this follows the sum over all (3^images)^3 copies that its
-// direct check computes.)  One workgroup: 4 waves share the M2L offsets, each
-// in a fixed order, their partial sums added in wave order.
-__global__ __launch_bounds__(256) void k_periodic_far(const double *Mroot, double *Lroot,
-                                                      double cycle, int images) {
-  critical_path_priority();
-  __shared__ cd Ms[NTERM], Mn[NTERM], Yl[NTERM];
-  __shared__ cd Ys[4][NTERM];
-  __shared__ cd part[4][NTERM];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  int j = 0, k = 0;
-  if (lane < NTERM) untri(lane, j, k);
-  const cd *M0 = reinterpret_cast<const cd *>(Mroot);
-  if (threadIdx.x < NTERM) Ms[threadIdx.x] = M0[threadIdx.x];
-  cd acc = mk(0, 0);
-  for (int level = 0; level + 1 < images; level++) {
-    __syncthreads();
-    for (int o = w; o < 26 * 27; o += 4) {
-      const int a = o / 27, ac = a < 13 ? a : a + 1;  // the 26 images other than the centre
-      int ix, iy, iz, cx, cy, cz;
-      image_of(ac, ix, iy, iz);
-      image_of(o % 27, cx, cy, cz);
-      __builtin_amdgcn_wave_barrier();
-      if (lane < P) {
-        const double dx = -((ix * 3 + cx) * cycle), dy = -((iy * 3 + cy) * cycle),
-                     dz = -((iz * 3 + cz) * cycle);
-        double rho, ca, sa;
-        cd ei;
-        sph_frame(dx, dy, dz, rho, ca, sa, ei);
-        local_column(lane, rho, ca, sa, ei, [&](int n, int m, cd Y) { Ys[w][tri(n, m)] = Y; });
-      }
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-      __builtin_amdgcn_wave_barrier();
-      if (lane < NTERM) acc = cadd(acc, m2l_entry(j, k, Ms, Ys[w]));
-    }
-    __syncthreads();
-    if (w == 0) {
-      cd mn = mk(0, 0);
-      for (int a = 0; a < 27; a++) {
-        int ix, iy, iz;
-        image_of(a, ix, iy, iz);
-        __builtin_amdgcn_wave_barrier();
-        if (lane == 0) {  // dX = parent - child centre = -(i cycle_l)
-          double rho, ca, sa;
-          cd ei;
-          sph_frame(-(ix * cycle), -(iy * cycle), -(iz * cycle), rho, ca, sa, ei);
-          multipole_all<false>(rho, ca, sa, ei, [&](int n, int m, cd v, cd) { Yl[tri(n, m)] = v; });
+// direct check computes.)
+//
+// Both translations are linear in the harmonics of dX, so the sum over the
+// copies is one translation by the sum of their harmonics.  The copies are the
+// lattice points of [-4,4]^3 less [-1,1]^3 (M2L) and of [-1,1]^3 (M2M) times
+// cycle_l: sets that a reflection of any axis and a quarter turn about z leave
+// as they are, so only even degrees p and orders q = 0, +-4, +-8 remain, all
+// real.  Those nine sums are numbers of the lattice alone (far_sums);
+// cycle_l^-(p+1) and cycle_l^p scale them.  One workgroup, a wave for each
+// translation: 4.4 us for one level of copies; with the copies taken one after
+// the other (702 M2L and 27 M2M a level in four waves) 3.2 ms.
+constexpr int NFAR = 9;
+__host__ __device__ constexpr int far_index(int p, int q) {  // p even, q = 0, 4, 8 <= p
+  return q == 0 ? p / 2 : q == 4 ? 5 + (p - 4) / 2 : 8;
+}
+static_assert(P == 10, "the far sums list the even degrees below 10");
+
+struct FarSums {
+  double sing[NFAR];  // singular harmonics (as local_column) over the M2L's points
+  double reg[NFAR];   // regular harmonics (as multipole_all) over the M2M's points
+};
+
+// The sums, in extended precision from the points of one octant: a point with
+// e coordinates other than 0 stands for its 2^e reflections.
+FarSums far_sums() {
+  long double sing[NFAR] = {}, reg[NFAR] = {};
+  for (int x = 0; x <= 4; x++)
+    for (int y = 0; y <= 4; y++)
+      for (int z = 0; z <= 4; z++) {
+        const bool near = x <= 1 && y <= 1 && z <= 1;
+        const long double copies = (long double)((x ? 2 : 1) * (y ? 2 : 1) * (z ? 2 : 1));
+        const long double rxy = sqrtl((long double)(x * x + y * y));
+        const long double r = sqrtl((long double)(x * x + y * y + z * z));
+        const long double ct = r > 0 ? z / r : 1, st = r > 0 ? rxy / r : 0;
+        const long double phi = atan2l((long double)y, (long double)x);
+        for (int m = 0; m < P; m += 4) {
+          long double p1 = 0, p = 1;  // P_(n-1)^m, P_n^m
+          for (int i = 1; i <= m; i++) p *= (2 * i - 1) * st;
+          for (int n = m; n < P; n++) {
+            if (n % 2 == 0) {
+              const long double v = copies * p * cosl(m * phi);
+              long double up = 1, down = 1;  // (n - m)!, (n + m)!
+              for (int i = 2; i <= n - m; i++) up *= i;
+              for (int i = 2; i <= n + m; i++) down *= i;
+              if (near)
+                reg[far_index(n, m)] += v * powl(r, n) / down;
+              else
+                sing[far_index(n, m)] += v * up / powl(r, n + 1);
+            }
+            const long double p2 = p1;
+            p1 = p;
+            p = (ct * (2 * n + 1) * p1 - (n + m) * p2) / (n - m + 1);
+          }
         }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_wave_barrier();
-        if (lane < NTERM) mn = cadd(mn, m2m_entry(j, k, Ms, Yl));
       }
-      if (lane < NTERM) Mn[lane] = mn;
-    }
-    __syncthreads();
-    if (threadIdx.x < NTERM) Ms[threadIdx.x] = Mn[threadIdx.x];
-    cycle *= 3;
+  FarSums f;
+  for (int i = 0; i < NFAR; i++) {
+    f.sing[i] = (double)sing[i];
+    f.reg[i] = (double)reg[i];
   }
-  if (lane < NTERM) part[w][lane] = acc;
-  __syncthreads();
-  if (threadIdx.x < NTERM) {
-    cd s = part[0][threadIdx.x];
-    for (int u = 1; u < 4; u++) s = cadd(s, part[u][threadIdx.x]);
+  return f;
+}
+
+__global__ __launch_bounds__(128) void k_periodic_far(const double *Mroot, double *Lroot,
+                                                      double cycle, int images, FarSums far) {
+  critical_path_priority();
+  __shared__ cd Ms[2][NTERM];  // M_l and M_(l+1), in turn
+  __shared__ double S[2][NFAR];
+  const int t = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (threadIdx.x < NFAR) {
+    S[0][threadIdx.x] = far.sing[threadIdx.x];
+    S[1][threadIdx.x] = far.reg[threadIdx.x];
+  }
+  if (threadIdx.x < NTERM) Ms[0][threadIdx.x] = reinterpret_cast<const cd *>(Mroot)[threadIdx.x];
+  int j = 0, k = 0;
+  if (t < NTERM) untri(t, j, k);
+  cd acc = mk(0, 0);
+  for (int level = 0; level + 1 < images; level++, cycle *= 3) {
+    __syncthreads();
+    const cd *M = Ms[level & 1];
+    const double ic = 1 / cycle;
+    if (t < NTERM && w == 0) {  // LaplaceSphericalCPU_tapas.h:227-250, mutual = 0
+      double scale = ic;
+      for (int p = 0; p < P; p += 2, scale *= ic * ic)
+        for (int q = -(p / 4 * 4); q <= p; q += 4) {
+          const int n = p - j, m = k + q;
+          if (n < 0 || m > n || -m > n) continue;
+          const cd c = m < 0 ? cconj(M[tri(n, -m)]) : M[tri(n, m)];
+          const int sign = sgn(j) * (m < 0 ? 1 : sgn(m));  // q is even
+          acc = cadd(acc, cscale(c, sign * scale * S[0][far_index(p, abs(q))]));
+        }
+    } else if (t < NTERM) {  // LaplaceSphericalCPU_tapas.h:178-200
+      cd next = mk(0, 0);
+      double scale = 1;
+      for (int n = 0; n <= j; n += 2, scale *= cycle * cycle)
+        for (int m = -(n / 4 * 4); m <= n; m += 4) {
+          const int d = j - n, e = k - m;
+          if (e > d || -e > d) continue;
+          const cd c = m < k ? M[tri(d, e)] : cconj(M[tri(d, -e)]);
+          const int sign = m < k ? 1 : sgn(k);  // m and n are even
+          next = cadd(next, cscale(c, sign * scale * S[1][far_index(n, abs(m))]));
+        }
+      Ms[(level + 1) & 1][t] = next;
+    }
+  }
+  if (t < NTERM && w == 0) {
     cd *L0 = reinterpret_cast<cd *>(Lroot);
-    L0[threadIdx.x] = cadd(L0[threadIdx.x], s);
+    L0[t] = cadd(L0[t], acc);
   }
 }
 
@@ -599,7 +620,8 @@ __global__ __launch_bounds__(256) void k_periodic_far(const double *Mroot, doubl
 hipError_t launch_periodic_far(const double *Mroot, double *Lroot, double cycle, int images,
                                hipStream_t s) {
   if (images < 2) return hipSuccess;
-  k_periodic_far<<<1, 256, 0, s>>>(Mroot, Lroot, cycle, images);
+  static const FarSums far = far_sums();
+  k_periodic_far<<<1, 128, 0, s>>>(Mroot, Lroot, cycle, images, far);
   return hipGetLastError();
 }
 
