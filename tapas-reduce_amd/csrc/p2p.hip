@@ -64,21 +64,36 @@ __device__ inline int lanes_per_target(int32_t nt) {
   return g_best;
 }
 
+// RINV / |dX| of a pair, and 0 for a negative argument (the R2 != 0 test above)
+template <typename T> constexpr T RINV = 1;
+template <> constexpr double RINV<double> = 2;
+
 __device__ inline float rsq_guarded(float r2) {
   return __builtin_fmaxf(__builtin_amdgcn_rsqf(r2), 0.f);
 }
 
-// 1/sqrt(x) in FP64: the hardware estimate (relative error 5.2e-8 at most,
-// about 24 bits) and one Newton step y <- y + y/2 (1 - x y^2), which squares
-// the error: 4.1e-15 at most, a few ulp (both measured on gfx950 over 2^20
-// arguments spread over [1e-12, 1e12]; a second step gives 1.4e-16 and costs
-// 4 of the pair's 23 VALU instructions).  A negative x gives NaN, and
-// max(NaN, 0) = 0.
+// 2/sqrt(x) in FP64: the hardware estimate y (relative error 5.2e-8 at most,
+// about 24 bits) and one Newton step y (3 - x y^2), which squares the error:
+// 4.1e-15 at most, a few ulp (both measured on gfx950 over 2^20 arguments spread
+// over [1e-12, 1e12]; a second step gives 1.4e-16 and costs 4 more VALU
+// instructions).  The pair's coordinates are scaled (p2p_scale) so that the value
+// never exceeds 1: the limits to [0, 1] are then the clamp of the last
+// multiplication, which is no instruction of its own and makes the NaN of a
+// negative x zero.  v_max_f64 takes as long as two other FP64 instructions, and
+// leaving the factor 2 in saves a third: 1M-body cube, ncrit 64, alone 2,227
+// us against 2,428.
 __device__ inline double rsq_guarded(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  const double e = __builtin_fma(-x * y, y, 1.0);
-  y = __builtin_fma(0.5 * y, e, y);
-  return __builtin_fmax(y, 0.0);
+  const double y = __builtin_amdgcn_rsq(x);
+  return __builtin_fmin(__builtin_fmax(y * __builtin_fma(-x * y, y, 3.0), 0.0), 1.0);
+}
+
+// The FP64 P2P works on coordinates times 2^p2p_scale, exact powers of two, in
+// which a cell's width is about 2^256: |dX| is then at least 2 for every pair
+// down to 2^-255 of the width, and |dX|^3 far below the largest double for the
+// farthest leaf of a list.
+__device__ inline int p2p_scale(double width) {
+  if (!(width > 0)) return 0;  // all bodies of the problem in one point
+  return max(-400, min(400, 256 - ilogb(width)));
 }
 
 __device__ inline float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
@@ -88,7 +103,7 @@ template <typename T> struct Vec4;
 template <> struct Vec4<float> { using type = float4; };
 template <> struct Vec4<double> { using type = double4; };
 
-// One pair: target xi, source xj (w = charge); p0 += q/r, p1..3 -= q dX / r^3
+// One pair: target xi, source xj (w = charge); p0 += RINV q/r, p1..3 -= RINV^3 q dX / r^3
 template <typename T, typename V4>
 __device__ inline void pair(const V4 &xi, const V4 &xj, T tiny, T &p0, T &p1, T &p2, T &p3) {
   const T dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
@@ -125,14 +140,18 @@ template <> struct Acc<float> {
     kahan_add(s3, c3, p3);
     p0 = p1 = p2 = p3 = 0;
   }
-  __device__ double4 total() {
+  __device__ double4 total(int) {
     return make_double4((double)s0 - c0, (double)s1 - c1, (double)s2 - c2, (double)s3 - c3);
   }
 };
 template <> struct Acc<double> {
   double p0 = 0, p1 = 0, p2 = 0, p3 = 0;
   __device__ void flush() {}
-  __device__ double4 total() { return make_double4(p0, p1, p2, p3); }
+  // scale: that of the coordinates
+  __device__ double4 total(int scale) {
+    const double s1 = ldexp(1.0 / RINV<double>, scale), s3 = ldexp(0.125, 2 * scale);
+    return make_double4(p0 * s1, p1 * s3, p2 * s3, p3 * s3);
+  }
 };
 
 template <typename T>
@@ -147,14 +166,18 @@ __device__ inline double4 load_body<double>(const Bodies &b, const float4 *, int
   return make_double4(b.x[i], b.y[i], b.z[i], b.q[i]);
 }
 
+__device__ inline double4 scaled(double4 v, double up) {
+  return make_double4(v.x * up, v.y * up, v.z * up, v.w);
+}
+
 // One pass over the source stream for the targets t (and t2 when TWO) of
 // every lane; see p2p_leaf.
 template <typename T, int RING, bool TWO>
 __device__ inline void p2p_pass(const Cells &c, const Csr &list, const Bodies &b,
                                 const float4 *rel, double *acc, typename Vec4<T>::type *ring,
                                 int32_t tb, int32_t lb, int32_t le, double tcx, double tcy,
-                                double tcz, double cycle, T tiny, int G, int32_t t, int32_t t2,
-                                bool tvalid, bool tvalid2) {
+                                double tcz, double cycle, T tiny, int scale, int G,
+                                int32_t t, int32_t t2, bool tvalid, bool tvalid2) {
   using V4 = typename Vec4<T>::type;
   constexpr bool MIX = sizeof(T) == 4;
   const int lane = threadIdx.x;
@@ -164,6 +187,11 @@ __device__ inline void p2p_pass(const Cells &c, const Csr &list, const Bodies &b
   V4 xi{}, xi2{};
   if (tvalid) xi = load_body<T>(b, rel, tb + t);
   if (TWO && tvalid2) xi2 = load_body<T>(b, rel, tb + t2);
+  const double up = ldexp(1.0, scale);  // FP64: of the coordinates
+  if constexpr (!MIX) {
+    xi = scaled(xi, up);
+    if (TWO) xi2 = scaled(xi2, up);
+  }
   Acc<T> a, a2;
   int32_t wpos = 0, cpos = 0;
   int since = 0;
@@ -230,9 +258,10 @@ __device__ inline void p2p_pass(const Cells &c, const Csr &list, const Bodies &b
         if constexpr (MIX)
           ring[ring_slot<RING>(wpos + lane)] = make_float4(v.x - kox, v.y - koy, v.z - koz, v.w);
         else if (cycle != 0)
-          ring[ring_slot<RING>(wpos + lane)] = make_double4(v.x + ksx, v.y + ksy, v.z + ksz, v.w);
+          ring[ring_slot<RING>(wpos + lane)] =
+              scaled(make_double4(v.x + ksx, v.y + ksy, v.z + ksz, v.w), up);
         else
-          ring[ring_slot<RING>(wpos + lane)] = v;
+          ring[ring_slot<RING>(wpos + lane)] = scaled(v, up);
       }
       __builtin_amdgcn_wave_barrier();
       wpos += n;
@@ -275,7 +304,7 @@ __device__ inline void p2p_pass(const Cells &c, const Csr &list, const Bodies &b
   if (TWO) a2.flush();
   // the G partials of a target, added in lane order
   for (int h = 0; h < (TWO ? 2 : 1); h++) {
-    const double4 d = h ? a2.total() : a.total();
+    const double4 d = h ? a2.total(scale) : a.total(scale);
     const int32_t th = h ? t2 : t;
     __builtin_amdgcn_wave_barrier();
     red[lane] = d;
@@ -327,6 +356,7 @@ __device__ inline void p2p_leaf(int32_t ti, const Cells &c, const Csr &list, con
   } else {
     tiny = 0x1p-1022;
   }
+  const int scale = MIX ? 0 : p2p_scale(c.width[ti]);
   const int G = lanes_per_target<GMAX>(nt);
   const int tpp = 64 / G;  // targets per lane set
   const int tloc = lane / G;
@@ -336,10 +366,10 @@ __device__ inline void p2p_leaf(int32_t ti, const Cells &c, const Csr &list, con
     const bool tvalid = tloc < tpp && t < nt, tvalid2 = tloc < tpp && t2 < nt;
     if (t0 + tpp < nt)
       p2p_pass<T, RING, true>(c, list, b, rel, acc, ring, tb, lb, le, tcx, tcy, tcz, cycle, tiny,
-                              G, t, t2, tvalid, tvalid2);
+                              scale, G, t, t2, tvalid, tvalid2);
     else
       p2p_pass<T, RING, false>(c, list, b, rel, acc, ring, tb, lb, le, tcx, tcy, tcz, cycle, tiny,
-                               G, t, t2, tvalid, false);
+                               scale, G, t, t2, tvalid, false);
   }
 }
 

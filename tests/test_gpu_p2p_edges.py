@@ -1,0 +1,60 @@
+"""The P2P where its list sort and its pair arithmetic change branch: source
+lists around the sizes of the in-register sorts, and FP64 pairs at widths and
+distances far from 1."""
+import numpy as np
+import pytest
+
+import oracle
+import tfmm
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = tfmm.Context(0)
+    yield c
+    c.close()
+
+
+def test_gpu_list_lengths(ctx):
+    """One target for each length; its sources come back in order."""
+    r = np.random.default_rng(5)
+    n = 6000
+    x, y, z = [r.random(n) for _ in range(3)]
+    ctx.set_bodies(x, y, z, r.uniform(-1, 1, n))
+    ctx.build_tree(tfmm.make_params(1, 0.4, tfmm.FP64))
+    c = ctx.cells()
+    leaves = np.flatnonzero((c["leaf"] == 1) & (c["nb"] > 0)).astype(np.int32)
+    lens = [1, 2, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513, 1025]
+    src = {int(t): r.choice(leaves, k, replace=False) for t, k in zip(leaves, lens)}
+    p2p = np.concatenate([np.stack([np.full(len(s), t, np.int32), s], 1) for t, s in src.items()])
+    r.shuffle(p2p)
+    print("list lengths %s" % lens, flush=True)
+    ctx.upward()
+    ctx.traverse_lists(np.zeros((0, 2), np.int32), p2p)
+    _, (po, ps) = ctx.lists()
+    for t, s in src.items():
+        assert np.array_equal(ps[po[t]:po[t + 1]], np.sort(s)), len(s)
+
+
+@pytest.mark.parametrize("width", [1e-60, 1e-6, 1.0, 1e12, 1e30])
+def test_gpu_fp64_pairs_at_any_width(ctx, width):
+    """One leaf: the P2P alone is the field.  Coincident bodies do not interact,
+    and bodies 1e-13 of the width apart do."""
+    r = np.random.default_rng(9)
+    n = 60
+    x, y, z = [width * r.uniform(-1, 1, n) for _ in range(3)]
+    q = r.random(n) + 0.5
+    x[1], y[1], z[1] = x[0], y[0], z[0]
+    x[2], y[2], z[2] = 0, 0, 0
+    x[3], y[3], z[3] = 1e-13 * width, 0, 0
+    print("one leaf of width %g" % width, flush=True)
+    ctx.set_bodies(x, y, z, q)
+    ctx.evaluate(tfmm.make_params(64, 0.4, tfmm.FP64))
+    f, ref = ctx.fields(), oracle.direct(x, y, z, q, np.arange(n))
+    # 1/r to 4.1e-15 and its cube in the acceleration, sums of 60 terms
+    assert np.allclose(f[:, 0], ref[:, 0], rtol=2e-14, atol=0)
+    far = np.arange(n) != 2
+    assert np.all(np.linalg.norm(f - ref, axis=1)[far] <=
+                  5e-14 * np.linalg.norm(np.abs(ref) + np.abs(ref).max(1, keepdims=True), axis=1)[far])
