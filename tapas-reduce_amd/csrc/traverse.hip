@@ -294,8 +294,8 @@ __global__ void k_csr_offsets(const uint64_t *keys, uint32_t n, int sbits, int32
 }
 
 // Leaf-pair list in CSR form, in two steps: a stable radix sort of the
-// pairs by target only, then every target's sources sorted by one wave
-// (rank = number of smaller sources, ties by position).  The result is the
+// pairs by target only, then every target's sources sorted by one wave.  The
+// result is the
 // (target, source) order of a sort of the whole pair, with half the radix
 // passes.
 __global__ void k_split_pairs(const int2 *pairs, uint32_t n, uint32_t *tgt, uint32_t *src,
@@ -322,49 +322,62 @@ __global__ void k_csr_offsets32(const uint32_t *tgt, uint32_t n, int32_t ncells,
   off[t] = (int32_t)lo;
 }
 
-constexpr int SEG_CAP = 2048;  // sources of one target staged in LDS
-
-template <class P>
-__device__ inline void rank_sources(P v, int32_t n, int lane, int32_t *out) {
-  for (int32_t i = lane; i < n; i += 64) {
-    const uint32_t x = v[i];
-    int32_t r = 0;
-    for (int32_t k = 0; k < n; k++) {
-      const uint32_t y = v[k];
-      r += (y < x || (y == x && k < i)) ? 1 : 0;
-    }
-    out[r] = (int32_t)x;
-  }
+// Ascending bitonic sort of 64 R words by one wave: word 64 r + lane in x[r],
+// exchanges across lanes below a distance of 64, in registers from there.
+template <int R>
+__device__ inline void wave_sort(uint32_t (&x)[R], int lane) {
+#pragma unroll
+  for (int k = 2; k <= 64 * R; k <<= 1)
+#pragma unroll
+    for (int j = k >> 1; j > 0; j >>= 1)
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        const bool up = k < 64 ? (lane & k) == 0 : (64 * r & k) == 0;
+        if (j >= 64) {
+          const int o = r ^ (j >> 6);
+          if (o < r) continue;
+          const uint32_t lo = min(x[r], x[o]), hi = max(x[r], x[o]);
+          x[r] = up ? lo : hi;
+          x[o] = up ? hi : lo;
+        } else {
+          const uint32_t y = __shfl_xor(x[r], j, 64);
+          x[r] = ((lane & j) == 0) == up ? min(x[r], y) : max(x[r], y);
+        }
+      }
 }
 
-// one wave per target: its sources in ascending order (up to 64 sorted in
-// registers, up to SEG_CAP ranked from LDS); a longer list is queued in
-// longq (word 0 the count, then the targets) for k_seg_sort_long
+template <int R>
+__device__ inline void sort_segment(const uint32_t *in, int32_t *out, int32_t n, int lane) {
+  uint32_t x[R];  // past n: a value above every source word
+#pragma unroll
+  for (int r = 0; r < R; r++) x[r] = 64 * r + lane < n ? in[64 * r + lane] : 0xffffffffu;
+  wave_sort<R>(x, lane);
+#pragma unroll
+  for (int r = 0; r < R; r++)
+    if (64 * r + lane < n) out[64 * r + lane] = (int32_t)x[r];
+}
+
+// One wave per target: its sources in ascending order, sorted in registers up to
+// SEG_CAP of them; a longer list is queued in longq (word 0 the count, then the
+// targets) for k_seg_sort_long.  The work of a sort grows as n log^2 n; ranking
+// every source against all others (n^2, which took its place above 64) had single
+// waves with lists of 1,764 run for 1.2 ms beside a 500K-body ellipsoid's usual 90.
+constexpr int SEG_CAP = 512;
 __global__ __launch_bounds__(64) void k_seg_sort(const int32_t *off, const uint32_t *in,
                                                  int32_t *out, uint32_t *longq) {
-  __shared__ uint32_t v[SEG_CAP];
   const int lane = threadIdx.x;
   const int32_t b = off[blockIdx.x], n = off[blockIdx.x + 1] - b;
   if (n <= 0) return;
-  if (n > SEG_CAP) {
-    if (lane == 0) longq[1 + atomicAdd(longq, 1u)] = blockIdx.x;
-    return;
-  }
   if (n <= 64) {
-    // one source per lane: bitonic sort across the wave, ascending (lanes
-    // past n hold a value above every cell index)
-    uint32_t x = lane < n ? in[b + lane] : 0xffffffffu;
-    for (int k = 2; k <= 64; k <<= 1)
-      for (int j = k >> 1; j > 0; j >>= 1) {
-        const uint32_t y = __shfl_xor(x, j, 64);
-        const bool keep_min = ((lane & j) == 0) == ((lane & k) == 0);
-        x = keep_min ? min(x, y) : max(x, y);
-      }
-    if (lane < n) out[b + lane] = (int32_t)x;
-  } else {
-    for (int32_t i = lane; i < n; i += 64) v[i] = in[b + i];
-    __syncthreads();
-    rank_sources(static_cast<const uint32_t *>(v), n, lane, out + b);
+    sort_segment<1>(in + b, out + b, n, lane);
+  } else if (n <= 128) {
+    sort_segment<2>(in + b, out + b, n, lane);
+  } else if (n <= 256) {
+    sort_segment<4>(in + b, out + b, n, lane);
+  } else if (n <= SEG_CAP) {
+    sort_segment<8>(in + b, out + b, n, lane);
+  } else if (lane == 0) {
+    longq[1 + atomicAdd(longq, 1u)] = blockIdx.x;
   }
 }
 
