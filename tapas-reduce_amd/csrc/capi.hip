@@ -325,6 +325,9 @@ int cart_tables(tfmm_ctx *c) {
   return TFMM_OK;
 }
 
+// waves that share a target leaf of the P2P
+int leaf_waves(const tfmm_ctx *c) { return p2p_waves_per_leaf(c->n, c->prm.ncrit); }
+
 // the direct sum's image range for the image sublevels (the reference's
 // prange, tapas_exafmm.cxx:314-317)
 int image_range(const tfmm_ctx *c) {
@@ -917,10 +920,10 @@ int run_lists(tfmm_ctx *c, bool given = false) {
     Csr pl{dp<int32_t>(c->p2p_off), dp<int32_t>(c->p2p_src)};
     if (mixed)
       TRY(launch_p2p_fp32(k, (int32_t)c->ncells, pl, sorted_bodies(c), dp<float4>(c->relpos),
-                          dp<double>(c->acc), p2p_resident(c), dp<uint32_t>(c->p2p_next),
+                          dp<double>(c->acc), leaf_waves(c), p2p_resident(c), dp<uint32_t>(c->p2p_next),
                           c->side, period(c)));
     else
-      TRY(launch_p2p_fp64(k, (int32_t)c->ncells, pl, sorted_bodies(c), dp<double>(c->acc),
+      TRY(launch_p2p_fp64(k, (int32_t)c->ncells, pl, sorted_bodies(c), dp<double>(c->acc), leaf_waves(c),
                           p2p_resident(c), dp<uint32_t>(c->p2p_next), c->side, period(c)));
     TRY(hipEventRecord(c->ev[EV_P2P1], c->side));
     return TFMM_OK;
@@ -1150,7 +1153,7 @@ int drain_p2p(tfmm_ctx *c, int64_t ncells, bool l2l_done) {
   const Cells k = cells_of(c);
   Csr pl{dp<int32_t>(c->p2p_off), dp<int32_t>(c->p2p_src)};
   TRY(launch_p2p_fp32_drain(k, (int32_t)ncells, pl, sorted_bodies(c), dp<float4>(c->relpos),
-                            dp<double>(c->acc), 8 * 4 * c->n_cu, dp<uint32_t>(c->p2p_next),
+                            dp<double>(c->acc), leaf_waves(c), 8 * 4 * c->n_cu, dp<uint32_t>(c->p2p_next),
                             c->stream, period(c)));
   return TFMM_OK;
 }
@@ -1173,14 +1176,14 @@ int fork_p2p(tfmm_ctx *c, int64_t ncells = -1) {
   Csr pl{dp<int32_t>(c->p2p_off), dp<int32_t>(c->p2p_src)};
   if (p2p_drains(c))
     TRY(launch_p2p_fp32_drain(k, (int32_t)ncells, pl, sorted_bodies(c), dp<float4>(c->relpos),
-                              dp<double>(c->acc), p2p_resident(c), dp<uint32_t>(c->p2p_next),
+                              dp<double>(c->acc), leaf_waves(c), p2p_resident(c), dp<uint32_t>(c->p2p_next),
                               ps, period(c)));
   else if (mixed)
     TRY(launch_p2p_fp32(k, (int32_t)ncells, pl, sorted_bodies(c), dp<float4>(c->relpos),
-                        dp<double>(c->acc), p2p_resident(c), dp<uint32_t>(c->p2p_next), ps,
-                        period(c)));
+                        dp<double>(c->acc), leaf_waves(c), p2p_resident(c),
+                        dp<uint32_t>(c->p2p_next), ps, period(c)));
   else
-    TRY(launch_p2p_fp64(k, (int32_t)ncells, pl, sorted_bodies(c), dp<double>(c->acc),
+    TRY(launch_p2p_fp64(k, (int32_t)ncells, pl, sorted_bodies(c), dp<double>(c->acc), leaf_waves(c),
                         p2p_resident(c), dp<uint32_t>(c->p2p_next), ps,
                         period(c)));
   TRY(rec(c, EV_P2P1, ps));

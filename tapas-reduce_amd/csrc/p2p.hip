@@ -27,6 +27,9 @@
 // (tiny far below the smallest distance the coordinates resolve), so a zero
 // distance gives a negative argument, rsqrt gives NaN, and max(NaN, 0) = 0
 // drops the pair exactly.
+#include <algorithm>
+#include <type_traits>
+
 #include "tfmm_device.h"
 #include "tfmm_kernels.h"
 
@@ -34,6 +37,7 @@ namespace tfmm {
 namespace {
 
 constexpr int SEG = 16;  // bodies per lane and chunk
+__host__ __device__ constexpr int ring_entries(int ring) { return ring + ring / 16; }
 
 // Bodies of the source stream live in the ring at slot(p); one pad slot per
 // 16 keeps the segments of one chunk (16 bodies apart) in different banks.
@@ -172,7 +176,7 @@ __device__ inline double4 scaled(double4 v, double up) {
 
 // One pass over the source stream for the targets t (and t2 when TWO) of
 // every lane; see p2p_leaf.
-template <typename T, int RING, bool TWO>
+template <typename T, int RING, int W, bool TWO>
 __device__ inline void p2p_pass(const Cells &c, const Csr &list, const Bodies &b,
                                 const float4 *rel, double *acc, typename Vec4<T>::type *ring,
                                 int32_t tb, int32_t lb, int32_t le, double tcx, double tcy,
@@ -180,7 +184,7 @@ __device__ inline void p2p_pass(const Cells &c, const Csr &list, const Bodies &b
                                 int32_t t, int32_t t2, bool tvalid, bool tvalid2) {
   using V4 = typename Vec4<T>::type;
   constexpr bool MIX = sizeof(T) == 4;
-  const int lane = threadIdx.x;
+  const int lane = W == 1 ? threadIdx.x : threadIdx.x & 63;
   const int B = SEG * G;
   const int seg = lane % G;
   double4 *red = reinterpret_cast<double4 *>(ring);
@@ -302,38 +306,52 @@ __device__ inline void p2p_pass(const Cells &c, const Csr &list, const Bodies &b
   }
   a.flush();
   if (TWO) a2.flush();
-  // the G partials of a target, added in lane order
+  // the G partials of a target, added in lane order, then the waves' in theirs
   for (int h = 0; h < (TWO ? 2 : 1); h++) {
-    const double4 d = h ? a2.total(scale) : a.total(scale);
+    double4 d = h ? a2.total(scale) : a.total(scale);
     const int32_t th = h ? t2 : t;
+    const bool mine = (h ? tvalid2 : tvalid) && seg == 0;
     __builtin_amdgcn_wave_barrier();
     red[lane] = d;
     __builtin_amdgcn_wave_barrier();
-    if ((h ? tvalid2 : tvalid) && seg == 0) {
-      double d0 = d.x, d1 = d.y, d2 = d.z, d3 = d.w;
+    if (mine) {
       for (int u = 1; u < G; u++) {
         const double4 e = red[lane + u];
-        d0 += e.x;
-        d1 += e.y;
-        d2 += e.z;
-        d3 += e.w;
+        d.x += e.x;
+        d.y += e.y;
+        d.z += e.z;
+        d.w += e.w;
+      }
+      if (W > 1) red[lane] = d;
+    }
+    if (W > 1) __syncthreads();
+    if (mine && (W == 1 || threadIdx.x < 64)) {
+      for (int w = 1; w < W; w++) {
+        const double4 e = *reinterpret_cast<const double4 *>(
+            reinterpret_cast<const char *>(red + lane) + w * sizeof(V4) * ring_entries(RING));
+        d.x += e.x;
+        d.y += e.y;
+        d.z += e.z;
+        d.w += e.w;
       }
       // stored as q_i * sum, the reference's P2P sum (divided by q_i in L2P)
       const double qi = b.q[tb + th];
       double *o = acc + 4 * (int64_t)(tb + th);
-      o[0] = d0 * qi;
-      o[1] = d1 * qi;
-      o[2] = d2 * qi;
-      o[3] = d3 * qi;
+      o[0] = d.x * qi;
+      o[1] = d.y * qi;
+      o[2] = d.z * qi;
+      o[3] = d.w * qi;
     }
+    if (W > 1) __syncthreads();
     __builtin_amdgcn_wave_barrier();
   }
 }
 
-// The work of one target leaf (one wave); returns at once for other cells.
-// ring: RING + RING / 16 entries of LDS; it also holds the lane partials at
-// the end of every pass.
-template <typename T, int RING>
+// The work of one target leaf (one workgroup of W waves, each with its share of
+// the leaf's source leaves); returns at once for other cells.
+// ring: W times RING + RING / 16 entries of LDS; each wave's also holds its lane
+// partials at the end of every pass.
+template <typename T, int RING, int W>
 __device__ inline void p2p_leaf(int32_t ti, const Cells &c, const Csr &list, const Bodies &b,
                                 const float4 *rel, double *acc, typename Vec4<T>::type *ring,
                                 double cycle) {
@@ -343,8 +361,12 @@ __device__ inline void p2p_leaf(int32_t ti, const Cells &c, const Csr &list, con
   const int32_t nt = c.nb[ti];
   if (nt == 0) return;
   const int32_t tb = c.beg[ti];
-  const int lane = threadIdx.x;
-  const int32_t lb = list.off[ti], le = list.off[ti + 1];
+  const int lane = W == 1 ? threadIdx.x : threadIdx.x & 63;
+  const int wave = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int32_t l0 = list.off[ti], ln = list.off[ti + 1] - l0;
+  const int32_t lb = l0 + (int32_t)((int64_t)ln * wave / W),
+                le = l0 + (int32_t)((int64_t)ln * (wave + 1) / W);
+  ring += wave * ring_entries(RING);
   const double tcx = c.center[3 * (int64_t)ti], tcy = c.center[3 * (int64_t)ti + 1],
                tcz = c.center[3 * (int64_t)ti + 2];
   // tiny: far below the square of the smallest resolved distance (FP32:
@@ -365,31 +387,32 @@ __device__ inline void p2p_leaf(int32_t ti, const Cells &c, const Csr &list, con
     const int32_t t = t0 + tloc, t2 = t + tpp;
     const bool tvalid = tloc < tpp && t < nt, tvalid2 = tloc < tpp && t2 < nt;
     if (t0 + tpp < nt)
-      p2p_pass<T, RING, true>(c, list, b, rel, acc, ring, tb, lb, le, tcx, tcy, tcz, cycle, tiny,
+      p2p_pass<T, RING, W, true>(c, list, b, rel, acc, ring, tb, lb, le, tcx, tcy, tcz, cycle, tiny,
                               scale, G, t, t2, tvalid, tvalid2);
     else
-      p2p_pass<T, RING, false>(c, list, b, rel, acc, ring, tb, lb, le, tcx, tcy, tcz, cycle, tiny,
+      p2p_pass<T, RING, W, false>(c, list, b, rel, acc, ring, tb, lb, le, tcx, tcy, tcz, cycle, tiny,
                                scale, G, t, t2, tvalid, false);
   }
 }
 
 constexpr int RING32 = 256;  // float4 entries: 4.25 KB with the pads
 constexpr int RING64 = 128;  // double4 entries: 4.25 KB with the pads
-constexpr int ring_entries(int ring) { return ring + ring / 16; }
 
-__global__ __launch_bounds__(64) void k_p2p_fp64(Cells c, Csr list, Bodies b, double *acc,
-                                                 double cycle) {
-  __shared__ double4 ring[ring_entries(RING64)];
-  p2p_leaf<double, RING64>(blockIdx.x, c, list, b, nullptr, acc, ring, cycle);
+template <int W>
+__global__ __launch_bounds__(64 * W) void k_p2p_fp64(Cells c, Csr list, Bodies b, double *acc,
+                                                     double cycle) {
+  __shared__ double4 ring[W * ring_entries(RING64)];
+  p2p_leaf<double, RING64, W>(blockIdx.x, c, list, b, nullptr, acc, ring, cycle);
 }
 
 // The FP64 P2P as resident waves taking target cells from a counter, as
 // k_p2p_fp32_resident below (each target computed by one wave exactly as by
 // k_p2p_fp64, so the fields do not change).
-__global__ __launch_bounds__(64) void k_p2p_fp64_resident(Cells c, int32_t ncells, Csr list,
-                                                         Bodies b, double *acc, uint32_t *next,
-                                                         double cycle) {
-  __shared__ double4 ring[ring_entries(RING64)];
+template <int W>
+__global__ __launch_bounds__(64 * W) void k_p2p_fp64_resident(Cells c, int32_t ncells, Csr list,
+                                                              Bodies b, double *acc,
+                                                              uint32_t *next, double cycle) {
+  __shared__ double4 ring[W * ring_entries(RING64)];
   __shared__ uint32_t take;
   while (true) {
     __syncthreads();
@@ -397,22 +420,51 @@ __global__ __launch_bounds__(64) void k_p2p_fp64_resident(Cells c, int32_t ncell
     __syncthreads();
     const uint32_t ti = take;
     if (ti >= (uint32_t)ncells) return;
-    p2p_leaf<double, RING64>((int32_t)ti, c, list, b, nullptr, acc, ring, cycle);
+    p2p_leaf<double, RING64, W>((int32_t)ti, c, list, b, nullptr, acc, ring, cycle);
   }
+}
+
+// launch(W) for the W waves a leaf that p2p_waves_per_leaf chose
+template <class F>
+void p2p_waves(int per_leaf, F launch) {
+  if (per_leaf >= 8) launch(std::integral_constant<int, 8>{});
+  else if (per_leaf >= 4) launch(std::integral_constant<int, 4>{});
+  else if (per_leaf >= 2) launch(std::integral_constant<int, 2>{});
+  else launch(std::integral_constant<int, 1>{});
+}
+
+int resident_blocks(int waves, int per_block, int32_t ncells) {
+  return std::min((waves + per_block - 1) / per_block, (int)ncells);
 }
 
 }  // namespace
 
+// With a wave a leaf, a problem of few leaves leaves SIMDs idle, and one of a
+// few thousand ends with single waves on its longest lists.  W waves shorten both
+// and cost a partial last chunk each.  Alone, us, with 1 / 2 / 4 / 8 waves, at ncrit
+// 64: 4,096-body cube 191 / 147 / 119 / 67, 16K cube 164 / 108 / 62 / 53, 64K
+// ellipsoid 223 / 141 / 121 / 141, 100K periodic 254 / 241 / 219 / 238, 256K
+// Plummer (FP32) 561 / 368 / 346 / 410, 500K ellipsoid 1,203 / 753 / 799 / 1,001,
+// 1M cube 2,165 / 2,173 / 2,175 / 2,405.  The number of bodies and ncrit alone
+// decide, so that every way to run an evaluation adds in the same order.
+int p2p_waves_per_leaf(int64_t n, int32_t ncrit) {
+  const int64_t leaves = n / ncrit;  // about
+  return leaves <= 512 ? 8 : leaves <= 2560 ? 4 : leaves <= 8192 ? 2 : 1;
+}
+
 hipError_t launch_p2p_fp64(Cells c, int32_t ncells, Csr list, Bodies b, double *acc,
-                           int resident, uint32_t *next, hipStream_t s, double cycle) {
+                           int per_leaf, int resident, uint32_t *next, hipStream_t s,
+                           double cycle) {
   if (ncells <= 0) return hipSuccess;
   if (resident > 0 && next) {
     hipError_t e = launch_fill_zero(next, 4, s);
     if (e != hipSuccess) return e;
-    const int grid = resident < ncells ? resident : ncells;
-    k_p2p_fp64_resident<<<grid, 64, 0, s>>>(c, ncells, list, b, acc, next, cycle);
+    p2p_waves(per_leaf, [&](auto w) {
+      const int grid = resident_blocks(resident, w, ncells);
+      k_p2p_fp64_resident<w><<<grid, 64 * w, 0, s>>>(c, ncells, list, b, acc, next, cycle);
+    });
   } else {
-    k_p2p_fp64<<<ncells, 64, 0, s>>>(c, list, b, acc, cycle);
+    p2p_waves(per_leaf, [&](auto w) { k_p2p_fp64<w><<<ncells, 64 * w, 0, s>>>(c, list, b, acc, cycle); });
   }
   return hipGetLastError();
 }
@@ -437,10 +489,11 @@ __global__ __launch_bounds__(64) void k_leaf_relpos(Cells c, Bodies b, float4 *r
                          (float)b.q[i]);
 }
 
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8)))
+template <int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(6, 8)))
 void k_p2p_fp32(Cells c, Csr list, Bodies b, const float4 *rel, double *acc, double cycle) {
-  __shared__ float4 ring[ring_entries(RING32)];
-  p2p_leaf<float, RING32>(blockIdx.x, c, list, b, rel, acc, ring, cycle);
+  __shared__ float4 ring[W * ring_entries(RING32)];
+  p2p_leaf<float, RING32, W>(blockIdx.x, c, list, b, rel, acc, ring, cycle);
 }
 
 // A fixed number of resident waves that take target cells from a counter
@@ -452,10 +505,11 @@ void k_p2p_fp32(Cells c, Csr list, Bodies b, const float4 *rel, double *acc, dou
 // kernel takes 232 of a SIMD's 512, which three waves of 94 would not leave, and
 // the M2L then ran mostly after the P2P (two clusters of 4M bodies 21.9 ms an
 // evaluation against 20.4, one cluster 12.2 against 11.5).
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8)))
+template <int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(6, 8)))
 void k_p2p_fp32_resident(Cells c, int32_t ncells, Csr list, Bodies b, const float4 *rel,
                          double *acc, uint32_t *next, double cycle) {
-  __shared__ float4 ring[ring_entries(RING32)];
+  __shared__ float4 ring[W * ring_entries(RING32)];
   __shared__ uint32_t take;
   while (true) {
     __syncthreads();
@@ -463,7 +517,7 @@ void k_p2p_fp32_resident(Cells c, int32_t ncells, Csr list, Bodies b, const floa
     __syncthreads();
     const uint32_t ti = take;
     if (ti >= (uint32_t)ncells) return;
-    p2p_leaf<float, RING32>((int32_t)ti, c, list, b, rel, acc, ring, cycle);
+    p2p_leaf<float, RING32, W>((int32_t)ti, c, list, b, rel, acc, ring, cycle);
   }
 }
 }  // namespace
@@ -478,25 +532,31 @@ hipError_t launch_leaf_relpos(Cells c, int32_t ncells, Bodies b, float4 *rel, hi
 // several such launches (on different streams) share the cells of one
 // cleared counter, each cell computed once by one wave
 hipError_t launch_p2p_fp32_drain(Cells c, int32_t ncells, Csr list, Bodies b, const float4 *rel,
-                                 double *acc, int waves, uint32_t *next, hipStream_t s,
-                                 double cycle) {
+                                 double *acc, int per_leaf, int waves, uint32_t *next,
+                                 hipStream_t s, double cycle) {
   if (ncells <= 0 || waves <= 0) return hipSuccess;
-  const int grid = waves < ncells ? waves : ncells;
-  k_p2p_fp32_resident<<<grid, 64, 0, s>>>(c, ncells, list, b, rel, acc, next, cycle);
+  p2p_waves(per_leaf, [&](auto w) {
+    const int grid = resident_blocks(waves, w, ncells);
+    k_p2p_fp32_resident<w><<<grid, 64 * w, 0, s>>>(c, ncells, list, b, rel, acc, next, cycle);
+  });
   return hipGetLastError();
 }
 
 hipError_t launch_p2p_fp32(Cells c, int32_t ncells, Csr list, Bodies b, const float4 *rel,
-                           double *acc, int resident, uint32_t *next, hipStream_t s,
-                           double cycle) {
+                           double *acc, int per_leaf, int resident, uint32_t *next,
+                           hipStream_t s, double cycle) {
   if (ncells <= 0) return hipSuccess;
   if (resident > 0 && next) {
     hipError_t e = launch_fill_zero(next, 4, s);
     if (e != hipSuccess) return e;
-    const int grid = resident < ncells ? resident : ncells;
-    k_p2p_fp32_resident<<<grid, 64, 0, s>>>(c, ncells, list, b, rel, acc, next, cycle);
+    p2p_waves(per_leaf, [&](auto w) {
+      const int grid = resident_blocks(resident, w, ncells);
+      k_p2p_fp32_resident<w><<<grid, 64 * w, 0, s>>>(c, ncells, list, b, rel, acc, next, cycle);
+    });
   } else {
-    k_p2p_fp32<<<ncells, 64, 0, s>>>(c, list, b, rel, acc, cycle);
+    p2p_waves(per_leaf, [&](auto w) {
+      k_p2p_fp32<w><<<ncells, 64 * w, 0, s>>>(c, list, b, rel, acc, cycle);
+    });
   }
   return hipGetLastError();
 }

@@ -208,7 +208,9 @@ hipError_t launch_m2l_fp64(Cells c, int32_t ncells, Csr list, int32_t npairs, co
 // (list sources are source words: leaf and periodic image, cycle the period)
 // resident > 0: that many resident waves take the target cells from *next
 // (cleared first), as launch_p2p_fp32
-hipError_t launch_p2p_fp64(Cells c, int32_t ncells, Csr list, Bodies b, double *acc,
+// per_leaf: waves that share a target leaf (p2p_waves_per_leaf)
+int p2p_waves_per_leaf(int64_t n, int32_t ncrit);
+hipError_t launch_p2p_fp64(Cells c, int32_t ncells, Csr list, Bodies b, double *acc, int per_leaf,
                            int resident, uint32_t *next, hipStream_t s, double cycle = 0);
 
 // direct.hip
@@ -307,10 +309,10 @@ hipError_t launch_leaf_relpos(Cells c, int32_t ncells, Bodies b, float4 *rel, hi
 // the resident FP32 P2P on a counter cleared by the caller (waves
 // workgroups of one wave each); launches sharing the counter split the cells
 hipError_t launch_p2p_fp32_drain(Cells c, int32_t ncells, Csr list, Bodies b, const float4 *rel,
-                                 double *acc, int waves, uint32_t *next, hipStream_t s,
+                                 double *acc, int per_leaf, int waves, uint32_t *next, hipStream_t s,
                                  double cycle);
 hipError_t launch_p2p_fp32(Cells c, int32_t ncells, Csr list, Bodies b, const float4 *rel,
-                           double *acc, int resident, uint32_t *next, hipStream_t s,
+                           double *acc, int per_leaf, int resident, uint32_t *next, hipStream_t s,
                            double cycle = 0);
 }  // namespace tfmm
 

@@ -58,3 +58,29 @@ def test_gpu_fp64_pairs_at_any_width(ctx, width):
     far = np.arange(n) != 2
     assert np.all(np.linalg.norm(f - ref, axis=1)[far] <=
                   5e-14 * np.linalg.norm(np.abs(ref) + np.abs(ref).max(1, keepdims=True), axis=1)[far])
+
+
+@pytest.mark.parametrize("n,ncrit", [(5, 8), (512, 1), (600, 1), (3000, 1), (9000, 1), (600, 300),
+                                     (20000, 16)])
+@pytest.mark.parametrize("precision,tol", [(tfmm.FP64, 1e-12), (tfmm.MIXED, 1e-6)])
+def test_gpu_waves_per_leaf(ctx, n, ncrit, precision, tol):
+    """Every number of waves a leaf (8, 4, 2 and 1, by n / ncrit), lists shorter
+    than it, and the resident form bit for bit the same."""
+    r = np.random.default_rng(n)
+    x, y, z = [r.random(n) for _ in range(3)]
+    q = r.random(n) + 0.5
+    print("n=%d ncrit=%d precision %d" % (n, ncrit, precision), flush=True)
+    ctx.set_bodies(x, y, z, q)
+    prm = tfmm.make_params(ncrit, 0.5, precision)
+    ctx.evaluate(prm)
+    f = ctx.fields()
+    ctx.set_tuning(tfmm.TUNE_P2P_WAVES, 2)
+    try:
+        ctx.evaluate(prm)
+        assert np.array_equal(ctx.fields(), f)
+    finally:
+        ctx.set_tuning(tfmm.TUNE_P2P_WAVES, 0)
+    # against the oracle's evaluation: FP64 differs by rounding, mixed by the
+    # rounding of FP32 pairs (6e-8) and, in the far field, of FP32 M2L
+    ep, ea = oracle.rel_l2(f, oracle.Run(x, y, z, q, ncrit, 0.5, phases=3).fields())
+    assert ep < tol and ea < 4 * tol, (ep, ea)
