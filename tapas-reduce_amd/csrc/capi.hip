@@ -28,7 +28,9 @@ namespace {
 enum Ev {
   EV_BEGIN,
   EV_TREE,
+  EV_UP0,
   EV_UP,
+  EV_UPJOIN,  // the early upward pass's end, for the join only
   EV_DTT0,
   EV_DTT1,
   EV_M2L0,
@@ -528,8 +530,7 @@ int sort_list(tfmm_ctx *c, DevBuf &pairs, uint32_t npairs, DevBuf &off, DevBuf &
 
 // The Cartesian basis's upward pass: P2M, then M2M level by level (Mc);
 // for the set kernel's route also the spherical images of the multipoles (M).
-int cart_upward(tfmm_ctx *c) {
-  hipStream_t s = c->stream;
+int cart_upward(tfmm_ctx *c, hipStream_t s) {
   const Cells k = cells_of(c);
   TRY(launch_fill_zero(c->Mc.ptr, cart_bytes(c->ncells), s));
   TRY(launch_cart_p2m(k, (int32_t)c->ncells, sorted_bodies(c), dp<double>(c->Mc), s));
@@ -593,7 +594,7 @@ int do_upward(tfmm_ctx *c) {
   if (cartesian(c)) {
     int rc = cart_tables(c);
     if (rc) return rc;
-    return cart_upward(c);
+    return cart_upward(c, c->stream);
   }
   const size_t bytes = sph_bytes(c->ncells);
   TRY(hipMemsetAsync(c->M.ptr, 0, bytes, s));
@@ -1191,7 +1192,72 @@ int fork_p2p(tfmm_ctx *c, int64_t ncells = -1) {
   return TFMM_OK;
 }
 
+// The upward pass on stream st, with the scaled multipoles of the M2L (the
+// Cartesian basis: in its own arrays, then the spherical images).
+int upward_pass(tfmm_ctx *c, hipStream_t st) {
+  const Cells k = cells_of(c);
+  const int nl = (int)c->lvl.size() - 1;
+  TRY(rec(c, EV_UP0, st));
+  if (cartesian(c)) {
+    const int rc = cart_upward(c, st);
+    if (rc) return rc;
+  } else {
+    TRY(launch_fill_zero(c->M.ptr, sph_bytes(c->ncells), st));
+    TRY(launch_p2m(k, (int32_t)c->ncells, sorted_bodies(c), dp<double>(c->M), st));
+    for (int d = nl - 2; d >= 0; d--)
+      TRY(launch_m2m(k, c->lvl[d + 1], (c->lvl[d + 2] - c->lvl[d + 1]) / 8,
+                     dp<double>(c->tops), dp<double>(c->M), st));
+  }
+  if (!cart_direct(c))
+    TRY(launch_m2l_scale_m(k, (int32_t)c->ncells, dp<double>(c->M), c->mq.ptr, m2l_fp32(c), st));
+  TRY(rec(c, EV_UP, st));
+  return TFMM_OK;
+}
+
+// The upward pass needs the tree only.  Where the P2P starts with the numeric
+// phase or later (schedules 0 and 1), it runs on the second stream from the end of
+// the tree build, beside the traversal and the list building: short kernels and
+// host round trips that leave most of the GPU idle, while a P2P that started
+// before it would hold its slots.  256K Plummer 2.86 to 2.57 ms, 500K ellipsoid
+// 4.91 to 4.59, 4M Plummer with schedule 0 12.97 to 12.63.  With the P2P started
+// beside the list building it stays in the numeric phase: it would delay the P2P
+// (4M Plummer, schedule 2, 11.25 ms against 11.64).  A numeric phase that is a
+// graph of its own (TFMM_TUNE_GRAPH 1) keeps it too.
+bool early_upward(const tfmm_ctx *c) { return c->use_graph != 1 && c->p2p_schedule < 2; }
+
+int fork_upward(tfmm_ctx *c) {
+  TRY(hipEventRecord(c->ev[EV_P2PREADY], c->stream));
+  TRY(hipStreamWaitEvent(c->side, c->ev[EV_P2PREADY], 0));
+  const int rc = upward_pass(c, c->side);
+  (void)hipEventRecord(c->ev[EV_UPJOIN], c->side);
+  return rc;
+}
+
+int fused_lists(tfmm_ctx *c);
+
 int fused_prepare(tfmm_ctx *c) {
+  hipStream_t s = c->stream;
+  TRY(reserve_expansions(c));
+  int rc = cartesian(c) ? cart_tables(c) : TFMM_OK;
+  if (rc) return rc;
+  if (!cart_direct(c)) {
+    if (!c->tops_ready) {
+      TRY(dev_reserve(c->tops, translation_ops_doubles() * 8));
+      TRY(launch_translation_ops(dp<double>(c->tops), s));
+      c->tops_ready = true;
+    }
+    TRY(dev_reserve(c->mq, m2l_mq_bytes(c->ncells, m2l_fp32(c))));
+  }
+  c->p2p_forked = false;
+  if (!early_upward(c)) return fused_lists(c);
+  rc = fork_upward(c);
+  if (!rc) rc = fused_lists(c);
+  // what was started on the second stream ends before anything that follows
+  if (rc) (void)hipStreamWaitEvent(s, c->ev[EV_UPJOIN], 0);
+  return rc;
+}
+
+int fused_lists(tfmm_ctx *c) {
   hipStream_t s = c->stream;
   const Cells k = cells_of(c);
   const bool mixed = c->prm.precision == TFMM_MIXED;
@@ -1205,7 +1271,6 @@ int fused_prepare(tfmm_ctx *c) {
     TRY(launch_leaf_relpos(k, (int32_t)c->ncells, sorted_bodies(c), dp<float4>(c->relpos), s));
   }
   TRY(dev_reserve(c->acc, (size_t)c->n * 32));
-  c->p2p_forked = false;
   if (c->p2p_schedule >= 2 && !c->use_graph) {
     // the P2P list is complete: start the P2P now, beside the M2L batch
     // building (with resident waves it leaves that work CU slots)
@@ -1214,25 +1279,17 @@ int fused_prepare(tfmm_ctx *c) {
     c->p2p_forked = true;
   }
   rc = cart_direct(c) ? cart_lists(c) : build_m2l_batches(c);
-  if (!rc && cartesian(c)) rc = cart_tables(c);
   if (rc) {
     if (c->p2p_forked) (void)hipStreamWaitEvent(s, c->ev[EV_P2PJOIN], 0);
     return rc;
   }
   TRY(hipMemcpyAsync(c->h_u64, static_cast<char *>(c->cnt.ptr) + 32, 16, hipMemcpyDeviceToHost, s));
-  TRY(reserve_expansions(c));
   if (cart_direct(c)) {
     TRY(dev_reserve(c->trg, (size_t)c->n * 32));
     TRY(dev_reserve(c->out, (size_t)c->n * 32));
     TRY(hipEventRecord(c->ev[EV_DTT1], s));
     return TFMM_OK;
   }
-  if (!c->tops_ready) {
-    TRY(dev_reserve(c->tops, translation_ops_doubles() * 8));
-    TRY(launch_translation_ops(dp<double>(c->tops), s));
-    c->tops_ready = true;
-  }
-  TRY(dev_reserve(c->mq, m2l_mq_bytes(c->ncells, m2l_fp32(c))));
   TRY(dev_reserve(c->trg, (size_t)c->n * 32));
   TRY(dev_reserve(c->out, (size_t)c->n * 32));
   TRY(dev_reserve(c->leaf_of, (size_t)c->n * 4));
@@ -1251,8 +1308,8 @@ int fused_numeric(tfmm_ctx *c) {
   int rc;
   if (!c->p2p_forked && c->p2p_schedule != 1 && (rc = fork_p2p(c))) return rc;
   if (cart_direct(c)) {
-    if ((rc = cart_upward(c))) return rc;
-    TRY(rec(c, EV_UP, s));
+    if (early_upward(c)) TRY(hipStreamWaitEvent(s, c->ev[EV_UPJOIN], 0));
+    else if ((rc = upward_pass(c, s))) return rc;
     if (!c->p2p_forked && c->p2p_schedule == 1 && (rc = fork_p2p(c))) return rc;
     if ((rc = cart_m2l(c))) return rc;
     TRY(rec(c, EV_M2L1, s));
@@ -1263,22 +1320,12 @@ int fused_numeric(tfmm_ctx *c) {
     TRY(rec(c, EV_DOWN, s));
     return TFMM_OK;
   }
-  // upward (the Cartesian basis: in its own arrays, then the spherical images)
-  const size_t ebytes = sph_bytes(c->ncells);
+  // upward
   const int nl = (int)c->lvl.size() - 1;
-  if (cartesian(c)) {
-    if ((rc = cart_upward(c))) return rc;
-  } else {
-    TRY(launch_fill_zero(c->M.ptr, ebytes, s));
-    TRY(launch_p2m(k, (int32_t)c->ncells, sorted_bodies(c), dp<double>(c->M), s));
-    for (int d = nl - 2; d >= 0; d--)
-      TRY(launch_m2m(k, c->lvl[d + 1], (c->lvl[d + 2] - c->lvl[d + 1]) / 8,
-                     dp<double>(c->tops), dp<double>(c->M), s));
-  }
-  TRY(rec(c, EV_UP, s));
+  if (early_upward(c)) TRY(hipStreamWaitEvent(s, c->ev[EV_UPJOIN], 0));
+  else if ((rc = upward_pass(c, s))) return rc;
   // M2L
   const bool mixed = m2l_fp32(c);
-  TRY(launch_m2l_scale_m(k, (int32_t)c->ncells, dp<double>(c->M), c->mq.ptr, mixed, s));
   TRY(rec(c, EV_M2L0, s));
   if (!c->p2p_forked && c->p2p_schedule == 1 && (rc = fork_p2p(c))) return rc;
   const int32_t tile = m2l_tile_size();
@@ -1640,6 +1687,24 @@ int whole_record(tfmm_ctx *c) {
   TRY(launch_tree_final(lev, pl.L, dp<uint32_t>(c->lev_status), m2l_tile_size(), sz, s));
   TRY(launch_pad_cells(k, sz, cells, s));
   TRY(rec(c, EV_TREE, s));
+  auto upward = [&](hipStream_t st) -> int {
+    TRY(rec(c, EV_UP0, st));
+    TRY(launch_fill_zero(c->M.ptr, (size_t)cells * NTERM * 16, st));
+    TRY(launch_p2m(k, cells, sorted_bodies(c), dp<double>(c->M), st));
+    for (int d = pl.L - 2; d >= 0; d--)
+      TRY(launch_m2m(k, 0, pl.grid[d + 1] / 8 + 1, dp<double>(c->tops), dp<double>(c->M), st, lev,
+                     d + 1));
+    TRY(launch_m2l_scale_m(k, cells, dp<double>(c->M), c->mq.ptr, mixed, st));
+    TRY(rec(c, EV_UP, st));
+    return TFMM_OK;
+  };
+  int rc;
+  if (early_upward(c)) {
+    TRY(hipEventRecord(c->ev[EV_P2PREADY], s));
+    TRY(hipStreamWaitEvent(c->side, c->ev[EV_P2PREADY], 0));
+    if ((rc = upward(c->side))) return rc;
+    TRY(hipEventRecord(c->ev[EV_UPJOIN], c->side));
+  }
   TRY(rec(c, EV_DTT0, s));
   // traversal
   uint32_t *cnt = dp<uint32_t>(c->cnt);
@@ -1675,7 +1740,6 @@ int whole_record(tfmm_ctx *c) {
   if (mixed)
     TRY(launch_leaf_relpos(k, cells, sorted_bodies(c), dp<float4>(c->relpos), s));
   // schedules 2 and 3: the P2P branches off here, beside the M2L batching
-  int rc;
   const bool early = c->p2p_schedule >= 2;
   if (early && (rc = fork_p2p(c, cells))) return rc;
   // M2L batches
@@ -1727,14 +1791,8 @@ int whole_record(tfmm_ctx *c) {
   TRY(rec(c, EV_DTT1, s));
   // the numeric phase
   if (!early && c->p2p_schedule != 1 && (rc = fork_p2p(c, cells))) return rc;
-  const size_t ebytes = (size_t)cells * NTERM * 16;
-  TRY(launch_fill_zero(c->M.ptr, ebytes, s));
-  TRY(launch_p2m(k, cells, sorted_bodies(c), dp<double>(c->M), s));
-  for (int d = pl.L - 2; d >= 0; d--)
-    TRY(launch_m2m(k, 0, pl.grid[d + 1] / 8 + 1, dp<double>(c->tops), dp<double>(c->M), s, lev,
-                   d + 1));
-  TRY(rec(c, EV_UP, s));
-  TRY(launch_m2l_scale_m(k, cells, dp<double>(c->M), c->mq.ptr, mixed, s));
+  if (early_upward(c)) TRY(hipStreamWaitEvent(s, c->ev[EV_UPJOIN], 0));
+  else if ((rc = upward(s))) return rc;
   TRY(rec(c, EV_M2L0, s));
   if (c->p2p_schedule == 1 && (rc = fork_p2p(c, cells))) return rc;
   TRY(launch_m2l_sets(dp<int32_t>(c->set_off), dp<int2>(c->units), dp<uint32_t>(c->u_cnt),
@@ -2513,8 +2571,9 @@ int tfmm_get_stats(tfmm_ctx *c, tfmm_stats_t *o) {
   }
   if (c->fused && c->stage >= 4) {
     // fused order: traversal and list building, then upward, M2L/P2P, downward
-    o->ms_upward = el(EV_DTT1, EV_UP);
-    o->ms_traverse = el(EV_DTT0, EV_DTT1) + el(EV_UP, EV_TRAV);
+    // the upward pass may run beside the traversal, on the second stream
+    o->ms_upward = el(EV_UP0, EV_UP);
+    o->ms_traverse = el(EV_DTT0, EV_TRAV);
   } else {
     if (c->stage >= 2) o->ms_upward = el(EV_TREE, EV_UP);
     if (c->stage >= 3) o->ms_traverse = el(EV_UP, EV_TRAV);
