@@ -312,6 +312,7 @@ __global__ __launch_bounds__(IT_THREADS) void k_items(const uint32_t *keys, cons
   if (lane == 63) wsum[wid] = inc;
   __syncthreads();
   uint32_t pre = 0, tot = 0;
+#pragma unroll 4
   for (int w = 0; w < IT_THREADS / 64; w++) {
     pre += w < wid ? wsum[w] : 0u;
     tot += wsum[w];

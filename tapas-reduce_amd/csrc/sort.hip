@@ -16,10 +16,15 @@ constexpr int SCAN_THREADS = 256;
 constexpr int SCAN_ITEMS = 8;
 constexpr int SCAN_TILE = SCAN_THREADS * SCAN_ITEMS;
 
-constexpr int RS_THREADS = 256;
+// A tile of 4,096 keys is a workgroup of 1,024 threads with 4 keys each: a tile's
+// time is the latency of its chain of rows (16 rows of 256 threads: see below).
+constexpr int RS_THREADS = 1024;
 constexpr int RS_WAVES = RS_THREADS / 64;
-constexpr int RS_ROWS = 16;  // keys per lane
+constexpr int RS_ROWS = 4;  // keys per lane
 constexpr int RS_TILE = RS_THREADS * RS_ROWS;
+// Up to this many tiles every tile's workgroup sums the counts of the tiles
+// before it by itself instead of a scan between the two kernels.
+constexpr int SELF_TILES = 32;
 constexpr int RS_MAXBITS = 9;
 constexpr int RS_BINS = 1 << RS_MAXBITS;
 
@@ -34,14 +39,16 @@ __device__ inline uint32_t wave_incl_scan(uint32_t v, int lane) {
 
 // block-wide exclusive scan of one value per thread; returns the exclusive
 // prefix and writes the block total to *total
+template <int THREADS>
 __device__ inline uint32_t block_excl_scan(uint32_t v, uint32_t *total) {
-  __shared__ uint32_t wsum[SCAN_THREADS / 64];
+  __shared__ uint32_t wsum[THREADS / 64];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   uint32_t inc = wave_incl_scan(v, lane);
   if (lane == 63) wsum[wid] = inc;
   __syncthreads();
   uint32_t off = 0, tot = 0;
-  for (int w = 0; w < SCAN_THREADS / 64; w++) {
+#pragma unroll 2
+  for (int w = 0; w < THREADS / 64; w++) {
     if (w < wid) off += wsum[w];
     tot += wsum[w];
   }
@@ -61,7 +68,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_reduce(const uint32_t *in
     if (j < n) s += in[j];
   }
   uint32_t tot;
-  block_excl_scan(s, &tot);
+  block_excl_scan<SCAN_THREADS>(s, &tot);
   if (threadIdx.x == 0) sums[blockIdx.x] = tot;
 }
 
@@ -79,7 +86,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_down(const uint32_t *in, 
     s += v[i];
   }
   uint32_t tot;
-  uint32_t run = block_excl_scan(s, &tot) + (block_off ? block_off[blockIdx.x] : 0u);
+  uint32_t run = block_excl_scan<SCAN_THREADS>(s, &tot) + (block_off ? block_off[blockIdx.x] : 0u);
 #pragma unroll
   for (int i = 0; i < SCAN_ITEMS; i++) {
     const int64_t j = base + i;
@@ -94,9 +101,13 @@ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // radix sort
 // ---------------------------------------------------------------------------
 // LSD passes of up to RS_MAXBITS bits; a pass = per-tile digit histogram,
-// device-wide exclusive scan of the (digit, tile) counts, and a stable
-// scatter that ranks each tile in LDS (wave ballots), stages it in digit
-// order and writes every digit run to consecutive positions.
+// device-wide exclusive scan of the (digit, tile) counts (for a few tiles inside
+// the scatter), and a stable scatter that ranks each tile in LDS (wave ballots),
+// stages it in digit order and writes every digit run to consecutive positions.
+// Before and after the wide tile, us per scatter beside nothing: 64-bit keys, 4,096
+// 15.2 and 8.8, 1M 20.6 and 13.4, 4M 43 and 31, 8M 70 and 55.  With the scan inside
+// (up to SELF_TILES tiles) a launch and its gap less a pass: 16K cube 1.02 to 0.78
+// ms an evaluation, both together.
 
 template <class K>
 __device__ inline uint32_t digit_of(K k, int shift, uint32_t mask) {
@@ -123,11 +134,15 @@ __global__ __launch_bounds__(RS_THREADS) void k_radix_hist(const K *__restrict__
     counts[(int64_t)d * nblocks + blockIdx.x] = hist[d];
 }
 
-template <class K>
+// counts: the histograms (SELF), else their exclusive scan.  At most 48 registers
+// (the loops over the waves are unrolled by two for that): a workgroup is four
+// waves a SIMD, and must fit beside four resident P2P waves of 80.  With more, a
+// sort of the few pairs outside the M2L groups waited 5 ms for the P2P's end.
+template <class K, bool SELF>
 __global__ __launch_bounds__(RS_THREADS) void k_radix_scatter(
     const K *__restrict__ keys_in, const uint32_t *__restrict__ vals_in, K *__restrict__ keys_out,
     uint32_t *__restrict__ vals_out, int64_t n, int shift, int nbits,
-    const uint32_t *__restrict__ offsets, int nblocks, const uint32_t *dn) {
+    const uint32_t *__restrict__ counts, int nblocks, const uint32_t *dn) {
   __builtin_amdgcn_s_setprio(2);  // as the kernels beside the early P2P (critical_path_priority)
   // The wave histograms are dead once every key knows its place in the tile,
   // so the tile's staging arrays reuse their LDS (more blocks per CU).
@@ -143,6 +158,42 @@ __global__ __launch_bounds__(RS_THREADS) void k_radix_scatter(
   const uint32_t mask = (1u << nbits) - 1u;
   if (dn) n = min(n, (int64_t)*dn);
   for (int i = lane; i < RS_BINS; i += 64) whist[wid][i] = 0;
+  // the digits' global positions, read here so that the write loop at the end
+  // waits on no global load
+  constexpr int DPT = (RS_BINS + RS_THREADS - 1) / RS_THREADS;  // consecutive digits of a thread
+  uint32_t unused;
+  if (SELF) {  // keys of smaller digits, and of the digit in the tiles before
+    uint32_t before[DPT], all[DPT], sum = 0;
+#pragma unroll
+    for (int u = 0; u < DPT; u++) {
+      const int d = threadIdx.x * DPT + u;
+      before[u] = all[u] = 0;
+      if (d > (int)mask) continue;
+      const uint32_t *c = counts + (int64_t)d * nblocks;
+#pragma unroll 1
+      for (int b0 = 0; b0 < nblocks; b0 += 4) {
+        uint32_t x[4];
+#pragma unroll
+        for (int b = 0; b < 4; b++) x[b] = b0 + b < nblocks ? c[b0 + b] : 0u;
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+          before[u] += b0 + b < (int)blockIdx.x ? x[b] : 0u;
+          all[u] += x[b];
+        }
+      }
+      sum += all[u];
+    }
+    uint32_t base = block_excl_scan<RS_THREADS>(sum, &unused);
+#pragma unroll
+    for (int u = 0; u < DPT; u++) {
+      const int d = threadIdx.x * DPT + u;
+      if (d <= (int)mask) gshift[d] = base + before[u];
+      base += all[u];
+    }
+  } else {
+    for (int d = threadIdx.x; d <= (int)mask; d += RS_THREADS)
+      gshift[d] = counts[(int64_t)d * nblocks + blockIdx.x];
+  }
   __syncthreads();
 
   const int64_t wbase = (int64_t)blockIdx.x * RS_TILE + (int64_t)wid * (64 * RS_ROWS);
@@ -172,31 +223,29 @@ __global__ __launch_bounds__(RS_THREADS) void k_radix_scatter(
   }
   __syncthreads();
   // per digit: offsets of the waves (exclusive, in wave order) and the tile's
-  // count; then the tile's digit starts (exclusive scan over digits).  Each
-  // thread owns RS_BINS / RS_THREADS consecutive digits.
-  constexpr int DPT = RS_BINS / RS_THREADS;
+  // count; then the tile's digit starts (exclusive scan over digits)
   uint32_t cnt[DPT];
   uint32_t mine = 0;
 #pragma unroll
   for (int u = 0; u < DPT; u++) {
     const int d = threadIdx.x * DPT + u;
     cnt[u] = 0;
-    for (int w = 0; w < RS_WAVES; w++) {
-      const uint32_t t = whist[w][d];
-      whist[w][d] = cnt[u];
-      cnt[u] += t;
-    }
+    if (d < RS_BINS)
+#pragma unroll 2
+      for (int w = 0; w < RS_WAVES; w++) {
+        const uint32_t t = whist[w][d];
+        whist[w][d] = cnt[u];
+        cnt[u] += t;
+      }
     mine += cnt[u];
   }
-  uint32_t unused;
-  uint32_t start = block_excl_scan(mine, &unused);
+  uint32_t start = block_excl_scan<RS_THREADS>(mine, &unused);
 #pragma unroll
   for (int u = 0; u < DPT; u++) {
     const int d = threadIdx.x * DPT + u;
+    if (d >= RS_BINS) continue;
     dstart[d] = start;
-    // the digit's global offsets, read once here so the write loop below
-    // waits on no global load
-    if (d <= (int)mask) gshift[d] = offsets[(int64_t)d * nblocks + blockIdx.x] - start;
+    if (d <= (int)mask) gshift[d] -= start;
     start += cnt[u];
   }
   __syncthreads();
@@ -334,11 +383,17 @@ static hipError_t radix_sort_impl(K *keys, uint32_t *vals, K *keys_alt, uint32_t
     const int nbits = (bit_hi - lo + (passes - ps) - 1) / (passes - ps);  // balanced widths
     const uint32_t mask = (1u << nbits) - 1u;
     const int64_t nc = (int64_t)nb * (mask + 1);
+    hipError_t e = hipSuccess;
     k_radix_hist<K><<<nb, RS_THREADS, 0, s>>>(kin, n, lo, mask, counts, nb, dn);
-    hipError_t e = scan_exclusive_u32(counts, offs, nc, stmp, s);
-    if (e != hipSuccess) return e;
-    k_radix_scatter<K><<<nb, RS_THREADS, 0, s>>>(kin, vin, kout, vout, n, lo, nbits, offs, nb,
-                                                  dn);
+    if (nb <= SELF_TILES) {
+      k_radix_scatter<K, true><<<nb, RS_THREADS, 0, s>>>(kin, vin, kout, vout, n, lo, nbits,
+                                                         counts, nb, dn);
+    } else {
+      e = scan_exclusive_u32(counts, offs, nc, stmp, s);
+      if (e != hipSuccess) return e;
+      k_radix_scatter<K, false><<<nb, RS_THREADS, 0, s>>>(kin, vin, kout, vout, n, lo, nbits,
+                                                          offs, nb, dn);
+    }
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     K *tk = kin; kin = kout; kout = tk;
