@@ -41,8 +41,8 @@ namespace tfmm {
 namespace {
 
 constexpr int DTT_THREADS = 1024;
-constexpr int DTT_PPT = 4;  // frontier pairs per thread
 constexpr int DTT_WAVES = DTT_THREADS / 64;
+constexpr uint32_t DTT_ONE = 1 << 19;  // frontiers up to this take one pair per thread
 
 // per-cell traversal records: (centre, R) with R = (width / 2 * 1.00001) / theta
 // (tapas_exafmm.cxx:222-226), and (first child, body count)
@@ -60,6 +60,8 @@ __global__ void k_dtt_cells(Cells c, int32_t ncells, double theta, double4 *geo,
 // Kind of a frontier pair after the MAC: what the step emits for it.
 enum : int { DK_NONE = 0, DK_M2L, DK_FAR_EMPTY, DK_P2P, DK_SPLIT_I, DK_SPLIT_J, DK_SPLIT_BOTH };
 
+// DTT_PPT: frontier pairs per thread (launch_dtt_step chooses)
+template <int DTT_PPT>
 __global__ __launch_bounds__(DTT_THREADS) void k_dtt_step(const int2 *in, const uint32_t *nin_dev,
                                                   uint32_t nin_max, int2 *out, uint32_t out_cap,
                                                   uint32_t *nout, int2 *m2l, uint32_t m2l_cap,
@@ -470,11 +472,20 @@ hipError_t launch_dtt_step(const int2 *in, const uint32_t *nin_dev, uint32_t nin
                            int32_t *m2l_slot, uint32_t *used, uint32_t *n_outside, int mutual,
                            hipStream_t s, double cycle) {
   if (nin_max == 0) return hipSuccess;
-  const uint32_t per = DTT_THREADS * DTT_PPT;
-  k_dtt_step<<<(nin_max + per - 1) / per, DTT_THREADS, 0, s>>>(
-      in, nin_dev, nin_max, out, out_cap, nout, m2l, m2l_cap, p2p, p2p_cap, cnt, geo, topo, depth,
-      width, m2l_slot, used, n_outside, mutual, cycle);
-  return hipGetLastError();
+  // Four pairs per thread spare a large frontier same-address atomics, which bound
+  // it then; a smaller one they leave on a quarter of the CUs it could use, for
+  // four times the chain of gathers.  All steps of a traversal, us, at 4 / the
+  // better by size: 4,096-body cube 81 / 48, 64K ellipsoid 230 / 164, 256K Plummer
+  // 484 / 326, 500K ellipsoid 586 / 530, 1M cube 444 / 404, 4M Plummer 1,673 /
+  // 1,605; the line at 2^17 or 2^20 pairs lies between on most of them.
+  auto go = [&](auto kernel, uint32_t ppt) {
+    const uint32_t per = DTT_THREADS * ppt;
+    kernel<<<(nin_max + per - 1) / per, DTT_THREADS, 0, s>>>(
+        in, nin_dev, nin_max, out, out_cap, nout, m2l, m2l_cap, p2p, p2p_cap, cnt, geo, topo, depth,
+        width, m2l_slot, used, n_outside, mutual, cycle);
+    return hipGetLastError();
+  };
+  return nin_max <= DTT_ONE ? go(k_dtt_step<1>, 1) : go(k_dtt_step<4>, 4);
 }
 
 hipError_t launch_pair_slots(const int2 *pairs, uint32_t n, const double4 *geo,
