@@ -59,6 +59,7 @@ struct Plan {
   // capacities
   int L = 0;                        // tree levels
   std::vector<int32_t> grid;        // cells per level
+  int top = 0;                      // leading levels built by one workgroup
   int64_t cells = 0;                // cells in all
   int max_depth = 0, nsteps = 0, cwords = 0;
   int32_t nslots = 0, ntiles = 0;
@@ -144,6 +145,7 @@ struct tfmm_ctx {
   Plan plan;                      // the whole-evaluation graph (use_graph == 2)
   DevBuf gsz, gstep;              // its device sizes and traversal step grids
   uint32_t *h_plan = nullptr;     // pinned read-back of the whole graph (PLAN_HOST_BYTES)
+  bool upward_pending = false;  // the early upward pass is still to be enqueued
   bool one_graph = false;         // the last tfmm_evaluate was one launch of it
   // periodic images (tfmm_set_periodic): image sublevels, 0 = none, and the
   // period; the root cell is then the periodic cell
@@ -385,12 +387,12 @@ int build_levels_hinted(tfmm_ctx *c, int64_t n, const int64_t *off, int np,
   TRY(dev_reserve(c->flag, (size_t)gmax * 4 + 1024));
   TRY(dev_reserve(c->slot, (size_t)gmax * 4 + 1024));
   TRY(dev_reserve(c->lev_bsum, (size_t)level_blocks((int32_t)gmax) * 4 + 4));
-  TRY(hipMemsetAsync(c->lev.ptr, 0, (size_t)2 * (L + 1) * 4, s));
-  TRY(hipMemsetAsync(c->lev_status.ptr, 0, 4, s));
   const Cells k = cells_of(c);
   int32_t *lev = dp<int32_t>(c->lev);
-  TRY(launch_roots(k, n, off, np, dp<double>(c->region), lev, s));
-  for (int d = 0; d < L; d++)
+  const int top = tree_top_levels(c->tree_hint.data(), L);
+  TRY(launch_tree_top(k, n, off, np, lev, L, top, c->prm.ncrit, cap, dp<uint32_t>(c->lev_status),
+                      skeys, dp<double>(c->region), sprob, s));
+  for (int d = top; d < L; d++)
     TRY(launch_level_step(k, lev, d, grid[d], c->prm.ncrit, cap, dp<uint32_t>(c->flag),
                           dp<uint32_t>(c->slot), dp<uint32_t>(c->lev_bsum),
                           dp<uint32_t>(c->lev_status), skeys, dp<double>(c->region), sprob, s));
@@ -489,7 +491,7 @@ int do_build_tree(tfmm_ctx *c) {
     }
   }
   TRY(reserve_cells(c, std::max<size_t>(4096, 8 * (size_t)np), 0, s));
-  TRY(launch_roots(cells_of(c), n, off, np, dp<double>(c->region), nullptr, s));
+  TRY(launch_roots(cells_of(c), n, off, np, dp<double>(c->region), s));
   c->lvl.assign(1, 0);
   int32_t lbeg = 0, lcnt = np;
   int64_t nleaves = 0;
@@ -638,6 +640,8 @@ int sort_list(tfmm_ctx *c, DevBuf &pairs, uint32_t npairs, DevBuf &off, DevBuf &
   return TFMM_OK;
 }
 
+int run_pending_upward(tfmm_ctx *c);
+
 // The traversal runs 2 max_depth + 2 breadth-first steps (every step refines
 // one side of a pair by one level, so no pair survives longer), each reading
 // its input size on the device: one host round trip for the whole traversal.
@@ -656,8 +660,6 @@ int do_dtt(tfmm_ctx *c) {
   if (cwords > H_U32_WORDS) return fail(c, TFMM_EINVAL, "tree too deep");
   TRY(dev_reserve(c->dtt_geo, (size_t)c->ncells * 32));
   TRY(dev_reserve(c->dtt_topo, (size_t)c->ncells * 8));
-  TRY(launch_dtt_cells(k, (int32_t)c->ncells, c->prm.theta, dp<double4>(c->dtt_geo),
-                       dp<int2>(c->dtt_topo), s));
   // A frontier that overflowed truncates every later step, so the counts
   // seen after an overflow are lower bounds: capacities at least double.
   // M2L group-table flags (one per slot), then the count of M2L pairs
@@ -667,13 +669,13 @@ int do_dtt(tfmm_ctx *c) {
   for (int attempt = 0; attempt < 12; attempt++) {
     TRY(dev_reserve(c->m2l_pairs, (size_t)c->m2l_cap * 8));
     TRY(dev_reserve(c->slot_of, (size_t)c->m2l_cap * 4));
-    TRY(hipMemsetAsync(c->g_used.ptr, 0, (size_t)(nslots + 1) * 4, s));
     TRY(dev_reserve(c->p2p_pairs, (size_t)c->p2p_cap * 8));
     TRY(dev_reserve(c->front_a, (size_t)c->front_cap * 8));
     TRY(dev_reserve(c->front_b, (size_t)c->front_cap * 8));
     uint32_t *cnt = dp<uint32_t>(c->cnt);
-    TRY(hipMemsetAsync(cnt, 0, (size_t)cwords * 4, s));
-    TRY(launch_root_pairs(dp<int2>(c->front_a), c->nprob, cnt + 16, s, c->images > 0));
+    TRY(launch_dtt_begin(k, (int32_t)c->ncells, c->prm.theta, dp<double4>(c->dtt_geo),
+                         dp<int2>(c->dtt_topo), dp<uint32_t>(c->g_used), nslots + 1, cnt, cwords,
+                         dp<int2>(c->front_a), c->nprob, s, c->images > 0));
     // grid of step st: the frontier size of the previous traversal of the same
     // tree shape when there is one (checked below), else the capacity
     const bool hint = (int)c->dtt_hint.size() == nsteps + 1 && c->dtt_hint_cells == c->ncells;
@@ -689,6 +691,8 @@ int do_dtt(tfmm_ctx *c) {
       std::swap(c->front_a, c->front_b);
     }
     TRY(hipMemcpyAsync(c->h_u32, cnt, (size_t)cwords * 4, hipMemcpyDeviceToHost, s));
+    const int rc = run_pending_upward(c);
+    if (rc) return rc;
     TRY(hipStreamSynchronize(s));
     uint32_t fmax = 0;
     c->dtt_steps = 0;
@@ -797,7 +801,7 @@ int build_m2l_batches(tfmm_ctx *c, bool given = false) {
   TRY(dev_reserve(c->fkeys_alt, nn * 8));
   TRY(dev_reserve(c->fvals_alt, nn * 4));
   TRY(dev_reserve(c->g_cnt, 16));
-  TRY(hipMemsetAsync(c->g_cnt.ptr, 0, 16, s));
+  if (n_outside || given) TRY(hipMemsetAsync(c->g_cnt.ptr, 0, 16, s));
   const int gbits = bits_for(ngr);
   const int sbits = bits_for(c->ncells);
   {
@@ -854,27 +858,29 @@ int build_m2l_batches(tfmm_ctx *c, bool given = false) {
   c->n_items = nitems;
   c->group_bits = gbits;
   TRY(dev_reserve(c->set_off, (size_t)(ntiles + 1) * 4));
-  TRY(launch_m2l_set_offsets(dp<uint32_t>(c->items), nitems, gbits, ntiles, dp<int32_t>(c->set_off),
-                             s));
   c->unit_chunk = m2l_unit_chunk(nitems, ntiles, c->m2l_unit_factor);
   c->units_bound = m2l_units_bound(nitems, ntiles, c->unit_chunk);
   TRY(dev_reserve(c->u_cnt, (size_t)ntiles * 4));
   TRY(dev_reserve(c->u_off, (size_t)ntiles * 4));
   TRY(dev_reserve(c->units, (size_t)c->units_bound * 8));
   TRY(dev_reserve(c->u_part, m2l_unit_part_bytes(c->units_bound, ntiles)));
+  TRY(launch_m2l_set_offsets(dp<uint32_t>(c->items), nitems, gbits, ntiles, dp<int32_t>(c->set_off),
+                             c->unit_chunk, dp<uint32_t>(c->u_cnt), s));
   TRY(dev_reserve(c->scan_tmp, scan_tmp_bytes(std::max<int64_t>(ntiles, std::max<int64_t>(nslots, n)))));
-  TRY(launch_m2l_units(dp<int32_t>(c->set_off), ntiles, c->unit_chunk, dp<uint32_t>(c->u_cnt),
-                       dp<uint32_t>(c->u_off), dp<int2>(c->units), c->scan_tmp.ptr, s));
+  TRY(launch_m2l_units(ntiles, dp<uint32_t>(c->u_cnt), dp<uint32_t>(c->u_off), dp<int2>(c->units),
+                       c->scan_tmp.ptr, s));
   // fallback pairs: per-target list sorted by (target, source)
-  bool falt = false;
-  TRY(radix_sort_pairs(dp<uint64_t>(c->fkeys), dp<uint32_t>(c->fvals), dp<uint64_t>(c->fkeys_alt),
-                       dp<uint32_t>(c->fvals_alt), nfb, 0, FB_SRC_BITS + sbits, c->sort_tmp.ptr, s,
-                       &falt));
-  const uint64_t *fk = dp<uint64_t>(falt ? c->fkeys_alt : c->fkeys);
-  TRY(dev_reserve(c->fb_off, (size_t)(c->ncells + 1) * 4));
-  TRY(dev_reserve(c->fb_src, (size_t)std::max<uint32_t>(nfb, 1) * 4));
-  TRY(launch_csr_offsets(fk, nfb, FB_SRC_BITS, (int32_t)c->ncells, dp<int32_t>(c->fb_off), s));
-  TRY(launch_unpack_pairs(fk, nfb, FB_SRC_BITS, dp<int32_t>(c->fb_src), s));
+  if (nfb) {
+    bool falt = false;
+    TRY(radix_sort_pairs(dp<uint64_t>(c->fkeys), dp<uint32_t>(c->fvals), dp<uint64_t>(c->fkeys_alt),
+                         dp<uint32_t>(c->fvals_alt), nfb, 0, FB_SRC_BITS + sbits, c->sort_tmp.ptr,
+                         s, &falt));
+    const uint64_t *fk = dp<uint64_t>(falt ? c->fkeys_alt : c->fkeys);
+    TRY(dev_reserve(c->fb_off, (size_t)(c->ncells + 1) * 4));
+    TRY(dev_reserve(c->fb_src, (size_t)nfb * 4));
+    TRY(launch_csr_offsets(fk, nfb, FB_SRC_BITS, (int32_t)c->ncells, dp<int32_t>(c->fb_off), s));
+    TRY(launch_unpack_pairs(fk, nfb, FB_SRC_BITS, dp<int32_t>(c->fb_src), s));
+  }
   if (!c->codes_ready) {
     TRY(dev_reserve(c->codes, m2l_codes_bytes()));
     hipError_t e = m2l_upload_codes(dp<uint32_t>(c->codes), s);
@@ -1066,8 +1072,8 @@ int traverse_given(tfmm_ctx *c, const int32_t *m2l, int64_t nm, const int32_t *p
     TRY(hipMemcpyAsync(c->m2l_pairs.ptr, me.data(), me.size() * 8, hipMemcpyHostToDevice, s));
   if (!pe.empty())
     TRY(hipMemcpyAsync(c->p2p_pairs.ptr, pe.data(), pe.size() * 8, hipMemcpyHostToDevice, s));
-  TRY(launch_dtt_cells(k, (int32_t)nc, c->prm.theta, dp<double4>(c->dtt_geo),
-                       dp<int2>(c->dtt_topo), s));
+  TRY(launch_dtt_begin(k, (int32_t)nc, c->prm.theta, dp<double4>(c->dtt_geo),
+                       dp<int2>(c->dtt_topo), nullptr, 0, nullptr, 0, nullptr, 0, s));
   TRY(launch_pair_slots(dp<int2>(c->m2l_pairs), (uint32_t)me.size(), dp<double4>(c->dtt_geo),
                         k.depth, k.width, dp<int32_t>(c->slot_of), dp<uint32_t>(c->g_used),
                         dp<uint32_t>(c->g_used) + nslots, s));
@@ -1095,6 +1101,7 @@ int do_downward(tfmm_ctx *c) {
   TRY(dev_reserve(c->trg, (size_t)c->n * 32));
   TRY(dev_reserve(c->out, (size_t)c->n * 32));
   TRY(dev_reserve(c->leaf_of, (size_t)c->n * 4));
+  TRY(launch_body_leaf(k, (int32_t)c->ncells, dp<int32_t>(c->leaf_of), s));
   TRY(launch_l2p(k, (int32_t)c->ncells, sorted_bodies(c), dp<double>(c->L), dp<double>(c->acc),
                  dp<int32_t>(c->perm), dp<int32_t>(c->leaf_of), dp<double>(c->trg),
                  dp<double>(c->out), s));
@@ -1210,6 +1217,8 @@ int upward_pass(tfmm_ctx *c, hipStream_t st) {
   }
   if (!cart_direct(c))
     TRY(launch_m2l_scale_m(k, (int32_t)c->ncells, dp<double>(c->M), c->mq.ptr, m2l_fp32(c), st));
+  if (!cartesian(c))  // for the L2P
+    TRY(launch_body_leaf(k, (int32_t)c->ncells, dp<int32_t>(c->leaf_of), st));
   TRY(rec(c, EV_UP, st));
   return TFMM_OK;
 }
@@ -1225,9 +1234,11 @@ int upward_pass(tfmm_ctx *c, hipStream_t st) {
 // graph of its own (TFMM_TUNE_GRAPH 1) keeps it too.
 bool early_upward(const tfmm_ctx *c) { return c->use_graph != 1 && c->p2p_schedule < 2; }
 
-int fork_upward(tfmm_ctx *c) {
-  TRY(hipEventRecord(c->ev[EV_P2PREADY], c->stream));
-  TRY(hipStreamWaitEvent(c->side, c->ev[EV_P2PREADY], 0));
+// The host enqueues it after the traversal's steps, while those run: the steps are
+// what the next read-back waits for.
+int run_pending_upward(tfmm_ctx *c) {
+  if (!c->upward_pending) return TFMM_OK;
+  c->upward_pending = false;
   const int rc = upward_pass(c, c->side);
   (void)hipEventRecord(c->ev[EV_UPJOIN], c->side);
   return rc;
@@ -1238,6 +1249,7 @@ int fused_lists(tfmm_ctx *c);
 int fused_prepare(tfmm_ctx *c) {
   hipStream_t s = c->stream;
   TRY(reserve_expansions(c));
+  TRY(dev_reserve(c->leaf_of, (size_t)c->n * 4));
   int rc = cartesian(c) ? cart_tables(c) : TFMM_OK;
   if (rc) return rc;
   if (!cart_direct(c)) {
@@ -1250,8 +1262,11 @@ int fused_prepare(tfmm_ctx *c) {
   }
   c->p2p_forked = false;
   if (!early_upward(c)) return fused_lists(c);
-  rc = fork_upward(c);
-  if (!rc) rc = fused_lists(c);
+  TRY(hipEventRecord(c->ev[EV_UPJOIN], s));  // the tree; again once the pass is enqueued
+  TRY(hipStreamWaitEvent(c->side, c->ev[EV_UPJOIN], 0));
+  c->upward_pending = true;
+  rc = fused_lists(c);
+  c->upward_pending = false;
   // what was started on the second stream ends before anything that follows
   if (rc) (void)hipStreamWaitEvent(s, c->ev[EV_UPJOIN], 0);
   return rc;
@@ -1292,7 +1307,6 @@ int fused_lists(tfmm_ctx *c) {
   }
   TRY(dev_reserve(c->trg, (size_t)c->n * 32));
   TRY(dev_reserve(c->out, (size_t)c->n * 32));
-  TRY(dev_reserve(c->leaf_of, (size_t)c->n * 4));
   if (c->n_fallback)
     TRY(dev_reserve(c->fb_part, m2l_pairs_scratch_bytes((int32_t)c->n_fallback)));
   TRY(hipEventRecord(c->ev[EV_DTT1], s));
@@ -1472,6 +1486,7 @@ void plan_make(tfmm_ctx *c) {
     pl.grid[d] = (int32_t)std::min<int64_t>(g, INT32_MAX / 16);
     pl.cells += pl.grid[d];
   }
+  pl.top = tree_top_levels(c->tree_hint.data(), L0);
   if (pl.cells > INT32_MAX / 4) return;
   pl.max_depth = pl.L - 1;
   pl.nsteps = 2 * pl.max_depth + 2;
@@ -1677,10 +1692,10 @@ int whole_record(tfmm_ctx *c) {
                      dp<int32_t>(c->perm), s));
   // cells, level by level, every size on the device
   int32_t *lev = dp<int32_t>(c->lev);
-  TRY(launch_fill_zero(c->lev.ptr, (size_t)2 * (pl.L + 1) * 4, s));
-  TRY(launch_fill_zero(c->lev_status.ptr, 4, s));
-  TRY(launch_roots(k, n, off, np, region, lev, s));
-  for (int d = 0; d < pl.L; d++)
+  TRY(launch_tree_top(k, n, off, np, lev, pl.L, pl.top, pl.prm.ncrit, cells,
+                      dp<uint32_t>(c->lev_status), skeys, region, sprob, s, true,
+                      pl.grid.data()));
+  for (int d = pl.top; d < pl.L; d++)
     TRY(launch_level_step(k, lev, d, pl.grid[d], pl.prm.ncrit, cells, dp<uint32_t>(c->flag),
                           dp<uint32_t>(c->slot), dp<uint32_t>(c->lev_bsum),
                           dp<uint32_t>(c->lev_status), skeys, region, sprob, s, d == pl.L - 1));
@@ -1695,6 +1710,7 @@ int whole_record(tfmm_ctx *c) {
       TRY(launch_m2m(k, 0, pl.grid[d + 1] / 8 + 1, dp<double>(c->tops), dp<double>(c->M), st, lev,
                      d + 1));
     TRY(launch_m2l_scale_m(k, cells, dp<double>(c->M), c->mq.ptr, mixed, st));
+    TRY(launch_body_leaf(k, cells, dp<int32_t>(c->leaf_of), st));
     TRY(rec(c, EV_UP, st));
     return TFMM_OK;
   };
@@ -1709,11 +1725,8 @@ int whole_record(tfmm_ctx *c) {
   // traversal
   uint32_t *cnt = dp<uint32_t>(c->cnt);
   uint32_t *used = dp<uint32_t>(c->g_used);
-  TRY(launch_dtt_cells(k, cells, pl.prm.theta, dp<double4>(c->dtt_geo), dp<int2>(c->dtt_topo),
-                       s));
-  TRY(launch_fill_zero(used, (size_t)(pl.nslots + 1) * 4, s));
-  TRY(launch_fill_zero(cnt, (size_t)pl.cwords * 4, s));
-  TRY(launch_root_pairs(dp<int2>(c->front_a), np, cnt + 16, s));
+  TRY(launch_dtt_begin(k, cells, pl.prm.theta, dp<double4>(c->dtt_geo), dp<int2>(c->dtt_topo),
+                       used, pl.nslots + 1, cnt, pl.cwords, dp<int2>(c->front_a), np, s));
   DevBuf *fa = &c->front_a, *fb = &c->front_b;
   for (int st = 0; st < pl.nsteps; st++) {
     TRY(launch_dtt_step(dp<int2>(*fa), cnt + 16 + st, pl.step_grid[st], dp<int2>(*fb),
@@ -1767,13 +1780,13 @@ int whole_record(tfmm_ctx *c) {
                                    dp<uint32_t>(c->it_start), c->scan_tmp.ptr, sz + SZ_NITEMS, s));
     TRY(launch_m2l_write_items(gk, gv, nm, dp<uint32_t>(c->it_start), cells, dp<uint32_t>(c->items),
                                dp<uint32_t>(c->cols), s, gcnt, pl.caps.items));
-    TRY(launch_m2l_set_offsets(dp<uint32_t>(c->items), pl.caps.items, pl.gbits, pl.ntiles,
-                               dp<int32_t>(c->set_off), s, sz + SZ_NITEMS));
     int32_t *chunk = reinterpret_cast<int32_t *>(sz + SZ_CHUNK);
     TRY(launch_m2l_unit_chunk(sz + SZ_NITEMS, sz + SZ_NTILES, c->m2l_unit_factor, chunk, s));
-    TRY(launch_m2l_units(dp<int32_t>(c->set_off), pl.ntiles, 0, dp<uint32_t>(c->u_cnt),
-                         dp<uint32_t>(c->u_off), dp<int2>(c->units), c->scan_tmp.ptr, s,
-                         pl.caps.units, chunk));
+    TRY(launch_m2l_set_offsets(dp<uint32_t>(c->items), pl.caps.items, pl.gbits, pl.ntiles,
+                               dp<int32_t>(c->set_off), 0, dp<uint32_t>(c->u_cnt), s,
+                               sz + SZ_NITEMS, chunk));
+    TRY(launch_m2l_units(pl.ntiles, dp<uint32_t>(c->u_cnt), dp<uint32_t>(c->u_off),
+                         dp<int2>(c->units), c->scan_tmp.ptr, s, pl.caps.units));
     // the pairs outside the groups (appended compactly): at most the
     // fallback capacity of them are sorted
     const uint32_t nfb = std::min<uint32_t>(nm, pl.caps.fallback);

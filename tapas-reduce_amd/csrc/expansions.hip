@@ -220,12 +220,17 @@ hipError_t launch_p2m(Cells c, int32_t ncells, Bodies b, double *M, hipStream_t 
   return hipGetLastError();
 }
 
-// leaf_of: scratch of b.n int32
+hipError_t launch_body_leaf(Cells c, int32_t ncells, int32_t *leaf_of, hipStream_t s) {
+  if (ncells <= 0) return hipSuccess;
+  k_body_leaf<<<(ncells + 3) / 4, 256, 0, s>>>(c, ncells, leaf_of);
+  return hipGetLastError();
+}
+
+// leaf_of: the leaf of every sorted body (launch_body_leaf)
 hipError_t launch_l2p(Cells c, int32_t ncells, Bodies b, const double *L, const double *p2p,
-                      const int32_t *perm, int32_t *leaf_of, double *trg, double *out,
+                      const int32_t *perm, const int32_t *leaf_of, double *trg, double *out,
                       hipStream_t s) {
   if (ncells <= 0 || b.n <= 0) return hipSuccess;
-  k_body_leaf<<<(ncells + 3) / 4, 256, 0, s>>>(c, ncells, leaf_of);
   k_l2p<<<(unsigned)((b.n + 255) / 256), 256, 0, s>>>(c, b, leaf_of, L, p2p, perm, trg, out);
   return hipGetLastError();
 }

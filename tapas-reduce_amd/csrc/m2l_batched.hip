@@ -158,33 +158,34 @@ __global__ void k_classify_all(const int2 *pairs, const int32_t *slot_of, uint32
 // 2^(p dl), dl = l_t - l_s, i.e. the harmonics of the offset measured in
 // target widths.  Stored as NR reals (re/im interleaved, index 2 tri(p, q)),
 // in FP64 and FP32.
+constexpr int HARM_BITS = 4;
 __global__ void k_group_harmonics(const uint32_t *used, const uint32_t *gid_of_slot, double *Y64,
                                   float *Y32, int8_t *gdl, uint32_t gcap) {
   critical_path_priority();
-  const int32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
-  if (slot >= m2lg::SLOTS || !used[slot]) return;
+  const int32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int32_t slot = t >> HARM_BITS;
+  const int m = t & ((1 << HARM_BITS) - 1);  // one column of one slot per thread
+  if (m >= P || slot >= m2lg::SLOTS || !used[slot]) return;
   const uint32_t g = gid_of_slot[slot];
   if (g >= gcap) return;  // more groups than the buffers hold (checked by the caller)
   int sl, o[3];  // source level less target level
   m2lg::slot_decode(slot, sl, o);
   const double half = ldexp(0.5, -max(sl, 0));  // half the finer width, target width = 1
   const double dx = o[0] * half, dy = o[1] * half, dz = o[2] * half;
-  double rho, alpha, beta;
-  cart2sph(dx, dy, dz, rho, alpha, beta);
-  const double x = cos(alpha), y = sin(alpha);
-  const cd ei = mk(cos(beta), sin(beta));
+  double rho, x, y;
+  cd ei;
+  sph_frame(dx, dy, dz, rho, x, y, ei);
   double *yo = Y64 + (int64_t)g * NR;
   float *yf = Y32 + (int64_t)g * NR;
-  for (int m = 0; m < P; m++) {
-    local_column(m, rho, x, y, ei, [&](int n, int mm, cd v) {
-      const double sc = ldexp(1.0, -n * sl);  // 2^(n dl)
-      const int t = tri(n, mm);
-      yo[2 * t] = v.re * sc;
-      yo[2 * t + 1] = v.im * sc;
-      yf[2 * t] = (float)(v.re * sc);
-      yf[2 * t + 1] = (float)(v.im * sc);
-    });
-  }
+  local_column(m, rho, x, y, ei, [&](int n, int mm, cd v) {
+    const double sc = ldexp(1.0, -n * sl);  // 2^(n dl)
+    const int t = tri(n, mm);
+    yo[2 * t] = v.re * sc;
+    yo[2 * t + 1] = v.im * sc;
+    yf[2 * t] = (float)(v.re * sc);
+    yf[2 * t + 1] = (float)(v.im * sc);
+  });
+  if (m > 0) return;
   yo[110] = yo[111] = 0;
   yf[110] = yf[111] = 0;
   gdl[g] = (int8_t)-sl;
@@ -350,20 +351,35 @@ __global__ __launch_bounds__(IT_THREADS) void k_items(const uint32_t *keys, cons
   }
 }
 
-// first item of every set
+// first item of every set, and the set's work units (of chunk items, *dchunk
+// with dchunk; at least one)
 __global__ void k_set_offsets(const uint32_t *ikey, uint32_t nitems, int gbits, int32_t nsets,
-                              int32_t *off, const uint32_t *dnitems) {
+                              int32_t *off, int32_t chunk, uint32_t *ucnt,
+                              const uint32_t *dnitems, const int32_t *dchunk) {
   critical_path_priority();
   const int32_t t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t > nsets) return;
   if (dnitems) nitems = min(nitems, *dnitems);
-  uint32_t lo = 0, hi = nitems;
-  while (lo < hi) {
-    const uint32_t mid = lo + ((hi - lo) >> 1);
-    if ((ikey[mid] >> gbits) < (uint32_t)t) lo = mid + 1;
-    else hi = mid;
+  if (dchunk) chunk = *dchunk;
+  // the first items of sets t and t + 1, their searches in step
+  uint32_t lo = 0, hi = nitems, lo1 = 0, hi1 = nitems;
+  while (lo < hi || lo1 < hi1) {
+    const uint32_t mid = lo + ((hi - lo) >> 1), mid1 = lo1 + ((hi1 - lo1) >> 1);
+    const uint32_t k = lo < hi ? ikey[mid] : 0u, k1 = lo1 < hi1 ? ikey[mid1] : 0u;
+    if (lo < hi) {
+      if ((k >> gbits) < (uint32_t)t) lo = mid + 1;
+      else hi = mid;
+    }
+    if (lo1 < hi1) {
+      if ((k1 >> gbits) <= (uint32_t)t) lo1 = mid1 + 1;
+      else hi1 = mid1;
+    }
   }
   off[t] = (int32_t)lo;
+  if (t < nsets) {
+    const int32_t n = (int32_t)(lo1 - lo);
+    ucnt[t] = n > chunk ? (uint32_t)((n + chunk - 1) / chunk) : 1u;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -618,23 +634,15 @@ __device__ inline int unit_of_block(int b, int nunits, int run) {
 // unit writes the set's L, the others leave theirs in part[] (one 16 x 110 slab
 // per extra unit, FP64), which k_unit_combine adds in unit order after the
 // launch, so the sums do not depend on timing.
-__global__ void k_unit_counts(const int32_t *tile_off, int32_t ntiles, int32_t chunk,
-                              uint32_t *ucnt, const int32_t *dchunk) {
-  critical_path_priority();
-  const int32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= ntiles) return;
-  if (dchunk) chunk = *dchunk;
-  const int32_t n = tile_off[t + 1] - tile_off[t];
-  ucnt[t] = n > chunk ? (uint32_t)((n + chunk - 1) / chunk) : 1u;
-}
-
+// (set, number) of every unit: 16 threads a set
 __global__ void k_unit_map(const uint32_t *ucnt, const uint32_t *uoff, int32_t ntiles,
                            int2 *units, uint32_t units_cap) {
   critical_path_priority();
-  const int32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int32_t t = (blockIdx.x * blockDim.x + threadIdx.x) >> 4;
   if (t >= ntiles) return;
-  for (uint32_t k = 0; k < ucnt[t] && uoff[t] + k < units_cap; k++)
-    units[uoff[t] + k] = make_int2(t, (int)k);
+  const uint32_t n = ucnt[t], o = uoff[t];
+  for (uint32_t k = threadIdx.x & 15; k < n && o + k < units_cap; k += 16)
+    units[o + k] = make_int2(t, (int)k);
 }
 
 // slab of extra unit k >= 1 of tile t: every tile has at least one unit
@@ -868,7 +876,7 @@ hipError_t launch_m2l_classify(const int2 *pairs, const int32_t *slot_of, uint32
 hipError_t launch_m2l_group_harmonics(const uint32_t *used, const uint32_t *gid_of_slot,
                                       double *Y64, float *Y32, int8_t *gdl, hipStream_t s,
                                       uint32_t gcap) {
-  k_group_harmonics<<<(m2lg::SLOTS + 63) / 64, 64, 0, s>>>(used, gid_of_slot, Y64, Y32, gdl, gcap);
+  k_group_harmonics<<<((m2lg::SLOTS << HARM_BITS) + 255) / 256, 256, 0, s>>>(used, gid_of_slot, Y64, Y32, gdl, gcap);
   return hipGetLastError();
 }
 
@@ -942,8 +950,10 @@ hipError_t launch_m2l_write_items(const uint32_t *keys, const uint32_t *vals, ui
 }
 
 hipError_t launch_m2l_set_offsets(const uint32_t *ikey, uint32_t nitems, int gbits, int32_t nsets,
-                                  int32_t *off, hipStream_t s, const uint32_t *dnitems) {
-  k_set_offsets<<<(nsets + 1 + 255) / 256, 256, 0, s>>>(ikey, nitems, gbits, nsets, off, dnitems);
+                                  int32_t *off, int32_t chunk, uint32_t *ucnt, hipStream_t s,
+                                  const uint32_t *dnitems, const int32_t *dchunk) {
+  k_set_offsets<<<(nsets + 1 + 255) / 256, 256, 0, s>>>(ikey, nitems, gbits, nsets, off, chunk,
+                                                        ucnt, dnitems, dchunk);
   return hipGetLastError();
 }
 
@@ -996,14 +1006,12 @@ size_t m2l_unit_part_bytes(uint32_t units_bound, int32_t ntiles) {
   return std::max<size_t>(extra, 1) * TILE * 110 * 8;
 }
 
-hipError_t launch_m2l_units(const int32_t *tile_off, int32_t ntiles, int32_t chunk,
-                            uint32_t *ucnt, uint32_t *uoff, int2 *units, void *scan_tmp,
-                            hipStream_t s, uint32_t units_cap, const int32_t *dchunk) {
+hipError_t launch_m2l_units(int32_t ntiles, const uint32_t *ucnt, uint32_t *uoff, int2 *units,
+                            void *scan_tmp, hipStream_t s, uint32_t units_cap) {
   if (ntiles <= 0) return hipSuccess;
-  k_unit_counts<<<(ntiles + 255) / 256, 256, 0, s>>>(tile_off, ntiles, chunk, ucnt, dchunk);
   hipError_t e = scan_exclusive_u32(ucnt, uoff, ntiles, scan_tmp, s);
   if (e != hipSuccess) return e;
-  k_unit_map<<<(ntiles + 255) / 256, 256, 0, s>>>(ucnt, uoff, ntiles, units, units_cap);
+  k_unit_map<<<(ntiles + 15) / 16, 256, 0, s>>>(ucnt, uoff, ntiles, units, units_cap);
   return hipGetLastError();
 }
 

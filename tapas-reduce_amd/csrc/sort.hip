@@ -95,6 +95,33 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_down(const uint32_t *in, 
   }
 }
 
+// A scan of up to SCAN_ONE values in one launch of one workgroup (three launches
+// with tiles of 2,048).
+constexpr int SCAN_ONE_THREADS = 1024;
+constexpr int SCAN_ONE_ITEMS = 16;
+constexpr int SCAN_ONE = SCAN_ONE_THREADS * SCAN_ONE_ITEMS;
+
+__global__ __launch_bounds__(SCAN_ONE_THREADS) void k_scan_one(const uint32_t *in, int n,
+                                                               uint32_t *out) {
+  __builtin_amdgcn_s_setprio(2);  // as the kernels beside the early P2P (critical_path_priority)
+  __shared__ uint32_t part[SCAN_ONE + SCAN_ONE / 32];  // a pad word per 32: a thread's 16 in a row
+  auto at = [](int i) { return i + (i >> 5); };
+  for (int i = threadIdx.x; i < n; i += SCAN_ONE_THREADS) part[at(i)] = in[i];
+  __syncthreads();
+  const int base = threadIdx.x * SCAN_ONE_ITEMS;
+  uint32_t s = 0;
+  for (int i = base; i < min(n, base + SCAN_ONE_ITEMS); i++) s += part[at(i)];
+  uint32_t tot;
+  uint32_t run = block_excl_scan<SCAN_ONE_THREADS>(s, &tot);
+  for (int i = base; i < min(n, base + SCAN_ONE_ITEMS); i++) {
+    const uint32_t v = part[at(i)];
+    part[at(i)] = run;
+    run += v;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += SCAN_ONE_THREADS) out[i] = part[at(i)];
+}
+
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // ---------------------------------------------------------------------------
@@ -339,6 +366,10 @@ hipError_t scan_exclusive_u32(const uint32_t *in, uint32_t *out, int64_t n, void
   const int64_t nb = ceil_div(n, SCAN_TILE);
   if (nb == 1) {
     k_scan_down<<<1, SCAN_THREADS, 0, s>>>(in, n, nullptr, out);
+    return hipGetLastError();
+  }
+  if (n <= SCAN_ONE) {
+    k_scan_one<<<1, SCAN_ONE_THREADS, 0, s>>>(in, (int)n, out);
     return hipGetLastError();
   }
   uint32_t *sums = reinterpret_cast<uint32_t *>(tmp);

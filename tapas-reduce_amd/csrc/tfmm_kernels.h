@@ -80,12 +80,10 @@ hipError_t launch_problem_gather(const uint32_t *pos, const uint64_t *keys1,
                                  uint32_t *order, hipStream_t s);
 // the first traversal frontier: each root with itself, or (periodic) the one
 // root with its 27 images
-hipError_t launch_root_pairs(int2 *front, int nroots, uint32_t *count, hipStream_t s,
-                             bool periodic = false);
 hipError_t launch_permute(const uint32_t *order, const double4 *rec, int64_t n, double *sx,
                           double *sy, double *sz, double *sq, int32_t *perm, hipStream_t s);
 hipError_t launch_roots(Cells c, int64_t n, const int64_t *off, int nprob,
-                        const double *regions, int32_t *lev, hipStream_t s);
+                        const double *regions, hipStream_t s);
 // one level of the cell build with sizes on the device (lev: first cell and
 // count per level); grid_cells bounds the level's size; status bit 1: cell
 // capacity cap exceeded, bit 2: level larger than grid_cells
@@ -94,6 +92,11 @@ int32_t level_blocks(int32_t cells);
 // side cycle around the bodies' bounding cube; *flag = 1 if they span more
 hipError_t launch_periodic_region(double *region, double cycle, uint32_t *flag, hipStream_t s);
 // last: the planned tree has no level after d (splits there set ST_DEPTH)
+hipError_t launch_tree_top(Cells c, int64_t n, const int64_t *off, int nprob, int32_t *lev, int L,
+                           int levels, int ncrit, int32_t cap, uint32_t *status,
+                           const uint64_t *keys, const double *regions, const uint32_t *sprob,
+                           hipStream_t s, bool last = false, const int32_t *most = nullptr);
+int tree_top_levels(const int32_t *sizes, int L);
 hipError_t launch_level_step(Cells c, int32_t *lev, int d, int32_t grid_cells, int ncrit,
                              int32_t cap, uint32_t *flag, uint32_t *loc, uint32_t *bsum,
                              uint32_t *status, const uint64_t *keys, const double *regions,
@@ -130,8 +133,9 @@ hipError_t launch_m2m(Cells c, int32_t first_child, int32_t npar, const double *
                       hipStream_t s, const int32_t *lev = nullptr, int dl = 0);
 hipError_t launch_l2l(Cells c, int32_t first_child, int32_t npar, const double *ops, double *L,
                       hipStream_t s, const int32_t *lev = nullptr, int dl = 0);
+hipError_t launch_body_leaf(Cells c, int32_t ncells, int32_t *leaf_of, hipStream_t s);
 hipError_t launch_l2p(Cells c, int32_t ncells, Bodies b, const double *L, const double *p2p,
-                      const int32_t *perm, int32_t *leaf_of, double *trg, double *out,
+                      const int32_t *perm, const int32_t *leaf_of, double *trg, double *out,
                       hipStream_t s);
 
 // cartesian.hip: the Cartesian Taylor basis, CART_TERMS doubles per
@@ -167,8 +171,10 @@ struct DttCounters {
   uint32_t *cnt;
 };
 // per-cell records the traversal steps read (geo: centre + MAC radius)
-hipError_t launch_dtt_cells(Cells c, int32_t ncells, double theta, double4 *geo, int2 *topo,
-                            hipStream_t s);
+// (per-cell records, the counters and flags cleared, the first frontier)
+hipError_t launch_dtt_begin(Cells c, int32_t ncells, double theta, double4 *geo, int2 *topo,
+                            uint32_t *used, int32_t nused, uint32_t *cnt, int32_t cwords,
+                            int2 *front, int nroots, hipStream_t s, bool periodic = false);
 // One breadth-first traversal step.  Every M2L pair stored also gets its
 // group-table slot (m2l_slot, -1 outside the table), marks used[slot] and
 // counts the pairs outside the table in *n_outside.
@@ -272,8 +278,9 @@ hipError_t launch_m2l_write_items(const uint32_t *keys, const uint32_t *vals, ui
                                   uint32_t *cols, hipStream_t s, const uint32_t *dn = nullptr,
                                   uint32_t items_cap = UINT32_MAX);
 hipError_t launch_m2l_set_offsets(const uint32_t *ikey, uint32_t nitems, int gbits, int32_t nsets,
-                                  int32_t *off, hipStream_t s,
-                                  const uint32_t *dnitems = nullptr);
+                                  int32_t *off, int32_t chunk, uint32_t *ucnt, hipStream_t s,
+                                  const uint32_t *dnitems = nullptr,
+                                  const int32_t *dchunk = nullptr);
 // m2l_unit_chunk of the device's item and tile counts, into *chunk
 hipError_t launch_m2l_unit_chunk(const uint32_t *nitems, const uint32_t *ntiles, double factor,
                                  int32_t *chunk, hipStream_t s);
@@ -282,12 +289,9 @@ int32_t m2l_unit_chunk(uint32_t nitems, int32_t ntiles, double factor);
 uint32_t m2l_units_bound(uint32_t nitems, int32_t ntiles, int32_t chunk);
 uint32_t m2l_units_cap(uint32_t nitems, int32_t nsets, double factor);
 size_t m2l_unit_part_bytes(uint32_t units_bound, int32_t ntiles);
-// units at or past units_cap are not written; with dchunk the chunk is read
-// on the device
-hipError_t launch_m2l_units(const int32_t *tile_off, int32_t ntiles, int32_t chunk,
-                            uint32_t *ucnt, uint32_t *uoff, int2 *units, void *scan_tmp,
-                            hipStream_t s, uint32_t units_cap = UINT32_MAX,
-                            const int32_t *dchunk = nullptr);
+// (set, number) of every unit; units at or past units_cap are not written
+hipError_t launch_m2l_units(int32_t ntiles, const uint32_t *ucnt, uint32_t *uoff, int2 *units,
+                            void *scan_tmp, hipStream_t s, uint32_t units_cap = UINT32_MAX);
 // A fragments of every group (the set kernel's operand order, row factors
 // 2^(-j dl) included) from the group harmonics (FP32 or FP64), the operand
 // codes of both types and the groups' level differences

@@ -33,6 +33,8 @@
 // and one 8-byte record (first child, body count), built once per traversal,
 // instead of six separate arrays: the traversal gathers cells at random, so
 // the number of cache lines a pair touches sets its cost.
+#include <algorithm>
+
 #include "m2l_groups.h"
 #include "tfmm_device.h"
 #include "tfmm_kernels.h"
@@ -44,11 +46,23 @@ constexpr int DTT_THREADS = 1024;
 constexpr int DTT_WAVES = DTT_THREADS / 64;
 constexpr uint32_t DTT_ONE = 1 << 19;  // frontiers up to this take one pair per thread
 
-// per-cell traversal records: (centre, R) with R = (width / 2 * 1.00001) / theta
-// (tapas_exafmm.cxx:222-226), and (first child, body count)
-__global__ void k_dtt_cells(Cells c, int32_t ncells, double theta, double4 *geo, int2 *topo) {
+// The traversal's start: per-cell records (centre, R) with R = (width / 2 *
+// 1.00001) / theta (tapas_exafmm.cxx:222-226) and (first child, body count); with
+// cnt also the cleared group flags (nused words) and counters (cwords words), and
+// the first frontier, its size in cnt[16]: every root with itself, or with periodic
+// images the one root with each of its 27 images (EX/include/traversal.h:256-266).
+__global__ void k_dtt_begin(Cells c, int32_t ncells, double theta, double4 *geo, int2 *topo,
+                            uint32_t *used, int32_t nused, uint32_t *cnt, int32_t cwords,
+                            int2 *front, int nroots, int periodic) {
 #pragma clang fp contract(off)
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (cnt) {
+    const int nf = periodic ? 27 : nroots;
+    if (i < nused) used[i] = 0;
+    if (i < cwords) cnt[i] = i == 16 ? (uint32_t)nf : 0u;
+    if (i < nf)
+      front[i] = periodic ? make_int2(0, (int32_t)((uint32_t)i << IMG_SHIFT)) : make_int2(i, i);
+  }
   if (i >= ncells) return;
   double R = c.width[i];
   R = (R / 2 * 1.00001) / theta;
@@ -458,10 +472,13 @@ hipError_t launch_csr_sorted_sources(const uint32_t *tgt, const uint32_t *in, ui
   return hipGetLastError();
 }
 
-hipError_t launch_dtt_cells(Cells c, int32_t ncells, double theta, double4 *geo, int2 *topo,
-                            hipStream_t s) {
-  if (ncells <= 0) return hipSuccess;
-  k_dtt_cells<<<(ncells + 255) / 256, 256, 0, s>>>(c, ncells, theta, geo, topo);
+hipError_t launch_dtt_begin(Cells c, int32_t ncells, double theta, double4 *geo, int2 *topo,
+                            uint32_t *used, int32_t nused, uint32_t *cnt, int32_t cwords,
+                            int2 *front, int nroots, hipStream_t s, bool periodic) {
+  const int32_t most = std::max(std::max(ncells, nroots), std::max(nused, std::max(cwords, 27)));
+  if (most <= 0) return hipSuccess;
+  k_dtt_begin<<<(most + 255) / 256, 256, 0, s>>>(c, ncells, theta, geo, topo, used, nused, cnt,
+                                                 cwords, front, nroots, periodic ? 1 : 0);
   return hipGetLastError();
 }
 

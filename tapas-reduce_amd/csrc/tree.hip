@@ -194,15 +194,9 @@ __global__ void k_permute(const uint32_t *order, const double4 *rec, int64_t n, 
   perm[i] = (int32_t)o;
 }
 
-// Root cells: one per problem (off == nullptr: the single root 0 of n bodies).
-__global__ void k_roots(Cells c, int64_t n, const int64_t *off, int nprob,
-                        const double *regions, int32_t *lev) {
-  const int pb = blockIdx.x * blockDim.x + threadIdx.x;
-  if (pb == 0 && lev) {
-    lev[0] = 0;
-    lev[1] = nprob;
-  }
-  if (pb >= nprob) return;
+// Root cell of problem pb (off == nullptr: the single root 0 of n bodies).
+__device__ inline void make_root(const Cells &c, int pb, int64_t n, const int64_t *off,
+                                 const double *regions) {
   const int64_t b = off ? off[pb] : 0, e = off ? off[pb + 1] : n;
   c.key[pb] = 0;
   c.beg[pb] = (int32_t)b;
@@ -220,15 +214,10 @@ __global__ void k_roots(Cells c, int64_t n, const int64_t *off, int nprob,
   c.width[pb] = w;
 }
 
-// Traversal start: the pair (root, root) of every problem.
-// The traversal's first frontier: every root with itself, or with periodic
-// images the one root with each of its 27 images (EX/include/traversal.h:
-// 256-266).
-__global__ void k_root_pairs(int2 *front, int nroots, uint32_t *count, int periodic) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int n = periodic ? 27 : nroots;
-  if (i < n) front[i] = periodic ? make_int2(0, (int32_t)((uint32_t)i << IMG_SHIFT)) : make_int2(i, i);
-  if (i == 0) *count = (uint32_t)n;
+__global__ void k_roots(Cells c, int64_t n, const int64_t *off, int nprob,
+                        const double *regions) {
+  const int pb = blockIdx.x * blockDim.x + threadIdx.x;
+  if (pb < nprob) make_root(c, pb, n, off, regions);
 }
 
 __global__ void k_split_flags(Cells c, int32_t lbeg, int32_t lcnt, int ncrit, uint32_t *flag) {
@@ -392,6 +381,74 @@ __global__ void k_level_children(Cells c, const int32_t *lev, int d, const uint3
   make_child(c, lbeg + i, ch, next_beg + 8 * (int32_t)slot, keys, regions, sprob);
 }
 
+// The roots and the first `levels` level steps in one workgroup: levels of a few
+// hundred cells are three launches of a few microseconds each otherwise, most of it
+// the gaps between them.  lev and *status are initialised here.  A level may hold
+// any number of cells (each takes its turn); status as k_level_scan, bit 2 for a
+// level larger than most.cells (what later launches over that level cover).
+// With the other launches taken out beside it, a 4,096-body cube 650 to 565 us an
+// evaluation, a 64K ellipsoid 1,760 to 1,680.
+constexpr int TOP_THREADS = 1024;
+
+struct LevelSizes {
+  int32_t cells[MAXDEPTH + 2];
+};
+
+__global__ __launch_bounds__(TOP_THREADS) void k_tree_top(Cells c, int64_t n, const int64_t *off,
+                                                          int nprob, int32_t *lev, int L,
+                                                          int levels, int ncrit, int32_t cap,
+                                                          uint32_t *status, const uint64_t *keys,
+                                                          const double *regions,
+                                                          const uint32_t *sprob, int last,
+                                                          LevelSizes most) {
+  __shared__ int32_t parent[TOP_THREADS];  // the split cells of a turn
+  __shared__ uint32_t wsum[TOP_THREADS / 64];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  for (int i = threadIdx.x; i < 2 * (L + 1); i += TOP_THREADS)
+    lev[i] = i == 1 ? nprob : 0;
+  for (int pb = threadIdx.x; pb < nprob; pb += TOP_THREADS) make_root(c, pb, n, off, regions);
+  int32_t lbeg = 0, lcnt = nprob;
+  uint32_t st = 0;
+  for (int d = 0; d < levels; d++) {
+    if (lcnt > most.cells[d]) st |= 2u;
+    const int32_t next_beg = lbeg + lcnt;
+    int64_t total = 0;  // split cells so far
+    for (int32_t base = 0; base < lcnt; base += TOP_THREADS) {
+      __syncthreads();  // the cells of this level are written; the last turn is over
+      const int32_t i = base + threadIdx.x, ci = lbeg + i;
+      bool split = false;
+      if (i < lcnt) {
+        split = c.nb[ci] > ncrit && c.depth[ci] < MAXDEPTH;
+        if (!split) c.child[ci] = -1;
+      }
+      const uint64_t m = __ballot(split);
+      if (lane == 0) wsum[wid] = (uint32_t)__popcll(m);
+      __syncthreads();
+      uint32_t pre = 0, tot = 0;
+      for (int w = 0; w < TOP_THREADS / 64; w++) {
+        pre += w < wid ? wsum[w] : 0u;
+        tot += wsum[w];
+      }
+      if (split) parent[pre + (uint32_t)__popcll(m & (lane == 0 ? 0ull : ~0ull >> (64 - lane)))] = ci;
+      __syncthreads();
+      if (next_beg + 8 * (total + tot) > cap) st |= 1u;
+      if (!st)
+        for (uint32_t t = threadIdx.x; t < tot * 8; t += TOP_THREADS)
+          make_child(c, parent[t >> 3], (int)(t & 7),
+                     next_beg + 8 * (int32_t)(total + (t >> 3)), keys, regions, sprob);
+      total += tot;
+    }
+    if (last && d == L - 1 && total > 0) st |= 4u;
+    lbeg = next_beg;
+    lcnt = st ? 0 : (int32_t)(8 * total);
+    if (threadIdx.x == 0) {
+      lev[2 * (d + 1)] = lbeg;
+      lev[2 * (d + 1) + 1] = lcnt;
+    }
+  }
+  if (threadIdx.x == 0) *status = st;
+}
+
 // flag = 1 when a coordinate or charge of the n bodies is not finite (the
 // host path rejects such bodies while unpacking them; device arrays are
 // checked here)
@@ -473,13 +530,6 @@ hipError_t launch_problem_gather(const uint32_t *pos, const uint64_t *keys1,
   return hipGetLastError();
 }
 
-hipError_t launch_root_pairs(int2 *front, int nroots, uint32_t *count, hipStream_t s,
-                             bool periodic) {
-  const int n = periodic ? 27 : nroots;
-  k_root_pairs<<<(n + 255) / 256, 256, 0, s>>>(front, nroots, count, periodic ? 1 : 0);
-  return hipGetLastError();
-}
-
 hipError_t launch_permute(const uint32_t *order, const double4 *rec, int64_t n, double *sx,
                           double *sy, double *sz, double *sq, int32_t *perm, hipStream_t s) {
   if (n <= 0) return hipSuccess;
@@ -488,8 +538,29 @@ hipError_t launch_permute(const uint32_t *order, const double4 *rec, int64_t n, 
 }
 
 hipError_t launch_roots(Cells c, int64_t n, const int64_t *off, int nprob,
-                        const double *regions, int32_t *lev, hipStream_t s) {
-  k_roots<<<(nprob + 255) / 256, 256, 0, s>>>(c, n, off, nprob, regions, lev);
+                        const double *regions, hipStream_t s) {
+  k_roots<<<(nprob + 255) / 256, 256, 0, s>>>(c, n, off, nprob, regions);
+  return hipGetLastError();
+}
+
+// the leading levels that launch_tree_top takes, from the L level sizes of an earlier
+// tree: those whose cells and children are one turn of its workgroup (a child costs a
+// chain of keys read at random, which more workgroups hide better)
+int tree_top_levels(const int32_t *sizes, int L) {
+  auto one_turn = [&](int d) { return d >= L || sizes[d] <= TOP_THREADS; };
+  int t = 0;
+  while (t < L && t < MAXDEPTH + 2 && one_turn(t) && one_turn(t + 1)) t++;
+  return t;
+}
+
+hipError_t launch_tree_top(Cells c, int64_t n, const int64_t *off, int nprob, int32_t *lev, int L,
+                           int levels, int ncrit, int32_t cap, uint32_t *status,
+                           const uint64_t *keys, const double *regions, const uint32_t *sprob,
+                           hipStream_t s, bool last, const int32_t *most) {
+  LevelSizes m;
+  for (int d = 0; d < MAXDEPTH + 2; d++) m.cells[d] = most && d < levels ? most[d] : INT32_MAX;
+  k_tree_top<<<1, TOP_THREADS, 0, s>>>(c, n, off, nprob, lev, L, levels, ncrit, cap, status, keys,
+                                       regions, sprob, last ? 1 : 0, m);
   return hipGetLastError();
 }
 
