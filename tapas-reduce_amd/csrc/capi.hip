@@ -60,6 +60,7 @@ struct Plan {
   int L = 0;                        // tree levels
   std::vector<int32_t> grid;        // cells per level
   int top = 0;                      // leading levels built by one workgroup
+  int key_bits = 0;                 // leading key bits of the bodies' sort
   int64_t cells = 0;                // cells in all
   int max_depth = 0, nsteps = 0, cwords = 0;
   int32_t nslots = 0, ntiles = 0;
@@ -101,6 +102,7 @@ struct tfmm_ctx {
   DevBuf flag, slot, scan_tmp, lev, lev_bsum, lev_status;
   std::vector<int32_t> lvl;
   std::vector<int32_t> tree_hint;  // cells per level of the last tree
+  int sort_extra = 0;              // levels more to sort the bodies by (do_build_tree)
   int64_t ncells = 0, nleaves = 0;
   bool keys_in_alt = false;
   double h_region[6] = {0, 0, 0, 0, 0, 0};
@@ -364,7 +366,8 @@ int check_params(tfmm_ctx *c, const tfmm_params *p) {
 // last tree's levels (with headroom), one host round trip at the end.
 // Returns 0 when the tree is complete, 1 when it must be built the
 // synchronous way (a level outgrew its grid, the cell capacity or the
-// hinted depth), or an error.
+// hinted depth), 2 when the bodies have to be sorted again by their whole keys,
+// or an error.
 int build_levels_hinted(tfmm_ctx *c, int64_t n, const int64_t *off, int np,
                         const uint64_t *skeys, const uint32_t *sprob) {
   hipStream_t s = c->stream;
@@ -383,7 +386,6 @@ int build_levels_hinted(tfmm_ctx *c, int64_t n, const int64_t *off, int np,
   TRY(reserve_cells(c, (size_t)total + 4096, 0, s));
   const int32_t cap = (int32_t)std::min<size_t>(c->cell_cap, INT32_MAX / 2);
   TRY(dev_reserve(c->lev, (size_t)2 * (L + 1) * 4));
-  TRY(dev_reserve(c->lev_status, 4));
   TRY(dev_reserve(c->flag, (size_t)gmax * 4 + 1024));
   TRY(dev_reserve(c->slot, (size_t)gmax * 4 + 1024));
   TRY(dev_reserve(c->lev_bsum, (size_t)level_blocks((int32_t)gmax) * 4 + 4));
@@ -391,7 +393,7 @@ int build_levels_hinted(tfmm_ctx *c, int64_t n, const int64_t *off, int np,
   int32_t *lev = dp<int32_t>(c->lev);
   const int top = tree_top_levels(c->tree_hint.data(), L);
   TRY(launch_tree_top(k, n, off, np, lev, L, top, c->prm.ncrit, cap, dp<uint32_t>(c->lev_status),
-                      skeys, dp<double>(c->region), sprob, s));
+                      skeys, dp<double>(c->region), sprob, dp<uint32_t>(c->lev_status) + 1, s));
   for (int d = top; d < L; d++)
     TRY(launch_level_step(k, lev, d, grid[d], c->prm.ncrit, cap, dp<uint32_t>(c->flag),
                           dp<uint32_t>(c->slot), dp<uint32_t>(c->lev_bsum),
@@ -400,6 +402,7 @@ int build_levels_hinted(tfmm_ctx *c, int64_t n, const int64_t *off, int np,
   TRY(hipMemcpyAsync(c->h_u32 + 2 * (L + 1), c->lev_status.ptr, 4, hipMemcpyDeviceToHost, s));
   TRY(hipStreamSynchronize(s));
   const int32_t *hl = reinterpret_cast<const int32_t *>(c->h_u32);
+  if (c->h_u32[2 * (L + 1)] & ST_SORT) return 2;
   if (c->h_u32[2 * (L + 1)] != 0 || hl[2 * L + 1] != 0) return 1;
   c->lvl.assign(1, 0);
   int64_t nleaves = 0;
@@ -414,9 +417,35 @@ int build_levels_hinted(tfmm_ctx *c, int64_t n, const int64_t *off, int np,
   return 0;
 }
 
-int do_build_tree(tfmm_ctx *c) {
+// The bodies, sorted by the key bits above shift in the buffers that alt names, in
+// the order of their whole keys in the others.
+hipError_t sort_runs(tfmm_ctx *c, bool alt, const uint32_t *sprob, int shift, uint32_t *long_run) {
+  return launch_sort_runs(dp<uint64_t>(alt ? c->keys_alt : c->keys),
+                          dp<uint32_t>(alt ? c->idx_alt : c->idx), sprob, c->n, shift,
+                          dp<uint64_t>(alt ? c->keys : c->keys_alt),
+                          dp<uint32_t>(alt ? c->idx : c->idx_alt), long_run, c->stream);
+}
+
+// Leading key bits to sort the bodies by before the runs that agree on them
+// (launch_sort_runs), 63 for all of them.  At the depth of the last tree a cell
+// holds at most ncrit bodies; bodies spread evenly agree in a few at n's bits.
+// Whole passes of 9 bits; with six or more the runs would save nothing.
+int key_prefix_bits(const tfmm_ctx *c) {
+  if (c->tree_hint.empty()) return 3 * MAXDEPTH;
+  int levels = (int)c->tree_hint.size() - 1 + c->sort_extra;
+  for (int64_t m = c->prm.ncrit; m > 128; m /= 4) levels++;
+  const int bits = std::max({3 * levels, bits_for(c->n) - 4, 1});
+  const int passes = (bits + 8) / 9;
+  return passes >= 6 ? 3 * MAXDEPTH : 9 * passes;
+}
+
+int do_build_tree(tfmm_ctx *c, bool whole_keys = false) {
   hipStream_t s = c->stream;
   const int64_t n = c->n;
+  TRY(dev_reserve(c->lev_status, 8));
+  uint32_t *long_run = dp<uint32_t>(c->lev_status) + 1;
+  const int prefix = whole_keys ? 3 * MAXDEPTH : key_prefix_bits(c);
+  const int key_end = DEPTHBITS + 3 * MAXDEPTH;
   TRY(dev_reserve(c->keys, n * 8));
   TRY(dev_reserve(c->keys_alt, n * 8));
   TRY(dev_reserve(c->idx, n * 4));
@@ -448,11 +477,11 @@ int do_build_tree(tfmm_ctx *c) {
   TRY(dev_reserve(c->brec, n * 32));
   TRY(launch_keys(c->bx, c->by, c->bz, c->bq, n, dp<double>(c->region), off, np,
                   dp<uint64_t>(c->keys), dp<uint32_t>(c->idx),
-                  forest ? dp<uint32_t>(c->bprob) : nullptr, dp<double4>(c->brec), s));
+                  forest ? dp<uint32_t>(c->bprob) : nullptr, dp<double4>(c->brec), long_run, s));
   bool alt = false;
   TRY(radix_sort_pairs(dp<uint64_t>(c->keys), dp<uint32_t>(c->idx), dp<uint64_t>(c->keys_alt),
-                       dp<uint32_t>(c->idx_alt), n, DEPTHBITS, DEPTHBITS + 3 * MAXDEPTH,
-                       c->sort_tmp.ptr, s, &alt));
+                       dp<uint32_t>(c->idx_alt), n, key_end - prefix, key_end, c->sort_tmp.ptr, s,
+                       &alt));
   const uint32_t *sprob = nullptr;
   if (forest) {
     // (problem, key) order: a stable sort by problem of the key-sorted bodies
@@ -474,6 +503,10 @@ int do_build_tree(tfmm_ctx *c) {
                               dp<uint32_t>(alt ? c->idx : c->idx_alt), s));
     alt = !alt;
   }
+  if (prefix < 3 * MAXDEPTH) {
+    TRY(sort_runs(c, alt, sprob, key_end - prefix, long_run));
+    alt = !alt;
+  }
   c->keys_in_alt = alt;
   const uint64_t *skeys = dp<uint64_t>(alt ? c->keys_alt : c->keys);
   const uint32_t *order = dp<uint32_t>(alt ? c->idx_alt : c->idx);
@@ -485,6 +518,10 @@ int do_build_tree(tfmm_ctx *c) {
   if (!c->tree_hint.empty()) {
     int rc = build_levels_hinted(c, n, off, np, skeys, sprob);
     if (rc < 0) return rc;
+    if (rc == 2) {  // these bodies are closer together than the last ones
+      c->sort_extra += 2;
+      return do_build_tree(c, true);
+    }
     if (rc == 0) {
       TRY(hipMemcpyAsync(c->h_region, c->region.ptr, 48, hipMemcpyDeviceToHost, s));
       return TFMM_OK;
@@ -1487,6 +1524,7 @@ void plan_make(tfmm_ctx *c) {
     pl.cells += pl.grid[d];
   }
   pl.top = tree_top_levels(c->tree_hint.data(), L0);
+  pl.key_bits = key_prefix_bits(c);
   if (pl.cells > INT32_MAX / 4) return;
   pl.max_depth = pl.L - 1;
   pl.nsteps = 2 * pl.max_depth + 2;
@@ -1555,7 +1593,7 @@ int plan_reserve(tfmm_ctx *c) {
   int32_t gmax = 0;
   for (int32_t g : pl.grid) gmax = std::max(gmax, g);
   TRY(dev_reserve(c->lev, (size_t)2 * (pl.L + 1) * 4));
-  TRY(dev_reserve(c->lev_status, 4));
+  TRY(dev_reserve(c->lev_status, 8));
   TRY(dev_reserve(c->flag, (size_t)gmax * 4 + 1024));
   TRY(dev_reserve(c->slot, (size_t)gmax * 4 + 1024));
   TRY(dev_reserve(c->lev_bsum, (size_t)level_blocks(gmax) * 4 + 4));
@@ -1655,6 +1693,8 @@ int whole_record(tfmm_ctx *c) {
   TRY(launch_fill_zero(c->gsz.ptr, SZ_WORDS * 4, s));
   // bodies to sorted keys
   double *region = dp<double>(c->region);
+  uint32_t *long_run = dp<uint32_t>(c->lev_status) + 1;
+  const int key_end = DEPTHBITS + 3 * MAXDEPTH;
   const int64_t *off = forest ? dp<int64_t>(c->d_prob_off) : nullptr;
   if (forest) {
     TRY(launch_bbox_forest(c->bx, c->by, c->bz, off, np, region, s));
@@ -1664,10 +1704,10 @@ int whole_record(tfmm_ctx *c) {
   }
   TRY(launch_keys(c->bx, c->by, c->bz, c->bq, n, region, off, np, dp<uint64_t>(c->keys),
                   dp<uint32_t>(c->idx), forest ? dp<uint32_t>(c->bprob) : nullptr,
-                  dp<double4>(c->brec), s));
+                  dp<double4>(c->brec), long_run, s));
   bool alt = false;
   TRY(radix_sort_pairs(dp<uint64_t>(c->keys), dp<uint32_t>(c->idx), dp<uint64_t>(c->keys_alt),
-                       dp<uint32_t>(c->idx_alt), n, DEPTHBITS, DEPTHBITS + 3 * MAXDEPTH,
+                       dp<uint32_t>(c->idx_alt), n, key_end - pl.key_bits, key_end,
                        c->sort_tmp.ptr, s, &alt));
   const uint32_t *sprob = nullptr;
   if (forest) {
@@ -1685,6 +1725,10 @@ int whole_record(tfmm_ctx *c) {
                               dp<uint32_t>(alt ? c->idx : c->idx_alt), s));
     alt = !alt;
   }
+  if (pl.key_bits < 3 * MAXDEPTH) {
+    TRY(sort_runs(c, alt, sprob, key_end - pl.key_bits, long_run));
+    alt = !alt;
+  }
   pl.keys_alt = alt;
   const uint64_t *skeys = dp<uint64_t>(alt ? c->keys_alt : c->keys);
   TRY(launch_permute(dp<uint32_t>(alt ? c->idx_alt : c->idx), dp<double4>(c->brec), n,
@@ -1693,7 +1737,7 @@ int whole_record(tfmm_ctx *c) {
   // cells, level by level, every size on the device
   int32_t *lev = dp<int32_t>(c->lev);
   TRY(launch_tree_top(k, n, off, np, lev, pl.L, pl.top, pl.prm.ncrit, cells,
-                      dp<uint32_t>(c->lev_status), skeys, region, sprob, s, true,
+                      dp<uint32_t>(c->lev_status), skeys, region, sprob, long_run, s, true,
                       pl.grid.data()));
   for (int d = pl.top; d < pl.L; d++)
     TRY(launch_level_step(k, lev, d, pl.grid[d], pl.prm.ncrit, cells, dp<uint32_t>(c->flag),

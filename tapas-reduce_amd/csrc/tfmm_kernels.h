@@ -53,7 +53,8 @@ enum : uint32_t {
   ST_GROUPS = 16,
   ST_ITEMS = 32,
   ST_UNITS = 64,
-  ST_FALLBACK = 128
+  ST_FALLBACK = 128,
+  ST_SORT = 256       // bodies out of order (a run too long for launch_sort_runs)
 };
 struct PlanCaps {
   uint32_t m2l, p2p, front, items, units, fallback;
@@ -69,7 +70,12 @@ hipError_t launch_bbox(const double *x, const double *y, const double *z, int64_
 hipError_t launch_keys(const double *x, const double *y, const double *z, const double *q,
                        int64_t n, const double *regions, const int64_t *off, int nprob,
                        uint64_t *keys, uint32_t *idx, uint32_t *bprob, double4 *rec,
-                       hipStream_t s);
+                       uint32_t *long_run, hipStream_t s);
+// bodies sorted by the key bits above shift (and, with sprob, by problem), in the
+// order of the whole key; *long_run set when a run was too long to be sorted
+hipError_t launch_sort_runs(const uint64_t *keys, const uint32_t *idx, const uint32_t *sprob,
+                            int64_t n, int shift, uint64_t *keys_out, uint32_t *idx_out,
+                            uint32_t *long_run, hipStream_t s);
 // forest of nprob problems, problem p = bodies [off[p], off[p+1])
 hipError_t launch_bbox_forest(const double *x, const double *y, const double *z,
                               const int64_t *off, int nprob, double *regions, hipStream_t s);
@@ -95,7 +101,8 @@ hipError_t launch_periodic_region(double *region, double cycle, uint32_t *flag, 
 hipError_t launch_tree_top(Cells c, int64_t n, const int64_t *off, int nprob, int32_t *lev, int L,
                            int levels, int ncrit, int32_t cap, uint32_t *status,
                            const uint64_t *keys, const double *regions, const uint32_t *sprob,
-                           hipStream_t s, bool last = false, const int32_t *most = nullptr);
+                           const uint32_t *long_run, hipStream_t s, bool last = false,
+                           const int32_t *most = nullptr);
 int tree_top_levels(const int32_t *sizes, int L);
 hipError_t launch_level_step(Cells c, int32_t *lev, int d, int32_t grid_cells, int ncrit,
                              int32_t cap, uint32_t *flag, uint32_t *loc, uint32_t *bsum,
