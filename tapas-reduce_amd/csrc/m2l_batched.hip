@@ -411,9 +411,10 @@ struct Mfma<double> {
 // columns; the step (row block, k-step) is non-zero only while the smallest
 // degrees of its rows and columns add up to at most P - 1, which leaves 61 of
 // the 196 (18 whole 16 x 16 blocks would be 72): the first RB_STEPS[rb] k-steps
-// of row block rb.  They are taken row block by row block, the last three
-// (6 steps) in turn: an MFMA's results take a while to arrive, and a row block
-// is added to the sums some steps after its last one.
+// of row block rb.  The last three row blocks (6 steps) are taken in turn, then
+// the others upwards, the first, which needs every k-step, last: a B vector then
+// has its last use early enough to be loaded over itself for the next item at
+// least 24 steps before that item's first use of it.
 constexpr int NRB = 7;
 constexpr int RB_STEPS[NRB] = {28, 14, 8, 5, 3, 2, 1};
 constexpr int NST = 61;
@@ -444,17 +445,17 @@ struct StepTab {
 constexpr StepTab make_steps() {
   StepTab s{};
   int n = 0;
-  for (int rb = 0; rb < 4; rb++)
-    for (int t = 0; t < RB_STEPS[rb]; t++, n++) {
-      s.rb[n] = (int16_t)rb;
-      s.t[n] = (int16_t)t;
-    }
   for (int t = 0; t < 3; t++)
     for (int rb = 4; rb < NRB; rb++)
       if (t < RB_STEPS[rb]) {
         s.rb[n] = (int16_t)rb;
         s.t[n++] = (int16_t)t;
       }
+  for (int rb = 3; rb >= 0; rb--)
+    for (int t = 0; t < RB_STEPS[rb]; t++, n++) {
+      s.rb[n] = (int16_t)rb;
+      s.t[n] = (int16_t)t;
+    }
   for (int i = 0; i < n; i++)
     for (int b = 0; b < NBLK; b++)
       if (BLK_RB[b] == s.rb[i] && BLK_CB[b] == s.t[i] / 4) s.code[i] = (int16_t)(4 * b + s.t[i] % 4);
@@ -463,6 +464,23 @@ constexpr StepTab make_steps() {
 }
 constexpr StepTab STEP = make_steps();
 __constant__ StepTab c_steps = make_steps();
+// first step of k-step t, last step that uses B vector v, and the last step of row
+// block rb
+constexpr int first_use(int t) {
+  int i = 0;
+  while (STEP.t[i] != t) i++;
+  return i;
+}
+constexpr int last_use(int v) {
+  int i = NST - 1;
+  while (STEP.t[i] / 4 != v) i--;
+  return i;
+}
+constexpr int last_step(int rb) {
+  int i = NST - 1;
+  while (STEP.rb[i] != rb) i--;
+  return i;
+}
 
 __device__ inline int row_degree(int r) {
   if (r >= 110) return 0;
@@ -539,77 +557,70 @@ __device__ inline double flip(double x, uint32_t mask, int at) {
                           __double2loint(x));
 }
 
-// sums of row block rb += products, with their signs
+// sums of row block rb += products, with their signs: result i
 template <class T>
-__device__ inline void add_products(typename Mfma<T>::V (&sum)[NRB], int rb,
-                                    const typename Mfma<T>::V &v, uint32_t signs) {
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    sum[rb][i] += flip(v[i], signs, 4 * rb + i);
-    asm volatile("" : "+v"(sum[rb][i]));  // added here, not when the sum is next needed
-  }
+__device__ inline void add_product(typename Mfma<T>::V (&sum)[NRB], int rb,
+                                   const typename Mfma<T>::V &v, uint32_t signs, int i) {
+  sum[rb][i] += flip(v[i], signs, 4 * rb + i);
+  asm volatile("" : "+v"(sum[rb][i]));  // added here, not when the sum is next needed
 }
 
-// One wave's registers: the operands of the current group, the sums, and the
-// products of the last three row blocks of the item before (with their signs),
+// One wave's registers: the A operands of the next steps, the B operands, the
+// sums, and the products of the item before's last row block (with their signs),
 // which are added during this one.
+constexpr int RING = 4;  // A vectors held: 16 steps ahead
+static_assert(NAV % RING == 0, "an A vector's place is the same in every item");
 template <class T>
 struct SetRegs {
-  typename Vec4<T>::V a[NAV];
-  typename Mfma<T>::V sum[NRB], late[3];
+  typename Vec4<T>::V a[RING], b[NBV];
+  typename Mfma<T>::V sum[NRB], late;
   uint32_t late_signs;
 };
 
-// One item: 61 MFMAs, and between them the loads of the next item's B operands
-// (from next into bn) and, when its group differs (change), of its A operands
-// (from af, each vector over itself once its last step is issued): they have
-// most of an item to arrive.  A wave issues in order and waits at an MFMA until
-// the matrix unit is free, so what is written between two MFMAs costs no time
-// as long as it is short, and what is loaded after the last one is waited for.
-// The loads over a vector in use stand in branches of their own because the
-// compiler would otherwise lift them above the vector's last use and move the
-// values back at the end, waiting for them.
+// One item: 61 MFMAs, and between them the loads of what comes next, every vector
+// over itself once its last step is issued: the A operands RING vectors ahead
+// (af, then the next item's afn), the next item's B operands from next.  A wave
+// issues in order and waits at an MFMA until the matrix unit is free, so what is
+// written between two MFMAs costs little as long as it is short.  The steps are
+// kept in this order (sched_barrier): the compiler would lift the loads above the
+// vectors' last uses, into registers of their own, and move the values back at
+// the end, waiting for them.  The A operands are read again for an item of the
+// same group: holding all 61 for as long as a group lasts took 225 registers (446
+// in FP64) instead of 128 (217), two waves a SIMD instead of four (one instead of
+// two).  Alone, us, then and now (the shortest units last, see k_unit_map,
+// included): 4M Plummer 2,830 and 2,610, 256 x 16K 3,020 and 2,820, 1M cube FP64
+// 1,420 and 1,255, 500K ellipsoid FP64 1,770 and 1,700.
 // Every row block's products are summed from zero over the item and then added
 // to the target's sums: long chains into the sums themselves would lose more to
 // rounding in FP32 (relative 1.2e-6 between two groupings of one problem's
-// pairs, against 6e-7).  bs, ss: signs of b and of the products.
+// pairs, against 6e-7).  They are added four steps after their last one (an
+// MFMA's results take a while to arrive), one result a step.  bs, ss: signs of b and of the products.
 template <class T, int S>
-__device__ inline void set_step(SetRegs<T> &r, typename Vec4<T>::V (&b)[NBV],
-                                typename Vec4<T>::V (&bn)[NBV], typename Mfma<T>::V (&p)[NRB],
-                                uint32_t bs, uint32_t ss, const T *next, bool change,
-                                const T *af) {
+__device__ inline void set_step(SetRegs<T> &r, typename Mfma<T>::V (&p)[NRB], uint32_t bs,
+                                uint32_t ss, const T *next, const T *af, const T *afn) {
   typedef typename Vec4<T>::V V;
-  constexpr int rb = STEP.rb[S], t = STEP.t[S];
-  if constexpr (S < 28 && S % 4 == 0) {
-    bn[S / 4] = *reinterpret_cast<const V *>(next + 4 * S);
-#pragma unroll
-    for (int k = 0; k < 4; k++) b[S / 4][k] = flip(b[S / 4][k], bs, S + k);
-  }
+  constexpr int rb = STEP.rb[S], t = STEP.t[S], v = t / 4, k = S / 4;
+  if constexpr (S == first_use(t)) r.b[v][t % 4] = flip(r.b[v][t % 4], bs, t);
   if constexpr (t == 0) p[rb] = (typename Mfma<T>::V){0, 0, 0, 0};
-  p[rb] = Mfma<T>::step(r.a[S / 4][S % 4], b[t / 4][t % 4], p[rb]);
-  if constexpr (S == 11) {
+  p[rb] = Mfma<T>::step(r.a[k % RING][S % 4], r.b[v][t % 4], p[rb]);
+  if constexpr (S >= 4 && S < 8) add_product<T>(r.sum, 0, r.late, r.late_signs, S - 4);
 #pragma unroll
-    for (int i = 0; i < 3; i++) add_products<T>(r.sum, 4 + i, r.late[i], r.late_signs);
-  }
-  // row block rb is added four steps into the next one
-  constexpr int end[4] = {28, 28 + 14, 28 + 14 + 8, 28 + 14 + 8 + 5};
-#pragma unroll
-  for (int k = 0; k < 4; k++)
-    if (S == end[k] + 3) add_products<T>(r.sum, k, p[k], ss);
-  if constexpr (S % 4 == 3 || S == NST - 1) {
-    if (change) r.a[S / 4] = *reinterpret_cast<const V *>(af + (S / 4) * 256);
-  }
+  for (int i = 1; i < NRB; i++)
+    if (S >= last_step(i) + 4 && S < last_step(i) + 8)
+      add_product<T>(r.sum, i, p[i], ss, S - last_step(i) - 4);
+  if constexpr (S == last_use(v)) r.b[v] = *reinterpret_cast<const V *>(next + 16 * v);
+  if constexpr (S % 4 == 3 || S == NST - 1)
+    r.a[k % RING] = *reinterpret_cast<const V *>(
+        k + RING < NAV ? af + (k + RING) * 256 : afn + (k + RING - NAV) * 256);
+  __builtin_amdgcn_sched_barrier(0);
 }
 
 template <class T, int... S>
-__device__ inline void set_steps(std::integer_sequence<int, S...>, SetRegs<T> &r,
-                                 typename Vec4<T>::V (&b)[NBV], typename Vec4<T>::V (&bn)[NBV],
-                                 uint32_t bs, uint32_t ss, const T *next, bool change,
-                                 const T *af) {
+__device__ inline void set_steps(std::integer_sequence<int, S...>, SetRegs<T> &r, uint32_t bs,
+                                 uint32_t ss, const T *next, const T *af, const T *afn) {
   typename Mfma<T>::V p[NRB];
-  (set_step<T, S>(r, b, bn, p, bs, ss, next, change, af), ...);
-#pragma unroll
-  for (int i = 0; i < 3; i++) r.late[i] = p[4 + i];
+  (set_step<T, S>(r, p, bs, ss, next, af, afn), ...);
+  r.late = p[0];
   r.late_signs = ss;
 }
 
@@ -634,15 +645,19 @@ __device__ inline int unit_of_block(int b, int nunits, int run) {
 // unit writes the set's L, the others leave theirs in part[] (one 16 x 110 slab
 // per extra unit, FP64), which k_unit_combine adds in unit order after the
 // launch, so the sums do not depend on timing.
-// (set, number) of every unit: 16 threads a set
+// (set, number) of every unit, 16 threads a set: all whole units first, then every
+// set's last one, which is the shortest: the launch ends on short units.
 __global__ void k_unit_map(const uint32_t *ucnt, const uint32_t *uoff, int32_t ntiles,
                            int2 *units, uint32_t units_cap) {
   critical_path_priority();
   const int32_t t = (blockIdx.x * blockDim.x + threadIdx.x) >> 4;
   if (t >= ntiles) return;
-  const uint32_t n = ucnt[t], o = uoff[t];
-  for (uint32_t k = threadIdx.x & 15; k < n && o + k < units_cap; k += 16)
-    units[o + k] = make_int2(t, (int)k);
+  const uint32_t n = ucnt[t], o = uoff[t] - (uint32_t)t;
+  const uint32_t total = uoff[ntiles - 1] + ucnt[ntiles - 1];
+  for (uint32_t k = threadIdx.x & 15; k < n; k += 16) {
+    const uint32_t at = k + 1 < n ? o + k : total - (uint32_t)(ntiles - t);
+    if (at < units_cap) units[at] = make_int2(t, (int)k);
+  }
 }
 
 // slab of extra unit k >= 1 of tile t: every tile has at least one unit
@@ -734,7 +749,7 @@ __device__ inline int result_degree(int rb, int i, int q) {
 
 // One work unit per wave.
 template <class T>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 2 : 1)))
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 2)))
 void k_m2l_sets(
     const int32_t *set_off, const int2 *units, const uint32_t *ucnt, const uint32_t *uoff,
     int32_t nsets, int32_t chunk, int xcd_run, const uint32_t *ikey, int gbits,
@@ -769,38 +784,30 @@ void k_m2l_sets(
     };
     auto operands = [&](uint32_t g) { return Af + (int64_t)g * AF_PER_GROUP + lane * 4; };
     const LaneSigns signs = lane_signs<T>(q);
-    V b0[NBV], b1[NBV];
     // keys and column words are loaded two items ahead of their use
-    uint32_t w0 = word(ib), w1 = word(ib + 1), k1 = key(ib + 1), k0 = key(ib + 2);
-    uint32_t g = group(key(ib));
+    uint32_t w0 = word(ib), w1 = word(ib + 1), k1 = key(ib + 1);
+    const T *af = operands(group(key(ib)));
     {
-      const T *m = source(w0), *af = operands(g);
+      const T *m = source(w0);
 #pragma unroll
-      for (int v = 0; v < NBV; v++) b0[v] = *reinterpret_cast<const V *>(m + 16 * v);
+      for (int v = 0; v < NBV; v++) r.b[v] = *reinterpret_cast<const V *>(m + 16 * v);
 #pragma unroll
-      for (int v = 0; v < NAV; v++) r.a[v] = *reinterpret_cast<const V *>(af + v * 256);
+      for (int v = 0; v < RING; v++) r.a[v] = *reinterpret_cast<const V *>(af + v * 256);
     }
-#pragma unroll
-    for (int i = 0; i < 3; i++) r.late[i] = (typename Mfma<T>::V){0, 0, 0, 0};
+    r.late = (typename Mfma<T>::V){0, 0, 0, 0};
     r.late_signs = 0;
-    // wa, wb: column words of this item and the next; kb: the next item's key
-    auto item = [&](V (&b)[NBV], V (&bn)[NBV], uint32_t &wa, uint32_t wb, uint32_t &kb,
-                    int32_t it) {
-      const uint32_t gn = group(kb), m = wa >> MIR_AT;
-      kb = key(it + 3);
-      wa = word(it + 2);
-      set_steps<T>(std::make_integer_sequence<int, NST>{}, r, b, bn, LaneSigns::of(signs.b, m),
-                   LaneSigns::of(signs.p, m), source(wb), gn != g, operands(gn));
-      g = gn;
-    };
-    for (int32_t it = ib;; it += 2) {
-      item(b0, b1, w0, w1, k1, it);
-      if (it + 1 >= ie) break;
-      item(b1, b0, w1, w0, k0, it + 1);
-      if (it + 2 >= ie) break;
+    for (int32_t it = ib; it < ie; it++) {
+      const uint32_t m = w0 >> MIR_AT;
+      const T *afn = operands(group(k1)), *next = source(w1);
+      w0 = w1;
+      w1 = word(it + 2);
+      k1 = key(it + 2);
+      set_steps<T>(std::make_integer_sequence<int, NST>{}, r, LaneSigns::of(signs.b, m),
+                   LaneSigns::of(signs.p, m), next, af, afn);
+      af = afn;
     }
 #pragma unroll
-    for (int i = 0; i < 3; i++) add_products<T>(r.sum, 4 + i, r.late[i], r.late_signs);
+    for (int i = 0; i < 4; i++) add_product<T>(r.sum, 0, r.late, r.late_signs, i);
   }
   // L_j = L~_j / sigma_t^(j+1)
   const int32_t ci = set * TILE + j;
