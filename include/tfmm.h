@@ -257,15 +257,17 @@ int tfmm_get_lists(tfmm_ctx *ctx, int32_t *m2l_off, int32_t *m2l_src, int32_t *p
  * expansions). */
 #define TFMM_TUNE_M2L_XCD_RUN 2
 /* TFMM_TUNE_P2P_SCHEDULE: where the P2P kernel (second stream) starts.  In
- * tfmm_evaluate, 0 starts it with the numeric phase, beside the upward pass
- * and the M2L kernels; 1 starts it with the M2L set kernel; 2 as soon as
+ * tfmm_evaluate, 0 (default) starts it with the numeric phase, beside the M2L
+ * kernels, or, without resident waves (TFMM_TUNE_P2P_WAVES 0) and where the
+ * traversal finds that the P2P outweighs the M2L, as 2 with a few resident
+ * waves of the library's choice; 1 starts it with the M2L set kernel; 2 as soon as
  * its list is sorted, beside the M2L batch building (also inside the
  * one-launch graph of TFMM_TUNE_GRAPH 2; with TFMM_TUNE_GRAPH 1 as 0); 3 as 2.  A
- * resident FP32 P2P (TFMM_TUNE_P2P_WAVES > 0, mixed precision) holds its few
- * waves until the critical path beside it is done; a full-occupancy launch of
- * the same kernel on the context stream then takes the target cells still left
- * on its counter (each cell is computed by one wave either way: the fields do
- * not change), with schedule 3 after the M2L, else after the L2L; 4 runs it on the context
+ * resident P2P (TFMM_TUNE_P2P_WAVES > 0) holds its few waves until the critical
+ * path beside it is done; a full-occupancy launch of the same kernel on the
+ * context stream then takes the target cells still left on its counter (each
+ * cell is computed the same way by either: the fields do not change), with
+ * schedule 3 after the M2L, else after the L2L; 4 runs it on the context
  * stream with nothing beside it (from phase A, serially: for timing the
  * kernel alone).  In the separate
  * tfmm_traverse, 1 starts it with the set kernel, any other value as soon
@@ -293,8 +295,7 @@ int tfmm_get_lists(tfmm_ctx *ctx, int32_t *m2l_off, int32_t *m2l_src, int32_t *p
 /* TFMM_TUNE_P2P_WAVES: 0 (default) runs the P2P (FP32 or FP64) as one
  * workgroup per cell; k in 1..8 runs it as k resident waves per SIMD that
  * take target leaves from a counter, so it holds a bounded share of the CUs
- * and the kernels beside it keep slots (see TFMM_TUNE_P2P_SCHEDULE; the
- * drain is the FP32 P2P's). */
+ * and the kernels beside it keep slots (see TFMM_TUNE_P2P_SCHEDULE). */
 #define TFMM_TUNE_P2P_WAVES 5
 /* TFMM_TUNE_DEVICE_LIMIT: a limit in bytes (0 = none, the default) on the
  * device memory the library's buffers hold, over all contexts of the

@@ -59,6 +59,7 @@ struct Plan {
   // capacities
   int L = 0;                        // tree levels
   std::vector<int32_t> grid;        // cells per level
+  int run_schedule = 0, run_waves = 0;
   int top = 0;                      // leading levels built by one workgroup
   int key_bits = 0;                 // leading key bits of the bodies' sort
   int64_t cells = 0;                // cells in all
@@ -122,6 +123,7 @@ struct tfmm_ctx {
   uint32_t n_m2l_exec = 0, n_p2p = 0;
   uint64_t n_m2l_all = 0, n_p2p_calls = 0, n_p2p_self = 0;
   uint64_t n_p2p_calls_leaf = 0;  // P2P leaf-pair calls (a mutual pair once)
+  uint64_t n_p2p_pairs = 0;  // body pairs of the traversal (counted as numP2P)
   uint32_t dtt_steps = 0;
 
   // batched M2L (offset groups)
@@ -136,6 +138,7 @@ struct tfmm_ctx {
   int p2p_schedule = 0;          // where the P2P starts (TFMM_TUNE_P2P_SCHEDULE)
   int use_graph = 0;             // tfmm_evaluate's numeric phase as one hipGraph
   int p2p_waves = 0;             // resident P2P waves per SIMD (0: one workgroup per cell)
+  int run_schedule = 0, run_waves = 0;  // the two as the running evaluation takes them
   int n_cu = 0;                  // compute units of the device
   DevBuf p2p_next;               // the resident P2P's work counter
   int ext_events = -1;           // external event records in a capture: -1 not probed
@@ -147,6 +150,8 @@ struct tfmm_ctx {
   Plan plan;                      // the whole-evaluation graph (use_graph == 2)
   DevBuf gsz, gstep;              // its device sizes and traversal step grids
   uint32_t *h_plan = nullptr;     // pinned read-back of the whole graph (PLAN_HOST_BYTES)
+  bool upward_early = false;  // the running evaluation's upward pass (early_upward)
+  bool p2p_heavy = false;     // the last evaluation's p2p_outweighs
   bool upward_pending = false;  // the early upward pass is still to be enqueued
   bool one_graph = false;         // the last tfmm_evaluate was one launch of it
   // periodic images (tfmm_set_periodic): image sublevels, 0 = none, and the
@@ -748,6 +753,7 @@ int do_dtt(tfmm_ctx *c) {
     if (c->h_u32[16 + nsteps] != 0) return fail(c, TFMM_EHIP, "traversal did not terminate");
     const uint32_t nm = c->h_u32[1], np = c->h_u32[2];
     if (nm <= c->m2l_cap && np <= c->p2p_cap && fmax <= c->front_cap) {
+      c->n_p2p_pairs = (uint64_t)c->h_u32[9] << 32 | c->h_u32[8];
       c->dtt_hint.assign(c->h_u32 + 16, c->h_u32 + 16 + nsteps + 1);
       c->dtt_hint_cells = c->ncells;
       c->n_m2l_exec = nm;
@@ -1182,55 +1188,79 @@ void probe_external_events(tfmm_ctx *c) {
 
 // The P2P on the second stream (forked from and later joined to the context
 // stream by events).
-// The resident FP32 P2P holds few waves so that the kernels of the critical path
+// A resident P2P holds few waves so that the kernels of the critical path
 // find room beside it.  When those are done, nothing is left to make room for: a
 // full-occupancy launch of the same kernel on the context stream then takes the
 // target cells still left on its counter, after the L2L, or with schedule 3
 // already once the set kernel is done.  (Two clusters of 4M bodies, mixed, 3
 // resident waves: 19.9 ms with the drain, 20.3 without, where the 3 waves
 // ended alone.)
-bool p2p_drains(const tfmm_ctx *c) {
-  return c->p2p_schedule != 4 && c->p2p_waves > 0 && c->prm.precision == TFMM_MIXED;
+bool p2p_drains(const tfmm_ctx *c) { return c->run_schedule != 4 && c->run_waves > 0; }
+
+// one launch of resident waves on the shared counter
+hipError_t p2p_on_counter(tfmm_ctx *c, int64_t ncells, int waves, hipStream_t st) {
+  const Cells k = cells_of(c);
+  Csr pl{dp<int32_t>(c->p2p_off), dp<int32_t>(c->p2p_src)};
+  if (c->prm.precision == TFMM_MIXED)
+    return launch_p2p_fp32_drain(k, (int32_t)ncells, pl, sorted_bodies(c), dp<float4>(c->relpos),
+                                 dp<double>(c->acc), leaf_waves(c), waves,
+                                 dp<uint32_t>(c->p2p_next), st, period(c));
+  return launch_p2p_fp64_drain(k, (int32_t)ncells, pl, sorted_bodies(c), dp<double>(c->acc),
+                               leaf_waves(c), waves, dp<uint32_t>(c->p2p_next), st, period(c));
 }
 
 int drain_p2p(tfmm_ctx *c, int64_t ncells, bool l2l_done) {
-  if (!p2p_drains(c) || l2l_done == (c->p2p_schedule == 3)) return TFMM_OK;
-  const Cells k = cells_of(c);
-  Csr pl{dp<int32_t>(c->p2p_off), dp<int32_t>(c->p2p_src)};
-  TRY(launch_p2p_fp32_drain(k, (int32_t)ncells, pl, sorted_bodies(c), dp<float4>(c->relpos),
-                            dp<double>(c->acc), leaf_waves(c), 8 * 4 * c->n_cu, dp<uint32_t>(c->p2p_next),
-                            c->stream, period(c)));
+  if (!p2p_drains(c) || l2l_done == (c->run_schedule == 3)) return TFMM_OK;
+  TRY(p2p_on_counter(c, ncells, 8 * 4 * c->n_cu, c->stream));
   return TFMM_OK;
+}
+
+// With neither P2P knob set (schedule 0, no resident waves) the library chooses.
+// Where the P2P is the larger part of the work beside the M2L, it starts as soon as
+// its list is sorted, as schedule 2, as resident waves that leave the M2L's waves
+// room (3 a SIMD in FP32, 2 in FP64), and a full launch takes the rest at the end:
+// 1M cube FP64 4.69 to 4.2 ms, 4M Plummer mixed 11.58 to 10.9.  Where the M2L is
+// larger, it would only be delayed (500K ellipsoid FP64 4.06 to 4.15), and with
+// several waves a leaf the P2P is over too soon.  Cycles of a SIMD: 60 (FP32) or
+// 120 a 64 body pairs with the usual idle lanes, 44 or 80 an M2L step, 11 pairs an
+// item.
+constexpr double P2P_HEAVY = 1.3;
+bool p2p_chosen(const tfmm_ctx *c) {
+  return c->p2p_schedule == 0 && c->p2p_waves == 0 && c->use_graph != 1;
+}
+
+bool p2p_outweighs(const tfmm_ctx *c, uint64_t body_pairs, uint32_t m2l) {
+  const bool mixed = c->prm.precision == TFMM_MIXED, fp32 = m2l_fp32(c);
+  const double p2p = (double)body_pairs * (c->prm.mutual ? 2 : 1) / 64 * (mixed ? 60 : 120);
+  const double far = (double)m2l / 11 * 61 * (fp32 ? 44 : 80);
+  return leaf_waves(c) == 1 && p2p > P2P_HEAVY * far;
 }
 
 int fork_p2p(tfmm_ctx *c, int64_t ncells = -1) {
   hipStream_t s = c->stream;
   const Cells k = cells_of(c);
   if (ncells < 0) ncells = c->ncells;
-  const bool mixed = c->prm.precision == TFMM_MIXED;
-  // the drained schedule clears the shared counter on this stream, before
-  // either launch can take from it
+  // the launches on the counter share it: cleared on this stream, before either
+  // can take from it
   if (p2p_drains(c)) TRY(launch_fill_zero(c->p2p_next.ptr, 4, s));
   // schedule 4: on the context stream, alone (the kernel's own time)
-  hipStream_t ps = c->p2p_schedule == 4 ? s : c->side;
+  hipStream_t ps = c->run_schedule == 4 ? s : c->side;
   if (ps != s) {
     TRY(hipEventRecord(c->ev[EV_P2PREADY], s));
     TRY(hipStreamWaitEvent(ps, c->ev[EV_P2PREADY], 0));
   }
   TRY(rec(c, EV_P2P0, ps));
+  const int resident = c->run_waves > 0 ? c->run_waves * 4 * c->n_cu : 0;
   Csr pl{dp<int32_t>(c->p2p_off), dp<int32_t>(c->p2p_src)};
   if (p2p_drains(c))
-    TRY(launch_p2p_fp32_drain(k, (int32_t)ncells, pl, sorted_bodies(c), dp<float4>(c->relpos),
-                              dp<double>(c->acc), leaf_waves(c), p2p_resident(c), dp<uint32_t>(c->p2p_next),
-                              ps, period(c)));
-  else if (mixed)
+    TRY(p2p_on_counter(c, ncells, resident, ps));
+  else if (c->prm.precision == TFMM_MIXED)
     TRY(launch_p2p_fp32(k, (int32_t)ncells, pl, sorted_bodies(c), dp<float4>(c->relpos),
-                        dp<double>(c->acc), leaf_waves(c), p2p_resident(c),
-                        dp<uint32_t>(c->p2p_next), ps, period(c)));
-  else
-    TRY(launch_p2p_fp64(k, (int32_t)ncells, pl, sorted_bodies(c), dp<double>(c->acc), leaf_waves(c),
-                        p2p_resident(c), dp<uint32_t>(c->p2p_next), ps,
+                        dp<double>(c->acc), leaf_waves(c), resident, dp<uint32_t>(c->p2p_next), ps,
                         period(c)));
+  else
+    TRY(launch_p2p_fp64(k, (int32_t)ncells, pl, sorted_bodies(c), dp<double>(c->acc),
+                        leaf_waves(c), resident, dp<uint32_t>(c->p2p_next), ps, period(c)));
   TRY(rec(c, EV_P2P1, ps));
   TRY(hipEventRecord(c->ev[EV_P2PJOIN], ps));
   return TFMM_OK;
@@ -1269,7 +1299,7 @@ int upward_pass(tfmm_ctx *c, hipStream_t st) {
 // beside the list building it stays in the numeric phase: it would delay the P2P
 // (4M Plummer, schedule 2, 11.25 ms against 11.64).  A numeric phase that is a
 // graph of its own (TFMM_TUNE_GRAPH 1) keeps it too.
-bool early_upward(const tfmm_ctx *c) { return c->use_graph != 1 && c->p2p_schedule < 2; }
+bool early_upward(const tfmm_ctx *c) { return c->use_graph != 1 && c->run_schedule < 2; }
 
 // The host enqueues it after the traversal's steps, while those run: the steps are
 // what the next read-back waits for.
@@ -1285,6 +1315,11 @@ int fused_lists(tfmm_ctx *c);
 
 int fused_prepare(tfmm_ctx *c) {
   hipStream_t s = c->stream;
+  c->run_schedule = c->p2p_schedule;
+  c->run_waves = c->p2p_waves;
+  // the P2P's start is chosen after the traversal; until then as the last time
+  if (p2p_chosen(c) && c->p2p_heavy) c->run_schedule = 2;
+  c->upward_early = early_upward(c);
   TRY(reserve_expansions(c));
   TRY(dev_reserve(c->leaf_of, (size_t)c->n * 4));
   int rc = cartesian(c) ? cart_tables(c) : TFMM_OK;
@@ -1298,7 +1333,7 @@ int fused_prepare(tfmm_ctx *c) {
     TRY(dev_reserve(c->mq, m2l_mq_bytes(c->ncells, m2l_fp32(c))));
   }
   c->p2p_forked = false;
-  if (!early_upward(c)) return fused_lists(c);
+  if (!c->upward_early) return fused_lists(c);
   TRY(hipEventRecord(c->ev[EV_UPJOIN], s));  // the tree; again once the pass is enqueued
   TRY(hipStreamWaitEvent(c->side, c->ev[EV_UPJOIN], 0));
   c->upward_pending = true;
@@ -1323,7 +1358,12 @@ int fused_lists(tfmm_ctx *c) {
     TRY(launch_leaf_relpos(k, (int32_t)c->ncells, sorted_bodies(c), dp<float4>(c->relpos), s));
   }
   TRY(dev_reserve(c->acc, (size_t)c->n * 32));
-  if (c->p2p_schedule >= 2 && !c->use_graph) {
+  if (p2p_chosen(c)) {
+    c->p2p_heavy = p2p_outweighs(c, c->n_p2p_pairs, c->n_m2l_exec);
+    c->run_schedule = c->p2p_heavy ? 2 : 0;
+    c->run_waves = c->p2p_heavy ? (mixed ? 3 : 2) : 0;
+  }
+  if (c->run_schedule >= 2 && c->use_graph != 1) {
     // the P2P list is complete: start the P2P now, beside the M2L batch
     // building (with resident waves it leaves that work CU slots)
     rc = fork_p2p(c);
@@ -1357,14 +1397,14 @@ int fused_numeric(tfmm_ctx *c) {
   // start of the phase (schedule 0), at the set kernel (1), or already in
   // phase A (2)
   int rc;
-  if (!c->p2p_forked && c->p2p_schedule != 1 && (rc = fork_p2p(c))) return rc;
+  if (!c->p2p_forked && c->run_schedule != 1 && (rc = fork_p2p(c))) return rc;
   if (cart_direct(c)) {
-    if (early_upward(c)) TRY(hipStreamWaitEvent(s, c->ev[EV_UPJOIN], 0));
+    if (c->upward_early) TRY(hipStreamWaitEvent(s, c->ev[EV_UPJOIN], 0));
     else if ((rc = upward_pass(c, s))) return rc;
-    if (!c->p2p_forked && c->p2p_schedule == 1 && (rc = fork_p2p(c))) return rc;
+    if (!c->p2p_forked && c->run_schedule == 1 && (rc = fork_p2p(c))) return rc;
     if ((rc = cart_m2l(c))) return rc;
     TRY(rec(c, EV_M2L1, s));
-    if ((rc = drain_p2p(c, c->ncells, c->p2p_schedule != 3))) return rc;
+    if ((rc = drain_p2p(c, c->ncells, c->run_schedule != 3))) return rc;
     TRY(hipStreamWaitEvent(s, c->ev[EV_P2PJOIN], 0));
     TRY(rec(c, EV_TRAV, s));
     if ((rc = cart_downward(c))) return rc;
@@ -1373,12 +1413,12 @@ int fused_numeric(tfmm_ctx *c) {
   }
   // upward
   const int nl = (int)c->lvl.size() - 1;
-  if (early_upward(c)) TRY(hipStreamWaitEvent(s, c->ev[EV_UPJOIN], 0));
+  if (c->upward_early) TRY(hipStreamWaitEvent(s, c->ev[EV_UPJOIN], 0));
   else if ((rc = upward_pass(c, s))) return rc;
   // M2L
   const bool mixed = m2l_fp32(c);
   TRY(rec(c, EV_M2L0, s));
-  if (!c->p2p_forked && c->p2p_schedule == 1 && (rc = fork_p2p(c))) return rc;
+  if (!c->p2p_forked && c->run_schedule == 1 && (rc = fork_p2p(c))) return rc;
   const int32_t tile = m2l_tile_size();
   const int32_t ntiles = (int32_t)((c->ncells + tile - 1) / tile);
   TRY(launch_m2l_sets(dp<int32_t>(c->set_off), dp<int2>(c->units), dp<uint32_t>(c->u_cnt),
@@ -1513,6 +1553,8 @@ void plan_make(tfmm_ctx *c) {
   pl.xcd_run = c->m2l_xcd_run;
   pl.p2p_schedule = c->p2p_schedule;
   pl.p2p_waves = c->p2p_waves;
+  pl.run_schedule = c->run_schedule;
+  pl.run_waves = c->run_waves;
   pl.L = L0 + 1;
   pl.grid.resize(pl.L);
   pl.cells = 4096;
@@ -1687,6 +1729,8 @@ int whole_record(tfmm_ctx *c) {
   const int np = c->nprob;
   const bool forest = np > 1;
   const bool mixed = pl.prm.precision == TFMM_MIXED;
+  c->run_schedule = pl.run_schedule;
+  c->run_waves = pl.run_waves;
   const Cells k = cells_of(c);
   const int32_t cells = (int32_t)pl.cells;
   uint32_t *sz = dp<uint32_t>(c->gsz);
@@ -1797,7 +1841,7 @@ int whole_record(tfmm_ctx *c) {
   if (mixed)
     TRY(launch_leaf_relpos(k, cells, sorted_bodies(c), dp<float4>(c->relpos), s));
   // schedules 2 and 3: the P2P branches off here, beside the M2L batching
-  const bool early = c->p2p_schedule >= 2;
+  const bool early = c->run_schedule >= 2;
   if (early && (rc = fork_p2p(c, cells))) return rc;
   // M2L batches
   {
@@ -1847,11 +1891,11 @@ int whole_record(tfmm_ctx *c) {
   }
   TRY(rec(c, EV_DTT1, s));
   // the numeric phase
-  if (!early && c->p2p_schedule != 1 && (rc = fork_p2p(c, cells))) return rc;
+  if (!early && c->run_schedule != 1 && (rc = fork_p2p(c, cells))) return rc;
   if (early_upward(c)) TRY(hipStreamWaitEvent(s, c->ev[EV_UPJOIN], 0));
   else if ((rc = upward(s))) return rc;
   TRY(rec(c, EV_M2L0, s));
-  if (c->p2p_schedule == 1 && (rc = fork_p2p(c, cells))) return rc;
+  if (c->run_schedule == 1 && (rc = fork_p2p(c, cells))) return rc;
   TRY(launch_m2l_sets(dp<int32_t>(c->set_off), dp<int2>(c->units), dp<uint32_t>(c->u_cnt),
                       dp<uint32_t>(c->u_off), pl.ntiles, 0, c->m2l_xcd_run, pl.caps.units,
                       dp<uint32_t>(c->items), pl.gbits, dp<uint32_t>(c->cols), c->g_af.ptr,

@@ -452,6 +452,20 @@ int p2p_waves_per_leaf(int64_t n, int32_t ncrit) {
   return leaves <= 512 ? 8 : leaves <= 2560 ? 4 : leaves <= 8192 ? 2 : 1;
 }
 
+// resident waves taking target cells from *next without clearing it first:
+// several such launches (on different streams) share the cells of one
+// cleared counter, each cell computed once by one workgroup
+hipError_t launch_p2p_fp64_drain(Cells c, int32_t ncells, Csr list, Bodies b, double *acc,
+                                 int per_leaf, int waves, uint32_t *next, hipStream_t s,
+                                 double cycle) {
+  if (ncells <= 0 || waves <= 0) return hipSuccess;
+  p2p_waves(per_leaf, [&](auto w) {
+    const int grid = resident_blocks(waves, w, ncells);
+    k_p2p_fp64_resident<w><<<grid, 64 * w, 0, s>>>(c, ncells, list, b, acc, next, cycle);
+  });
+  return hipGetLastError();
+}
+
 hipError_t launch_p2p_fp64(Cells c, int32_t ncells, Csr list, Bodies b, double *acc,
                            int per_leaf, int resident, uint32_t *next, hipStream_t s,
                            double cycle) {
@@ -459,13 +473,10 @@ hipError_t launch_p2p_fp64(Cells c, int32_t ncells, Csr list, Bodies b, double *
   if (resident > 0 && next) {
     hipError_t e = launch_fill_zero(next, 4, s);
     if (e != hipSuccess) return e;
-    p2p_waves(per_leaf, [&](auto w) {
-      const int grid = resident_blocks(resident, w, ncells);
-      k_p2p_fp64_resident<w><<<grid, 64 * w, 0, s>>>(c, ncells, list, b, acc, next, cycle);
-    });
-  } else {
-    p2p_waves(per_leaf, [&](auto w) { k_p2p_fp64<w><<<ncells, 64 * w, 0, s>>>(c, list, b, acc, cycle); });
+    return launch_p2p_fp64_drain(c, ncells, list, b, acc, per_leaf, resident, next, s, cycle);
   }
+  p2p_waves(per_leaf,
+            [&](auto w) { k_p2p_fp64<w><<<ncells, 64 * w, 0, s>>>(c, list, b, acc, cycle); });
   return hipGetLastError();
 }
 
@@ -528,9 +539,6 @@ hipError_t launch_leaf_relpos(Cells c, int32_t ncells, Bodies b, float4 *rel, hi
   return hipGetLastError();
 }
 
-// resident waves taking target cells from *next without clearing it first:
-// several such launches (on different streams) share the cells of one
-// cleared counter, each cell computed once by one wave
 hipError_t launch_p2p_fp32_drain(Cells c, int32_t ncells, Csr list, Bodies b, const float4 *rel,
                                  double *acc, int per_leaf, int waves, uint32_t *next,
                                  hipStream_t s, double cycle) {
@@ -549,15 +557,11 @@ hipError_t launch_p2p_fp32(Cells c, int32_t ncells, Csr list, Bodies b, const fl
   if (resident > 0 && next) {
     hipError_t e = launch_fill_zero(next, 4, s);
     if (e != hipSuccess) return e;
-    p2p_waves(per_leaf, [&](auto w) {
-      const int grid = resident_blocks(resident, w, ncells);
-      k_p2p_fp32_resident<w><<<grid, 64 * w, 0, s>>>(c, ncells, list, b, rel, acc, next, cycle);
-    });
-  } else {
-    p2p_waves(per_leaf, [&](auto w) {
-      k_p2p_fp32<w><<<ncells, 64 * w, 0, s>>>(c, list, b, rel, acc, cycle);
-    });
+    return launch_p2p_fp32_drain(c, ncells, list, b, rel, acc, per_leaf, resident, next, s, cycle);
   }
+  p2p_waves(per_leaf, [&](auto w) {
+    k_p2p_fp32<w><<<ncells, 64 * w, 0, s>>>(c, list, b, rel, acc, cycle);
+  });
   return hipGetLastError();
 }
 

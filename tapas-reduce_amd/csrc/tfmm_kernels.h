@@ -225,6 +225,10 @@ hipError_t launch_m2l_fp64(Cells c, int32_t ncells, Csr list, int32_t npairs, co
 int p2p_waves_per_leaf(int64_t n, int32_t ncrit);
 hipError_t launch_p2p_fp64(Cells c, int32_t ncells, Csr list, Bodies b, double *acc, int per_leaf,
                            int resident, uint32_t *next, hipStream_t s, double cycle = 0);
+// resident waves on a counter that another launch clears and shares
+hipError_t launch_p2p_fp64_drain(Cells c, int32_t ncells, Csr list, Bodies b, double *acc,
+                                 int per_leaf, int waves, uint32_t *next, hipStream_t s,
+                                 double cycle = 0);
 
 // direct.hip
 // target t sums over the n bodies at x, y, z, q: index targets[t] - tbase

@@ -84,3 +84,31 @@ def test_gpu_waves_per_leaf(ctx, n, ncrit, precision, tol):
     # rounding of FP32 pairs (6e-8) and, in the far field, of FP32 M2L
     ep, ea = oracle.rel_l2(f, oracle.Run(x, y, z, q, ncrit, 0.5, phases=3).fields())
     assert ep < tol and ea < 4 * tol, (ep, ea)
+
+
+@pytest.mark.parametrize("precision", [tfmm.FP64, tfmm.MIXED])
+def test_gpu_chosen_p2p_start(ctx, precision):
+    """Where the P2P outweighs the M2L the library starts it early by itself; the
+    fields are those of a start that the caller sets, bit for bit, with and without
+    the one-launch graph, and after bodies for which it chooses otherwise."""
+    r = np.random.default_rng(4)
+    big = [r.random(600000) for _ in range(3)] + [r.random(600000) + 0.5]
+    small = [v[:3000] for v in big]
+    prm = tfmm.make_params(64, 0.5, precision)
+    print("chosen P2P start, precision %d" % precision, flush=True)
+    ctx.set_bodies(*big)
+    ctx.set_tuning(tfmm.TUNE_P2P_SCHEDULE, 1)
+    try:
+        ctx.evaluate(prm)
+        ref = ctx.fields()
+        ctx.set_tuning(tfmm.TUNE_P2P_SCHEDULE, 0)
+        for graph in (0, 2):
+            ctx.set_tuning(tfmm.TUNE_GRAPH, graph)
+            for bodies in (big, big, small, big, big):
+                ctx.set_bodies(*bodies)
+                ctx.evaluate(prm)
+                if bodies is big:
+                    assert np.array_equal(ctx.fields(), ref), graph
+    finally:
+        ctx.set_tuning(tfmm.TUNE_P2P_SCHEDULE, 0)
+        ctx.set_tuning(tfmm.TUNE_GRAPH, 0)
