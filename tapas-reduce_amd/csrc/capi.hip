@@ -65,7 +65,7 @@ struct Plan {
   int64_t cells = 0;                // cells in all
   int max_depth = 0, nsteps = 0, cwords = 0;
   int32_t nslots = 0, ntiles = 0;
-  std::vector<uint32_t> step_grid;  // pairs per traversal step
+  std::vector<uint32_t> step_grid;  // frontier entries per traversal step
   PlanCaps caps{};
   uint32_t groups = 0;
   int gbits = 0, sbits = 0, tbits = 0;
@@ -118,7 +118,7 @@ struct tfmm_ctx {
   DevBuf m2l_off, m2l_src, p2p_off, p2p_src;
   DevBuf seg_long;  // queue of the per-target lists too long for one wave's sort
   uint32_t m2l_cap = 0, p2p_cap = 0, front_cap = 0;
-  std::vector<uint32_t> dtt_hint;  // frontier sizes of the last traversal
+  std::vector<uint32_t> dtt_hint;  // frontier entries of the last traversal
   int64_t dtt_hint_cells = -1;
   uint32_t n_m2l_exec = 0, n_p2p = 0;
   uint64_t n_m2l_all = 0, n_p2p_calls = 0, n_p2p_self = 0;
@@ -698,10 +698,10 @@ int do_dtt(tfmm_ctx *c) {
   TRY(dev_reserve(c->cnt, (size_t)cwords * 4));
   if (c->m2l_cap == 0) c->m2l_cap = (uint32_t)std::min<int64_t>(UINT32_MAX / 2, std::max<int64_t>(1 << 16, 200 * c->ncells));
   if (c->p2p_cap == 0) c->p2p_cap = (uint32_t)std::min<int64_t>(UINT32_MAX / 2, std::max<int64_t>(1 << 16, 40 * c->nleaves));
-  if (c->front_cap == 0) c->front_cap = (uint32_t)std::min<int64_t>(UINT32_MAX / 2, std::max<int64_t>(1 << 20, 256 * c->ncells));
+  if (c->front_cap == 0) c->front_cap = (uint32_t)std::min<int64_t>(UINT32_MAX / 2, std::max<int64_t>(1 << 17, 32 * c->ncells));
   if (cwords > H_U32_WORDS) return fail(c, TFMM_EINVAL, "tree too deep");
   TRY(dev_reserve(c->dtt_geo, (size_t)c->ncells * 32));
-  TRY(dev_reserve(c->dtt_topo, (size_t)c->ncells * 8));
+  TRY(dev_reserve(c->dtt_topo, (size_t)c->ncells * 16));
   // A frontier that overflowed truncates every later step, so the counts
   // seen after an overflow are lower bounds: capacities at least double.
   // M2L group-table flags (one per slot), then the count of M2L pairs
@@ -716,7 +716,7 @@ int do_dtt(tfmm_ctx *c) {
     TRY(dev_reserve(c->front_b, (size_t)c->front_cap * 8));
     uint32_t *cnt = dp<uint32_t>(c->cnt);
     TRY(launch_dtt_begin(k, (int32_t)c->ncells, c->prm.theta, dp<double4>(c->dtt_geo),
-                         dp<int2>(c->dtt_topo), dp<uint32_t>(c->g_used), nslots + 1, cnt, cwords,
+                         dp<int4>(c->dtt_topo), dp<uint32_t>(c->g_used), nslots + 1, cnt, cwords,
                          dp<int2>(c->front_a), c->nprob, s, c->images > 0));
     // grid of step st: the frontier size of the previous traversal of the same
     // tree shape when there is one (checked below), else the capacity
@@ -727,7 +727,7 @@ int do_dtt(tfmm_ctx *c) {
       TRY(launch_dtt_step(dp<int2>(c->front_a), cnt + 16 + st, grid[st], dp<int2>(c->front_b),
                           c->front_cap, cnt + 16 + st + 1, dp<int2>(c->m2l_pairs), c->m2l_cap,
                           dp<int2>(c->p2p_pairs), c->p2p_cap, cnt, dp<double4>(c->dtt_geo),
-                          dp<int2>(c->dtt_topo), k.depth, k.width, dp<int32_t>(c->slot_of),
+                          dp<int4>(c->dtt_topo), c->prm.theta, dp<int32_t>(c->slot_of),
                           dp<uint32_t>(c->g_used), dp<uint32_t>(c->g_used) + nslots,
                           c->prm.mutual, s, period(c)));
       std::swap(c->front_a, c->front_b);
@@ -1106,7 +1106,7 @@ int traverse_given(tfmm_ctx *c, const int32_t *m2l, int64_t nm, const int32_t *p
   TRY(dev_reserve(c->slot_of, nme * 4));
   TRY(dev_reserve(c->p2p_pairs, npe * 8));
   TRY(dev_reserve(c->dtt_geo, (size_t)nc * 32));
-  TRY(dev_reserve(c->dtt_topo, (size_t)nc * 8));
+  TRY(dev_reserve(c->dtt_topo, (size_t)nc * 16));
   TRY(hipMemsetAsync(c->g_used.ptr, 0, (size_t)(nslots + 1) * 4, s));
   c->h_u64[0] = pairs;
   c->h_u64[1] = self;
@@ -1116,7 +1116,7 @@ int traverse_given(tfmm_ctx *c, const int32_t *m2l, int64_t nm, const int32_t *p
   if (!pe.empty())
     TRY(hipMemcpyAsync(c->p2p_pairs.ptr, pe.data(), pe.size() * 8, hipMemcpyHostToDevice, s));
   TRY(launch_dtt_begin(k, (int32_t)nc, c->prm.theta, dp<double4>(c->dtt_geo),
-                       dp<int2>(c->dtt_topo), nullptr, 0, nullptr, 0, nullptr, 0, s));
+                       dp<int4>(c->dtt_topo), nullptr, 0, nullptr, 0, nullptr, 0, s));
   TRY(launch_pair_slots(dp<int2>(c->m2l_pairs), (uint32_t)me.size(), dp<double4>(c->dtt_geo),
                         k.depth, k.width, dp<int32_t>(c->slot_of), dp<uint32_t>(c->g_used),
                         dp<uint32_t>(c->g_used) + nslots, s));
@@ -1577,7 +1577,7 @@ void plan_make(tfmm_ctx *c) {
   pl.step_grid.resize(pl.nsteps);
   for (int st = 0; st < pl.nsteps; st++) {
     const int64_t h = st < (int)c->dtt_hint.size() ? c->dtt_hint[st] : 0;
-    pl.step_grid[st] = (uint32_t)std::min<int64_t>(UINT32_MAX / 4, more(h, 4096));
+    pl.step_grid[st] = (uint32_t)std::min<int64_t>(UINT32_MAX / 16, more(h, 1024));
     fmax = std::max<int64_t>(fmax, pl.step_grid[st]);
   }
   auto cap32 = [](int64_t v) { return (uint32_t)std::min<int64_t>(UINT32_MAX / 4, v); };
@@ -1642,7 +1642,7 @@ int plan_reserve(tfmm_ctx *c) {
   // traversal and P2P list
   TRY(dev_reserve(c->cnt, (size_t)pl.cwords * 4));
   TRY(dev_reserve(c->dtt_geo, cells * 32));
-  TRY(dev_reserve(c->dtt_topo, cells * 8));
+  TRY(dev_reserve(c->dtt_topo, cells * 16));
   TRY(dev_reserve(c->g_used, (size_t)(pl.nslots + 1) * 4));
   TRY(dev_reserve(c->m2l_pairs, nm * 8));
   TRY(dev_reserve(c->slot_of, nm * 4));
@@ -1813,14 +1813,14 @@ int whole_record(tfmm_ctx *c) {
   // traversal
   uint32_t *cnt = dp<uint32_t>(c->cnt);
   uint32_t *used = dp<uint32_t>(c->g_used);
-  TRY(launch_dtt_begin(k, cells, pl.prm.theta, dp<double4>(c->dtt_geo), dp<int2>(c->dtt_topo),
+  TRY(launch_dtt_begin(k, cells, pl.prm.theta, dp<double4>(c->dtt_geo), dp<int4>(c->dtt_topo),
                        used, pl.nslots + 1, cnt, pl.cwords, dp<int2>(c->front_a), np, s));
   DevBuf *fa = &c->front_a, *fb = &c->front_b;
   for (int st = 0; st < pl.nsteps; st++) {
     TRY(launch_dtt_step(dp<int2>(*fa), cnt + 16 + st, pl.step_grid[st], dp<int2>(*fb),
                         pl.caps.front, cnt + 16 + st + 1, dp<int2>(c->m2l_pairs), pl.caps.m2l,
                         dp<int2>(c->p2p_pairs), pl.caps.p2p, cnt, dp<double4>(c->dtt_geo),
-                        dp<int2>(c->dtt_topo), k.depth, k.width, dp<int32_t>(c->slot_of), used,
+                        dp<int4>(c->dtt_topo), pl.prm.theta, dp<int32_t>(c->slot_of), used,
                         used + pl.nslots, pl.prm.mutual, s));
     std::swap(fa, fb);
   }

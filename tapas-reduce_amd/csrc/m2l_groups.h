@@ -68,19 +68,23 @@ __host__ __device__ constexpr int mirror_sign(int d, int r) {
   return d == 2 ? (n + m) & 1 : d == 1 ? r & 1 : (m + r) & 1;
 }
 
-// slot of an M2L pair (target t, source s) from the cells' depths, widths
-// (max over the dimensions) and centres: the offset in half widths of the
-// finer cell; -1 outside the table
+// slot of an M2L pair from the cells' depths and the offset of target less source
+// in half widths of the finer cell, up to rounding; -1 outside the table
+__device__ inline int32_t offset_slot(int lt, int ls, const double *v) {
+  int o[3];
+  for (int d = 0; d < 3; d++) {
+    if (!(fabs(v[d]) < 64.0)) return -1;
+    o[d] = (int)rint(v[d]);
+  }
+  return group_slot(lt, ls, o);
+}
+
+// the same from the cells' depths, widths (max over the dimensions) and centres
 __device__ inline int32_t pair_slot(int lt, int ls, double wt, double ws, const double *ct,
                                     const double *cs) {
   const double half = 0.5 * fmin(wt, ws);
-  int o[3];
-  for (int d = 0; d < 3; d++) {
-    const double v = (ct[d] - cs[d]) / half;
-    if (!(fabs(v) < 64.0)) return -1;
-    o[d] = (int)rint(v);
-  }
-  return group_slot(lt, ls, o);
+  const double v[3] = {(ct[0] - cs[0]) / half, (ct[1] - cs[1]) / half, (ct[2] - cs[2]) / half};
+  return offset_slot(lt, ls, v);
 }
 
 }  // namespace m2lg

@@ -179,18 +179,18 @@ struct DttCounters {
 };
 // per-cell records the traversal steps read (geo: centre + MAC radius)
 // (per-cell records, the counters and flags cleared, the first frontier)
-hipError_t launch_dtt_begin(Cells c, int32_t ncells, double theta, double4 *geo, int2 *topo,
+hipError_t launch_dtt_begin(Cells c, int32_t ncells, double theta, double4 *geo, int4 *topo,
                             uint32_t *used, int32_t nused, uint32_t *cnt, int32_t cwords,
                             int2 *front, int nroots, hipStream_t s, bool periodic = false);
-// One breadth-first traversal step.  Every M2L pair stored also gets its
+// One breadth-first traversal step; nin_max, out_cap and the counts are frontier
+// entries, each up to eight pairs.  Every M2L pair stored also gets its
 // group-table slot (m2l_slot, -1 outside the table), marks used[slot] and
 // counts the pairs outside the table in *n_outside.
 hipError_t launch_dtt_step(const int2 *in, const uint32_t *nin_dev, uint32_t nin_max, int2 *out,
                            uint32_t out_cap, uint32_t *nout, int2 *m2l, uint32_t m2l_cap,
                            int2 *p2p, uint32_t p2p_cap, uint32_t *cnt, const double4 *geo,
-                           const int2 *topo, const int32_t *depth, const double *width,
-                           int32_t *m2l_slot, uint32_t *used, uint32_t *n_outside, int mutual,
-                           hipStream_t s, double cycle = 0);
+                           const int4 *topo, double theta, int32_t *m2l_slot, uint32_t *used,
+                           uint32_t *n_outside, int mutual, hipStream_t s, double cycle = 0);
 // group-table slots of M2L pairs given from outside the traversal
 hipError_t launch_pair_slots(const int2 *pairs, uint32_t n, const double4 *geo,
                              const int32_t *depth, const double *width, int32_t *slot,

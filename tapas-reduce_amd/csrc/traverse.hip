@@ -30,9 +30,15 @@
 // operation order, so every decision is bit-identical to the reference's.
 //
 // The step reads each cell through one 32-byte record (centre, MAC radius R)
-// and one 8-byte record (first child, body count), built once per traversal,
-// instead of six separate arrays: the traversal gathers cells at random, so
-// the number of cache lines a pair touches sets its cost.
+// and one 16-byte record (first child, body count, depth), built once per
+// traversal, instead of six separate arrays: the traversal gathers cells at
+// random, so the number of cache lines a pair touches sets its cost.
+//
+// A frontier holds split pairs, not their eight successors: an entry names the
+// cell that stays, the first child of the one that was split, and which of them
+// (ENTRY_*), and the next step's eight threads of the entry are its successors.
+// The frontier is an eighth of what it would be, and is written and read in
+// whole lines.
 #include <algorithm>
 
 #include "m2l_groups.h"
@@ -47,11 +53,11 @@ constexpr int DTT_WAVES = DTT_THREADS / 64;
 constexpr uint32_t DTT_ONE = 1 << 19;  // frontiers up to this take one pair per thread
 
 // The traversal's start: per-cell records (centre, R) with R = (width / 2 *
-// 1.00001) / theta (tapas_exafmm.cxx:222-226) and (first child, body count); with
+// 1.00001) / theta (tapas_exafmm.cxx:222-226) and (first child, body count, depth); with
 // cnt also the cleared group flags (nused words) and counters (cwords words), and
 // the first frontier, its size in cnt[16]: every root with itself, or with periodic
 // images the one root with each of its 27 images (EX/include/traversal.h:256-266).
-__global__ void k_dtt_begin(Cells c, int32_t ncells, double theta, double4 *geo, int2 *topo,
+__global__ void k_dtt_begin(Cells c, int32_t ncells, double theta, double4 *geo, int4 *topo,
                             uint32_t *used, int32_t nused, uint32_t *cnt, int32_t cwords,
                             int2 *front, int nroots, int periodic) {
 #pragma clang fp contract(off)
@@ -68,54 +74,73 @@ __global__ void k_dtt_begin(Cells c, int32_t ncells, double theta, double4 *geo,
   R = (R / 2 * 1.00001) / theta;
   geo[i] = make_double4(c.center[3 * (int64_t)i], c.center[3 * (int64_t)i + 1],
                         c.center[3 * (int64_t)i + 2], R);
-  topo[i] = make_int2(c.child[i], c.nb[i]);
+  topo[i] = make_int4(c.child[i], c.nb[i], c.depth[i], 0);
 }
 
-// Kind of a frontier pair after the MAC: what the step emits for it.
+// Kind of a pair after the MAC: what the step emits for it.
 enum : int { DK_NONE = 0, DK_M2L, DK_FAR_EMPTY, DK_P2P, DK_SPLIT_I, DK_SPLIT_J, DK_SPLIT_BOTH };
 
-// DTT_PPT: frontier pairs per thread (launch_dtt_step chooses)
-template <int DTT_PPT>
-__global__ __launch_bounds__(DTT_THREADS) void k_dtt_step(const int2 *in, const uint32_t *nin_dev,
-                                                  uint32_t nin_max, int2 *out, uint32_t out_cap,
-                                                  uint32_t *nout, int2 *m2l, uint32_t m2l_cap,
-                                                  int2 *p2p, uint32_t p2p_cap, uint32_t *cnt,
-                                                  const double4 *geo, const int2 *topo,
-                                                  const int32_t *depth, const double *width,
-                                                  int32_t *m2l_slot, uint32_t *used,
-                                                  uint32_t *n_outside, int mutual, double cycle) {
+// Kind of a frontier entry (x, y), in the top two bits of x: the pair itself
+// (roots), the children x .. x + 7 with y, x with the children y .. y + 7, or of
+// those only the ones from x on (a cell with itself under mutual).
+enum : uint32_t { ENTRY_PAIR = 0, ENTRY_I, ENTRY_J, ENTRY_UPPER };
+constexpr int ENTRY_SHIFT = 30;
+static_assert(CELL_MASK < 1u << ENTRY_SHIFT, "a cell and the kind share a word");
+
+// PPT: pairs per thread (launch_dtt_step chooses).  inv_half: 1.00001 / theta, over
+// R half the inverse of half a cell's width.
+template <int PPT, bool MUTUAL>
+__global__ __launch_bounds__(DTT_THREADS) __attribute__((amdgpu_waves_per_eu(MUTUAL ? 4 : 8)))
+void k_dtt_step(
+    const int2 *in, const uint32_t *nin_dev, uint32_t nin_max, int2 *out, uint32_t out_cap,
+    uint32_t *nout, int2 *m2l, uint32_t m2l_cap, int2 *p2p, uint32_t p2p_cap, uint32_t *cnt,
+    const double4 *geo, const int4 *topo, double inv_half, int32_t *m2l_slot, uint32_t *used,
+    uint32_t *n_outside, double cycle) {
 #pragma clang fp contract(off)
-  const uint32_t nin = nin_dev ? *nin_dev : nin_max;
+  const uint32_t nin = min(nin_dev ? *nin_dev : nin_max, nin_max);
+  const uint32_t block_first = blockIdx.x * (DTT_THREADS / 8) * PPT;
+  if (block_first >= nin) return;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
-  // Each thread takes DTT_PPT pairs (rows r: pair blockIdx.x * DTT_THREADS *
-  // DTT_PPT + r * DTT_THREADS + threadIdx.x).  Pass 1 classifies them and
-  // counts the block's appends to the four lists (0 next frontier, 8 entries
-  // per pair; 1 executed M2L; 2 P2P; 3 all M2L, counted only) per row and
-  // wave; one global atomic per list per block reserves the block's ranges
-  // (same-address atomics are what bound this kernel); pass 2 writes.
-  __shared__ uint32_t wc[DTT_PPT][DTT_WAVES][5];
+  // Thread t's row r is successor t % 8 of an entry.  Pass 1 classifies the pairs
+  // and counts the block's appends to the four lists (0 next frontier; 1 executed
+  // M2L; 2 P2P; 3 all M2L, counted only; 4 P2P calls) per row and wave; one global
+  // atomic per list per block reserves the block's ranges (same-address atomics
+  // bound this kernel with more of them); pass 2 writes.  The group flags of the
+  // block's M2L pairs are gathered in LDS: millions of stores to the same few lines
+  // otherwise.
+  constexpr int FLAGS = (m2lg::SLOTS + 31) / 32;
+  __shared__ uint32_t wc[PPT][DTT_WAVES][5];
   __shared__ unsigned long long ws[DTT_WAVES][2];
-  int32_t pi[DTT_PPT], pj[DTT_PPT], kind[DTT_PPT], fch[DTT_PPT], grp[DTT_PPT], grp2[DTT_PPT];
-  bool dbl[DTT_PPT];
+  __shared__ uint32_t flags[FLAGS];
+  for (int i = threadIdx.x; i < FLAGS; i += DTT_THREADS) flags[i] = 0;
+  int32_t pi[PPT], pj[PPT], kind[PPT], arg[PPT], arg2[PPT];  // arg: first child, or group slot
   unsigned long long v = 0, self = 0;
 #pragma unroll
-  for (int r = 0; r < DTT_PPT; r++) {
-    const uint32_t t = (blockIdx.x * DTT_PPT + r) * DTT_THREADS + threadIdx.x;
-    const bool valid = t < nin && t < nin_max;
-    int32_t i = 0, j = 0, k = DK_NONE, f = 0, g = -1, g2 = -1;
+  for (int r = 0; r < PPT; r++) {
+    const uint32_t e = block_first + (uint32_t)r * (DTT_THREADS / 8) + (threadIdx.x >> 3);
+    const int l = threadIdx.x & 7;
+    int32_t i = 0, j = 0, k = DK_NONE, f = -1, f2 = -1;
     bool two = false;  // the pair's entries go into the lists in both directions
+    bool valid = e < nin;
     if (valid) {
-      const int2 pr = in[t];
-      i = pr.x;
-      j = pr.y;  // source cell and image (periodic images)
+      const int2 en = in[e];
+      const uint32_t what = (uint32_t)en.x >> ENTRY_SHIFT;
+      i = (int32_t)((uint32_t)en.x & ((1u << ENTRY_SHIFT) - 1u));
+      j = en.y;  // source cell and image (periodic images)
+      if (what == ENTRY_PAIR) valid = l == 0;
+      else if (what == ENTRY_I) i += l;
+      else j += l;
+      if (MUTUAL && what == ENTRY_UPPER) valid = j >= i;
+    }
+    if (valid) {
       const int32_t jc = (int32_t)((uint32_t)j & CELL_MASK);
       const uint32_t img = (uint32_t)j >> IMG_SHIFT;
+      const double4 gi = geo[i], gj = geo[jc];
+      const int4 ti = topo[i], tj = topo[jc];
       double sx, sy, sz;
       image_shift(img, cycle, sx, sy, sz);
       const bool same = i == jc && (cycle == 0 || img == IMG_CENTRE);  // a cell with itself
-      const double4 gi = geo[i], gj = geo[jc];
-      const int2 ti = topo[i], tj = topo[jc];
       // dX = Xi - Xj - Xperiodic (EX/include/traversal.h:37)
       const double d0 = gi.x - gj.x - sx;
       const double d1 = gi.y - gj.y - sy;
@@ -129,19 +154,19 @@ __global__ __launch_bounds__(DTT_THREADS) void k_dtt_step(const int2 *in, const 
       const bool nonempty = ti.y > 0 && tj.y > 0;
       if (R2 > (Ri + Rj) * (Ri + Rj)) {
         k = nonempty ? DK_M2L : DK_FAR_EMPTY;
-        two = mutual != 0;
-        if (nonempty) {
-          // the pair's M2L offset group (same arithmetic on the same centres
-          // as a separate pass over the list would do)
-          const double ci[3] = {gi.x, gi.y, gi.z}, cj[3] = {gj.x + sx, gj.y + sy, gj.z + sz};
-          g = m2lg::pair_slot(depth[i], depth[jc], width[i], width[jc], ci, cj);
-          if (two) g2 = m2lg::pair_slot(depth[jc], depth[i], width[jc], width[i], cj, ci);
+        two = MUTUAL;
+        if (nonempty) {  // the pair's M2L offset group
+          // (an R too small for its digits says nothing: outside the table)
+          const double rmin = fmin(Ri, Rj), ih = rmin < 2.3e-308 ? INFINITY : inv_half / rmin;
+          const double o[3] = {d0 * ih, d1 * ih, d2 * ih}, b[3] = {-o[0], -o[1], -o[2]};
+          f = m2lg::offset_slot(ti.z, tj.z, o);
+          if (two) f2 = m2lg::offset_slot(tj.z, ti.z, b);
         }
       } else if (leaf_i && leaf_j) {
         if (nonempty) {
           k = DK_P2P;
-          two = mutual != 0 && !same;
-          if (mutual != 0 && same) {
+          two = MUTUAL && !same;
+          if (MUTUAL && same) {
             v += (unsigned long long)ti.y * (unsigned long long)(ti.y + 1) / 2;
           } else {
             v += (unsigned long long)ti.y * (unsigned long long)tj.y;
@@ -154,7 +179,7 @@ __global__ __launch_bounds__(DTT_THREADS) void k_dtt_step(const int2 *in, const 
       } else if (leaf_i) {
         k = DK_SPLIT_J;
         f = tj.x | (int32_t)(img << IMG_SHIFT);
-      } else if (mutual != 0 && same) {
+      } else if (MUTUAL && same) {
         k = DK_SPLIT_BOTH;
         f = ti.x;
       } else if (Ri >= Rj) {
@@ -167,18 +192,16 @@ __global__ __launch_bounds__(DTT_THREADS) void k_dtt_step(const int2 *in, const 
     }
     pi[r] = i;
     pj[r] = j;
-    kind[r] = k;
-    fch[r] = f;
-    grp[r] = g;
-    grp2[r] = g2;
-    dbl[r] = two;
+    kind[r] = k | (two ? 8 : 0);
+    arg[r] = f;
+    arg2[r] = f2;
     const uint64_t m0 = __ballot(k == DK_SPLIT_I || k == DK_SPLIT_J);
-    const uint64_t m0b = __ballot(k == DK_SPLIT_BOTH);
-    const uint64_t m1 = __ballot(k == DK_M2L), m1d = __ballot(k == DK_M2L && two);
-    const uint64_t m2 = __ballot(k == DK_P2P), m2d = __ballot(k == DK_P2P && two);
+    const uint64_t m0b = MUTUAL ? __ballot(k == DK_SPLIT_BOTH) : 0;
+    const uint64_t m1 = __ballot(k == DK_M2L), m1d = MUTUAL ? __ballot(k == DK_M2L && two) : 0;
+    const uint64_t m2 = __ballot(k == DK_P2P), m2d = MUTUAL ? __ballot(k == DK_P2P && two) : 0;
     const uint64_t m3 = __ballot(k == DK_M2L || k == DK_FAR_EMPTY);
     if (lane == 0) {
-      wc[r][wid][0] = (uint32_t)__popcll(m0) * 8u + (uint32_t)__popcll(m0b) * 36u;
+      wc[r][wid][0] = (uint32_t)__popcll(m0) + (uint32_t)__popcll(m0b) * 8u;
       wc[r][wid][1] = (uint32_t)(__popcll(m1) + __popcll(m1d));
       wc[r][wid][2] = (uint32_t)(__popcll(m2) + __popcll(m2d));
       wc[r][wid][3] = (uint32_t)__popcll(m3);
@@ -199,10 +222,10 @@ __global__ __launch_bounds__(DTT_THREADS) void k_dtt_step(const int2 *in, const 
   if (threadIdx.x < 5) {
     const int q = threadIdx.x;
     uint32_t tot = 0;
-    for (int r = 0; r < DTT_PPT; r++)
+    for (int r = 0; r < PPT; r++)
       for (int w = 0; w < DTT_WAVES; w++) tot += wc[r][w][q];
     uint32_t run = tot ? atomicAdd(q == 0 ? nout : &cnt[q], tot) : 0u;
-    for (int r = 0; r < DTT_PPT; r++)
+    for (int r = 0; r < PPT; r++)
       for (int w = 0; w < DTT_WAVES; w++) {
         const uint32_t c = wc[r][w][q];
         wc[r][w][q] = run;
@@ -221,24 +244,25 @@ __global__ __launch_bounds__(DTT_THREADS) void k_dtt_step(const int2 *in, const 
   __syncthreads();
   uint32_t outside = 0;
 #pragma unroll
-  for (int r = 0; r < DTT_PPT; r++) {
-    const int k = kind[r];
+  for (int r = 0; r < PPT; r++) {
+    const int k = kind[r] & 7;
     const int32_t i = pi[r], j = pj[r];
-    const bool two = dbl[r];
+    const bool two = MUTUAL && (kind[r] & 8);
     const bool split = k == DK_SPLIT_I || k == DK_SPLIT_J;
-    const uint64_t m0 = __ballot(split), m0b = __ballot(k == DK_SPLIT_BOTH);
-    const uint64_t m1 = __ballot(k == DK_M2L), m1d = __ballot(k == DK_M2L && two);
-    const uint64_t m2 = __ballot(k == DK_P2P), m2d = __ballot(k == DK_P2P && two);
+    const uint64_t m0 = __ballot(split), m0b = MUTUAL ? __ballot(k == DK_SPLIT_BOTH) : 0;
+    const uint64_t m1 = __ballot(k == DK_M2L), m1d = MUTUAL ? __ballot(k == DK_M2L && two) : 0;
+    const uint64_t m2 = __ballot(k == DK_P2P), m2d = MUTUAL ? __ballot(k == DK_P2P && two) : 0;
     if (k == DK_M2L) {
       const uint32_t sl =
           wc[r][wid][1] + (uint32_t)(__popcll(m1 & lt) + __popcll(m1d & lt));
       for (int e = 0; e < (two ? 2 : 1); e++) {
-        const int32_t ge = e ? grp2[r] : grp[r];
+        const int32_t ge = e ? arg2[r] : arg[r];
         if (sl + e < m2l_cap) {
           m2l[sl + e] = e ? make_int2(j, i) : make_int2(i, j);
           m2l_slot[sl + e] = ge;
-          if (ge >= 0) used[ge >> m2lg::MIRROR_BITS] = 1u;
-          else outside++;
+          const int32_t g = ge >> m2lg::MIRROR_BITS;
+          if (ge < 0) outside++;
+          else if (!(flags[g >> 5] >> (g & 31) & 1u)) atomicOr(&flags[g >> 5], 1u << (g & 31));
         }
       }
     } else if (k == DK_P2P) {
@@ -248,25 +272,23 @@ __global__ __launch_bounds__(DTT_THREADS) void k_dtt_step(const int2 *in, const 
       if (two && sl + 1 < p2p_cap) p2p[sl + 1] = make_int2(j, i);
     } else if (split || k == DK_SPLIT_BOTH) {
       const uint32_t sl =
-          wc[r][wid][0] + (uint32_t)__popcll(m0 & lt) * 8u + (uint32_t)__popcll(m0b & lt) * 36u;
-      const int32_t f = fch[r];
+          wc[r][wid][0] + (uint32_t)__popcll(m0 & lt) + (uint32_t)__popcll(m0b & lt) * 8u;
+      const int32_t f = arg[r];
       if (k == DK_SPLIT_BOTH) {
-        if (sl + 36 <= out_cap) {
-          uint32_t o = sl;
-          for (int a = 0; a < 8; a++)
-            for (int b = a; b < 8; b++) out[o++] = make_int2(f + a, f + b);
-        }
-      } else if (sl + 8 <= out_cap) {
-        if (k == DK_SPLIT_I) {
-          for (int c = 0; c < 8; c++) out[sl + c] = make_int2(f + c, j);
-        } else {
-          for (int c = 0; c < 8; c++) out[sl + c] = make_int2(i, f + c);
-        }
+        for (int a = 0; a < 8; a++)
+          if (sl + a < out_cap)
+            out[sl + a] = make_int2((int32_t)((uint32_t)(f + a) | ENTRY_UPPER << ENTRY_SHIFT), f);
+      } else if (sl < out_cap) {
+        out[sl] = k == DK_SPLIT_I ? make_int2((int32_t)((uint32_t)f | ENTRY_I << ENTRY_SHIFT), j)
+                                  : make_int2((int32_t)((uint32_t)i | ENTRY_J << ENTRY_SHIFT), f);
       }
     }
   }
   for (int o = 32; o > 0; o >>= 1) outside += __shfl_xor(outside, o, 64);
   if (lane == 0 && outside) atomicAdd(n_outside, outside);
+  __syncthreads();
+  for (int i = threadIdx.x; i < FLAGS; i += DTT_THREADS)
+    for (uint32_t m = flags[i]; m; m &= m - 1) used[32 * i + __ffs((int)m) - 1] = 1u;
 }
 
 // Group-table slots of M2L pairs that come from outside the traversal (the
@@ -472,7 +494,7 @@ hipError_t launch_csr_sorted_sources(const uint32_t *tgt, const uint32_t *in, ui
   return hipGetLastError();
 }
 
-hipError_t launch_dtt_begin(Cells c, int32_t ncells, double theta, double4 *geo, int2 *topo,
+hipError_t launch_dtt_begin(Cells c, int32_t ncells, double theta, double4 *geo, int4 *topo,
                             uint32_t *used, int32_t nused, uint32_t *cnt, int32_t cwords,
                             int2 *front, int nroots, hipStream_t s, bool periodic) {
   const int32_t most = std::max(std::max(ncells, nroots), std::max(nused, std::max(cwords, 27)));
@@ -485,24 +507,27 @@ hipError_t launch_dtt_begin(Cells c, int32_t ncells, double theta, double4 *geo,
 hipError_t launch_dtt_step(const int2 *in, const uint32_t *nin_dev, uint32_t nin_max, int2 *out,
                            uint32_t out_cap, uint32_t *nout, int2 *m2l, uint32_t m2l_cap,
                            int2 *p2p, uint32_t p2p_cap, uint32_t *cnt, const double4 *geo,
-                           const int2 *topo, const int32_t *depth, const double *width,
-                           int32_t *m2l_slot, uint32_t *used, uint32_t *n_outside, int mutual,
-                           hipStream_t s, double cycle) {
+                           const int4 *topo, double theta, int32_t *m2l_slot, uint32_t *used,
+                           uint32_t *n_outside, int mutual, hipStream_t s, double cycle) {
   if (nin_max == 0) return hipSuccess;
   // Four pairs per thread spare a large frontier same-address atomics, which bound
   // it then; a smaller one they leave on a quarter of the CUs it could use, for
-  // four times the chain of gathers.  All steps of a traversal, us, at 4 / the
-  // better by size: 4,096-body cube 81 / 48, 64K ellipsoid 230 / 164, 256K Plummer
-  // 484 / 326, 500K ellipsoid 586 / 530, 1M cube 444 / 404, 4M Plummer 1,673 /
-  // 1,605; the line at 2^17 or 2^20 pairs lies between on most of them.
+  // four times the chain of gathers.  All steps of a traversal, us, with the line at
+  // 2^17, 2^19 and 2^21 pairs: 256K Plummer 257, 234, 237, 500K ellipsoid 420, 427,
+  // 444, 4M Plummer 553, 555, 591.  With the eight successors of a split written out,
+  // flags stored pair by pair and depths and widths gathered by the pairs in the
+  // group table: 484, 586 and 1,673.  64 registers, two workgroups a CU instead of
+  // one, are worth 15 % on the largest steps, spills included.
   auto go = [&](auto kernel, uint32_t ppt) {
-    const uint32_t per = DTT_THREADS * ppt;
+    const uint32_t per = DTT_THREADS / 8 * ppt;  // entries
     kernel<<<(nin_max + per - 1) / per, DTT_THREADS, 0, s>>>(
-        in, nin_dev, nin_max, out, out_cap, nout, m2l, m2l_cap, p2p, p2p_cap, cnt, geo, topo, depth,
-        width, m2l_slot, used, n_outside, mutual, cycle);
+        in, nin_dev, nin_max, out, out_cap, nout, m2l, m2l_cap, p2p, p2p_cap, cnt, geo, topo,
+        1.00001 / theta, m2l_slot, used, n_outside, cycle);
     return hipGetLastError();
   };
-  return nin_max <= DTT_ONE ? go(k_dtt_step<1>, 1) : go(k_dtt_step<4>, 4);
+  const bool one = nin_max <= DTT_ONE / 8;
+  if (mutual) return one ? go(k_dtt_step<1, true>, 1) : go(k_dtt_step<4, true>, 4);
+  return one ? go(k_dtt_step<1, false>, 1) : go(k_dtt_step<4, false>, 4);
 }
 
 hipError_t launch_pair_slots(const int2 *pairs, uint32_t n, const double4 *geo,
