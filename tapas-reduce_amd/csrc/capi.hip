@@ -346,15 +346,15 @@ int image_range(const tfmm_ctx *c) {
   for (int i = 0; i < c->images; i++, p3 *= 3) r += p3;
   return r;
 }
-// source field of the fallback M2L keys (target << FB_SRC_BITS | source word):
-// the whole 32-bit source word, cell and periodic image
-constexpr int FB_SRC_BITS = 32;
-
 int bits_for(int64_t v) {
   int b = 1;
   while (b < 62 && (((int64_t)1 << b) <= v)) b++;
   return b;
 }
+
+// source field of the fallback M2L keys (target << bits | source word): the cell,
+// with periodic images the whole 32-bit source word
+int fallback_src_bits(const tfmm_ctx *c, int cell_bits) { return c->images > 0 ? 32 : cell_bits; }
 
 int check_params(tfmm_ctx *c, const tfmm_params *p) {
   if (!p) return fail(c, TFMM_EINVAL, "params is null");
@@ -846,7 +846,7 @@ int build_m2l_batches(tfmm_ctx *c, bool given = false) {
   TRY(dev_reserve(c->g_cnt, 16));
   if (n_outside || given) TRY(hipMemsetAsync(c->g_cnt.ptr, 0, 16, s));
   const int gbits = bits_for(ngr);
-  const int sbits = bits_for(c->ncells);
+  const int sbits = bits_for(c->ncells), fbits = fallback_src_bits(c, sbits);
   {
     const int64_t nt = (c->ncells + m2l_tile_size() - 1) / m2l_tile_size();
     if (bits_for(nt) + gbits > 32 || c->ncells >= ((int64_t)1 << m2l_src_bits()))
@@ -858,7 +858,7 @@ int build_m2l_batches(tfmm_ctx *c, bool given = false) {
                                 dp<uint32_t>(c->g_gid), gbits, dp<uint32_t>(c->gkeys),
                                 dp<uint32_t>(c->gvals), s));
   } else {
-    TRY(launch_m2l_classify(dp<int2>(c->m2l_pairs), dp<int32_t>(c->slot_of), n, dp<uint32_t>(c->g_gid), gbits, FB_SRC_BITS,
+    TRY(launch_m2l_classify(dp<int2>(c->m2l_pairs), dp<int32_t>(c->slot_of), n, dp<uint32_t>(c->g_gid), gbits, fbits,
                             dp<uint32_t>(c->gkeys), dp<uint32_t>(c->gvals), dp<uint64_t>(c->fkeys),
                             dp<uint32_t>(c->fvals), dp<uint32_t>(c->g_cnt), s));
     TRY(hipMemcpyAsync(c->h_u32, c->g_cnt.ptr, 8, hipMemcpyDeviceToHost, s));
@@ -916,13 +916,13 @@ int build_m2l_batches(tfmm_ctx *c, bool given = false) {
   if (nfb) {
     bool falt = false;
     TRY(radix_sort_pairs(dp<uint64_t>(c->fkeys), dp<uint32_t>(c->fvals), dp<uint64_t>(c->fkeys_alt),
-                         dp<uint32_t>(c->fvals_alt), nfb, 0, FB_SRC_BITS + sbits, c->sort_tmp.ptr,
+                         dp<uint32_t>(c->fvals_alt), nfb, 0, fbits + sbits, c->sort_tmp.ptr,
                          s, &falt));
     const uint64_t *fk = dp<uint64_t>(falt ? c->fkeys_alt : c->fkeys);
     TRY(dev_reserve(c->fb_off, (size_t)(c->ncells + 1) * 4));
     TRY(dev_reserve(c->fb_src, (size_t)nfb * 4));
-    TRY(launch_csr_offsets(fk, nfb, FB_SRC_BITS, (int32_t)c->ncells, dp<int32_t>(c->fb_off), s));
-    TRY(launch_unpack_pairs(fk, nfb, FB_SRC_BITS, dp<int32_t>(c->fb_src), s));
+    TRY(launch_csr_offsets(fk, nfb, fbits, (int32_t)c->ncells, dp<int32_t>(c->fb_off), s));
+    TRY(launch_unpack_pairs(fk, nfb, fbits, dp<int32_t>(c->fb_src), s));
   }
   if (!c->codes_ready) {
     TRY(dev_reserve(c->codes, m2l_codes_bytes()));
@@ -1585,14 +1585,17 @@ void plan_make(tfmm_ctx *c) {
   pl.caps.m2l = cap32(more(c->n_m2l_exec, 65536));
   pl.caps.p2p = cap32(more(c->n_p2p, 65536));
   pl.caps.items = cap32(more(c->n_items, 4096));
-  pl.caps.fallback = cap32(more(c->n_fallback, 4096));
+  // none the last time: 17 launches fewer (16K cube 575 to 536 us); the first
+  // evaluation with one runs again, and the plan made after it has room for more
+  pl.caps.fallback = c->n_fallback ? cap32(more(c->n_fallback, 4096)) : 0;
   pl.groups = cap32(more(c->n_groups, 256));
   pl.ntiles = (int32_t)((pl.cells + m2l_tile_size() - 1) / m2l_tile_size());
   pl.caps.units = m2l_units_cap(pl.caps.items, pl.ntiles, c->m2l_unit_factor);
   pl.gbits = bits_for(pl.groups);
   pl.sbits = bits_for(pl.cells);
   pl.tbits = bits_for(pl.ntiles);
-  if (pl.tbits + pl.gbits > 32 || pl.cells >= ((int64_t)1 << m2l_src_bits()) || FB_SRC_BITS + pl.sbits > 64 ||
+  if (pl.tbits + pl.gbits > 32 || pl.cells >= ((int64_t)1 << m2l_src_bits()) ||
+      2 * pl.sbits > 64 ||
       (int64_t)pl.caps.fallback > (1 << 22))
     return;
   pl.valid = true;
@@ -1853,7 +1856,7 @@ int whole_record(tfmm_ctx *c) {
                                    dp<float>(c->g_y32), dp<int8_t>(c->g_dl), s, pl.groups));
     TRY(launch_fill_zero(gcnt, 16, s));
     TRY(launch_m2l_classify(dp<int2>(c->m2l_pairs), dp<int32_t>(c->slot_of), nm,
-                            dp<uint32_t>(c->g_gid), pl.gbits, FB_SRC_BITS, dp<uint32_t>(c->gkeys),
+                            dp<uint32_t>(c->g_gid), pl.gbits, pl.sbits, dp<uint32_t>(c->gkeys),
                             dp<uint32_t>(c->gvals), dp<uint64_t>(c->fkeys),
                             dp<uint32_t>(c->fvals), gcnt, s, cnt + 1, pl.groups));
     bool galt = false;
@@ -1877,14 +1880,15 @@ int whole_record(tfmm_ctx *c) {
                          dp<int2>(c->units), c->scan_tmp.ptr, s, pl.caps.units));
     // the pairs outside the groups (appended compactly): at most the
     // fallback capacity of them are sorted
-    const uint32_t nfb = std::min<uint32_t>(nm, pl.caps.fallback);
-    bool falt = false;
-    TRY(radix_sort_pairs(dp<uint64_t>(c->fkeys), dp<uint32_t>(c->fvals), dp<uint64_t>(c->fkeys_alt),
-                         dp<uint32_t>(c->fvals_alt), nfb, 0, FB_SRC_BITS + pl.sbits, c->sort_tmp.ptr, s,
-                         &falt, gcnt + 1));
-    const uint64_t *fk = dp<uint64_t>(falt ? c->fkeys_alt : c->fkeys);
-    TRY(launch_csr_offsets(fk, nfb, FB_SRC_BITS, cells, dp<int32_t>(c->fb_off), s, gcnt + 1));
-    TRY(launch_unpack_pairs(fk, nfb, FB_SRC_BITS, dp<int32_t>(c->fb_src), s, gcnt + 1));
+    if (const uint32_t nfb = std::min<uint32_t>(nm, pl.caps.fallback)) {
+      bool falt = false;
+      TRY(radix_sort_pairs(dp<uint64_t>(c->fkeys), dp<uint32_t>(c->fvals),
+                           dp<uint64_t>(c->fkeys_alt), dp<uint32_t>(c->fvals_alt), nfb, 0,
+                           2 * pl.sbits, c->sort_tmp.ptr, s, &falt, gcnt + 1));
+      const uint64_t *fk = dp<uint64_t>(falt ? c->fkeys_alt : c->fkeys);
+      TRY(launch_csr_offsets(fk, nfb, pl.sbits, cells, dp<int32_t>(c->fb_off), s, gcnt + 1));
+      TRY(launch_unpack_pairs(fk, nfb, pl.sbits, dp<int32_t>(c->fb_src), s, gcnt + 1));
+    }
     TRY(launch_m2l_group_afrag(mixed ? (const void *)c->g_y32.ptr : (const void *)c->g_y64.ptr,
                                pl.groups, dp<uint32_t>(c->codes), dp<int8_t>(c->g_dl),
                                c->g_af.ptr, mixed, s, sz + SZ_NG));

@@ -85,7 +85,8 @@ __global__ void k_list_targets(const int32_t *off, int32_t ncells, int32_t npair
 }
 
 // L_t += partials of t's pairs within the chunk [p0, p1), in list order; one
-// wave per target
+// wave per target.  The longest list is the kernel's time, one load after another;
+// eight in flight: 500K ellipsoid (7,230 pairs) 116 to 23 us.
 __global__ __launch_bounds__(256) void k_m2l_reduce(Csr list, int32_t ncells, int32_t p0,
                                                     int32_t p1, const cd *part, double *L) {
   critical_path_priority();
@@ -95,7 +96,16 @@ __global__ __launch_bounds__(256) void k_m2l_reduce(Csr list, int32_t ncells, in
   const int32_t b = max(list.off[ti], p0), e = min(list.off[ti + 1], p1);
   if (b >= e) return;
   cd acc = mk(0, 0);
-  for (int32_t p = b; p < e; p++) acc = cadd(acc, part[(int64_t)(p - p0) * NTERM + lane]);
+  const cd *v = part + (int64_t)(b - p0) * NTERM + lane;
+  int32_t p = b;
+  for (; p + 8 <= e; p += 8, v += 8 * NTERM) {
+    cd t[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) t[i] = v[i * NTERM];
+#pragma unroll
+    for (int i = 0; i < 8; i++) acc = cadd(acc, t[i]);
+  }
+  for (; p < e; p++, v += NTERM) acc = cadd(acc, *v);
   cd *Li = reinterpret_cast<cd *>(L) + (int64_t)ti * NTERM;
   Li[lane] = cadd(Li[lane], acc);
 }
