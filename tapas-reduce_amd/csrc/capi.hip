@@ -140,7 +140,7 @@ struct tfmm_ctx {
   int p2p_waves = 0;             // resident P2P waves per SIMD (0: one workgroup per cell)
   int run_schedule = 0, run_waves = 0;  // the two as the running evaluation takes them
   int n_cu = 0;                  // compute units of the device
-  DevBuf p2p_next;               // the resident P2P's work counter
+  DevBuf p2p_next, p2p_order;    // the resident P2P's counters and targets
   int ext_events = -1;           // external event records in a capture: -1 not probed
   bool fused = false;            // last evaluation ran the fused order
   bool capturing = false;        // inside the numeric phase's stream capture
@@ -275,7 +275,7 @@ std::vector<DevBuf *> all_buffers(tfmm_ctx *c) {
           &c->feat_acc, &c->feat_x, &c->feat_out, &c->d_prob_off, &c->bprob,
           &c->pkey, &c->pkey_alt, &c->ppos, &c->ppos_alt, &c->brec, &c->lev,
           &c->lev_bsum, &c->lev_status, &c->dtt_geo, &c->dtt_topo, &c->u_cnt,
-          &c->u_off, &c->units, &c->u_part, &c->p2p_next, &c->finite_flag, &c->gsz, &c->gstep,
+          &c->u_off, &c->units, &c->u_part, &c->p2p_next, &c->p2p_order, &c->finite_flag, &c->gsz, &c->gstep,
           &c->pflag, &c->cart_tab, &c->Mc, &c->Lc, &c->seg_long};
 }
 
@@ -337,6 +337,18 @@ int cart_tables(tfmm_ctx *c) {
 }
 
 // waves that share a target leaf of the P2P
+// Resident waves take the leaves of at least the average's work (bodies times source
+// leaves, by the last traversal) first, or a long one that is taken late is the end
+// of the evaluation.  Evaluations, ms, in the cells' order / from 1, 2, 3, 5 times
+// the average: 4M Plummer 10.85 / 10.43, 10.63, 10.81, 10.98, two clusters of 8M
+// 19.05 / 18.74, 18.78, 19.17, 19.18, 256 problems 12.29 / 12.27, 12.30, 11.98,
+// 12.32, 1M cube 4.28 / 4.13, 4.16, 4.17, 4.19.
+P2pQueue p2p_queue(tfmm_ctx *c) {
+  const double leaves = (double)std::max<int64_t>(c->nleaves, 1);
+  return {dp<uint32_t>(c->p2p_next), dp<int32_t>(c->p2p_order),
+          (float)(c->n / leaves * (c->n_p2p / leaves))};
+}
+
 int leaf_waves(const tfmm_ctx *c) { return p2p_waves_per_leaf(c->n, c->prm.ncrit); }
 
 // the direct sum's image range for the image sublevels (the reference's
@@ -963,6 +975,7 @@ int run_lists(tfmm_ctx *c, bool given = false) {
   // VALU) and the M2L (MFMA) share the CUs.  Joined before the
   // downward pass.
   TRY(dev_reserve(c->acc, (size_t)c->n * 32));
+  TRY(dev_reserve(c->p2p_order, (size_t)c->ncells * 4));
   auto launch_p2p = [&]() -> int {
     TRY(hipEventRecord(c->ev[EV_P2PREADY], s));
     TRY(hipStreamWaitEvent(c->side, c->ev[EV_P2PREADY], 0));
@@ -970,11 +983,11 @@ int run_lists(tfmm_ctx *c, bool given = false) {
     Csr pl{dp<int32_t>(c->p2p_off), dp<int32_t>(c->p2p_src)};
     if (mixed)
       TRY(launch_p2p_fp32(k, (int32_t)c->ncells, pl, sorted_bodies(c), dp<float4>(c->relpos),
-                          dp<double>(c->acc), leaf_waves(c), p2p_resident(c), dp<uint32_t>(c->p2p_next),
-                          c->side, period(c)));
+                          dp<double>(c->acc), leaf_waves(c), p2p_resident(c), p2p_queue(c), c->side,
+                          period(c)));
     else
       TRY(launch_p2p_fp64(k, (int32_t)c->ncells, pl, sorted_bodies(c), dp<double>(c->acc), leaf_waves(c),
-                          p2p_resident(c), dp<uint32_t>(c->p2p_next), c->side, period(c)));
+                          p2p_resident(c), p2p_queue(c), c->side, period(c)));
     TRY(hipEventRecord(c->ev[EV_P2P1], c->side));
     return TFMM_OK;
   };
@@ -1191,22 +1204,22 @@ void probe_external_events(tfmm_ctx *c) {
 // A resident P2P holds few waves so that the kernels of the critical path
 // find room beside it.  When those are done, nothing is left to make room for: a
 // full-occupancy launch of the same kernel on the context stream then takes the
-// target cells still left on its counter, after the L2L, or with schedule 3
+// target cells still left in its queue, after the L2L, or with schedule 3
 // already once the set kernel is done.  (Two clusters of 4M bodies, mixed, 3
 // resident waves: 19.9 ms with the drain, 20.3 without, where the 3 waves
 // ended alone.)
 bool p2p_drains(const tfmm_ctx *c) { return c->run_schedule != 4 && c->run_waves > 0; }
 
-// one launch of resident waves on the shared counter
+// one launch of resident waves on the shared queue
 hipError_t p2p_on_counter(tfmm_ctx *c, int64_t ncells, int waves, hipStream_t st) {
   const Cells k = cells_of(c);
   Csr pl{dp<int32_t>(c->p2p_off), dp<int32_t>(c->p2p_src)};
   if (c->prm.precision == TFMM_MIXED)
     return launch_p2p_fp32_drain(k, (int32_t)ncells, pl, sorted_bodies(c), dp<float4>(c->relpos),
-                                 dp<double>(c->acc), leaf_waves(c), waves,
-                                 dp<uint32_t>(c->p2p_next), st, period(c));
+                                 dp<double>(c->acc), leaf_waves(c), waves, p2p_queue(c), st,
+                                 period(c));
   return launch_p2p_fp64_drain(k, (int32_t)ncells, pl, sorted_bodies(c), dp<double>(c->acc),
-                               leaf_waves(c), waves, dp<uint32_t>(c->p2p_next), st, period(c));
+                               leaf_waves(c), waves, p2p_queue(c), st, period(c));
 }
 
 int drain_p2p(tfmm_ctx *c, int64_t ncells, bool l2l_done) {
@@ -1240,9 +1253,11 @@ int fork_p2p(tfmm_ctx *c, int64_t ncells = -1) {
   hipStream_t s = c->stream;
   const Cells k = cells_of(c);
   if (ncells < 0) ncells = c->ncells;
-  // the launches on the counter share it: cleared on this stream, before either
-  // can take from it
-  if (p2p_drains(c)) TRY(launch_fill_zero(c->p2p_next.ptr, 4, s));
+  // the launches on the queue share it: made on this stream, before either can take
+  // from it
+  Csr pl{dp<int32_t>(c->p2p_off), dp<int32_t>(c->p2p_src)};
+  TRY(dev_reserve(c->p2p_order, (size_t)ncells * 4));
+  if (p2p_drains(c)) TRY(launch_p2p_order(k, (int32_t)ncells, pl, p2p_queue(c), s));
   // schedule 4: on the context stream, alone (the kernel's own time)
   hipStream_t ps = c->run_schedule == 4 ? s : c->side;
   if (ps != s) {
@@ -1251,16 +1266,14 @@ int fork_p2p(tfmm_ctx *c, int64_t ncells = -1) {
   }
   TRY(rec(c, EV_P2P0, ps));
   const int resident = c->run_waves > 0 ? c->run_waves * 4 * c->n_cu : 0;
-  Csr pl{dp<int32_t>(c->p2p_off), dp<int32_t>(c->p2p_src)};
   if (p2p_drains(c))
     TRY(p2p_on_counter(c, ncells, resident, ps));
   else if (c->prm.precision == TFMM_MIXED)
     TRY(launch_p2p_fp32(k, (int32_t)ncells, pl, sorted_bodies(c), dp<float4>(c->relpos),
-                        dp<double>(c->acc), leaf_waves(c), resident, dp<uint32_t>(c->p2p_next), ps,
-                        period(c)));
+                        dp<double>(c->acc), leaf_waves(c), resident, p2p_queue(c), ps, period(c)));
   else
     TRY(launch_p2p_fp64(k, (int32_t)ncells, pl, sorted_bodies(c), dp<double>(c->acc),
-                        leaf_waves(c), resident, dp<uint32_t>(c->p2p_next), ps, period(c)));
+                        leaf_waves(c), resident, p2p_queue(c), ps, period(c)));
   TRY(rec(c, EV_P2P1, ps));
   TRY(hipEventRecord(c->ev[EV_P2PJOIN], ps));
   return TFMM_OK;
@@ -1647,6 +1660,7 @@ int plan_reserve(tfmm_ctx *c) {
   TRY(dev_reserve(c->dtt_geo, cells * 32));
   TRY(dev_reserve(c->dtt_topo, cells * 16));
   TRY(dev_reserve(c->g_used, (size_t)(pl.nslots + 1) * 4));
+  TRY(dev_reserve(c->p2p_order, cells * 4));
   TRY(dev_reserve(c->m2l_pairs, nm * 8));
   TRY(dev_reserve(c->slot_of, nm * 4));
   TRY(dev_reserve(c->p2p_pairs, npp * 8));

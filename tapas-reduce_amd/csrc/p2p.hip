@@ -405,22 +405,40 @@ __global__ __launch_bounds__(64 * W) void k_p2p_fp64(Cells c, Csr list, Bodies b
   p2p_leaf<double, RING64, W>(blockIdx.x, c, list, b, nullptr, acc, ring, cycle);
 }
 
-// The FP64 P2P as resident waves taking target cells from a counter, as
+// The targets of resident waves, in the order in which they are taken: the leaves
+// of much work (bodies times source leaves) from the front, the others from the
+// back of order (10 us beside nothing; the order within a part is that of the blocks'
+// arrival, and no result depends on it).
+__global__ __launch_bounds__(1024) void k_p2p_order(Cells c, int32_t ncells, Csr list, P2pQueue q) {
+  critical_path_priority();
+  __shared__ uint32_t scratch[2][17];
+  const int32_t i = blockIdx.x * 1024 + threadIdx.x;
+  const bool leaf = i < ncells && c.child[i] < 0 && c.nb[i] > 0;
+  const bool much =
+      leaf && (float)c.nb[i] * (float)(list.off[i + 1] - list.off[i]) >= q.much;
+  const uint32_t f = block_append<16>(&q.next[1], much, 1, scratch[0]);
+  const uint32_t l = block_append<16>(&q.next[2], leaf && !much, 1, scratch[1]);
+  if (leaf) q.order[much ? f : (uint32_t)ncells - 1u - l] = i;
+}
+
+// The FP64 P2P as resident waves taking target cells from a queue, as
 // k_p2p_fp32_resident below (each target computed by one wave exactly as by
 // k_p2p_fp64, so the fields do not change).
 template <int W>
 __global__ __launch_bounds__(64 * W) void k_p2p_fp64_resident(Cells c, int32_t ncells, Csr list,
                                                               Bodies b, double *acc,
-                                                              uint32_t *next, double cycle) {
+                                                              P2pQueue q, double cycle) {
   __shared__ double4 ring[W * ring_entries(RING64)];
   __shared__ uint32_t take;
+  const uint32_t much = q.next[1], all = much + q.next[2];
   while (true) {
     __syncthreads();
-    if (threadIdx.x == 0) take = atomicAdd(next, 1u);
+    if (threadIdx.x == 0) take = atomicAdd(q.next, 1u);
     __syncthreads();
-    const uint32_t ti = take;
-    if (ti >= (uint32_t)ncells) return;
-    p2p_leaf<double, RING64, W>((int32_t)ti, c, list, b, nullptr, acc, ring, cycle);
+    const uint32_t t = take;
+    if (t >= all) return;
+    const int32_t ti = q.order[t < much ? t : (uint32_t)ncells - 1u - (t - much)];
+    p2p_leaf<double, RING64, W>(ti, c, list, b, nullptr, acc, ring, cycle);
   }
 }
 
@@ -452,28 +470,36 @@ int p2p_waves_per_leaf(int64_t n, int32_t ncrit) {
   return leaves <= 512 ? 8 : leaves <= 2560 ? 4 : leaves <= 8192 ? 2 : 1;
 }
 
-// resident waves taking target cells from *next without clearing it first:
-// several such launches (on different streams) share the cells of one
-// cleared counter, each cell computed once by one workgroup
+hipError_t launch_p2p_order(Cells c, int32_t ncells, Csr list, P2pQueue q, hipStream_t s) {
+  if (ncells <= 0) return hipSuccess;
+  hipError_t e = launch_fill_zero(q.next, 12, s);
+  if (e != hipSuccess) return e;
+  k_p2p_order<<<(ncells + 1023) / 1024, 1024, 0, s>>>(c, ncells, list, q);
+  return hipGetLastError();
+}
+
+// resident waves taking target cells from a queue made before: several such
+// launches (on different streams) share its cells, each computed once by one
+// workgroup
 hipError_t launch_p2p_fp64_drain(Cells c, int32_t ncells, Csr list, Bodies b, double *acc,
-                                 int per_leaf, int waves, uint32_t *next, hipStream_t s,
+                                 int per_leaf, int waves, P2pQueue q, hipStream_t s,
                                  double cycle) {
   if (ncells <= 0 || waves <= 0) return hipSuccess;
   p2p_waves(per_leaf, [&](auto w) {
     const int grid = resident_blocks(waves, w, ncells);
-    k_p2p_fp64_resident<w><<<grid, 64 * w, 0, s>>>(c, ncells, list, b, acc, next, cycle);
+    k_p2p_fp64_resident<w><<<grid, 64 * w, 0, s>>>(c, ncells, list, b, acc, q, cycle);
   });
   return hipGetLastError();
 }
 
 hipError_t launch_p2p_fp64(Cells c, int32_t ncells, Csr list, Bodies b, double *acc,
-                           int per_leaf, int resident, uint32_t *next, hipStream_t s,
+                           int per_leaf, int resident, P2pQueue q, hipStream_t s,
                            double cycle) {
   if (ncells <= 0) return hipSuccess;
-  if (resident > 0 && next) {
-    hipError_t e = launch_fill_zero(next, 4, s);
+  if (resident > 0) {
+    hipError_t e = launch_p2p_order(c, ncells, list, q, s);
     if (e != hipSuccess) return e;
-    return launch_p2p_fp64_drain(c, ncells, list, b, acc, per_leaf, resident, next, s, cycle);
+    return launch_p2p_fp64_drain(c, ncells, list, b, acc, per_leaf, resident, q, s, cycle);
   }
   p2p_waves(per_leaf,
             [&](auto w) { k_p2p_fp64<w><<<ncells, 64 * w, 0, s>>>(c, list, b, acc, cycle); });
@@ -507,8 +533,8 @@ void k_p2p_fp32(Cells c, Csr list, Bodies b, const float4 *rel, double *acc, dou
   p2p_leaf<float, RING32, W>(blockIdx.x, c, list, b, rel, acc, ring, cycle);
 }
 
-// A fixed number of resident waves that take target cells from a counter
-// (zeroed before the launch) until none are left: the P2P then holds a
+// A fixed number of resident waves that take target cells from a queue
+// (launch_p2p_order) until none are left: the P2P then holds a
 // bounded share of the CUs, and kernels on the other stream still find
 // slots.  Each target is computed by one wave exactly as above, so the order
 // in which the waves take them does not change any result.  80 registers (3
@@ -519,16 +545,18 @@ void k_p2p_fp32(Cells c, Csr list, Bodies b, const float4 *rel, double *acc, dou
 template <int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(6, 8)))
 void k_p2p_fp32_resident(Cells c, int32_t ncells, Csr list, Bodies b, const float4 *rel,
-                         double *acc, uint32_t *next, double cycle) {
+                         double *acc, P2pQueue q, double cycle) {
   __shared__ float4 ring[W * ring_entries(RING32)];
   __shared__ uint32_t take;
+  const uint32_t much = q.next[1], all = much + q.next[2];
   while (true) {
     __syncthreads();
-    if (threadIdx.x == 0) take = atomicAdd(next, 1u);
+    if (threadIdx.x == 0) take = atomicAdd(q.next, 1u);
     __syncthreads();
-    const uint32_t ti = take;
-    if (ti >= (uint32_t)ncells) return;
-    p2p_leaf<float, RING32, W>((int32_t)ti, c, list, b, rel, acc, ring, cycle);
+    const uint32_t t = take;
+    if (t >= all) return;
+    const int32_t ti = q.order[t < much ? t : (uint32_t)ncells - 1u - (t - much)];
+    p2p_leaf<float, RING32, W>(ti, c, list, b, rel, acc, ring, cycle);
   }
 }
 }  // namespace
@@ -540,24 +568,24 @@ hipError_t launch_leaf_relpos(Cells c, int32_t ncells, Bodies b, float4 *rel, hi
 }
 
 hipError_t launch_p2p_fp32_drain(Cells c, int32_t ncells, Csr list, Bodies b, const float4 *rel,
-                                 double *acc, int per_leaf, int waves, uint32_t *next,
+                                 double *acc, int per_leaf, int waves, P2pQueue q,
                                  hipStream_t s, double cycle) {
   if (ncells <= 0 || waves <= 0) return hipSuccess;
   p2p_waves(per_leaf, [&](auto w) {
     const int grid = resident_blocks(waves, w, ncells);
-    k_p2p_fp32_resident<w><<<grid, 64 * w, 0, s>>>(c, ncells, list, b, rel, acc, next, cycle);
+    k_p2p_fp32_resident<w><<<grid, 64 * w, 0, s>>>(c, ncells, list, b, rel, acc, q, cycle);
   });
   return hipGetLastError();
 }
 
 hipError_t launch_p2p_fp32(Cells c, int32_t ncells, Csr list, Bodies b, const float4 *rel,
-                           double *acc, int per_leaf, int resident, uint32_t *next,
+                           double *acc, int per_leaf, int resident, P2pQueue q,
                            hipStream_t s, double cycle) {
   if (ncells <= 0) return hipSuccess;
-  if (resident > 0 && next) {
-    hipError_t e = launch_fill_zero(next, 4, s);
+  if (resident > 0) {
+    hipError_t e = launch_p2p_order(c, ncells, list, q, s);
     if (e != hipSuccess) return e;
-    return launch_p2p_fp32_drain(c, ncells, list, b, rel, acc, per_leaf, resident, next, s, cycle);
+    return launch_p2p_fp32_drain(c, ncells, list, b, rel, acc, per_leaf, resident, q, s, cycle);
   }
   p2p_waves(per_leaf, [&](auto w) {
     k_p2p_fp32<w><<<ncells, 64 * w, 0, s>>>(c, list, b, rel, acc, cycle);

@@ -219,15 +219,24 @@ hipError_t launch_m2l_fp64(Cells c, int32_t ncells, Csr list, int32_t npairs, co
 
 // p2p.hip
 // (list sources are source words: leaf and periodic image, cycle the period)
-// resident > 0: that many resident waves take the target cells from *next
-// (cleared first), as launch_p2p_fp32
+// resident > 0: that many resident waves take the target cells from a queue (made
+// first), as launch_p2p_fp32
 // per_leaf: waves that share a target leaf (p2p_waves_per_leaf)
 int p2p_waves_per_leaf(int64_t n, int32_t ncrit);
+// The targets of resident waves (launch_p2p_order): next[0] counts those taken,
+// next[1] and next[2] the two parts of order (a word per cell); much: the work of a
+// leaf, bodies times source leaves, from which it is taken first.
+struct P2pQueue {
+  uint32_t *next;
+  int32_t *order;
+  float much;
+};
+hipError_t launch_p2p_order(Cells c, int32_t ncells, Csr list, P2pQueue q, hipStream_t s);
 hipError_t launch_p2p_fp64(Cells c, int32_t ncells, Csr list, Bodies b, double *acc, int per_leaf,
-                           int resident, uint32_t *next, hipStream_t s, double cycle = 0);
-// resident waves on a counter that another launch clears and shares
+                           int resident, P2pQueue q, hipStream_t s, double cycle = 0);
+// resident waves on a queue made before, which several launches share
 hipError_t launch_p2p_fp64_drain(Cells c, int32_t ncells, Csr list, Bodies b, double *acc,
-                                 int per_leaf, int waves, uint32_t *next, hipStream_t s,
+                                 int per_leaf, int waves, P2pQueue q, hipStream_t s,
                                  double cycle = 0);
 
 // direct.hip
@@ -319,15 +328,14 @@ hipError_t launch_m2l_sets(const int32_t *set_off, const int2 *units, const uint
 
 // p2p.hip (mixed precision)
 hipError_t launch_leaf_relpos(Cells c, int32_t ncells, Bodies b, float4 *rel, hipStream_t s);
-// resident > 0: that many resident waves take target cells from the counter
-// next (4 bytes, zeroed here); 0: one workgroup per cell
-// the resident FP32 P2P on a counter cleared by the caller (waves
-// workgroups of one wave each); launches sharing the counter split the cells
+// resident > 0: that many resident waves take target cells from a queue (made
+// first); 0: one workgroup per cell.  launch_p2p_fp32_drain: waves resident waves on
+// a queue made before; launches that share one split its cells
 hipError_t launch_p2p_fp32_drain(Cells c, int32_t ncells, Csr list, Bodies b, const float4 *rel,
-                                 double *acc, int per_leaf, int waves, uint32_t *next, hipStream_t s,
+                                 double *acc, int per_leaf, int waves, P2pQueue q, hipStream_t s,
                                  double cycle);
 hipError_t launch_p2p_fp32(Cells c, int32_t ncells, Csr list, Bodies b, const float4 *rel,
-                           double *acc, int per_leaf, int resident, uint32_t *next, hipStream_t s,
+                           double *acc, int per_leaf, int resident, P2pQueue q, hipStream_t s,
                            double cycle = 0);
 }  // namespace tfmm
 
