@@ -21,15 +21,68 @@ __device__ inline void untri(int t, int &j, int &k) {
 }
 
 // P2M: M[n,m] += q * conj(Y_n^m(body - centre)), summed over the leaf's
-// bodies.  One wave per leaf, one body per lane (chunks of 64 bodies).  The
-// harmonics come out of the recurrence in a fixed visit order; every 16 real
-// values (8 terms) are staged through LDS as a 64 x 16 block whose columns
-// the wave sums (16 rows per quarter-wave, then across quarters), so the
-// body sum costs 16 LDS writes + 16 LDS reads per 16 values instead of a
-// full wave reduction per value.  Summation order is fixed.
+// bodies.  One wave per leaf, one body per lane (chunks of 64 bodies).  The 110
+// real values come out of the recurrence in a fixed visit order and are summed over
+// the lanes by halving: two values become one register, in which half the lanes hold
+// the pairwise sums of the one and half those of the other, and two such registers
+// become one as soon as both are there (six levels, at most seven registers
+// waiting).  Value v ends in the lane of v's six bits reversed.  The sums' order is
+// fixed.  (Through LDS, 16 values at a time, each summed by 16 serial reads: 4M
+// Plummer 789 us beside the P2P against 343, 500K ellipsoid 131 against 89.)  Bound
+// by FP64 issue: some 500 instructions of harmonics and 440 of sums per 64 bodies.
 constexpr int P2M_WAVES = 4;
-constexpr int NVAL = 2 * NTERM;          // 110 real values per cell
-constexpr int NCHUNK = (NVAL + 15) / 16;  // 7
+constexpr int NVAL = 2 * NTERM;  // 110 real values per cell
+
+// lanes with bit 5 - LEVEL of their number clear: a summed over the two lanes that
+// differ there (below bit 4: in the lower bits too); the others: b
+template <int LEVEL>
+__device__ inline double halve(double a, double b, int lane) {
+  union {
+    double d;
+    uint32_t u[2];
+  } p, q;
+  if constexpr (LEVEL < 2) {
+    p.d = a;
+    q.d = b;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const auto r = LEVEL == 0 ? __builtin_amdgcn_permlane32_swap(p.u[h], q.u[h], false, false)
+                                : __builtin_amdgcn_permlane16_swap(p.u[h], q.u[h], false, false);
+      p.u[h] = r[0];
+      q.u[h] = r[1];
+    }
+    return p.d + q.d;
+  } else {
+    // lane ^ 15, 7, 3, 1
+    constexpr int CTRL = LEVEL == 2 ? 0x140 : LEVEL == 3 ? 0x141 : LEVEL == 4 ? 0x1b : 0xb1;
+    const bool other = lane >> (5 - LEVEL) & 1;
+    p.d = other ? a : b;
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+      q.u[h] = (uint32_t)__builtin_amdgcn_mov_dpp((int)p.u[h], CTRL, 0xf, 0xf, true);
+    return (other ? b : a) + q.d;
+  }
+}
+
+// The waiting registers: value v of 64 (a constant) goes in; at the last one, or with
+// flush at the end of fewer, out holds a value per lane.
+struct LaneSums {
+  double wait[6];
+  template <int LEVEL>
+  __device__ inline void carry(int v, double x, int lane, double &out) {
+    if constexpr (LEVEL == 6) out = x;
+    else if (v >> LEVEL & 1) carry<LEVEL + 1>(v, halve<LEVEL>(wait[LEVEL], x, lane), lane, out);
+    else wait[LEVEL] = x;
+  }
+  template <int LEVEL>
+  __device__ inline void flush(int n, double x, bool have, int lane, double &out) {
+    if constexpr (LEVEL == 6) out = x;
+    else if (n >> LEVEL & 1)
+      flush<LEVEL + 1>(n, halve<LEVEL>(wait[LEVEL], x, lane), true, lane, out);
+    else if (have) flush<LEVEL + 1>(n, halve<LEVEL>(x, 0.0, lane), true, lane, out);
+    else flush<LEVEL + 1>(n, 0.0, false, lane, out);
+  }
+};
 
 // (n, m) of the v-th term of multipole_all's visit order (m outer, n inner)
 __device__ inline int visit_term(int v) {
@@ -44,19 +97,15 @@ __device__ inline int visit_term(int v) {
 __global__ __launch_bounds__(64 * P2M_WAVES) void k_p2m(Cells c, int32_t ncells, Bodies b,
                                                         double *M) {
   critical_path_priority();
-  __shared__ double stage[P2M_WAVES][64][17];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int32_t ci = blockIdx.x * P2M_WAVES + w;
-  if (ci >= ncells || c.child[ci] >= 0 || c.nb[ci] == 0) return;  // per wave; no block barrier
-  double (*st)[17] = stage[w];
-  const int col = lane & 15, rg = lane >> 4;
+  if (ci >= ncells || c.child[ci] >= 0 || c.nb[ci] == 0) return;
   const double cx = c.center[3 * (int64_t)ci], cy = c.center[3 * (int64_t)ci + 1],
                cz = c.center[3 * (int64_t)ci + 2];
   const int32_t beg = c.beg[ci], end = beg + c.nb[ci];
-  double own0 = 0, own1 = 0;  // this lane's sums of chunks rg and rg + 4
+  double own[2] = {0, 0};  // this lane's values of the first 64 and of the others
   for (int32_t base = beg; base < end; base += 64) {
     const int32_t i = base + lane;
-    const int rows = min(64, end - base);
     double dx = 1, dy = 0, dz = 0, q = 0;
     if (i < end) {
       dx = b.x[i] - cx;
@@ -67,39 +116,23 @@ __global__ __launch_bounds__(64 * P2M_WAVES) void k_p2m(Cells c, int32_t ncells,
     double rho, ca, sa;
     cd ei;
     sph_frame(dx, dy, dz, rho, ca, sa, ei);
-    double buf[16];
+    LaneSums sums;
+    double got[2];
     int v = 0;  // visit counter (a constant after unrolling)
     multipole_all<false>(rho, ca, sa, ei, [&](int, int, cd Y, cd) {
-      buf[(2 * v) & 15] = q * Y.re;
-      buf[(2 * v + 1) & 15] = -q * Y.im;
-      const int filled = 2 * v + 2;
-      if ((filled & 15) == 0 || filled == NVAL) {
-        const int ch = (filled - 1) >> 4;
-        const int nval = filled - 16 * ch;
-#pragma unroll
-        for (int k = 0; k < 16; k++)
-          if (k < nval) st[lane][k] = buf[k];
-        __builtin_amdgcn_wave_barrier();
-        double sum = 0;
-        if (col < nval) {
-          const int r1 = min(rows, 16 * rg + 16);
-          for (int r = 16 * rg; r < r1; r++) sum += st[r][col];
-        }
-        sum += __shfl_xor(sum, 16, 64);
-        sum += __shfl_xor(sum, 32, 64);
-        if (ch == rg) own0 += sum;
-        if (ch == rg + 4) own1 += sum;
-        __builtin_amdgcn_wave_barrier();
-      }
-      v++;
-    });
+      sums.carry<0>(v & 63, Y.re, lane, got[v >> 6]);
+      sums.carry<0>((v + 1) & 63, -Y.im, lane, got[(v + 1) >> 6]);
+      v += 2;
+    }, 0.0, q);
+    sums.flush<0>(NVAL & 63, 0.0, false, lane, got[1]);
+    own[0] += got[0];
+    own[1] += got[1];
   }
   double *Mc = M + 2 * (int64_t)NTERM * ci;
 #pragma unroll
   for (int h = 0; h < 2; h++) {
-    const int ch = rg + 4 * h;
-    const int f = 16 * ch + col;  // value index in visit order
-    if (ch < NCHUNK && f < NVAL) Mc[2 * visit_term(f >> 1) + (f & 1)] += h ? own1 : own0;
+    const int f = 64 * h + (int)(__brev((uint32_t)lane) >> 26);  // value, in visit order
+    if (f < NVAL) Mc[2 * visit_term(f >> 1) + (f & 1)] += own[h];
   }
 }
 

@@ -188,8 +188,8 @@ __host__ __device__ constexpr double recip_int(int k) { return 1.0 / (double)k; 
 // only formed if WithTheta (inv_y = 1 / sin(theta) is then required).
 template <bool WithTheta, class Store>
 __device__ inline void multipole_all(double rho, double x, double y, cd ei, Store store,
-                                     double inv_y = 0.0) {
-  double fact = 1, pn = 1, rhom = 1;
+                                     double inv_y = 0.0, double scale = 1.0) {
+  double fact = 1, pn = scale, rhom = 1;
   cd eim = mk(1.0, 0.0);
 #pragma unroll
   for (int m = 0; m < P; m++) {
