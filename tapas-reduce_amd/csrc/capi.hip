@@ -1256,7 +1256,6 @@ int fork_p2p(tfmm_ctx *c, int64_t ncells = -1) {
   // the launches on the queue share it: made on this stream, before either can take
   // from it
   Csr pl{dp<int32_t>(c->p2p_off), dp<int32_t>(c->p2p_src)};
-  TRY(dev_reserve(c->p2p_order, (size_t)ncells * 4));
   if (p2p_drains(c)) TRY(launch_p2p_order(k, (int32_t)ncells, pl, p2p_queue(c), s));
   // schedule 4: on the context stream, alone (the kernel's own time)
   hipStream_t ps = c->run_schedule == 4 ? s : c->side;
@@ -1371,6 +1370,7 @@ int fused_lists(tfmm_ctx *c) {
     TRY(launch_leaf_relpos(k, (int32_t)c->ncells, sorted_bodies(c), dp<float4>(c->relpos), s));
   }
   TRY(dev_reserve(c->acc, (size_t)c->n * 32));
+  TRY(dev_reserve(c->p2p_order, (size_t)c->ncells * 4));
   if (p2p_chosen(c)) {
     c->p2p_heavy = p2p_outweighs(c, c->n_p2p_pairs, c->n_m2l_exec);
     c->run_schedule = c->p2p_heavy ? 2 : 0;
@@ -2222,14 +2222,14 @@ int tfmm_set_tuning(tfmm_ctx *c, int knob, double value) {
 
 // Candidates of the set-kernel knobs, tried jointly; the evaluation's time
 // (HIP events around it) decides, median over the repetitions.  The P2P
-// schedule stays as set: running the P2P beside the tiles measured within
+// schedule stays as set: running the P2P beside the M2L measured within
 // noise of running it beside the batch building, and it would fold the
 // P2P's time into the set kernel's.
 // Candidates of the kernel knobs, timed in two stages: the set kernel's
 // (unit factor x XCD run) at the current P2P setting, then where the P2P
-// starts and how many resident waves it holds, at the best tile setting
+// starts and how many resident waves it holds, at the best set-kernel setting
 // (running the P2P from phase A with a few resident waves lets the upward
-// pass and the tiles have CU slots beside it: on the 4M Plummer 12.96 ms
+// pass and the M2L have CU slots beside it: on the 4M Plummer 12.96 ms
 // against 13.82 with the P2P taking every slot).
 int tfmm_autotune(tfmm_ctx *c, const tfmm_params *p, int reps, double *chosen) {
   if (!c) return TFMM_EINVAL;
