@@ -83,9 +83,9 @@ def parse():
     ap.add_argument("--xcd-run", type=int, default=None,
                     help="groups of 8 M2L work units dealt to one XCD in a row")
     ap.add_argument("--p2p-schedule", type=int, default=None, choices=[0, 1, 2, 3, 4],
-                    help="0: P2P from the numeric phase's start, 1: beside the M2L tiles, "
+                    help="0: P2P from the numeric phase's start, 1: beside the M2L sets, "
                          "2: from phase A, beside the M2L batch building, 3: as 2, drained "
-                         "by a full-occupancy launch after the tiles, 4: serially, alone")
+                         "by a full-occupancy launch after the M2L, 4: serially, alone")
     ap.add_argument("--p2p-waves", type=int, default=None, choices=[0, 1, 2, 3, 4, 5, 6, 7, 8],
                     help="fix the FP32 P2P's resident waves per SIMD (0: one workgroup per cell)")
     ap.add_argument("--graph", action="store_true",
@@ -244,7 +244,7 @@ def p2p_isolated(ctx, prm, st, roof):
     occupancy (no resident-wave cap) on the context stream with nothing
     beside it (TFMM_TUNE_P2P_SCHEDULE 4), outside the timed steps.  The
     headline's figure is over the P2P's span while the upward pass, the M2L
-    batching and the tiles share the GPU with it."""
+    batching and the M2L share the GPU with it."""
     import tfmm
     was = ctx.get_tuning(tfmm.TUNE_P2P_SCHEDULE), ctx.get_tuning(tfmm.TUNE_P2P_WAVES)
     ctx.set_tuning(tfmm.TUNE_P2P_SCHEDULE, 4)

@@ -265,7 +265,7 @@ int tfmm_get_lists(tfmm_ctx *ctx, int32_t *m2l_off, int32_t *m2l_src, int32_t *p
  * one-launch graph of TFMM_TUNE_GRAPH 2; with TFMM_TUNE_GRAPH 1 as 0); 3 as 2.  A
  * resident P2P (TFMM_TUNE_P2P_WAVES > 0) holds its few waves until the critical
  * path beside it is done; a full-occupancy launch of the same kernel on the
- * context stream then takes the target cells still left on its counter (each
+ * context stream then takes the target cells still left in its queue (each
  * cell is computed the same way by either: the fields do not change), with
  * schedule 3 after the M2L, else after the L2L; 4 runs it on the context
  * stream with nothing beside it (from phase A, serially: for timing the
@@ -294,7 +294,7 @@ int tfmm_get_lists(tfmm_ctx *ctx, int32_t *m2l_off, int32_t *m2l_src, int32_t *p
 #define TFMM_TUNE_GRAPH 4
 /* TFMM_TUNE_P2P_WAVES: 0 (default) runs the P2P (FP32 or FP64) as one
  * workgroup per cell; k in 1..8 runs it as k resident waves per SIMD that
- * take target leaves from a counter, so it holds a bounded share of the CUs
+ * take target leaves from a queue, so it holds a bounded share of the CUs
  * and the kernels beside it keep slots (see TFMM_TUNE_P2P_SCHEDULE). */
 #define TFMM_TUNE_P2P_WAVES 5
 /* TFMM_TUNE_DEVICE_LIMIT: a limit in bytes (0 = none, the default) on the
@@ -306,7 +306,7 @@ int tfmm_get_lists(tfmm_ctx *ctx, int32_t *m2l_off, int32_t *m2l_src, int32_t *p
 #define TFMM_TUNE_DEVICE_LIMIT 6
 /* TFMM_TUNE_CART_M2L: the M2L of the Cartesian basis (tfmm_set_basis).
  * 0 (default): through the spherical set kernel, exactly -- the Cartesian
- * multipoles turned into spherical ones per degree (T1), the FP64 tile
+ * multipoles turned into spherical ones per degree (T1), the FP64 set
  * kernel (and its per-pair FP64 fallback, and the far field of periodic
  * images), the spherical locals turned back (T2); both bases truncate the
  * same series and a contraction with derivatives of 1/r sees only the
