@@ -74,29 +74,6 @@ constexpr Inv make_inv() {
 __constant__ Inv c_inv = make_inv();
 #define kInv c_inv.v
 
-// M2M products: for each parent term n, the pairs (k, n - k), k <= n
-// componentwise (k | (n - k) << 8), term by term from m2m_off[n]
-constexpr int M2M_ENTRIES = 5005;
-struct M2mTab {
-  uint16_t off[CN + 1];
-  uint16_t ent[M2M_ENTRIES];
-};
-constexpr M2mTab make_m2m() {
-  M2mTab r{};
-  int e = 0;
-  for (int n = 0; n < CN; n++) {
-    r.off[n] = (uint16_t)e;
-    const int nx = term_part(n, 0), ny = term_part(n, 1), nz = term_part(n, 2);
-    for (int kx = 0; kx <= nx; kx++)
-      for (int ky = 0; ky <= ny; ky++)
-        for (int kz = 0; kz <= nz; kz++)
-          r.ent[e++] = (uint16_t)(cidx(kx, ky, kz) | cidx(nx - kx, ny - ky, nz - kz) << 8);
-  }
-  r.off[CN] = (uint16_t)e;
-  return r;
-}
-__constant__ M2mTab c_m2m = make_m2m();
-
 // ---------------------------------------------------------------------------
 // P2M: one wave per leaf, lane l owns terms l, l+64, l+128, l+192.  Every
 // body of a chunk of 64 writes its powers (X - x)^a / a! per axis (the
@@ -156,47 +133,69 @@ __global__ __launch_bounds__(64 * PW) void k_cart_p2m(Cells c, int32_t ncells, B
 }
 
 // ---------------------------------------------------------------------------
+// The shift of a Cartesian expansion is a product of shifts along x, y and z, so M2M
+// and L2L run as three passes of at most 10 products a term (2,145 a cell and child
+// instead of 5,005, and 10 after one another instead of 220 for the lowest term).
+
+// powers d^e / e! of the offsets of the 8 children c0 .. c0 + 7 of par (sign: +1 from
+// the parent to the child, -1 back)
+__device__ inline void sibling_powers(const Cells &c, int32_t par, int32_t c0, double sign,
+                                      double (*pw)[PWR]) {
+  if (threadIdx.x >= 24) return;
+  const int j = threadIdx.x / 3, a = threadIdx.x % 3;
+  const double d = sign * (c.center[3 * (int64_t)(c0 + j) + a] - c.center[3 * (int64_t)par + a]);
+  double p = 1;
+  pw[j][a * P] = p;
+  for (int e = 1; e < P; e++) {
+    p = p * d * kInv[e];
+    pw[j][a * P + e] = p;
+  }
+}
+
 // M2M: one block per group of 8 siblings (children [c0, c0 + 8) of one
-// parent); thread t owns term t of the parent.  Each child's multipole and
-// its shift powers (Xp - Xc)^m / m! (all terms) are staged in LDS; the
-// products of a term come from the (k, n - k) table.
+// parent); thread t owns term t of every child in turn and of the parent.  1M cube,
+// all levels: 258 us with the 5,005 products from a table, 300K (32,873 cells) 215 us, now 97.
 __global__ __launch_bounds__(256) void k_cart_m2m(Cells c, int32_t first_child, int32_t npar,
                                                   double *M) {
   critical_path_priority();
   __shared__ double Mc[8][CN];
-  __shared__ double Pw[8][CN];
   __shared__ double pw[8][PWR];
   const int32_t g = blockIdx.x;
   if (g >= npar) return;
   const int32_t c0 = first_child + 8 * g;
   const int32_t par = c.parent[c0];
   for (int e = threadIdx.x; e < 8 * CN; e += 256) Mc[e / CN][e % CN] = M[(int64_t)c0 * CN + e];
-  if (threadIdx.x < 24) {
-    const int j = threadIdx.x / 3, a = threadIdx.x % 3;
-    const double d = c.center[3 * (int64_t)par + a] - c.center[3 * (int64_t)(c0 + j) + a];
-    double p = 1;
-    pw[j][a * P] = p;
-    for (int e = 1; e < P; e++) {
-      p = p * d * kInv[e];
-      pw[j][a * P + e] = p;
-    }
-  }
+  sibling_powers(c, par, c0, -1.0, pw);
   __syncthreads();
   const int t = threadIdx.x;
-  if (t < CN) {
-    const int x = c_terms.x[t], y = c_terms.y[t], z = c_terms.z[t];
-    for (int j = 0; j < 8; j++) Pw[j][t] = pw[j][x] * pw[j][P + y] * pw[j][2 * P + z];
+  const bool own = t < CN;
+  int n[3] = {0, 0, 0};
+  if (own) {
+    n[0] = c_terms.x[t];
+    n[1] = c_terms.y[t];
+    n[2] = c_terms.z[t];
   }
-  __syncthreads();
-  if (t >= CN) return;
-  double s = 0;
-  const int e1 = c_m2m.off[t + 1];
-  for (int e = c_m2m.off[t]; e < e1; e++) {
-    const int en = c_m2m.ent[e], k = en & 0xff, m = en >> 8;
+  double v[8];
 #pragma unroll
-    for (int j = 0; j < 8; j++) s += Pw[j][m] * Mc[j][k];
+  for (int a = 0; a < 3; a++) {
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] = 0;
+    if (own)
+      for (int e = 0; e <= n[a]; e++) {
+        const int k = cidx(n[0] - (a == 0 ? e : 0), n[1] - (a == 1 ? e : 0), n[2] - (a == 2 ? e : 0));
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] += pw[j][a * P + e] * Mc[j][k];
+      }
+    if (a == 2) break;
+    __syncthreads();
+    if (own)
+#pragma unroll
+      for (int j = 0; j < 8; j++) Mc[j][t] = v[j];
+    __syncthreads();
   }
-  M[(int64_t)par * CN + t] += s;
+  if (own)
+    M[(int64_t)par * CN + t] +=
+        ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
 }
 
 // ---------------------------------------------------------------------------
@@ -392,36 +391,49 @@ __global__ __launch_bounds__(64 * BW) void k_sph_to_cart(int32_t ncells, const d
 }
 
 // ---------------------------------------------------------------------------
-// L2L: one block per child cell; thread t owns term t of the child.
-__global__ __launch_bounds__(256) void k_cart_l2l(Cells c, int32_t first_child, int32_t nchild,
+// L2L: one block per group of 8 siblings; thread t owns term t of every child.  1M
+// cube, all levels: 462 us with a block a child and 5,005 products, 300K (32,873 cells) 411 us, now 76.
+__global__ __launch_bounds__(256) void k_cart_l2l(Cells c, int32_t first_child, int32_t npar,
                                                   double *L) {
-  __shared__ double Lp[CN];
-  __shared__ double pw[PWR];
-  const int32_t ch = first_child + (int32_t)blockIdx.x;
-  if ((int32_t)blockIdx.x >= nchild) return;
-  const int32_t par = c.parent[ch];
-  for (int t = threadIdx.x; t < CN; t += 256) Lp[t] = L[(int64_t)par * CN + t];
-  if (threadIdx.x < 3) {
-    const int a = threadIdx.x;
-    const double d = c.center[3 * (int64_t)ch + a] - c.center[3 * (int64_t)par + a];
-    double p = 1;
-    pw[a * P] = p;
-    for (int e = 1; e < P; e++) {
-      p = p * d * kInv[e];
-      pw[a * P + e] = p;
-    }
-  }
-  __syncthreads();
+  __shared__ double Lc[8][CN];
+  __shared__ double pw[8][PWR];
+  const int32_t g = blockIdx.x;
+  if (g >= npar) return;
+  const int32_t c0 = first_child + 8 * g;
+  const int32_t par = c.parent[c0];
   const int t = threadIdx.x;
-  if (t >= CN) return;
-  const int nx = c_terms.x[t], ny = c_terms.y[t], nz = c_terms.z[t];
-  const int left = P - 1 - (nx + ny + nz);
-  double s = 0;
-  for (int kx = 0; kx <= left; kx++)
-    for (int ky = 0; ky <= left - kx; ky++)
-      for (int kz = 0; kz <= left - kx - ky; kz++)
-        s += pw[kx] * pw[P + ky] * pw[2 * P + kz] * Lp[cidx(nx + kx, ny + ky, nz + kz)];
-  L[(int64_t)ch * CN + t] += s;
+  const bool own = t < CN;
+  if (own) Lc[0][t] = L[(int64_t)par * CN + t];
+  sibling_powers(c, par, c0, 1.0, pw);
+  __syncthreads();
+  int n[3] = {0, 0, 0};
+  if (own) {
+    n[0] = c_terms.x[t];
+    n[1] = c_terms.y[t];
+    n[2] = c_terms.z[t];
+  }
+  const int left = P - 1 - (n[0] + n[1] + n[2]);
+  double v[8];
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] = 0;
+    if (own)
+      for (int e = 0; e <= left; e++) {
+        const int k = cidx(n[0] + (a == 0 ? e : 0), n[1] + (a == 1 ? e : 0), n[2] + (a == 2 ? e : 0));
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] += pw[j][a * P + e] * Lc[a == 0 ? 0 : j][k];
+      }
+    if (a == 2) break;
+    __syncthreads();
+    if (own)
+#pragma unroll
+      for (int j = 0; j < 8; j++) Lc[j][t] = v[j];
+    __syncthreads();
+  }
+  if (own)
+#pragma unroll
+    for (int j = 0; j < 8; j++) L[(int64_t)(c0 + j) * CN + t] += v[j];
 }
 
 // ---------------------------------------------------------------------------
@@ -632,7 +644,7 @@ hipError_t launch_cart_m2l(Cells c, Csr list, int32_t ncells, const double *M, d
 hipError_t launch_cart_l2l(Cells c, int32_t first_child, int32_t nchild, double *L,
                            hipStream_t s) {
   if (nchild <= 0) return hipSuccess;
-  k_cart_l2l<<<nchild, 256, 0, s>>>(c, first_child, nchild, L);
+  k_cart_l2l<<<nchild / 8, 256, 0, s>>>(c, first_child, nchild / 8, L);  // families of 8
   return hipGetLastError();
 }
 
