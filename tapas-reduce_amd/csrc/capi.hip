@@ -97,7 +97,8 @@ struct tfmm_ctx {
   int stage = 0;  // 0 none, 1 tree, 2 upward, 3 traverse, 4 downward
 
   // tree
-  DevBuf keys, keys_alt, idx, idx_alt, sort_tmp, sx, sy, sz, sq, perm, region, bbox_part, brec;
+  DevBuf keys, keys_alt, idx, idx_alt, sort_tmp, sx, sy, sz, sq, perm, region, range, bbox_part,
+      brec;
   DevBuf c_key, c_beg, c_nb, c_parent, c_child, c_depth, c_center, c_width;
   size_t cell_cap = 0;
   DevBuf flag, slot, scan_tmp, lev, lev_bsum, lev_status;
@@ -262,7 +263,7 @@ Bodies sorted_bodies(tfmm_ctx *c) {
 std::vector<DevBuf *> all_buffers(tfmm_ctx *c) {
   return {&c->own_x, &c->own_y, &c->own_z, &c->own_q, &c->keys, &c->keys_alt, &c->idx,
           &c->idx_alt, &c->sort_tmp, &c->sx, &c->sy, &c->sz, &c->sq, &c->perm,
-          &c->region, &c->bbox_part, &c->c_key, &c->c_beg, &c->c_nb, &c->c_parent,
+          &c->region, &c->range, &c->bbox_part, &c->c_key, &c->c_beg, &c->c_nb, &c->c_parent,
           &c->c_child, &c->c_depth, &c->c_center, &c->c_width, &c->flag, &c->slot,
           &c->scan_tmp, &c->M, &c->L, &c->front_a, &c->front_b, &c->m2l_pairs,
           &c->p2p_pairs, &c->cnt, &c->lkeys, &c->lkeys_alt, &c->lidx, &c->lidx_alt,
@@ -476,15 +477,17 @@ int do_build_tree(tfmm_ctx *c, bool whole_keys = false) {
   const int np = c->nprob;
   const bool forest = np > 1;
   TRY(dev_reserve(c->region, 6 * 8 * (size_t)np));
+  TRY(dev_reserve(c->range, sizeof(BodyRange) * ((size_t)np + 1)));
   const int64_t *off = forest ? dp<int64_t>(c->d_prob_off) : nullptr;
   if (forest) {
     TRY(dev_reserve(c->bprob, n * 4));
-    TRY(launch_bbox_forest(c->bx, c->by, c->bz, off, np, dp<double>(c->region), s));
+    TRY(launch_bbox_forest(c->bx, c->by, c->bz, c->bq, off, np, dp<double>(c->region),
+                           dp<BodyRange>(c->range), s));
   } else {
     const int nparts = (int)std::min<int64_t>(1024, (n + 255) / 256);
-    TRY(dev_reserve(c->bbox_part, 2 * 8 * (size_t)nparts));
-    TRY(launch_bbox(c->bx, c->by, c->bz, n, dp<double>(c->bbox_part), nparts,
-                    dp<double>(c->region), s));
+    TRY(dev_reserve(c->bbox_part, bbox_part_bytes(nparts)));
+    TRY(launch_bbox(c->bx, c->by, c->bz, c->bq, n, c->bbox_part.ptr, nparts,
+                    dp<double>(c->region), dp<BodyRange>(c->range), s));
     if (c->images > 0) {
       TRY(dev_reserve(c->pflag, 4));
       TRY(launch_fill_zero(c->pflag.ptr, 4, s));
@@ -986,8 +989,9 @@ int run_lists(tfmm_ctx *c, bool given = false) {
                           dp<double>(c->acc), leaf_waves(c), p2p_resident(c), p2p_queue(c), c->side,
                           period(c)));
     else
-      TRY(launch_p2p_fp64(k, (int32_t)c->ncells, pl, sorted_bodies(c), dp<double>(c->acc), leaf_waves(c),
-                          p2p_resident(c), p2p_queue(c), c->side, period(c)));
+      TRY(launch_p2p_fp64(k, (int32_t)c->ncells, pl, sorted_bodies(c), dp<double>(c->acc),
+                          dp<BodyRange>(c->range), leaf_waves(c), p2p_resident(c), p2p_queue(c),
+                          c->side, period(c)));
     TRY(hipEventRecord(c->ev[EV_P2P1], c->side));
     return TFMM_OK;
   };
@@ -1219,7 +1223,8 @@ hipError_t p2p_on_counter(tfmm_ctx *c, int64_t ncells, int waves, hipStream_t st
                                  dp<double>(c->acc), leaf_waves(c), waves, p2p_queue(c), st,
                                  period(c));
   return launch_p2p_fp64_drain(k, (int32_t)ncells, pl, sorted_bodies(c), dp<double>(c->acc),
-                               leaf_waves(c), waves, p2p_queue(c), st, period(c));
+                               dp<BodyRange>(c->range), leaf_waves(c), waves, p2p_queue(c), st,
+                               period(c));
 }
 
 int drain_p2p(tfmm_ctx *c, int64_t ncells, bool l2l_done) {
@@ -1272,7 +1277,8 @@ int fork_p2p(tfmm_ctx *c, int64_t ncells = -1) {
                         dp<double>(c->acc), leaf_waves(c), resident, p2p_queue(c), ps, period(c)));
   else
     TRY(launch_p2p_fp64(k, (int32_t)ncells, pl, sorted_bodies(c), dp<double>(c->acc),
-                        leaf_waves(c), resident, p2p_queue(c), ps, period(c)));
+                        dp<BodyRange>(c->range), leaf_waves(c), resident, p2p_queue(c), ps,
+                        period(c)));
   TRY(rec(c, EV_P2P1, ps));
   TRY(hipEventRecord(c->ev[EV_P2PJOIN], ps));
   return TFMM_OK;
@@ -1636,6 +1642,7 @@ int plan_reserve(tfmm_ctx *c) {
   TRY(dev_reserve(c->sq, n * 8));
   TRY(dev_reserve(c->perm, n * 4));
   TRY(dev_reserve(c->region, 6 * 8 * (size_t)c->nprob));
+  TRY(dev_reserve(c->range, sizeof(BodyRange) * ((size_t)c->nprob + 1)));
   TRY(dev_reserve(c->brec, n * 32));
   if (c->nprob > 1) {
     TRY(dev_reserve(c->bprob, n * 4));
@@ -1645,7 +1652,7 @@ int plan_reserve(tfmm_ctx *c) {
     TRY(dev_reserve(c->ppos_alt, n * 4));
   } else {
     const int nparts = (int)std::min<int64_t>(1024, (n + 255) / 256);
-    TRY(dev_reserve(c->bbox_part, 2 * 8 * (size_t)nparts));
+    TRY(dev_reserve(c->bbox_part, bbox_part_bytes(nparts)));
   }
   TRY(reserve_cells(c, cells, 0, s));
   int32_t gmax = 0;
@@ -1758,10 +1765,11 @@ int whole_record(tfmm_ctx *c) {
   const int key_end = DEPTHBITS + 3 * MAXDEPTH;
   const int64_t *off = forest ? dp<int64_t>(c->d_prob_off) : nullptr;
   if (forest) {
-    TRY(launch_bbox_forest(c->bx, c->by, c->bz, off, np, region, s));
+    TRY(launch_bbox_forest(c->bx, c->by, c->bz, c->bq, off, np, region, dp<BodyRange>(c->range), s));
   } else {
     const int nparts = (int)std::min<int64_t>(1024, (n + 255) / 256);
-    TRY(launch_bbox(c->bx, c->by, c->bz, n, dp<double>(c->bbox_part), nparts, region, s));
+    TRY(launch_bbox(c->bx, c->by, c->bz, c->bq, n, c->bbox_part.ptr, nparts, region,
+                    dp<BodyRange>(c->range), s));
   }
   TRY(launch_keys(c->bx, c->by, c->bz, c->bq, n, region, off, np, dp<uint64_t>(c->keys),
                   dp<uint32_t>(c->idx), forest ? dp<uint32_t>(c->bprob) : nullptr,

@@ -23,10 +23,10 @@
 // are added in lane order at the end of its pass, so results do not depend
 // on timing.
 //
-// The R2 != 0 test costs one instruction: R2 is formed as dX.dX - tiny
+// The R2 != 0 test costs one instruction at most: R2 is formed as dX.dX - tiny
 // (tiny far below the smallest distance the coordinates resolve), so a zero
 // distance gives a negative argument, rsqrt gives NaN, and max(NaN, 0) = 0
-// drops the pair exactly.
+// drops the pair exactly (FP64: a clamp, see rsq_guarded).
 #include <algorithm>
 #include <type_traits>
 
@@ -68,10 +68,12 @@ __device__ inline int lanes_per_target(int32_t nt) {
   return g_best;
 }
 
-// RINV / |dX| of a pair, and 0 for a negative argument (the R2 != 0 test above)
-template <typename T> constexpr T RINV = 1;
-template <> constexpr double RINV<double> = 2;
+// RINV / |dX| of a pair, and 0 for a negative argument (the R2 != 0 test above).
+// WIDE: for distances of any size (FP64; p2p_frame says when it is needed).
+template <typename T, bool WIDE> constexpr T RINV = 1;
+template <> constexpr double RINV<double, false> = 2;
 
+template <bool WIDE>
 __device__ inline float rsq_guarded(float r2) {
   return __builtin_fmaxf(__builtin_amdgcn_rsqf(r2), 0.f);
 }
@@ -80,24 +82,20 @@ __device__ inline float rsq_guarded(float r2) {
 // about 24 bits) and one Newton step y (3 - x y^2), which squares the error:
 // 4.1e-15 at most, a few ulp (both measured on gfx950 over 2^20 arguments spread
 // over [1e-12, 1e12]; a second step gives 1.4e-16 and costs 4 more VALU
-// instructions).  The pair's coordinates are scaled (p2p_scale) so that the value
+// instructions).  The pair's coordinates are scaled (p2p_frame) so that the value
 // never exceeds 1: the limits to [0, 1] are then the clamp of the last
 // multiplication, which is no instruction of its own and makes the NaN of a
 // negative x zero.  v_max_f64 takes as long as two other FP64 instructions, and
 // leaving the factor 2 in saves a third: 1M-body cube, ncrit 64, alone 2,227
 // us against 2,428.
+// WIDE: 1/sqrt(x) for every x of the double range, max(NaN, 0) = 0.
+template <bool WIDE>
 __device__ inline double rsq_guarded(double x) {
   const double y = __builtin_amdgcn_rsq(x);
-  return __builtin_fmin(__builtin_fmax(y * __builtin_fma(-x * y, y, 3.0), 0.0), 1.0);
-}
-
-// The FP64 P2P works on coordinates times 2^p2p_scale, exact powers of two, in
-// which a cell's width is about 2^256: |dX| is then at least 2 for every pair
-// down to 2^-255 of the width, and |dX|^3 far below the largest double for the
-// farthest leaf of a list.
-__device__ inline int p2p_scale(double width) {
-  if (!(width > 0)) return 0;  // all bodies of the problem in one point
-  return max(-400, min(400, 256 - ilogb(width)));
+  if constexpr (WIDE)
+    return __builtin_fmax(__builtin_fma(0.5 * y, __builtin_fma(-x * y, y, 1.0), y), 0.0);
+  else
+    return __builtin_fmin(__builtin_fmax(y * __builtin_fma(-x * y, y, 3.0), 0.0), 1.0);
 }
 
 __device__ inline float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
@@ -108,13 +106,13 @@ template <> struct Vec4<float> { using type = float4; };
 template <> struct Vec4<double> { using type = double4; };
 
 // One pair: target xi, source xj (w = charge); p0 += RINV q/r, p1..3 -= RINV^3 q dX / r^3
-template <typename T, typename V4>
+template <typename T, bool WIDE, typename V4>
 __device__ inline void pair(const V4 &xi, const V4 &xj, T tiny, T &p0, T &p1, T &p2, T &p3) {
   const T dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
   T r2 = fma_t(dx, dx, -tiny);
   r2 = fma_t(dy, dy, r2);
   r2 = fma_t(dz, dz, r2);
-  const T rinv = rsq_guarded(r2);
+  const T rinv = rsq_guarded<WIDE>(r2);
   const T qr = xj.w * rinv;
   const T f = qr * (rinv * rinv);
   p0 += qr;
@@ -133,8 +131,8 @@ __device__ inline void kahan_add(float &s, float &c, float v) {
 
 // Running sums of one lane: FP32 partials over at most 64 pairs, folded into
 // Kahan-compensated FP32 sums (mixed); plain FP64 sums (FP64).
-template <typename T> struct Acc;
-template <> struct Acc<float> {
+template <typename T, bool WIDE> struct Acc;
+template <> struct Acc<float, false> {
   float p0 = 0, p1 = 0, p2 = 0, p3 = 0;
   float s0 = 0, s1 = 0, s2 = 0, s3 = 0, c0 = 0, c1 = 0, c2 = 0, c3 = 0;
   __device__ void flush() {
@@ -148,12 +146,13 @@ template <> struct Acc<float> {
     return make_double4((double)s0 - c0, (double)s1 - c1, (double)s2 - c2, (double)s3 - c3);
   }
 };
-template <> struct Acc<double> {
+template <bool WIDE> struct Acc<double, WIDE> {
   double p0 = 0, p1 = 0, p2 = 0, p3 = 0;
   __device__ void flush() {}
   // scale: that of the coordinates
   __device__ double4 total(int scale) {
-    const double s1 = ldexp(1.0 / RINV<double>, scale), s3 = ldexp(0.125, 2 * scale);
+    constexpr double R = 1 / RINV<double, WIDE>;
+    const double s1 = ldexp(R, scale), s3 = ldexp(R * R * R, 2 * scale);
     return make_double4(p0 * s1, p1 * s3, p2 * s3, p3 * s3);
   }
 };
@@ -176,8 +175,8 @@ __device__ inline double4 scaled(double4 v, double up) {
 
 // One pass over the source stream for the targets t (and t2 when TWO) of
 // every lane; see p2p_leaf.
-template <typename T, int RING, int W, bool TWO>
-__device__ inline void p2p_pass(const Cells &c, const Csr &list, const Bodies &b,
+template <typename T, int RING, int W, bool WIDE, bool TWO>
+__device__ __forceinline__ void p2p_pass(const Cells &c, const Csr &list, const Bodies &b,
                                 const float4 *rel, double *acc, typename Vec4<T>::type *ring,
                                 int32_t tb, int32_t lb, int32_t le, double tcx, double tcy,
                                 double tcz, double cycle, T tiny, int scale, int G,
@@ -196,7 +195,7 @@ __device__ inline void p2p_pass(const Cells &c, const Csr &list, const Bodies &b
     xi = scaled(xi, up);
     if (TWO) xi2 = scaled(xi2, up);
   }
-  Acc<T> a, a2;
+  Acc<T, WIDE> a, a2;
   int32_t wpos = 0, cpos = 0;
   int since = 0;
   // chunk [cpos, cpos + B) of the stream: segment seg of this lane
@@ -206,8 +205,8 @@ __device__ inline void p2p_pass(const Cells &c, const Csr &list, const Bodies &b
 #pragma unroll
       for (int k = 0; k < SEG; k++) {
         const V4 xj = sp[k];
-        pair<T>(xi, xj, tiny, a.p0, a.p1, a.p2, a.p3);
-        if (TWO) pair<T>(xi2, xj, tiny, a2.p0, a2.p1, a2.p2, a2.p3);
+        pair<T, WIDE>(xi, xj, tiny, a.p0, a.p1, a.p2, a.p3);
+        if (TWO) pair<T, WIDE>(xi2, xj, tiny, a2.p0, a2.p1, a2.p2, a2.p3);
       }
     }
     cpos += B;
@@ -350,11 +349,11 @@ __device__ inline void p2p_pass(const Cells &c, const Csr &list, const Bodies &b
 // The work of one target leaf (one workgroup of W waves, each with its share of
 // the leaf's source leaves); returns at once for other cells.
 // ring: W times RING + RING / 16 entries of LDS; each wave's also holds its lane
-// partials at the end of every pass.
-template <typename T, int RING, int W>
-__device__ inline void p2p_leaf(int32_t ti, const Cells &c, const Csr &list, const Bodies &b,
+// partials at the end of every pass.  scale: of the coordinates (FP64, p2p_frame).
+template <typename T, int RING, int W, bool WIDE>
+__device__ __forceinline__ void p2p_leaf(int32_t ti, const Cells &c, const Csr &list, const Bodies &b,
                                 const float4 *rel, double *acc, typename Vec4<T>::type *ring,
-                                double cycle) {
+                                double cycle, int scale) {
   constexpr bool MIX = sizeof(T) == 4;
   constexpr int GMAX = RING / (2 * SEG);  // a chunk (16 G) plus a 64-body piece fit the ring
   if (c.child[ti] >= 0) return;
@@ -378,7 +377,6 @@ __device__ inline void p2p_leaf(int32_t ti, const Cells &c, const Csr &list, con
   } else {
     tiny = 0x1p-1022;
   }
-  const int scale = MIX ? 0 : p2p_scale(c.width[ti]);
   const int G = lanes_per_target<GMAX>(nt);
   const int tpp = 64 / G;  // targets per lane set
   const int tloc = lane / G;
@@ -387,11 +385,11 @@ __device__ inline void p2p_leaf(int32_t ti, const Cells &c, const Csr &list, con
     const int32_t t = t0 + tloc, t2 = t + tpp;
     const bool tvalid = tloc < tpp && t < nt, tvalid2 = tloc < tpp && t2 < nt;
     if (t0 + tpp < nt)
-      p2p_pass<T, RING, W, true>(c, list, b, rel, acc, ring, tb, lb, le, tcx, tcy, tcz, cycle, tiny,
-                              scale, G, t, t2, tvalid, tvalid2);
+      p2p_pass<T, RING, W, WIDE, true>(c, list, b, rel, acc, ring, tb, lb, le, tcx, tcy, tcz, cycle,
+                                       tiny, scale, G, t, t2, tvalid, tvalid2);
     else
-      p2p_pass<T, RING, W, false>(c, list, b, rel, acc, ring, tb, lb, le, tcx, tcy, tcz, cycle, tiny,
-                               scale, G, t, t2, tvalid, false);
+      p2p_pass<T, RING, W, WIDE, false>(c, list, b, rel, acc, ring, tb, lb, le, tcx, tcy, tcz, cycle,
+                                        tiny, scale, G, t, t2, tvalid, false);
   }
 }
 
@@ -399,10 +397,19 @@ constexpr int RING32 = 256;  // float4 entries: 4.25 KB with the pads
 constexpr int RING64 = 128;  // double4 entries: 4.25 KB with the pads
 
 template <int W>
+__device__ __forceinline__ void p2p_leaf_fp64(int32_t ti, const Cells &c, const Csr &list, const Bodies &b,
+                                     double *acc, double4 *ring, double cycle, P2pFrame f) {
+  if (f.wide)
+    p2p_leaf<double, RING64, W, true>(ti, c, list, b, nullptr, acc, ring, cycle, 0);
+  else
+    p2p_leaf<double, RING64, W, false>(ti, c, list, b, nullptr, acc, ring, cycle, f.scale);
+}
+
+template <int W>
 __global__ __launch_bounds__(64 * W) void k_p2p_fp64(Cells c, Csr list, Bodies b, double *acc,
-                                                     double cycle) {
+                                                     const BodyRange *range, double cycle) {
   __shared__ double4 ring[W * ring_entries(RING64)];
-  p2p_leaf<double, RING64, W>(blockIdx.x, c, list, b, nullptr, acc, ring, cycle);
+  p2p_leaf_fp64<W>(blockIdx.x, c, list, b, acc, ring, cycle, p2p_frame(*range, cycle));
 }
 
 // The targets of resident waves, in the order in which they are taken: the leaves
@@ -427,9 +434,11 @@ __global__ __launch_bounds__(1024) void k_p2p_order(Cells c, int32_t ncells, Csr
 template <int W>
 __global__ __launch_bounds__(64 * W) void k_p2p_fp64_resident(Cells c, int32_t ncells, Csr list,
                                                               Bodies b, double *acc,
-                                                              P2pQueue q, double cycle) {
+                                                              const BodyRange *range, P2pQueue q,
+                                                              double cycle) {
   __shared__ double4 ring[W * ring_entries(RING64)];
   __shared__ uint32_t take;
+  const P2pFrame f = p2p_frame(*range, cycle);
   const uint32_t much = q.next[1], all = much + q.next[2];
   while (true) {
     __syncthreads();
@@ -438,7 +447,7 @@ __global__ __launch_bounds__(64 * W) void k_p2p_fp64_resident(Cells c, int32_t n
     const uint32_t t = take;
     if (t >= all) return;
     const int32_t ti = q.order[t < much ? t : (uint32_t)ncells - 1u - (t - much)];
-    p2p_leaf<double, RING64, W>(ti, c, list, b, nullptr, acc, ring, cycle);
+    p2p_leaf_fp64<W>(ti, c, list, b, acc, ring, cycle, f);
   }
 }
 
@@ -482,27 +491,28 @@ hipError_t launch_p2p_order(Cells c, int32_t ncells, Csr list, P2pQueue q, hipSt
 // launches (on different streams) share its cells, each computed once by one
 // workgroup
 hipError_t launch_p2p_fp64_drain(Cells c, int32_t ncells, Csr list, Bodies b, double *acc,
-                                 int per_leaf, int waves, P2pQueue q, hipStream_t s,
-                                 double cycle) {
+                                 const BodyRange *range, int per_leaf, int waves, P2pQueue q,
+                                 hipStream_t s, double cycle) {
   if (ncells <= 0 || waves <= 0) return hipSuccess;
   p2p_waves(per_leaf, [&](auto w) {
     const int grid = resident_blocks(waves, w, ncells);
-    k_p2p_fp64_resident<w><<<grid, 64 * w, 0, s>>>(c, ncells, list, b, acc, q, cycle);
+    k_p2p_fp64_resident<w><<<grid, 64 * w, 0, s>>>(c, ncells, list, b, acc, range, q, cycle);
   });
   return hipGetLastError();
 }
 
 hipError_t launch_p2p_fp64(Cells c, int32_t ncells, Csr list, Bodies b, double *acc,
-                           int per_leaf, int resident, P2pQueue q, hipStream_t s,
-                           double cycle) {
+                           const BodyRange *range, int per_leaf, int resident, P2pQueue q,
+                           hipStream_t s, double cycle) {
   if (ncells <= 0) return hipSuccess;
   if (resident > 0) {
     hipError_t e = launch_p2p_order(c, ncells, list, q, s);
     if (e != hipSuccess) return e;
-    return launch_p2p_fp64_drain(c, ncells, list, b, acc, per_leaf, resident, q, s, cycle);
+    return launch_p2p_fp64_drain(c, ncells, list, b, acc, range, per_leaf, resident, q, s, cycle);
   }
-  p2p_waves(per_leaf,
-            [&](auto w) { k_p2p_fp64<w><<<ncells, 64 * w, 0, s>>>(c, list, b, acc, cycle); });
+  p2p_waves(per_leaf, [&](auto w) {
+    k_p2p_fp64<w><<<ncells, 64 * w, 0, s>>>(c, list, b, acc, range, cycle);
+  });
   return hipGetLastError();
 }
 
@@ -530,7 +540,7 @@ template <int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(6, 8)))
 void k_p2p_fp32(Cells c, Csr list, Bodies b, const float4 *rel, double *acc, double cycle) {
   __shared__ float4 ring[W * ring_entries(RING32)];
-  p2p_leaf<float, RING32, W>(blockIdx.x, c, list, b, rel, acc, ring, cycle);
+  p2p_leaf<float, RING32, W, false>(blockIdx.x, c, list, b, rel, acc, ring, cycle, 0);
 }
 
 // A fixed number of resident waves that take target cells from a queue
@@ -556,7 +566,7 @@ void k_p2p_fp32_resident(Cells c, int32_t ncells, Csr list, Bodies b, const floa
     const uint32_t t = take;
     if (t >= all) return;
     const int32_t ti = q.order[t < much ? t : (uint32_t)ncells - 1u - (t - much)];
-    p2p_leaf<float, RING32, W>(ti, c, list, b, rel, acc, ring, cycle);
+    p2p_leaf<float, RING32, W, false>(ti, c, list, b, rel, acc, ring, cycle, 0);
   }
 }
 }  // namespace

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "p2p_range.h"
+
 namespace tfmm {
 
 // Cells in breadth-first order (level-contiguous, siblings adjacent).
@@ -64,8 +66,12 @@ struct PlanCaps {
 // *flag |= 1 when any x, y, z or q of the n bodies is not finite
 hipError_t launch_check_finite(const double *x, const double *y, const double *z,
                                const double *q, int64_t n, uint32_t *flag, hipStream_t s);
-hipError_t launch_bbox(const double *x, const double *y, const double *z, int64_t n,
-                       double *partial, int nparts, double *region, hipStream_t s);
+// the box, and the exponents of all coordinates and charges (p2p_range.h) in *range;
+// part: bbox_part_bytes of scratch
+size_t bbox_part_bytes(int nparts);
+hipError_t launch_bbox(const double *x, const double *y, const double *z, const double *q,
+                       int64_t n, void *part, int nparts, double *region, BodyRange *range,
+                       hipStream_t s);
 // keys, and the bodies packed as (x, y, z, q) records for the permutation
 hipError_t launch_keys(const double *x, const double *y, const double *z, const double *q,
                        int64_t n, const double *regions, const int64_t *off, int nprob,
@@ -77,8 +83,10 @@ hipError_t launch_sort_runs(const uint64_t *keys, const uint32_t *idx, const uin
                             int64_t n, int shift, uint64_t *keys_out, uint32_t *idx_out,
                             uint32_t *long_run, hipStream_t s);
 // forest of nprob problems, problem p = bodies [off[p], off[p+1])
-hipError_t launch_bbox_forest(const double *x, const double *y, const double *z,
-                              const int64_t *off, int nprob, double *regions, hipStream_t s);
+// (range: nprob + 1 of them, the first over all problems)
+hipError_t launch_bbox_forest(const double *x, const double *y, const double *z, const double *q,
+                              const int64_t *off, int nprob, double *regions, BodyRange *range,
+                              hipStream_t s);
 hipError_t launch_problem_keys(const uint32_t *order, const uint32_t *bprob, int64_t n,
                                uint32_t *pkey, uint32_t *pos, hipStream_t s);
 hipError_t launch_problem_gather(const uint32_t *pos, const uint64_t *keys1,
@@ -232,12 +240,14 @@ struct P2pQueue {
   float much;
 };
 hipError_t launch_p2p_order(Cells c, int32_t ncells, Csr list, P2pQueue q, hipStream_t s);
-hipError_t launch_p2p_fp64(Cells c, int32_t ncells, Csr list, Bodies b, double *acc, int per_leaf,
-                           int resident, P2pQueue q, hipStream_t s, double cycle = 0);
+// range: the exponents of the bodies' coordinates and charges (on the device)
+hipError_t launch_p2p_fp64(Cells c, int32_t ncells, Csr list, Bodies b, double *acc,
+                           const BodyRange *range, int per_leaf, int resident, P2pQueue q,
+                           hipStream_t s, double cycle = 0);
 // resident waves on a queue made before, which several launches share
 hipError_t launch_p2p_fp64_drain(Cells c, int32_t ncells, Csr list, Bodies b, double *acc,
-                                 int per_leaf, int waves, P2pQueue q, hipStream_t s,
-                                 double cycle = 0);
+                                 const BodyRange *range, int per_leaf, int waves, P2pQueue q,
+                                 hipStream_t s, double cycle = 0);
 
 // direct.hip
 // target t sums over the n bodies at x, y, z, q: index targets[t] - tbase

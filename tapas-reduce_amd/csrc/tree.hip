@@ -23,62 +23,91 @@ namespace tfmm {
 namespace {
 
 constexpr int BB_THREADS = 256;
+constexpr int BB_WAVES = BB_THREADS / 64;
+
+// What one pass over the bodies finds: the box (lo, hi), which leaves out the first
+// body's x and y, and the exponents of all coordinates and charges.
+struct BoxRange {
+  double lo, hi;
+  BodyRange r;
+
+  static __device__ inline BoxRange none() {
+    return {INFINITY, -INFINITY, {BodyRange::NONE, 0, BodyRange::NONE, 0}};
+  }
+  static __device__ inline void widen(uint32_t &a, uint32_t &b, double v) {
+    const uint32_t e = (uint32_t)__double2hiint(v) >> 20 & 0x7ffu;
+    a = v != 0 ? min(a, e) : a;
+    b = max(b, e);
+  }
+  __device__ inline void box(double v) {
+    lo = fmin(lo, v);
+    hi = fmax(hi, v);
+  }
+  __device__ inline void body(double x, double y, double z, double q, bool first) {
+    box(z);
+    if (!first) {
+      box(x);
+      box(y);
+    }
+    widen(r.lo, r.hi, x);
+    widen(r.lo, r.hi, y);
+    widen(r.lo, r.hi, z);
+    widen(r.qlo, r.qhi, q);
+  }
+  __device__ inline void merge(const BoxRange &o) {
+    lo = fmin(lo, o.lo);
+    hi = fmax(hi, o.hi);
+    merge(o.r);
+  }
+  __device__ inline void merge(const BodyRange &o) {
+    r.lo = min(r.lo, o.lo);
+    r.hi = max(r.hi, o.hi);
+    r.qlo = min(r.qlo, o.qlo);
+    r.qhi = max(r.qhi, o.qhi);
+  }
+  // over the workgroup: whole in thread 0
+  __device__ inline void merge_block() {
+    __shared__ BoxRange part[BB_WAVES];
+    for (int o = 32; o > 0; o >>= 1) {
+      BoxRange b;
+      b.lo = __shfl_xor(lo, o, 64);
+      b.hi = __shfl_xor(hi, o, 64);
+      b.r = {__shfl_xor(r.lo, o, 64), __shfl_xor(r.hi, o, 64), __shfl_xor(r.qlo, o, 64),
+             __shfl_xor(r.qhi, o, 64)};
+      merge(b);
+    }
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = *this;
+    __syncthreads();
+    if (threadIdx.x == 0)
+      for (int w = 1; w < BB_WAVES; w++) merge(part[w]);
+  }
+  __device__ inline void write_region(double *region) const {
+    for (int d = 0; d < 3; d++) {
+      region[d] = lo;
+      region[3 + d] = hi;
+    }
+  }
+};
 
 __global__ __launch_bounds__(BB_THREADS) void k_bbox_partial(const double *x, const double *y,
-                                                             const double *z, int64_t n,
-                                                             double *pmin, double *pmax) {
-  double lo = INFINITY, hi = -INFINITY;
+                                                             const double *z, const double *q,
+                                                             int64_t n, BoxRange *part) {
+  BoxRange b = BoxRange::none();
   for (int64_t i = (int64_t)blockIdx.x * BB_THREADS + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * BB_THREADS) {
-    const double vz = z[i];
-    lo = fmin(lo, vz);
-    hi = fmax(hi, vz);
-    if (i != 0) {
-      const double vx = x[i], vy = y[i];
-      lo = fmin(lo, fmin(vx, vy));
-      hi = fmax(hi, fmax(vx, vy));
-    }
-  }
-  __shared__ double slo[BB_THREADS], shi[BB_THREADS];
-  slo[threadIdx.x] = lo;
-  shi[threadIdx.x] = hi;
-  __syncthreads();
-  for (int o = BB_THREADS / 2; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) {
-      slo[threadIdx.x] = fmin(slo[threadIdx.x], slo[threadIdx.x + o]);
-      shi[threadIdx.x] = fmax(shi[threadIdx.x], shi[threadIdx.x + o]);
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    pmin[blockIdx.x] = slo[0];
-    pmax[blockIdx.x] = shi[0];
-  }
+       i += (int64_t)gridDim.x * BB_THREADS)
+    b.body(x[i], y[i], z[i], q[i], i == 0);
+  b.merge_block();
+  if (threadIdx.x == 0) part[blockIdx.x] = b;
 }
 
-__global__ __launch_bounds__(BB_THREADS) void k_bbox_final(const double *pmin,
-                                                           const double *pmax, int nparts,
-                                                           double *region) {
-  __shared__ double slo[BB_THREADS], shi[BB_THREADS];
-  double lo = INFINITY, hi = -INFINITY;
-  for (int i = threadIdx.x; i < nparts; i += BB_THREADS) {
-    lo = fmin(lo, pmin[i]);
-    hi = fmax(hi, pmax[i]);
-  }
-  slo[threadIdx.x] = lo;
-  shi[threadIdx.x] = hi;
-  __syncthreads();
-  for (int o = BB_THREADS / 2; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) {
-      slo[threadIdx.x] = fmin(slo[threadIdx.x], slo[threadIdx.x + o]);
-      shi[threadIdx.x] = fmax(shi[threadIdx.x], shi[threadIdx.x + o]);
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x < 3) {
-    region[threadIdx.x] = slo[0];
-    region[3 + threadIdx.x] = shi[0];
-  }
+__global__ __launch_bounds__(BB_THREADS) void k_bbox_final(const BoxRange *part, int nparts,
+                                                           double *region, BodyRange *range) {
+  BoxRange b = BoxRange::none();
+  for (int i = threadIdx.x; i < nparts; i += BB_THREADS) b.merge(part[i]);
+  b.merge_block();
+  if (threadIdx.x > 0) return;
+  b.write_region(region);
+  *range = b.r;
 }
 
 // Problem of body i of a forest: the last p with off[p] <= i.
@@ -128,36 +157,27 @@ __global__ void k_keys(const double *x, const double *y, const double *z, const 
 // the same scalar-cube rule as the single-problem box: problem p is its own
 // Partition, so its first body's x and y are the ones left out.
 __global__ __launch_bounds__(BB_THREADS) void k_bbox_forest(const double *x, const double *y,
-                                                            const double *z, const int64_t *off,
-                                                            double *regions) {
+                                                            const double *z, const double *q,
+                                                            const int64_t *off, double *regions,
+                                                            BodyRange *ranges) {
   const int pb = blockIdx.x;
-  const int64_t b = off[pb], e = off[pb + 1];
-  double lo = INFINITY, hi = -INFINITY;
-  for (int64_t i = b + threadIdx.x; i < e; i += BB_THREADS) {
-    const double vz = z[i];
-    lo = fmin(lo, vz);
-    hi = fmax(hi, vz);
-    if (i != b) {
-      const double vx = x[i], vy = y[i];
-      lo = fmin(lo, fmin(vx, vy));
-      hi = fmax(hi, fmax(vx, vy));
-    }
-  }
-  __shared__ double slo[BB_THREADS], shi[BB_THREADS];
-  slo[threadIdx.x] = lo;
-  shi[threadIdx.x] = hi;
-  __syncthreads();
-  for (int o = BB_THREADS / 2; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) {
-      slo[threadIdx.x] = fmin(slo[threadIdx.x], slo[threadIdx.x + o]);
-      shi[threadIdx.x] = fmax(shi[threadIdx.x], shi[threadIdx.x + o]);
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x < 3) {
-    regions[6 * pb + threadIdx.x] = slo[0];
-    regions[6 * pb + 3 + threadIdx.x] = shi[0];
-  }
+  const int64_t first = off[pb], e = off[pb + 1];
+  BoxRange b = BoxRange::none();
+  for (int64_t i = first + threadIdx.x; i < e; i += BB_THREADS)
+    b.body(x[i], y[i], z[i], q[i], i == first);
+  b.merge_block();
+  if (threadIdx.x > 0) return;
+  b.write_region(regions + 6 * pb);
+  ranges[pb] = b.r;
+}
+
+// the forest's range from its problems'
+__global__ __launch_bounds__(BB_THREADS) void k_range_forest(const BodyRange *ranges, int nprob,
+                                                             BodyRange *range) {
+  BoxRange b = BoxRange::none();
+  for (int i = threadIdx.x; i < nprob; i += BB_THREADS) b.merge(ranges[i]);
+  b.merge_block();
+  if (threadIdx.x == 0) *range = b.r;
 }
 
 // Forest order, step 1: after the bodies are sorted by key, the problem of
@@ -564,10 +584,14 @@ hipError_t launch_check_finite(const double *x, const double *y, const double *z
   return hipGetLastError();
 }
 
-hipError_t launch_bbox(const double *x, const double *y, const double *z, int64_t n,
-                       double *partial, int nparts, double *region, hipStream_t s) {
-  k_bbox_partial<<<nparts, BB_THREADS, 0, s>>>(x, y, z, n, partial, partial + nparts);
-  k_bbox_final<<<1, BB_THREADS, 0, s>>>(partial, partial + nparts, nparts, region);
+size_t bbox_part_bytes(int nparts) { return (size_t)nparts * sizeof(BoxRange); }
+
+hipError_t launch_bbox(const double *x, const double *y, const double *z, const double *q,
+                       int64_t n, void *part, int nparts, double *region, BodyRange *range,
+                       hipStream_t s) {
+  BoxRange *p = static_cast<BoxRange *>(part);
+  k_bbox_partial<<<nparts, BB_THREADS, 0, s>>>(x, y, z, q, n, p);
+  k_bbox_final<<<1, BB_THREADS, 0, s>>>(p, nparts, region, range);
   return hipGetLastError();
 }
 
@@ -581,10 +605,12 @@ hipError_t launch_keys(const double *x, const double *y, const double *z, const 
   return hipGetLastError();
 }
 
-hipError_t launch_bbox_forest(const double *x, const double *y, const double *z,
-                              const int64_t *off, int nprob, double *regions, hipStream_t s) {
+hipError_t launch_bbox_forest(const double *x, const double *y, const double *z, const double *q,
+                              const int64_t *off, int nprob, double *regions, BodyRange *range,
+                              hipStream_t s) {
   if (nprob <= 0) return hipSuccess;
-  k_bbox_forest<<<nprob, BB_THREADS, 0, s>>>(x, y, z, off, regions);
+  k_bbox_forest<<<nprob, BB_THREADS, 0, s>>>(x, y, z, q, off, regions, range + 1);
+  k_range_forest<<<1, BB_THREADS, 0, s>>>(range + 1, nprob, range);
   return hipGetLastError();
 }
 
