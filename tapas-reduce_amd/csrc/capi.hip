@@ -174,6 +174,7 @@ struct tfmm_ctx {
   bool codes_ready = false;
   uint32_t n_groups = 0, n_grouped = 0, n_fallback = 0, n_items = 0;
   int group_bits = 0;  // of a key's group field
+  bool repeats = false;  // the last lists repeated a target's place in a group
   bool grouped_keys_in_alt = false;
 
   // picker
@@ -789,9 +790,9 @@ int do_dtt(tfmm_ctx *c) {
   return fail(c, TFMM_EHIP, "traversal lists did not converge");
 }
 
-// An item takes one source per target and mirrored offset, which is all the
-// traversal makes.  Lists that the caller gives (given) may hold more: all but
-// one of them then go to the per-pair kernel.
+// An item takes one source per target and mirrored offset.  Lists that the caller
+// gives may hold more, and so may the traversal's where the centres of neighbouring
+// cells round to one point: all but one of them then go to the per-pair kernel.
 int repeats_to_fallback(tfmm_ctx *c) {
   hipStream_t s = c->stream;
   const uint32_t n = c->n_m2l_exec;
@@ -822,7 +823,7 @@ int repeats_to_fallback(tfmm_ctx *c) {
 
 // Group the executed M2L pairs by (level difference, offset up to mirrors), build
 // the MFMA work items and the per-target list of the pairs outside the groups.
-int build_m2l_batches(tfmm_ctx *c, bool given = false) {
+int build_m2l_batches(tfmm_ctx *c) {
   hipStream_t s = c->stream;
   const Cells k = cells_of(c);
   const uint32_t n = c->n_m2l_exec;
@@ -859,7 +860,7 @@ int build_m2l_batches(tfmm_ctx *c, bool given = false) {
   TRY(dev_reserve(c->fkeys_alt, nn * 8));
   TRY(dev_reserve(c->fvals_alt, nn * 4));
   TRY(dev_reserve(c->g_cnt, 16));
-  if (n_outside || given) TRY(hipMemsetAsync(c->g_cnt.ptr, 0, 16, s));
+  if (n_outside) TRY(hipMemsetAsync(c->g_cnt.ptr, 0, 16, s));
   const int gbits = bits_for(ngr);
   const int sbits = bits_for(c->ncells), fbits = fallback_src_bits(c, sbits);
   {
@@ -871,7 +872,7 @@ int build_m2l_batches(tfmm_ctx *c, bool given = false) {
   if (n_outside == 0) {  // the usual case: no compaction, no read-back
     TRY(launch_m2l_classify_all(dp<int2>(c->m2l_pairs), dp<int32_t>(c->slot_of), n,
                                 dp<uint32_t>(c->g_gid), gbits, dp<uint32_t>(c->gkeys),
-                                dp<uint32_t>(c->gvals), s));
+                                dp<uint32_t>(c->gvals), dp<uint32_t>(c->g_cnt), s));
   } else {
     TRY(launch_m2l_classify(dp<int2>(c->m2l_pairs), dp<int32_t>(c->slot_of), n, dp<uint32_t>(c->g_gid), gbits, fbits,
                             dp<uint32_t>(c->gkeys), dp<uint32_t>(c->gvals), dp<uint64_t>(c->fkeys),
@@ -900,14 +901,14 @@ int build_m2l_batches(tfmm_ctx *c, bool given = false) {
   const size_t nblk = m2l_item_blocks(ngp);
   TRY(dev_reserve(c->it_cnt, nblk * 4));
   TRY(dev_reserve(c->it_start, nblk * 4));
-  uint32_t nitems = 0;
   TRY(launch_m2l_count_items(gk, gvs, ngp, dp<uint32_t>(c->it_cnt), dp<uint32_t>(c->it_start),
-                             c->scan_tmp.ptr, c->h_u32, &nitems, s,
-                             given ? dp<uint32_t>(c->g_cnt) + 2 : nullptr));
-  if (given && c->h_u32[2]) {
+                             c->scan_tmp.ptr, dp<uint32_t>(c->g_cnt), c->h_u32, s));
+  if (c->h_u32[0]) {
+    c->repeats = true;
     const int rc = repeats_to_fallback(c);
     return rc ? rc : build_m2l_batches(c);
   }
+  const uint32_t nitems = c->h_u32[1];
   const size_t ni1 = std::max<uint32_t>(nitems, 1);
   TRY(dev_reserve(c->items, ni1 * 4));
   TRY(dev_reserve(c->cols, ni1 * 16 * 4));
@@ -961,7 +962,7 @@ int p2p_resident(tfmm_ctx *c) { return c->p2p_waves > 0 ? c->p2p_waves * 4 * c->
 // The M2L and P2P pairs of the traversal (c->m2l_pairs with their group
 // slots, c->p2p_pairs, the counters) into sorted lists, M2L batches and the
 // M2L and P2P kernels.
-int run_lists(tfmm_ctx *c, bool given = false) {
+int run_lists(tfmm_ctx *c) {
   hipStream_t s = c->stream;
   const Cells k = cells_of(c);
   const bool mixed = c->prm.precision == TFMM_MIXED;
@@ -1014,7 +1015,8 @@ int run_lists(tfmm_ctx *c, bool given = false) {
                        hipMemcpyDeviceToHost, s));
     return TFMM_OK;
   }
-  rc = build_m2l_batches(c, given);
+  c->repeats = false;
+  rc = build_m2l_batches(c);
   if (rc) {
     if (p2p_early) (void)hipStreamWaitEvent(s, c->ev[EV_P2P1], 0);
     return rc;
@@ -1143,7 +1145,7 @@ int traverse_given(tfmm_ctx *c, const int32_t *m2l, int64_t nm, const int32_t *p
   c->n_m2l_all = m2l_calls;
   c->n_p2p = (uint32_t)pe.size();
   c->n_p2p_calls_leaf = p2p_calls;
-  return run_lists(c, true);
+  return run_lists(c);
 }
 
 int do_downward(tfmm_ctx *c) {
@@ -1389,6 +1391,7 @@ int fused_lists(tfmm_ctx *c) {
     if (rc) return rc;
     c->p2p_forked = true;
   }
+  c->repeats = false;
   rc = cart_direct(c) ? cart_lists(c) : build_m2l_batches(c);
   if (rc) {
     if (c->p2p_forked) (void)hipStreamWaitEvent(s, c->ev[EV_P2PJOIN], 0);
@@ -1561,6 +1564,7 @@ void plan_drop(tfmm_ctx *c) {
 // of everything else.  No plan when the sizes leave no room in the keys.
 void plan_make(tfmm_ctx *c) {
   plan_drop(c);
+  if (c->repeats) return;  // the graph has no way to take them apart
   Plan pl;
   const int L0 = (int)c->tree_hint.size();
   if (L0 < 1 || L0 + 1 > PLAN_MAX_LEVELS || c->dtt_hint.empty()) return;
@@ -1890,7 +1894,8 @@ int whole_record(tfmm_ctx *c) {
     const uint32_t *gk = dp<uint32_t>(galt ? c->gkeys_alt : c->gkeys);
     const uint32_t *gv = dp<uint32_t>(galt ? c->gvals_alt : c->gvals);
     TRY(launch_m2l_count_items_dev(gk, gv, nm, gcnt, dp<uint32_t>(c->it_cnt),
-                                   dp<uint32_t>(c->it_start), c->scan_tmp.ptr, sz + SZ_NITEMS, s));
+                                   dp<uint32_t>(c->it_start), c->scan_tmp.ptr, gcnt, sz + SZ_NITEMS,
+                                   s));
     TRY(launch_m2l_write_items(gk, gv, nm, dp<uint32_t>(c->it_start), cells, dp<uint32_t>(c->items),
                                dp<uint32_t>(c->cols), s, gcnt, pl.caps.items));
     int32_t *chunk = reinterpret_cast<int32_t *>(sz + SZ_CHUNK);

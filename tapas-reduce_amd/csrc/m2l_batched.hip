@@ -111,6 +111,7 @@ __global__ __launch_bounds__(1024) void k_classify(const int2 *pairs, const int3
   critical_path_priority();
   __shared__ uint32_t scratch[17];
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) counters[2] = 0;  // no repeats (k_items)
   if (dn) n = min(n, *dn);
   const bool valid = i < n;
   int2 p = make_int2(0, 0);
@@ -144,9 +145,10 @@ __global__ void k_grouped_count(uint32_t n, const uint32_t *dn, uint32_t *counte
 // k_classify when every pair is in the table: keys and values in pair order
 __global__ void k_classify_all(const int2 *pairs, const int32_t *slot_of, uint32_t n,
                                const uint32_t *gid_of_slot, int gbits, uint32_t *gkeys,
-                               uint32_t *gvals) {
+                               uint32_t *gvals, uint32_t *counters) {
   critical_path_priority();
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) counters[2] = 0;  // no repeats (k_items)
   if (i >= n) return;
   const int2 p = pairs[i];
   const uint32_t slot = (uint32_t)slot_of[i];
@@ -233,10 +235,11 @@ __global__ void k_scale_m(Cells c, int32_t ncells, const double *M, T *Mq) {
 // the second, with the exclusive prefix of the blocks' counts in bstart,
 // writes every item's key and 16 column words (empty: empty).  With dn the
 // pair count is *dn (n its capacity); items at or past items_cap are not
-// written (a capacity the caller checks).  Lists that the caller of the library
-// gives may repeat a target's place in a group (a pair twice, or sources of two
-// problems); the counting pass then sets *repeats.  (A segment longer than the
-// block can see has a repeat among the 129 keys that it does see.)
+// written (a capacity the caller checks).  A target's place in a group may
+// repeat: in lists that the caller of the library gives, and in the library's own
+// where cells are as narrow as the last place of their coordinates, so that centres
+// round together.  The counting pass then sets *repeats.  (A segment longer than
+// the block can see has a repeat among the 129 keys that it does see.)
 constexpr int IT_THREADS = 1024;
 constexpr int IT_ROWS = IT_THREADS / 64 + 2;  // 2 rows after the block's own
 constexpr int SEG_WORDS = TILE * 8 / 32;      // words of a segment's mask
@@ -293,7 +296,7 @@ __global__ __launch_bounds__(IT_THREADS) void k_items(const uint32_t *keys, cons
     const uint32_t v = vals[w0 + t];
     const uint32_t sl = (v >> SRC_BITS) & (TILE - 1), mi = v >> MIR_AT;
     const uint32_t bit = 1u << (8 * (sl & 3) + mi);
-    if ((atomicOr(&mask[s * SEG_WORDS + (sl >> 2)], bit) & bit) && !WRITE && repeats) *repeats = 1;
+    if ((atomicOr(&mask[s * SEG_WORDS + (sl >> 2)], bit) & bit) && !WRITE) *repeats = 1;
     segkey[s] = sk[t];
   }
   __syncthreads();
@@ -860,10 +863,10 @@ int32_t m2l_group_slots() { return m2lg::SLOTS; }
 
 hipError_t launch_m2l_classify_all(const int2 *pairs, const int32_t *slot_of, uint32_t n,
                                    const uint32_t *gid_of_slot, int gbits, uint32_t *gkeys,
-                                   uint32_t *gvals, hipStream_t s) {
+                                   uint32_t *gvals, uint32_t *counters, hipStream_t s) {
   if (n == 0) return hipSuccess;
   k_classify_all<<<(n + 255) / 256, 256, 0, s>>>(pairs, slot_of, n, gid_of_slot, gbits, gkeys,
-                                                 gvals);
+                                                 gvals, counters);
   return hipGetLastError();
 }
 
@@ -903,30 +906,6 @@ uint32_t m2l_item_blocks(uint32_t n) {
   return std::max<uint32_t>(1, (n + IT_THREADS - 1) / IT_THREADS);
 }
 
-hipError_t launch_m2l_count_items(const uint32_t *keys, const uint32_t *vals, uint32_t n,
-                                  uint32_t *bcount, uint32_t *bstart, void *scan_tmp,
-                                  uint32_t *h_pinned, uint32_t *nitems_out, hipStream_t s,
-                                  uint32_t *repeats) {
-  *nitems_out = 0;
-  h_pinned[2] = 0;
-  if (n == 0) return hipSuccess;
-  const unsigned nb = m2l_item_blocks(n);
-  k_items<false><<<nb, IT_THREADS, 0, s>>>(keys, vals, n, bcount, nullptr, 0, nullptr, nullptr,
-                                           nullptr, 0, repeats);
-  hipError_t e = scan_exclusive_u32(bcount, bstart, nb, scan_tmp, s);
-  if (e != hipSuccess) return e;
-  e = hipMemcpyAsync(h_pinned, bstart + (nb - 1), 4, hipMemcpyDeviceToHost, s);
-  if (e != hipSuccess) return e;
-  e = hipMemcpyAsync(h_pinned + 1, bcount + (nb - 1), 4, hipMemcpyDeviceToHost, s);
-  if (e != hipSuccess) return e;
-  if (repeats) e = hipMemcpyAsync(h_pinned + 2, repeats, 4, hipMemcpyDeviceToHost, s);
-  if (e != hipSuccess) return e;
-  e = hipStreamSynchronize(s);
-  if (e != hipSuccess) return e;
-  *nitems_out = h_pinned[0] + h_pinned[1];
-  return hipGetLastError();
-}
-
 // the item count on the device: the block counts summed
 __global__ void k_items_total(const uint32_t *bcount, const uint32_t *bstart, uint32_t nb,
                               uint32_t *nitems) {
@@ -935,14 +914,28 @@ __global__ void k_items_total(const uint32_t *bcount, const uint32_t *bstart, ui
 
 hipError_t launch_m2l_count_items_dev(const uint32_t *keys, const uint32_t *vals, uint32_t n,
                                       const uint32_t *dn, uint32_t *bcount, uint32_t *bstart,
-                                      void *scan_tmp, uint32_t *nitems, hipStream_t s) {
+                                      void *scan_tmp, uint32_t *counters, uint32_t *nitems,
+                                      hipStream_t s) {
   const unsigned nb = m2l_item_blocks(n);
   k_items<false><<<nb, IT_THREADS, 0, s>>>(keys, vals, n, bcount, nullptr, 0, nullptr, nullptr, dn,
-                                           0, nullptr);
+                                           0, counters + 2);
   hipError_t e = scan_exclusive_u32(bcount, bstart, nb, scan_tmp, s);
   if (e != hipSuccess) return e;
   k_items_total<<<1, 64, 0, s>>>(bcount, bstart, nb, nitems);
   return hipGetLastError();
+}
+
+hipError_t launch_m2l_count_items(const uint32_t *keys, const uint32_t *vals, uint32_t n,
+                                  uint32_t *bcount, uint32_t *bstart, void *scan_tmp,
+                                  uint32_t *counters, uint32_t *h_pinned, hipStream_t s) {
+  h_pinned[0] = h_pinned[1] = 0;
+  if (n == 0) return hipSuccess;
+  hipError_t e = launch_m2l_count_items_dev(keys, vals, n, nullptr, bcount, bstart, scan_tmp,
+                                            counters, counters + 3, s);
+  if (e != hipSuccess) return e;
+  e = hipMemcpyAsync(h_pinned, counters + 2, 8, hipMemcpyDeviceToHost, s);
+  if (e != hipSuccess) return e;
+  return hipStreamSynchronize(s);
 }
 
 hipError_t launch_m2l_write_items(const uint32_t *keys, const uint32_t *vals, uint32_t n,

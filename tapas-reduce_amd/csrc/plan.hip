@@ -81,6 +81,7 @@ __global__ void k_plan_check(const uint32_t *cnt, int nsteps, const uint32_t *st
   }
   if (cnt[16 + nsteps] > caps.front) st |= ST_TRAVERSAL;
   if (gcnt[1] > caps.fallback) st |= ST_FALLBACK;
+  if (gcnt[2]) st |= ST_REPEATS;
   if (sz[SZ_NITEMS] > caps.items) st |= ST_ITEMS;
   const uint32_t units = ntiles > 0 ? uoff[ntiles - 1] + ucnt[ntiles - 1] : 0u;
   sz[SZ_NUNITS] = units;

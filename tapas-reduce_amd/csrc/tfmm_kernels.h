@@ -56,7 +56,8 @@ enum : uint32_t {
   ST_ITEMS = 32,
   ST_UNITS = 64,
   ST_FALLBACK = 128,
-  ST_SORT = 256       // bodies out of order (a run too long for launch_sort_runs)
+  ST_SORT = 256,      // bodies out of order (a run too long for launch_sort_runs)
+  ST_REPEATS = 512    // a target's place in an M2L group twice
 };
 struct PlanCaps {
   uint32_t m2l, p2p, front, items, units, fallback;
@@ -270,7 +271,7 @@ size_t m2l_codes_bytes();
 // every pair in the group table: grouped keys and values in pair order
 hipError_t launch_m2l_classify_all(const int2 *pairs, const int32_t *slot_of, uint32_t n,
                                    const uint32_t *gid_of_slot, int gbits, uint32_t *gkeys,
-                                   uint32_t *gvals, hipStream_t s);
+                                   uint32_t *gvals, uint32_t *counters, hipStream_t s);
 // Grouped keys and values at the pair's index, the key 0xffffffff (after
 // every grouped key) for a pair outside the groups, which is appended to
 // fkeys/fvals; counters[1] = pairs outside, counters[0] = grouped pairs.  A
@@ -290,17 +291,20 @@ hipError_t launch_m2l_scale_m(Cells c, int32_t ncells, const double *M, void *Mq
 // bytes of the scaled multipoles (one cell more: the source of empty columns)
 size_t m2l_mq_bytes(int64_t ncells, bool fp32);
 // items of the (set, group)-sorted grouped pairs, counted per block of pairs
-// (m2l_item_blocks words in bcount and bstart) and read back
+// (m2l_item_blocks words in bcount and bstart) and read back: h_pinned[0] is not 0
+// where a target's place in a group repeats (nothing that follows is then of use),
+// h_pinned[1] the items.  counters: the classification's, which clears its word 2,
+// the repeats; word 3 the items
 uint32_t m2l_item_blocks(uint32_t n);
 hipError_t launch_m2l_count_items(const uint32_t *keys, const uint32_t *vals, uint32_t n,
                                   uint32_t *bcount, uint32_t *bstart, void *scan_tmp,
-                                  uint32_t *h_pinned, uint32_t *nitems_out, hipStream_t s,
-                                  uint32_t *repeats = nullptr);
-// the same with the pair count *dn on the device (n its capacity) and the
-// item count left on the device in *nitems
+                                  uint32_t *counters, uint32_t *h_pinned, hipStream_t s);
+// the same with the pair count *dn on the device (n its capacity), nothing read
+// back and the item count in *nitems
 hipError_t launch_m2l_count_items_dev(const uint32_t *keys, const uint32_t *vals, uint32_t n,
                                       const uint32_t *dn, uint32_t *bcount, uint32_t *bstart,
-                                      void *scan_tmp, uint32_t *nitems, hipStream_t s);
+                                      void *scan_tmp, uint32_t *counters, uint32_t *nitems,
+                                      hipStream_t s);
 // every item's key and 16 column words (ncells: as the launch of the set
 // kernel); items at or past items_cap are not written
 hipError_t launch_m2l_write_items(const uint32_t *keys, const uint32_t *vals, uint32_t n,
