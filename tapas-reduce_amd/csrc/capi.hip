@@ -20,8 +20,11 @@
 #include "tfmm_device.h"
 #include "tfmm_internal.h"
 #include "tfmm_kernels.h"
+#include "tree_hints.h"
 
 using namespace tfmm;
+
+static_assert(KEY_LEVELS == MAXDEPTH, "a whole key sorts by every level");
 
 namespace {
 
@@ -360,12 +363,6 @@ int image_range(const tfmm_ctx *c) {
   for (int i = 0; i < c->images; i++, p3 *= 3) r += p3;
   return r;
 }
-int bits_for(int64_t v) {
-  int b = 1;
-  while (b < 62 && (((int64_t)1 << b) <= v)) b++;
-  return b;
-}
-
 // source field of the fallback M2L keys (target << bits | source word): the cell,
 // with periodic images the whole 32-bit source word
 int fallback_src_bits(const tfmm_ctx *c, int cell_bits) { return c->images > 0 ? 32 : cell_bits; }
@@ -387,34 +384,23 @@ int check_params(tfmm_ctx *c, const tfmm_params *p) {
 // synchronous way (a level outgrew its grid, the cell capacity or the
 // hinted depth), 2 when the bodies have to be sorted again by their whole keys,
 // or an error.
-int build_levels_hinted(tfmm_ctx *c, int64_t n, const int64_t *off, int np,
+int build_levels_hinted(tfmm_ctx *c, const LevelGrids &g, int64_t n, const int64_t *off, int np,
                         const uint64_t *skeys, const uint32_t *sprob) {
   hipStream_t s = c->stream;
-  const int L = (int)c->tree_hint.size();
-  if (2 * (L + 1) + 1 > H_U32_WORDS) return 1;
-  std::vector<int32_t> grid(L);
-  int64_t total = 0, gmax = 0;
-  for (int d = 0; d < L; d++) {
-    const int64_t h = c->tree_hint[d];
-    grid[d] = (int32_t)std::min<int64_t>(INT32_MAX / 16, h + h / 8 + 256);
-    if (d == 0) grid[d] = std::max<int32_t>(grid[d], np);
-    total += grid[d];
-    gmax = std::max<int64_t>(gmax, grid[d]);
-  }
-  if (total + 4096 > INT32_MAX / 2) return 1;
-  TRY(reserve_cells(c, (size_t)total + 4096, 0, s));
+  const int L = (int)g.grid.size();
+  TRY(reserve_cells(c, (size_t)g.cells + 4096, 0, s));
   const int32_t cap = (int32_t)std::min<size_t>(c->cell_cap, INT32_MAX / 2);
   TRY(dev_reserve(c->lev, (size_t)2 * (L + 1) * 4));
-  TRY(dev_reserve(c->flag, (size_t)gmax * 4 + 1024));
-  TRY(dev_reserve(c->slot, (size_t)gmax * 4 + 1024));
-  TRY(dev_reserve(c->lev_bsum, (size_t)level_blocks((int32_t)gmax) * 4 + 4));
+  TRY(dev_reserve(c->flag, (size_t)g.largest * 4 + 1024));
+  TRY(dev_reserve(c->slot, (size_t)g.largest * 4 + 1024));
+  TRY(dev_reserve(c->lev_bsum, (size_t)level_blocks((int32_t)g.largest) * 4 + 4));
   const Cells k = cells_of(c);
   int32_t *lev = dp<int32_t>(c->lev);
   const int top = tree_top_levels(c->tree_hint.data(), L);
   TRY(launch_tree_top(k, n, off, np, lev, L, top, c->prm.ncrit, cap, dp<uint32_t>(c->lev_status),
                       skeys, dp<double>(c->region), sprob, dp<uint32_t>(c->lev_status) + 1, s));
   for (int d = top; d < L; d++)
-    TRY(launch_level_step(k, lev, d, grid[d], c->prm.ncrit, cap, dp<uint32_t>(c->flag),
+    TRY(launch_level_step(k, lev, d, g.grid[d], c->prm.ncrit, cap, dp<uint32_t>(c->flag),
                           dp<uint32_t>(c->slot), dp<uint32_t>(c->lev_bsum),
                           dp<uint32_t>(c->lev_status), skeys, dp<double>(c->region), sprob, s));
   TRY(hipMemcpyAsync(c->h_u32, lev, (size_t)2 * (L + 1) * 4, hipMemcpyDeviceToHost, s));
@@ -445,17 +431,10 @@ hipError_t sort_runs(tfmm_ctx *c, bool alt, const uint32_t *sprob, int shift, ui
                           dp<uint32_t>(alt ? c->idx : c->idx_alt), long_run, c->stream);
 }
 
-// Leading key bits to sort the bodies by before the runs that agree on them
-// (launch_sort_runs), 63 for all of them.  At the depth of the last tree a cell
-// holds at most ncrit bodies; bodies spread evenly agree in a few at n's bits.
-// Whole passes of 9 bits; with six or more the runs would save nothing.
-int key_prefix_bits(const tfmm_ctx *c) {
-  if (c->tree_hint.empty()) return 3 * MAXDEPTH;
-  int levels = (int)c->tree_hint.size() - 1 + c->sort_extra;
-  for (int64_t m = c->prm.ncrit; m > 128; m /= 4) levels++;
-  const int bits = std::max({3 * levels, bits_for(c->n) - 4, 1});
-  const int passes = (bits + 8) / 9;
-  return passes >= 6 ? 3 * MAXDEPTH : 9 * passes;
+// key_prefix_bits for this context's bodies
+int key_prefix(const tfmm_ctx *c, bool on_device) {
+  return key_prefix_bits(on_device, (int)c->tree_hint.size() - 1 + c->sort_extra, c->n,
+                         c->prm.ncrit);
 }
 
 int do_build_tree(tfmm_ctx *c, bool whole_keys = false) {
@@ -463,7 +442,9 @@ int do_build_tree(tfmm_ctx *c, bool whole_keys = false) {
   const int64_t n = c->n;
   TRY(dev_reserve(c->lev_status, 8));
   uint32_t *long_run = dp<uint32_t>(c->lev_status) + 1;
-  const int prefix = whole_keys ? 3 * MAXDEPTH : key_prefix_bits(c);
+  const int np = c->nprob;
+  const LevelGrids grids = level_grids(c->tree_hint, np, H_U32_WORDS);
+  const int prefix = whole_keys ? WHOLE_KEY : key_prefix(c, grids.fits);
   const int key_end = DEPTHBITS + 3 * MAXDEPTH;
   TRY(dev_reserve(c->keys, n * 8));
   TRY(dev_reserve(c->keys_alt, n * 8));
@@ -475,7 +456,6 @@ int do_build_tree(tfmm_ctx *c, bool whole_keys = false) {
   TRY(dev_reserve(c->sz, n * 8));
   TRY(dev_reserve(c->sq, n * 8));
   TRY(dev_reserve(c->perm, n * 4));
-  const int np = c->nprob;
   const bool forest = np > 1;
   TRY(dev_reserve(c->region, 6 * 8 * (size_t)np));
   TRY(dev_reserve(c->range, sizeof(BodyRange) * ((size_t)np + 1)));
@@ -524,7 +504,7 @@ int do_build_tree(tfmm_ctx *c, bool whole_keys = false) {
                               dp<uint32_t>(alt ? c->idx : c->idx_alt), s));
     alt = !alt;
   }
-  if (prefix < 3 * MAXDEPTH) {
+  if (prefix < WHOLE_KEY) {
     TRY(sort_runs(c, alt, sprob, key_end - prefix, long_run));
     alt = !alt;
   }
@@ -536,8 +516,8 @@ int do_build_tree(tfmm_ctx *c, bool whole_keys = false) {
 
   // level-synchronous cell build: without a host round trip per level when
   // an earlier tree gives the level sizes to size the grids by
-  if (!c->tree_hint.empty()) {
-    int rc = build_levels_hinted(c, n, off, np, skeys, sprob);
+  if (grids.fits) {
+    int rc = build_levels_hinted(c, grids, n, off, np, skeys, sprob);
     if (rc < 0) return rc;
     if (rc == 2) {  // these bodies are closer together than the last ones
       c->sort_extra += 2;
@@ -1589,7 +1569,7 @@ void plan_make(tfmm_ctx *c) {
     pl.cells += pl.grid[d];
   }
   pl.top = tree_top_levels(c->tree_hint.data(), L0);
-  pl.key_bits = key_prefix_bits(c);
+  pl.key_bits = key_prefix(c, true);
   if (pl.cells > INT32_MAX / 4) return;
   pl.max_depth = pl.L - 1;
   pl.nsteps = 2 * pl.max_depth + 2;
@@ -1798,7 +1778,7 @@ int whole_record(tfmm_ctx *c) {
                               dp<uint32_t>(alt ? c->idx : c->idx_alt), s));
     alt = !alt;
   }
-  if (pl.key_bits < 3 * MAXDEPTH) {
+  if (pl.key_bits < WHOLE_KEY) {
     TRY(sort_runs(c, alt, sprob, key_end - pl.key_bits, long_run));
     alt = !alt;
   }
