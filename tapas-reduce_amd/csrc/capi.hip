@@ -107,7 +107,7 @@ struct tfmm_ctx {
   DevBuf flag, slot, scan_tmp, lev, lev_bsum, lev_status;
   std::vector<int32_t> lvl;
   std::vector<int32_t> tree_hint;  // cells per level of the last tree
-  int sort_extra = 0;              // levels more to sort the bodies by (do_build_tree)
+  SortDepth sort_depth;            // levels more to sort the bodies by
   int64_t ncells = 0, nleaves = 0;
   bool keys_in_alt = false;
   double h_region[6] = {0, 0, 0, 0, 0, 0};
@@ -433,7 +433,7 @@ hipError_t sort_runs(tfmm_ctx *c, bool alt, const uint32_t *sprob, int shift, ui
 
 // key_prefix_bits for this context's bodies
 int key_prefix(const tfmm_ctx *c, bool on_device) {
-  return key_prefix_bits(on_device, (int)c->tree_hint.size() - 1 + c->sort_extra, c->n,
+  return key_prefix_bits(on_device, (int)c->tree_hint.size() - 1 + c->sort_depth.extra, c->n,
                          c->prm.ncrit);
 }
 
@@ -519,8 +519,9 @@ int do_build_tree(tfmm_ctx *c, bool whole_keys = false) {
   if (grids.fits) {
     int rc = build_levels_hinted(c, grids, n, off, np, skeys, sprob);
     if (rc < 0) return rc;
+    if (rc != 2 && !whole_keys) c->sort_depth.sorted();
     if (rc == 2) {  // these bodies are closer together than the last ones
-      c->sort_extra += 2;
+      c->sort_depth.long_run();
       return do_build_tree(c, true);
     }
     if (rc == 0) {

@@ -53,4 +53,27 @@ inline int key_prefix_bits(bool on_device, int levels, int64_t n, int64_t ncrit)
   return passes >= 6 ? WHOLE_KEY : 9 * passes;
 }
 
+// Levels to sort by beyond the last tree's: two more for every build that met a run
+// too long, and two fewer again, on trial, after `patience` builds that met none (the
+// context may hold other bodies by then).  A trial that fails costs one sort, and
+// doubles the patience.
+struct SortDepth {
+  static constexpr int STEP = 2, CALM = 16, MOST = 1024;
+  int extra = 0, calm = 0, patience = CALM;
+  bool trial = false;
+
+  void long_run() {
+    extra += STEP;
+    calm = 0;
+    if (trial) patience = std::min(2 * patience, MOST);
+    trial = false;
+  }
+  void sorted() {
+    if (extra == 0 || ++calm < patience) return;
+    extra -= STEP;
+    calm = 0;
+    trial = true;
+  }
+};
+
 }  // namespace tfmm

@@ -38,7 +38,37 @@ static bool whole_keys_without_the_device_build() {
   return level_grids({1, 8}, 5000, 256).grid[0] == 5000;
 }
 
+// evaluations of bodies that need `need` levels more than the tree has; the long
+// runs among them
+static int evaluate(SortDepth &d, int need, int times) {
+  int longs = 0;
+  for (int i = 0; i < times; i++) {
+    if (d.extra < need) {
+      d.long_run();
+      longs++;
+    } else {
+      d.sorted();
+    }
+  }
+  return longs;
+}
+
+// A context that saw clustered bodies sorts even ones by few bits again; one that
+// keeps its clustered bodies seldom sorts twice.
+static bool depth_comes_back() {
+  SortDepth d;
+  if (evaluate(d, 0, 100) != 0 || d.extra != 0) return false;
+  if (evaluate(d, 8, 10) != 4 || d.extra != 8) return false;
+  evaluate(d, 0, 200);
+  if (d.extra != 0) return false;
+  evaluate(d, 8, 10);
+  if (evaluate(d, 8, 10000) > 20) return false;
+  evaluate(d, 0, 5000);
+  return d.extra == 0;
+}
+
 int main() {
+  if (!depth_comes_back()) return printf("depth\n"), 1;
   if (!whole_keys_without_the_device_build()) return printf("whole keys\n"), 1;
   printf("ok\n");
   return 0;
