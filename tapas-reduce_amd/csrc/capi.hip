@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../../include/tfmm.h"
+#include "p2p_outlook.h"
 #include "tfmm_device.h"
 #include "tfmm_internal.h"
 #include "tfmm_kernels.h"
@@ -155,7 +156,7 @@ struct tfmm_ctx {
   DevBuf gsz, gstep;              // its device sizes and traversal step grids
   uint32_t *h_plan = nullptr;     // pinned read-back of the whole graph (PLAN_HOST_BYTES)
   bool upward_early = false;  // the running evaluation's upward pass (early_upward)
-  bool p2p_heavy = false;     // the last evaluation's p2p_outweighs
+  P2pOutlook p2p_outlook;     // p2p_outweighs of the last evaluations
   bool upward_pending = false;  // the early upward pass is still to be enqueued
   bool one_graph = false;         // the last tfmm_evaluate was one launch of it
   // periodic images (tfmm_set_periodic): image sublevels, 0 = none, and the
@@ -1237,6 +1238,11 @@ bool p2p_outweighs(const tfmm_ctx *c, uint64_t body_pairs, uint32_t m2l) {
   return leaf_waves(c) == 1 && p2p > P2P_HEAVY * far;
 }
 
+P2pProblem p2p_problem(const tfmm_ctx *c) {
+  return {c->n, c->prm.theta, c->nprob, c->prm.ncrit, c->prm.precision, c->prm.mutual, c->basis,
+          c->images};
+}
+
 int fork_p2p(tfmm_ctx *c, int64_t ncells = -1) {
   hipStream_t s = c->stream;
   const Cells k = cells_of(c);
@@ -1319,7 +1325,7 @@ int fused_prepare(tfmm_ctx *c) {
   c->run_schedule = c->p2p_schedule;
   c->run_waves = c->p2p_waves;
   // the P2P's start is chosen after the traversal; until then as the last time
-  if (p2p_chosen(c) && c->p2p_heavy) c->run_schedule = 2;
+  if (p2p_chosen(c) && c->p2p_outlook.heavy(p2p_problem(c))) c->run_schedule = 2;
   c->upward_early = early_upward(c);
   TRY(reserve_expansions(c));
   TRY(dev_reserve(c->leaf_of, (size_t)c->n * 4));
@@ -1361,9 +1367,10 @@ int fused_lists(tfmm_ctx *c) {
   TRY(dev_reserve(c->acc, (size_t)c->n * 32));
   TRY(dev_reserve(c->p2p_order, (size_t)c->ncells * 4));
   if (p2p_chosen(c)) {
-    c->p2p_heavy = p2p_outweighs(c, c->n_p2p_pairs, c->n_m2l_exec);
-    c->run_schedule = c->p2p_heavy ? 2 : 0;
-    c->run_waves = c->p2p_heavy ? (mixed ? 3 : 2) : 0;
+    const bool heavy = p2p_outweighs(c, c->n_p2p_pairs, c->n_m2l_exec);
+    c->p2p_outlook.saw(p2p_problem(c), heavy);
+    c->run_schedule = heavy ? 2 : 0;
+    c->run_waves = heavy ? (mixed ? 3 : 2) : 0;
   }
   if (c->run_schedule >= 2 && c->use_graph != 1) {
     // the P2P list is complete: start the P2P now, beside the M2L batch
