@@ -260,7 +260,7 @@ int tfmm_get_lists(tfmm_ctx *ctx, int32_t *m2l_off, int32_t *m2l_src, int32_t *p
  * tfmm_evaluate, 0 (default) starts it with the numeric phase, beside the M2L
  * kernels, or, without resident waves (TFMM_TUNE_P2P_WAVES 0) and where the
  * traversal finds that the P2P outweighs the M2L, as 2 with a few resident
- * waves of the library's choice; 1 starts it with the M2L set kernel; 2 as soon as
+ * waves of the library's choice (TFMM_TUNE_P2P_CHOICE); 1 starts it with the M2L set kernel; 2 as soon as
  * its list is sorted, beside the M2L batch building (also inside the
  * one-launch graph of TFMM_TUNE_GRAPH 2; with TFMM_TUNE_GRAPH 1 as 0); 3 as 2.  A
  * resident P2P (TFMM_TUNE_P2P_WAVES > 0) holds its few waves until the critical
@@ -315,13 +315,18 @@ int tfmm_get_lists(tfmm_ctx *ctx, int32_t *m2l_off, int32_t *m2l_src, int32_t *p
  * (5005 multiply-adds per pair) on every pair of the list.  A change makes
  * the expansions again (as tfmm_set_basis). */
 #define TFMM_TUNE_CART_M2L 7
+/* TFMM_TUNE_P2P_CHOICE: 1 (default) lets the library choose the P2P's start
+ * and its resident waves where TFMM_TUNE_P2P_SCHEDULE and
+ * TFMM_TUNE_P2P_WAVES are both 0; 0 takes them as they are, the P2P as one
+ * workgroup per cell from the start of the numeric phase. */
+#define TFMM_TUNE_P2P_CHOICE 8
 int tfmm_set_tuning(tfmm_ctx *ctx, int knob, double value);
 int tfmm_get_tuning(tfmm_ctx *ctx, int knob, double *value);
 /* Autotuner: evaluates the current bodies with params, reps times per
  * candidate (after 2 uncounted evaluations of the candidate, which let the
  * device settle to the setting), in two stages -- the set-kernel knobs (unit factor {0, 1.5,
  * 2, 3} x XCD run {8, 16, 32, 64}) at the current P2P setting, then the
- * P2P's schedule {0, 1, 2} x resident waves {0, 3, 4} (waves for mixed
+ * P2P's schedule (0 without waves: as TFMM_TUNE_P2P_CHOICE is set) {0, 1, 2} x resident waves {0, 3, 4} (waves for mixed
  * precision only, schedule 2 not with TFMM_TUNE_GRAPH 1) at the best tile
  * setting --
  * and keeps the setting whose evaluation was fastest (median).  chosen (4

@@ -59,7 +59,7 @@ struct Plan {
   int nprob = 0;
   tfmm_params prm{};
   double unit_factor = 0;
-  int xcd_run = 0, p2p_schedule = 0, p2p_waves = 0;
+  int xcd_run = 0, p2p_schedule = 0, p2p_waves = 0, p2p_choice = 0;
   // capacities
   int L = 0;                        // tree levels
   std::vector<int32_t> grid;        // cells per level
@@ -143,6 +143,7 @@ struct tfmm_ctx {
   int p2p_schedule = 0;          // where the P2P starts (TFMM_TUNE_P2P_SCHEDULE)
   int use_graph = 0;             // tfmm_evaluate's numeric phase as one hipGraph
   int p2p_waves = 0;             // resident P2P waves per SIMD (0: one workgroup per cell)
+  int p2p_choice = 1;            // the library may choose the two (TFMM_TUNE_P2P_CHOICE)
   int run_schedule = 0, run_waves = 0;  // the two as the running evaluation takes them
   int n_cu = 0;                  // compute units of the device
   DevBuf p2p_next, p2p_order;    // the resident P2P's counters and targets
@@ -1217,7 +1218,8 @@ int drain_p2p(tfmm_ctx *c, int64_t ncells, bool l2l_done) {
   return TFMM_OK;
 }
 
-// With neither P2P knob set (schedule 0, no resident waves) the library chooses.
+// With neither P2P knob set (schedule 0, no resident waves) the library chooses,
+// unless TFMM_TUNE_P2P_CHOICE keeps it from that.
 // Where the P2P is the larger part of the work beside the M2L, it starts as soon as
 // its list is sorted, as schedule 2, as resident waves that leave the M2L's waves
 // room (3 a SIMD in FP32, 2 in FP64), and a full launch takes the rest at the end:
@@ -1228,7 +1230,7 @@ int drain_p2p(tfmm_ctx *c, int64_t ncells, bool l2l_done) {
 // item.
 constexpr double P2P_HEAVY = 1.3;
 bool p2p_chosen(const tfmm_ctx *c) {
-  return c->p2p_schedule == 0 && c->p2p_waves == 0 && c->use_graph != 1;
+  return c->p2p_choice && c->p2p_schedule == 0 && c->p2p_waves == 0 && c->use_graph != 1;
 }
 
 bool p2p_outweighs(const tfmm_ctx *c, uint64_t body_pairs, uint32_t m2l) {
@@ -1539,7 +1541,7 @@ bool plan_fits(tfmm_ctx *c, const tfmm_params *p) {
          pl.prm.theta == p->theta && pl.prm.precision == p->precision &&
          pl.prm.mutual == p->mutual && pl.unit_factor == c->m2l_unit_factor &&
          pl.xcd_run == c->m2l_xcd_run && pl.p2p_schedule == c->p2p_schedule &&
-         pl.p2p_waves == c->p2p_waves;
+         pl.p2p_waves == c->p2p_waves && pl.p2p_choice == c->p2p_choice;
 }
 
 void plan_drop(tfmm_ctx *c) {
@@ -1564,6 +1566,7 @@ void plan_make(tfmm_ctx *c) {
   pl.xcd_run = c->m2l_xcd_run;
   pl.p2p_schedule = c->p2p_schedule;
   pl.p2p_waves = c->p2p_waves;
+  pl.p2p_choice = c->p2p_choice;
   pl.run_schedule = c->run_schedule;
   pl.run_waves = c->run_waves;
   pl.L = L0 + 1;
@@ -2216,6 +2219,10 @@ int tfmm_set_tuning(tfmm_ctx *c, int knob, double value) {
         if (cartesian(c) && c->stage > 1) c->stage = 1;  // the expansions are made again
       }
       return TFMM_OK;
+    case TFMM_TUNE_P2P_CHOICE:
+      if (value != 0 && value != 1) return fail(c, TFMM_EINVAL, "P2P choice must be 0 or 1");
+      c->p2p_choice = (int)value;
+      return TFMM_OK;
     default:
       return fail(c, TFMM_EINVAL, "unknown tuning knob");
   }
@@ -2346,6 +2353,7 @@ int tfmm_get_tuning(tfmm_ctx *c, int knob, double *value) {
     case TFMM_TUNE_P2P_WAVES: *value = c->p2p_waves; return TFMM_OK;
     case TFMM_TUNE_DEVICE_LIMIT: *value = (double)dev_limit(); return TFMM_OK;
     case TFMM_TUNE_CART_M2L: *value = c->cart_direct; return TFMM_OK;
+    case TFMM_TUNE_P2P_CHOICE: *value = c->p2p_choice; return TFMM_OK;
     default: return fail(c, TFMM_EINVAL, "unknown tuning knob");
   }
 }
