@@ -100,7 +100,11 @@ typedef struct {
                                 j <= i of a leaf with itself) */
   uint64_t n_p2p_self;       /* r == 0 self pairs among them */
   /* milliseconds of the last evaluation, measured with HIP events on the
-   * context stream; kernel entries are summed over their launches */
+   * context stream; kernel entries are summed over their launches.
+   * ms_traverse: the traversal, the lists, the M2L and the wait for the P2P;
+   * ms_downward: L2L and L2P, wherever the L2L stands.  In tfmm_evaluate the
+   * upward pass may run on the second stream, beside the traversal: the
+   * phases then add up to more than ms_total. */
   double ms_tree, ms_upward, ms_traverse, ms_downward, ms_total;
   double ms_p2p, ms_m2l, ms_dtt;
   /* M2L batching: offset groups (offsets up to mirroring), MFMA work items

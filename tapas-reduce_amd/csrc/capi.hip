@@ -44,6 +44,8 @@ enum Ev {
   EV_P2P0,
   EV_P2P1,
   EV_P2PJOIN,  // the P2P stream's end, for the join only (never timed)
+  EV_L2L0,     // an L2L that stands before the join: its start, after a drain (else EV_M2L1)
+  EV_L2L1,     // and its end
   EV_TRAV,
   EV_DOWN,
   EV_COUNT
@@ -157,6 +159,7 @@ struct tfmm_ctx {
   DevBuf gsz, gstep;              // its device sizes and traversal step grids
   uint32_t *h_plan = nullptr;     // pinned read-back of the whole graph (PLAN_HOST_BYTES)
   bool upward_early = false;  // the running evaluation's upward pass (early_upward)
+  bool l2l_first = false;     // its L2L stands before the P2P's join (EV_L2L1)
   P2pOutlook p2p_outlook;     // p2p_outweighs of the last evaluations
   bool upward_pending = false;  // the early upward pass is still to be enqueued
   bool one_graph = false;         // the last tfmm_evaluate was one launch of it
@@ -1212,8 +1215,10 @@ hipError_t p2p_on_counter(tfmm_ctx *c, int64_t ncells, int waves, hipStream_t st
                                period(c));
 }
 
+bool drains_before_l2l(const tfmm_ctx *c) { return p2p_drains(c) && c->run_schedule == 3; }
+
 int drain_p2p(tfmm_ctx *c, int64_t ncells, bool l2l_done) {
-  if (!p2p_drains(c) || l2l_done == (c->run_schedule == 3)) return TFMM_OK;
+  if (!p2p_drains(c) || l2l_done == drains_before_l2l(c)) return TFMM_OK;
   TRY(p2p_on_counter(c, ncells, 8 * 4 * c->n_cu, c->stream));
   return TFMM_OK;
 }
@@ -1404,6 +1409,7 @@ int fused_lists(tfmm_ctx *c) {
 
 int fused_numeric(tfmm_ctx *c) {
   hipStream_t s = c->stream;
+  c->l2l_first = false;
   const Cells k = cells_of(c);
   // P2P on the second stream, joined before the downward pass; forked at the
   // start of the phase (schedule 0), at the set kernel (1), or already in
@@ -1449,10 +1455,14 @@ int fused_numeric(tfmm_ctx *c) {
   TRY(rec(c, EV_M2L1, s));
   // downward: the L2L needs no P2P, so the join stands before the L2P
   if ((rc = drain_p2p(c, c->ncells, false))) return rc;
-  if (!cartesian(c))
+  if (!cartesian(c)) {
+    if (drains_before_l2l(c)) TRY(rec(c, EV_L2L0, s));
     for (int d = 0; d + 1 < nl; d++)
       TRY(launch_l2l(k, c->lvl[d + 1], (c->lvl[d + 2] - c->lvl[d + 1]) / 8, dp<double>(c->tops),
                      dp<double>(c->L), s));
+    TRY(rec(c, EV_L2L1, s));
+    c->l2l_first = true;
+  }
   if ((rc = drain_p2p(c, c->ncells, true))) return rc;
   TRY(hipStreamWaitEvent(s, c->ev[EV_P2PJOIN], 0));
   TRY(rec(c, EV_TRAV, s));
@@ -1748,8 +1758,6 @@ int whole_record(tfmm_ctx *c) {
   const int np = c->nprob;
   const bool forest = np > 1;
   const bool mixed = pl.prm.precision == TFMM_MIXED;
-  c->run_schedule = pl.run_schedule;
-  c->run_waves = pl.run_waves;
   const Cells k = cells_of(c);
   const int32_t cells = (int32_t)pl.cells;
   uint32_t *sz = dp<uint32_t>(c->gsz);
@@ -1823,7 +1831,7 @@ int whole_record(tfmm_ctx *c) {
     return TFMM_OK;
   };
   int rc;
-  if (early_upward(c)) {
+  if (c->upward_early) {
     TRY(hipEventRecord(c->ev[EV_P2PREADY], s));
     TRY(hipStreamWaitEvent(c->side, c->ev[EV_P2PREADY], 0));
     if ((rc = upward(c->side))) return rc;
@@ -1914,7 +1922,7 @@ int whole_record(tfmm_ctx *c) {
   TRY(rec(c, EV_DTT1, s));
   // the numeric phase
   if (!early && c->run_schedule != 1 && (rc = fork_p2p(c, cells))) return rc;
-  if (early_upward(c)) TRY(hipStreamWaitEvent(s, c->ev[EV_UPJOIN], 0));
+  if (c->upward_early) TRY(hipStreamWaitEvent(s, c->ev[EV_UPJOIN], 0));
   else if ((rc = upward(s))) return rc;
   TRY(rec(c, EV_M2L0, s));
   if (c->run_schedule == 1 && (rc = fork_p2p(c, cells))) return rc;
@@ -1931,9 +1939,11 @@ int whole_record(tfmm_ctx *c) {
   }
   TRY(rec(c, EV_M2L1, s));
   if ((rc = drain_p2p(c, cells, false))) return rc;
+  if (drains_before_l2l(c)) TRY(rec(c, EV_L2L0, s));
   for (int d = 0; d + 1 < pl.L; d++)
     TRY(launch_l2l(k, 0, pl.grid[d + 1] / 8 + 1, dp<double>(c->tops), dp<double>(c->L), s, lev,
                    d + 1));
+  TRY(rec(c, EV_L2L1, s));
   if ((rc = drain_p2p(c, cells, true))) return rc;
   TRY(hipStreamWaitEvent(s, c->ev[EV_P2PJOIN], 0));
   TRY(rec(c, EV_TRAV, s));
@@ -2024,6 +2034,10 @@ int whole_run(tfmm_ctx *c, const tfmm_params *p) {
   TRY(hipSetDevice(c->device));
   c->prm = *p;
   Plan &pl = c->plan;
+  c->run_schedule = pl.run_schedule;
+  c->run_waves = pl.run_waves;
+  c->upward_early = early_upward(c);
+  c->l2l_first = true;
   if (!pl.exec || pl.signature != buffers_signature(c)) {
     const int rc = whole_capture(c);
     if (rc) return rc;
@@ -2698,10 +2712,13 @@ int tfmm_get_stats(tfmm_ctx *c, tfmm_stats_t *o) {
     return TFMM_OK;
   }
   if (c->fused && c->stage >= 4) {
-    // fused order: traversal and list building, then upward, M2L/P2P, downward
-    // the upward pass may run beside the traversal, on the second stream
+    // fused order: traversal and list building, then upward, M2L/P2P, downward.  The
+    // upward pass may run beside the traversal, on the second stream; on this one it
+    // stands inside it.  So does the L2L, before the P2P's join.
     o->ms_upward = el(EV_UP0, EV_UP);
-    o->ms_traverse = el(EV_DTT0, EV_TRAV);
+    o->ms_traverse = el(EV_DTT0, EV_TRAV) - (c->upward_early ? 0.0 : o->ms_upward);
+    if (c->l2l_first) o->ms_downward = el(drains_before_l2l(c) ? EV_L2L0 : EV_M2L1, EV_L2L1);
+    o->ms_traverse -= o->ms_downward;
   } else {
     if (c->stage >= 2) o->ms_upward = el(EV_TREE, EV_UP);
     if (c->stage >= 3) o->ms_traverse = el(EV_UP, EV_TRAV);
@@ -2713,7 +2730,7 @@ int tfmm_get_stats(tfmm_ctx *c, tfmm_stats_t *o) {
     o->ms_p2p = el(EV_P2P0, EV_P2P1);
   }
   if (c->stage >= 4) {
-    o->ms_downward = el(EV_TRAV, EV_DOWN);
+    o->ms_downward += el(EV_TRAV, EV_DOWN);
     o->ms_total = el(EV_BEGIN, EV_DOWN);
   }
   return TFMM_OK;
