@@ -252,9 +252,9 @@ int tfmm_get_lists(tfmm_ctx *ctx, int32_t *m2l_off, int32_t *m2l_src, int32_t *p
 /* Tuning knobs of the kernels (no counterpart in the reference; results do
  * not depend on them beyond the summation order).
  * TFMM_TUNE_M2L_UNIT: the batched M2L kernel runs each set of 16 target cells
- * as work units of at most factor x (mean items per set) items, so that a
- * few heavy sets do not hold the launch back; 0 = a size from the number of
- * items. */
+ * as work units of at most factor x (mean items per set) items, and no
+ * fewer than 8, so that a few heavy sets do not hold the launch back; 0 = a
+ * size from the number of items. */
 #define TFMM_TUNE_M2L_UNIT 1
 /* TFMM_TUNE_M2L_XCD_RUN: groups of 8 consecutive work units dealt to one of
  * the 8 XCDs (each has its own L2; neighbouring sets share source
@@ -330,9 +330,8 @@ int tfmm_get_tuning(tfmm_ctx *ctx, int knob, double *value);
  * candidate (after 2 uncounted evaluations of the candidate, which let the
  * device settle to the setting), in two stages -- the set-kernel knobs (unit factor {0, 1.5,
  * 2, 3} x XCD run {8, 16, 32, 64}) at the current P2P setting, then the
- * P2P's schedule (0 without waves: as TFMM_TUNE_P2P_CHOICE is set) {0, 1, 2} x resident waves {0, 3, 4} (waves for mixed
- * precision only, schedule 2 not with TFMM_TUNE_GRAPH 1) at the best tile
- * setting --
+ * P2P's schedule (0 without waves: as TFMM_TUNE_P2P_CHOICE is set) {0, 1, 2} x resident waves {0, 3, 4} (schedule
+ * 2 not with TFMM_TUNE_GRAPH 1) at the best set-kernel setting --
  * and keeps the setting whose evaluation was fastest (median).  chosen (4
  * doubles, may be null): unit factor, XCD run, P2P schedule, milliseconds
  * per evaluation; the P2P waves chosen stay set (tfmm_get_tuning). */

@@ -346,7 +346,6 @@ int cart_tables(tfmm_ctx *c) {
   return TFMM_OK;
 }
 
-// waves that share a target leaf of the P2P
 // Resident waves take the leaves of at least the average's work (bodies times source
 // leaves, by the last traversal) first, or a long one that is taken late is the end
 // of the evaluation.  Evaluations, ms, in the cells' order / from 1, 2, 3, 5 times
@@ -359,6 +358,7 @@ P2pQueue p2p_queue(tfmm_ctx *c) {
           (float)(c->n / leaves * (c->n_p2p / leaves))};
 }
 
+// waves that share a target leaf of the P2P
 int leaf_waves(const tfmm_ctx *c) { return p2p_waves_per_leaf(c->n, c->prm.ncrit); }
 
 // the direct sum's image range for the image sublevels (the reference's
@@ -616,7 +616,7 @@ int cart_lists(tfmm_ctx *c) {
 }
 
 // The set kernel's route: its spherical locals (L) into the Cartesian ones.
-hipError_t cart_from_tiles(tfmm_ctx *c) {
+hipError_t cart_from_sets(tfmm_ctx *c) {
   if (!cartesian(c) || c->cart_direct) return hipSuccess;
   return launch_sph_to_cart((int32_t)c->ncells, dp<double>(c->L), dp<double>(c->Lc),
                             c->cart_tab.ptr, c->stream);
@@ -1033,7 +1033,7 @@ int run_lists(tfmm_ctx *c) {
                         dp<double>(c->L), c->fb_part.ptr, s, nullptr, period(c)));
   }
   TRY(launch_periodic_far(dp<double>(c->M), dp<double>(c->L), c->cycle, c->images, s));
-  TRY(cart_from_tiles(c));
+  TRY(cart_from_sets(c));
   TRY(hipEventRecord(c->ev[EV_M2L1], s));
 
   TRY(hipStreamWaitEvent(s, c->ev[EV_P2P1], 0));
@@ -1451,7 +1451,7 @@ int fused_numeric(tfmm_ctx *c) {
                         dp<double>(c->L), c->fb_part.ptr, s, nullptr, period(c)));
   }
   TRY(launch_periodic_far(dp<double>(c->M), dp<double>(c->L), c->cycle, c->images, s));
-  TRY(cart_from_tiles(c));
+  TRY(cart_from_sets(c));
   TRY(rec(c, EV_M2L1, s));
   // downward: the L2L needs no P2P, so the join stands before the L2P
   if ((rc = drain_p2p(c, c->ncells, false))) return rc;
@@ -1768,7 +1768,8 @@ int whole_record(tfmm_ctx *c) {
   const int key_end = DEPTHBITS + 3 * MAXDEPTH;
   const int64_t *off = forest ? dp<int64_t>(c->d_prob_off) : nullptr;
   if (forest) {
-    TRY(launch_bbox_forest(c->bx, c->by, c->bz, c->bq, off, np, region, dp<BodyRange>(c->range), s));
+    TRY(launch_bbox_forest(c->bx, c->by, c->bz, c->bq, off, np, region,
+                           dp<BodyRange>(c->range), s));
   } else {
     const int nparts = (int)std::min<int64_t>(1024, (n + 255) / 256);
     TRY(launch_bbox(c->bx, c->by, c->bz, c->bq, n, c->bbox_part.ptr, nparts, region,
@@ -2242,11 +2243,6 @@ int tfmm_set_tuning(tfmm_ctx *c, int knob, double value) {
   }
 }
 
-// Candidates of the set-kernel knobs, tried jointly; the evaluation's time
-// (HIP events around it) decides, median over the repetitions.  The P2P
-// schedule stays as set: running the P2P beside the M2L measured within
-// noise of running it beside the batch building, and it would fold the
-// P2P's time into the set kernel's.
 // Candidates of the kernel knobs, timed in two stages: the set kernel's
 // (unit factor x XCD run) at the current P2P setting, then where the P2P
 // starts and how many resident waves it holds, at the best set-kernel setting

@@ -591,13 +591,14 @@ struct SetRegs {
 // same group: holding all 61 for as long as a group lasts took 225 registers (446
 // in FP64) instead of 128 (217), two waves a SIMD instead of four (one instead of
 // two).  Alone, us, then and now (the shortest units last, see k_unit_map,
-// included): 4M Plummer 2,830 and 2,610, 256 x 16K 3,020 and 2,820, 1M cube FP64
+// included): 4M Plummer 2,830 and 2,610, 256 problems 3,020 and 2,820, 1M cube FP64
 // 1,420 and 1,255, 500K ellipsoid FP64 1,770 and 1,700.
 // Every row block's products are summed from zero over the item and then added
 // to the target's sums: long chains into the sums themselves would lose more to
 // rounding in FP32 (relative 1.2e-6 between two groupings of one problem's
 // pairs, against 6e-7).  They are added four steps after their last one (an
-// MFMA's results take a while to arrive), one result a step.  bs, ss: signs of b and of the products.
+// MFMA's results take a while to arrive), one result a step.  bs, ss: signs of b and
+// of the products.
 template <class T, int S>
 __device__ inline void set_step(SetRegs<T> &r, typename Mfma<T>::V (&p)[NRB], uint32_t bs,
                                 uint32_t ss, const T *next, const T *af, const T *afn) {

@@ -20,7 +20,7 @@
 // supplies at k-step kk of block b is the sum of two table elements whose
 // byte offsets are packed into one 32-bit code (low 16 bits, high 16 bits).
 // Absent terms point at element 110, a zero.  The batched M2L forms every
-// group's A operands from these codes once, before the tile kernel.
+// group's A operands from these codes once, before the set kernel.
 #pragma once
 #include <stddef.h>
 #include <stdint.h>

@@ -177,10 +177,11 @@ __device__ inline double4 scaled(double4 v, double up) {
 // every lane; see p2p_leaf.
 template <typename T, int RING, int W, bool WIDE, bool TWO>
 __device__ __forceinline__ void p2p_pass(const Cells &c, const Csr &list, const Bodies &b,
-                                const float4 *rel, double *acc, typename Vec4<T>::type *ring,
-                                int32_t tb, int32_t lb, int32_t le, double tcx, double tcy,
-                                double tcz, double cycle, T tiny, int scale, int G,
-                                int32_t t, int32_t t2, bool tvalid, bool tvalid2) {
+                                         const float4 *rel, double *acc,
+                                         typename Vec4<T>::type *ring, int32_t tb, int32_t lb,
+                                         int32_t le, double tcx, double tcy, double tcz,
+                                         double cycle, T tiny, int scale, int G, int32_t t,
+                                         int32_t t2, bool tvalid, bool tvalid2) {
   using V4 = typename Vec4<T>::type;
   constexpr bool MIX = sizeof(T) == 4;
   const int lane = W == 1 ? threadIdx.x : threadIdx.x & 63;
@@ -351,9 +352,9 @@ __device__ __forceinline__ void p2p_pass(const Cells &c, const Csr &list, const 
 // ring: W times RING + RING / 16 entries of LDS; each wave's also holds its lane
 // partials at the end of every pass.  scale: of the coordinates (FP64, p2p_frame).
 template <typename T, int RING, int W, bool WIDE>
-__device__ __forceinline__ void p2p_leaf(int32_t ti, const Cells &c, const Csr &list, const Bodies &b,
-                                const float4 *rel, double *acc, typename Vec4<T>::type *ring,
-                                double cycle, int scale) {
+__device__ __forceinline__ void p2p_leaf(int32_t ti, const Cells &c, const Csr &list,
+                                         const Bodies &b, const float4 *rel, double *acc,
+                                         typename Vec4<T>::type *ring, double cycle, int scale) {
   constexpr bool MIX = sizeof(T) == 4;
   constexpr int GMAX = RING / (2 * SEG);  // a chunk (16 G) plus a 64-body piece fit the ring
   if (c.child[ti] >= 0) return;
@@ -385,11 +386,11 @@ __device__ __forceinline__ void p2p_leaf(int32_t ti, const Cells &c, const Csr &
     const int32_t t = t0 + tloc, t2 = t + tpp;
     const bool tvalid = tloc < tpp && t < nt, tvalid2 = tloc < tpp && t2 < nt;
     if (t0 + tpp < nt)
-      p2p_pass<T, RING, W, WIDE, true>(c, list, b, rel, acc, ring, tb, lb, le, tcx, tcy, tcz, cycle,
-                                       tiny, scale, G, t, t2, tvalid, tvalid2);
+      p2p_pass<T, RING, W, WIDE, true>(c, list, b, rel, acc, ring, tb, lb, le, tcx, tcy, tcz,
+                                       cycle, tiny, scale, G, t, t2, tvalid, tvalid2);
     else
-      p2p_pass<T, RING, W, WIDE, false>(c, list, b, rel, acc, ring, tb, lb, le, tcx, tcy, tcz, cycle,
-                                        tiny, scale, G, t, t2, tvalid, false);
+      p2p_pass<T, RING, W, WIDE, false>(c, list, b, rel, acc, ring, tb, lb, le, tcx, tcy, tcz,
+                                        cycle, tiny, scale, G, t, t2, tvalid, false);
   }
 }
 
@@ -397,8 +398,9 @@ constexpr int RING32 = 256;  // float4 entries: 4.25 KB with the pads
 constexpr int RING64 = 128;  // double4 entries: 4.25 KB with the pads
 
 template <int W>
-__device__ __forceinline__ void p2p_leaf_fp64(int32_t ti, const Cells &c, const Csr &list, const Bodies &b,
-                                     double *acc, double4 *ring, double cycle, P2pFrame f) {
+__device__ __forceinline__ void p2p_leaf_fp64(int32_t ti, const Cells &c, const Csr &list,
+                                              const Bodies &b, double *acc, double4 *ring,
+                                              double cycle, P2pFrame f) {
   if (f.wide)
     p2p_leaf<double, RING64, W, true>(ti, c, list, b, nullptr, acc, ring, cycle, 0);
   else
@@ -548,10 +550,11 @@ void k_p2p_fp32(Cells c, Csr list, Bodies b, const float4 *rel, double *acc, dou
 // bounded share of the CUs, and kernels on the other stream still find
 // slots.  Each target is computed by one wave exactly as above, so the order
 // in which the waves take them does not change any result.  80 registers (3
-// spilled, outside the pair loop) and not the 94 of a free choice: the M2L set
-// kernel takes 232 of a SIMD's 512, which three waves of 94 would not leave, and
-// the M2L then ran mostly after the P2P (two clusters of 4M bodies 21.9 ms an
-// evaluation against 20.4, one cluster 12.2 against 11.5).
+// spilled with one wave a leaf, 6 with more, outside the pair loop) and not the 94 of
+// a free choice, so that two waves of the M2L set kernel (128 registers) find room on
+// a SIMD of 512 beside three: with 94, and the 232 that kernel then took, the M2L ran
+// mostly after the P2P (two clusters of 4M bodies 21.9 ms an evaluation against 20.4,
+// one cluster 12.2 against 11.5).
 template <int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(6, 8)))
 void k_p2p_fp32_resident(Cells c, int32_t ncells, Csr list, Bodies b, const float4 *rel,

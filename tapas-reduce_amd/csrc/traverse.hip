@@ -517,7 +517,8 @@ hipError_t launch_dtt_step(const int2 *in, const uint32_t *nin_dev, uint32_t nin
   // 444, 4M Plummer 553, 555, 591.  With the eight successors of a split written out,
   // flags stored pair by pair and depths and widths gathered by the pairs in the
   // group table: 484, 586 and 1,673.  64 registers, two workgroups a CU instead of
-  // one, are worth 15 % on the largest steps, spills included.
+  // one, are worth 15 % on the largest steps, spills included (43 vector and 10 scalar
+  // registers with four pairs, 16 vector ones with one).
   auto go = [&](auto kernel, uint32_t ppt) {
     const uint32_t per = DTT_THREADS / 8 * ppt;  // entries
     kernel<<<(nin_max + per - 1) / per, DTT_THREADS, 0, s>>>(
