@@ -277,12 +277,14 @@ def errors(ctx, targets, direct):
 
 
 def kernels(st, phases, precision, workload, basis="spherical", cart_direct=False,
-            resident=False):
+            p2p_start=(0, 0)):
     """Achieved rates of the P2P kernel (20 flops per evaluated body pair)
     and the M2L set kernel (9,680 flops per grouped pair; the Cartesian
     basis's direct kernel k_cart_m2l: CART_M2L_FLOPS_PER_PAIR per pair, FP64
-    vector) over their HIP-event times on the streams they run on."""
+    vector) over their HIP-event times on the streams they run on.  p2p_start: the
+    schedule and resident waves that the evaluation ran the P2P with."""
     import tfmm
+    resident = p2p_start[1] > 0
     mixed = precision == tfmm.MIXED
     pairs = st["n_p2p_calls"] - st["n_p2p_self"]
     p2p_ms = phases["ms_p2p"]
@@ -437,6 +439,7 @@ def bench_single(args, dist, n, precision, use_picker, steps, warmup, fp64_steps
         targets = np.sort(rng.choice(n, size=min(args.targets, n), replace=False))
         direct = ctx.direct(targets)
         ms, phases, st = time_config(ctx, prm, steps, warmup)
+        p2p_start = ctx.p2p_start()
         ep, ea = errors(ctx, targets, direct)
         prec_name = "fp64" if precision == tfmm.FP64 else "mixed"
         workload = "%s N=%d P=10 ncrit=%d theta=%g %s%s%s" % (
@@ -449,8 +452,7 @@ def bench_single(args, dist, n, precision, use_picker, steps, warmup, fp64_steps
                          "against": "FP64 direct sum"},
                "picker": picked, "autotune": tuned, "phases_ms": phases, "counts": counts(st),
                "roofline": kernels(st, phases, precision, workload, args.basis,
-                                   cart and args.cart_m2l == 1,
-                                   ctx.get_tuning(tfmm.TUNE_P2P_WAVES) > 0),
+                                   cart and args.cart_m2l == 1, p2p_start),
                "basis": args.basis}
         if not args.graph and not cart:
             out["one_graph"] = one_graph(ctx, prm, steps, n)
@@ -471,7 +473,8 @@ def bench_single(args, dist, n, precision, use_picker, steps, warmup, fp64_steps
                                  "ncrit": args.ncrit or 64, "theta": args.theta,
                                  "rel_l2_pot": e64[0], "rel_l2_acc": e64[1],
                                  "phases_ms": ph64,
-                                 "roofline": kernels(st64, ph64, tfmm.FP64, None),
+                                 "roofline": kernels(st64, ph64, tfmm.FP64, None,
+                                                     p2p_start=ctx.p2p_start()),
                                  "speedup_of_headline": ms64 / ms}
         return out
     finally:
@@ -517,6 +520,7 @@ def bench_batch(args, nprob, precision, steps, warmup):
         targets = np.sort(rng.choice(n, size=min(args.targets, n), replace=False))
         direct = ctx.direct(targets)  # per problem: a target sees only its own problem
         ms, phases, st = time_config(ctx, prm, steps, warmup)
+        p2p_start = ctx.p2p_start()
         ep, ea = errors(ctx, targets, direct)
         graph_run = None if args.graph else one_graph(ctx, prm, steps, n)
         prec_name = "fp64" if precision == tfmm.FP64 else "mixed"
@@ -530,8 +534,7 @@ def bench_batch(args, nprob, precision, steps, warmup):
                 "error": {"rel_l2_pot": ep, "rel_l2_acc": ea, "targets": len(targets),
                           "against": "FP64 direct sum within each problem"},
                 "picker": picked, "autotune": tuned, "phases_ms": phases, "counts": counts(st),
-                "roofline": kernels(st, phases, precision, workload, resident=ctx.get_tuning(
-                    tfmm.TUNE_P2P_WAVES) > 0),
+                "roofline": kernels(st, phases, precision, workload, p2p_start=p2p_start),
                 "one_graph": graph_run}, probs
     finally:
         ctx.close()

@@ -101,10 +101,12 @@ typedef struct {
   uint64_t n_p2p_self;       /* r == 0 self pairs among them */
   /* milliseconds of the last evaluation, measured with HIP events on the
    * context stream; kernel entries are summed over their launches.
-   * ms_traverse: the traversal, the lists, the M2L and the wait for the P2P;
-   * ms_downward: L2L and L2P, wherever the L2L stands.  In tfmm_evaluate the
-   * upward pass may run on the second stream, beside the traversal: the
-   * phases then add up to more than ms_total. */
+   * ms_p2p: to the end of the launch that starts the P2P (as resident waves,
+   * a drain may end a little later).  ms_traverse: the traversal, the lists,
+   * the M2L and the wait for the P2P; ms_downward: L2L and L2P, wherever the
+   * L2L stands.  In tfmm_evaluate the upward pass may run on the second
+   * stream, beside the traversal: the phases then add up to more than
+   * ms_total. */
   double ms_tree, ms_upward, ms_traverse, ms_downward, ms_total;
   double ms_p2p, ms_m2l, ms_dtt;
   /* M2L batching: offset groups (offsets up to mirroring), MFMA work items
@@ -326,6 +328,10 @@ int tfmm_get_lists(tfmm_ctx *ctx, int32_t *m2l_off, int32_t *m2l_src, int32_t *p
 #define TFMM_TUNE_P2P_CHOICE 8
 int tfmm_set_tuning(tfmm_ctx *ctx, int knob, double value);
 int tfmm_get_tuning(tfmm_ctx *ctx, int knob, double *value);
+/* Where the P2P of the last evaluation started (a TFMM_TUNE_P2P_SCHEDULE) and as
+ * how many resident waves per SIMD it ran (0: one workgroup per cell), as set or
+ * as the library chose; either may be null. */
+int tfmm_get_p2p_start(tfmm_ctx *ctx, int *schedule, int *waves);
 /* Autotuner: evaluates the current bodies with params, reps times per
  * candidate (after 2 uncounted evaluations of the candidate, which let the
  * device settle to the setting), in two stages -- the set-kernel knobs (unit factor {0, 1.5,

@@ -2368,6 +2368,14 @@ int tfmm_get_tuning(tfmm_ctx *c, int knob, double *value) {
   }
 }
 
+int tfmm_get_p2p_start(tfmm_ctx *c, int *schedule, int *waves) {
+  const int rc = need_stage(c, 4, "tfmm_get_p2p_start");
+  if (rc) return rc;
+  if (schedule) *schedule = c->fused ? c->run_schedule : c->p2p_schedule;
+  if (waves) *waves = c->fused ? c->run_waves : c->p2p_waves;
+  return TFMM_OK;
+}
+
 void *tfmm_stream(tfmm_ctx *c) { return c ? (void *)c->stream : nullptr; }
 
 int tfmm_sync(tfmm_ctx *c) {

@@ -77,7 +77,7 @@ EXPORTED = [
     "tfmm_create", "tfmm_destroy", "tfmm_last_error", "tfmm_stream", "tfmm_sync",
     "tfmm_set_bodies", "tfmm_set_bodies_device", "tfmm_set_batch", "tfmm_set_batch_device",
     "tfmm_batch_evaluate", "tfmm_num_problems", "tfmm_set_tuning", "tfmm_get_tuning",
-    "tfmm_autotune",
+    "tfmm_autotune", "tfmm_get_p2p_start",
     "tfmm_build_tree", "tfmm_set_params",
     "tfmm_upward",
     "tfmm_traverse", "tfmm_downward", "tfmm_evaluate", "tfmm_get_fields", "tfmm_get_stats",
@@ -123,6 +123,8 @@ def lib():
         L.tfmm_get_basis.argtypes = [vp, ctypes.POINTER(ctypes.c_int)]
         L.tfmm_get_tuning.argtypes = [vp, ctypes.c_int, ctypes.POINTER(ctypes.c_double)]
         L.tfmm_autotune.argtypes = [vp, ctypes.POINTER(Params), ctypes.c_int, vp]
+        L.tfmm_get_p2p_start.argtypes = [vp, ctypes.POINTER(ctypes.c_int),
+                                         ctypes.POINTER(ctypes.c_int)]
         L.tfmm_build_tree.argtypes = [vp, ctypes.POINTER(Params)]
         L.tfmm_evaluate.argtypes = [vp, ctypes.POINTER(Params)]
         L.tfmm_set_params.argtypes = [vp, ctypes.POINTER(Params)]
@@ -275,6 +277,14 @@ class Context:
         v = ctypes.c_double()
         self._check(lib().tfmm_get_tuning(self._h, int(knob), ctypes.byref(v)), "tfmm_get_tuning")
         return v.value
+
+    def p2p_start(self):
+        """(schedule, resident waves) of the last evaluation's P2P, as set or as
+        the library chose"""
+        sched, waves = ctypes.c_int(), ctypes.c_int()
+        self._check(lib().tfmm_get_p2p_start(self._h, ctypes.byref(sched), ctypes.byref(waves)),
+                    "tfmm_get_p2p_start")
+        return sched.value, waves.value
 
     def autotune(self, params, reps=3):
         """Pick the kernel knobs for these bodies; returns (unit factor, XCD
